@@ -1,5 +1,5 @@
 // Multi-head self attention with Laplacian:  o = softmax(q k^T) v  and its Jacobian rows
-// and Laplacian, one workgroup per (walker, head).
+// and Laplacian, one workgroup per (walker, head): mhsa_small_kernel for n <= 16 (its mapping stands there), mhsa_kernel beyond.
 //
 // Algebra per Jacobian row c (the factored form of the rule):
 //   s'_c = q'_c k^T + q k'_c^T          p'_c = p * (s'_c - rowsum(p * s'_c))
@@ -11,7 +11,7 @@
 // bias e (s = q k^T + e) the rows e'_c and lap_e are added to s'_c and to the Laplacian's
 // first-order part; they have no second-order contribution.
 //
-// Mapping: wavefront w owns query rows [16 w, 16 w + 16) and every key column, so all
+// Mapping of mhsa_kernel: wavefront w owns query rows [16 w, 16 w + 16) and every key column, so all
 // row reductions stay inside 16-lane groups of one wavefront.  k, v and the current
 // k'_c, v'_c tiles are shared through LDS (the next pair waits in registers; a single LDS
 // copy keeps the workgroup under 40 KB, so four workgroups share a CU); q, q'_c and p live in
@@ -25,14 +25,24 @@ namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
+// Sum and maximum over the 16 lanes of a row, by DPP: quad permutes (lane ^ 1, lane ^ 2), then the two mirrors, which
+// meet equal values in every quad (half of 8) by then.  Vector instructions only, where a shuffle is a trip through LDS.
+template <int CTRL>
+__device__ __forceinline__ float dpp16(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float sum16(float v) {
-  v += __shfl_xor(v, 1, FOLX_WAVE); v += __shfl_xor(v, 2, FOLX_WAVE);
-  v += __shfl_xor(v, 4, FOLX_WAVE); v += __shfl_xor(v, 8, FOLX_WAVE);
+  v += dpp16<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  v += dpp16<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp16<0x141>(v);  // row_half_mirror
+  v += dpp16<0x140>(v);  // row_mirror
   return v;
 }
 __device__ __forceinline__ float max16(float v) {
-  v = fmaxf(v, __shfl_xor(v, 1, FOLX_WAVE)); v = fmaxf(v, __shfl_xor(v, 2, FOLX_WAVE));
-  v = fmaxf(v, __shfl_xor(v, 4, FOLX_WAVE)); v = fmaxf(v, __shfl_xor(v, 8, FOLX_WAVE));
+  v = fmaxf(v, dpp16<0xB1>(v));
+  v = fmaxf(v, dpp16<0x4E>(v));
+  v = fmaxf(v, dpp16<0x141>(v));
+  v = fmaxf(v, dpp16<0x140>(v));
   return v;
 }
 __device__ __forceinline__ float f4get(const float4& v, int r) {
@@ -376,6 +386,358 @@ __global__ __launch_bounds__(FOLX_WAVE * NW) void mhsa_kernel(MhsaArgs a) {
   out_store(a.ol, OL);
 }
 
+// n <= 16: one wavefront covers all query rows of a (walker, head) pair, so its rows c need nothing from its neighbours:
+// q'_c, k'_c and v'_c go from memory straight into MFMA operand registers and the W wavefronts of a workgroup take the rows
+// c = w, w + W, ... with every sum over rows in registers, added through LDS once at the end (k and v wait in LDS, the same
+// for all of them: 168 registers, twelve wavefronts on a CU).  Rows and columns of the padding are lanes whose buffer offset
+// lies past the descriptor's end: they read zeros and their stores are dropped, so no access is tested.  DT = 1, 2 or 4
+// blocks of 16 features.
+// Bound by HBM (16 n d bytes per pair and row, at 4.7-5.1 TB/s), for few pairs by the latency of a wavefront's rows.  One
+// wavefront per pair with the tiles of mhsa_kernel (two barriers and an LDS copy of k', v' per row) was bound by that chain:
+// 1200 pairs of 13 x 64, P = 39: 300 -> 139 us; 256 of 10 x 64, P = 30: 112 -> 24 us; 2048 of 16 x 16, P = 48: 146 -> 94 us;
+// 16000 of 16 x 64, P = 48: 2.69 -> 2.56 ms.
+constexpr int NXCD = 8;
+constexpr uint32_t FAR = 0x40000000u;  // past every descriptor's end, also with the row and piece offsets added
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+
+template <int DT, bool EDGE, bool MASKED>
+__global__ __launch_bounds__(512, 3) void mhsa_small_kernel(MhsaArgs a) {
+  constexpr float BIG = 1e20f;
+  constexpr int NS = 20;           // LDS row stride of a 16 x 16 tile
+  constexpr int NRED = 12 + 4 * DT;
+  const int W = blockDim.x / FOLX_WAVE;
+  constexpr int KS = 16 * DT + 4;  // row stride of the copies of k and v (the same for every wavefront; read once per row)
+  extern __shared__ __attribute__((aligned(16))) float lds[];  // [W][16 NS] tiles, later [W - 1][NRED][64] sums
+  __shared__ __attribute__((aligned(16))) float ksh[16 * KS];
+  __shared__ __attribute__((aligned(16))) float vsh[16 * KS];
+
+  const int lane = threadIdx.x % FOLX_WAVE;
+  const int w = folx_wave_id();
+  const int l16 = lane % 16;
+  const int lg = lane / 16;
+  // ids are dealt round-robin to the XCDs: consecutive pairs (the heads of a walker share cache lines when d < 32) go to one
+  const int64_t pairs = a.B * a.H, per = (pairs + NXCD - 1) / NXCD;
+  const int64_t pair = (int64_t)(blockIdx.x % NXCD) * per + blockIdx.x / NXCD;
+  if (pair >= pairs) return;
+  const int64_t b = pair / a.H;
+  const int h = (int)(pair % a.H);
+  const int n = a.n, d = a.d, H = a.H, P = a.P;
+  const int64_t B = a.B;
+  const int32_t tok = H * d;
+  const int64_t base = (b * n) * tok + (int64_t)h * d;
+  const int64_t slice = B * n * tok;
+  const uint32_t bytes = (uint32_t)(((int64_t)n * tok - (int64_t)h * d) * 4);  // from (b, 0, h, 0) to the walker's end
+
+  auto rsrc = [&](const float* p) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p) + base, 0, bytes, 0x00027000);
+  };
+  auto valid = [&](int i) __attribute__((always_inline)) -> bool {
+    return i < n && (!MASKED || a.mask == nullptr || a.mask[b * n + i] != 0);
+  };
+  // byte offsets of this lane: row l16, piece 4 lg of 16 t (A / k layout); rows 4 lg + r, columns DT l16 .. + DT - 1 (v and
+  // result: column l16 of block dt stands for DT l16 + dt, so that a lane's DT columns are one access)
+  uint32_t ao[DT], vo[4], aoj[DT], voj[4];  // ..j: rows of masked inputs read zeros as well
+  const bool arow = valid(l16);
+#pragma unroll
+  for (int t = 0; t < DT; ++t) {
+    const bool in = l16 < n && 16 * t + 4 * lg < d;
+    ao[t] = in ? (uint32_t)(l16 * tok + 16 * t + 4 * lg) * 4u : FAR;
+    aoj[t] = MASKED && !arow ? FAR : ao[t];
+  }
+  bool rvalid[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = 4 * lg + r;
+    rvalid[r] = valid(row);
+    vo[r] = row < n && DT * l16 < d ? (uint32_t)(row * tok + DT * l16) * 4u : FAR;
+    voj[r] = MASKED && !rvalid[r] ? FAR : vo[r];
+  }
+  auto load_rows = [&](const float* src, const uint32_t (&off)[DT], float4 (&reg)[DT]) __attribute__((always_inline)) {
+    const auto rs = rsrc(src);
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+      reg[t] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, off[t], 0, 0));
+  };
+  auto load_v = [&](const float* src, const uint32_t (&off)[4], float (&reg)[DT][4]) __attribute__((always_inline)) {
+    const auto rs = rsrc(src);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (DT == 4) {
+        const uintx4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, off[r], 0, 0);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) reg[dt][r] = __uint_as_float(v[dt]);
+      } else if constexpr (DT == 2) {
+        const uintx2 v = __builtin_amdgcn_raw_buffer_load_b64(rs, off[r], 0, 0);
+        reg[0][r] = __uint_as_float(v[0]);
+        reg[1][r] = __uint_as_float(v[1]);
+      } else {
+        reg[0][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off[r], 0, 0));
+      }
+    }
+  };
+  auto store = [&](float* dst, const floatx4 (&c)[DT]) __attribute__((always_inline)) {
+    const auto rs = rsrc(dst);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      unsigned x[DT];
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const float v = c[dt][r];
+        x[dt] = __float_as_uint(v);
+      }
+      if constexpr (DT == 4) {
+        uintx4 v;
+        v[0] = x[0]; v[1] = x[1]; v[2] = x[2]; v[3] = x[3];
+        __builtin_amdgcn_raw_buffer_store_b128(v, rs, vo[r], 0, 2);
+      } else if constexpr (DT == 2) {
+        uintx2 v;
+        v[0] = x[0]; v[1] = x[1];
+        __builtin_amdgcn_raw_buffer_store_b64(v, rs, vo[r], 0, 2);
+      } else {
+        __builtin_amdgcn_raw_buffer_store_b32(x[0], rs, vo[r], 0, 2);
+      }
+    }
+  };
+  const int64_t etok = (int64_t)H * n, ebase = (b * n) * etok + (int64_t)h * n, eslice = B * n * etok;
+  auto edge_add = [&](const float* src, floatx4& acc) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (4 * lg + r < n && l16 < n) acc[r] += src[ebase + (int64_t)(4 * lg + r) * etok + l16];
+  };
+  auto qk = [&](const float4 (&x)[DT], const float4 (&y)[DT], floatx4& acc) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(f4get(x[t], r), f4get(y[t], r), acc, 0, 0, 0);
+  };
+  auto pv = [&](const float4& p, const float (&y)[DT][4], floatx4 (&acc)[DT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4get(p, r), y[dt][r], acc[dt], 0, 0, 0);
+  };
+  float* st = lds + w * 16 * NS;
+  auto to_a = [&](const floatx4& c) __attribute__((always_inline)) -> float4 {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) st[(4 * lg + r) * NS + l16] = c[r];
+    // private to this wavefront, whose LDS accesses complete in issue order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const float4 v = *reinterpret_cast<const float4*>(&st[l16 * NS + 4 * lg]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return v;
+  };
+
+  // pass c < P: Jacobian row c; pass c == P: the Laplacians take the place of the row
+  auto active = [&](int c) __attribute__((always_inline)) -> bool {
+    return !MASKED || c == P || a.imask == nullptr || a.imask[(int64_t)c * B + b] != 0;
+  };
+  auto src_of = [&](const float* jac, const float* lap, int c) __attribute__((always_inline)) -> const float* {
+    return c == P ? lap : jac + (int64_t)c * slice;
+  };
+  // The next row's q', k' are asked for as soon as the products that read this row's are issued, and its v' behind the
+  // other three: half a row of matrix work ahead in the same registers, the rest of the latency is other wavefronts' time.
+  float4 qj[DT], kj[DT];
+  float vj[DT][4];
+  auto fetch_qk = [&](int c) __attribute__((always_inline)) {
+    load_rows(src_of(a.qj, a.ql, c), aoj, qj);
+    load_rows(src_of(a.kj, a.kl, c), aoj, kj);
+  };
+  auto fetch_v = [&](int c) __attribute__((always_inline)) { load_v(src_of(a.vj, a.vl, c), voj, vj); };
+
+  float4 qa[DT];
+  load_rows(a.q, ao, qa);
+  if (w == 0) {
+    float4 kr[DT];
+    float vr[DT][4];
+    load_rows(a.k, ao, kr);
+    load_v(a.v, vo, vr);
+#pragma unroll
+    for (int t = 0; t < DT; ++t) *reinterpret_cast<float4*>(&ksh[l16 * KS + 16 * t + 4 * lg]) = kr[t];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) vsh[(4 * lg + r) * KS + DT * l16 + dt] = vr[dt][r];
+  }
+  auto k_rows = [&](float4 (&kb)[DT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < DT; ++t) kb[t] = *reinterpret_cast<const float4*>(&ksh[l16 * KS + 16 * t + 4 * lg]);
+  };
+  auto v_rows = [&](float (&vb)[DT][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float* p = &vsh[(4 * lg + r) * KS + DT * l16];
+      if constexpr (DT == 4) {
+        const float4 x = *reinterpret_cast<const float4*>(p);
+        vb[0][r] = x.x; vb[1][r] = x.y; vb[2][r] = x.z; vb[3][r] = x.w;
+      } else {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) vb[dt][r] = p[dt];
+      }
+    }
+  };
+  if (w <= P && active(w)) {
+    fetch_qk(w);
+    fetch_v(w);
+  }
+
+  const bool cexist = l16 < n, cvalid = arow;
+  floatx4 pc = floatx4{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+  {
+    float4 kb[DT];
+    k_rows(kb);
+    qk(qa, kb, pc);
+  }
+  if constexpr (EDGE) edge_add(a.e, pc);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float sv = pc[r];
+    if (!cexist) sv = -INFINITY;
+    else if (!(rvalid[r] && cvalid)) sv = -BIG;
+    const float mx = max16(sv);
+    const float e = cexist ? expf(sv - mx) : 0.0f;
+    pc[r] = e * (1.0f / sum16(e));
+  }
+  const float4 pa = to_a(pc);
+  if (w == 0) {
+    floatx4 oc[DT];
+    float vb[DT][4];
+    v_rows(vb);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) oc[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    pv(pa, vb, oc);
+    store(a.o, oc);
+  }
+
+  floatx4 G = floatx4{0.f, 0.f, 0.f, 0.f}, X = G, O2[DT], OL[DT];
+  float u[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) { O2[dt] = G; OL[dt] = G; }
+  for (int c = w; c <= P; c += W) {
+    const bool act = active(c), next = c + W <= P && active(c + W);
+    floatx4 oj[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) oj[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (act) {
+      const bool is_lap = c == P;
+      floatx4 sj = floatx4{0.f, 0.f, 0.f, 0.f};
+      {
+        float4 kb[DT];
+        k_rows(kb);
+        qk(qj, kb, sj);
+      }
+      qk(qa, kj, sj);
+      if (!is_lap) qk(qj, kj, G);
+      if (next) fetch_qk(c + W);
+      if constexpr (EDGE) edge_add(is_lap ? a.el : a.ej + (int64_t)c * eslice, sj);
+      floatx4 pj;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float rs = sum16(pc[r] * sj[r]);
+        const float dlt = sj[r] - rs;
+        pj[r] = pc[r] * dlt;
+        if (!is_lap) {
+          X[r] += pj[r] * dlt;
+          u[r] += pj[r] * sj[r];  // lane-partial; reduced over the 16 lanes at the end
+        }
+      }
+      const float4 pja = to_a(pj);
+      {
+        float vb[DT][4];
+        v_rows(vb);
+        pv(pja, vb, oj);
+      }
+      pv(pa, vj, oj);
+      if (!is_lap) {
+        pv(pja, vj, O2);
+      } else {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) OL[dt] = oj[dt];
+      }
+    } else if (next) {
+      fetch_qk(c + W);
+    }
+    if (next) fetch_v(c + W);
+    if (c < P) store(a.oj + (int64_t)c * slice, oj);  // zeros for an inactive coordinate
+  }
+
+  // sums over rows: wavefronts 1 .. W - 1 leave theirs in LDS, wavefront 0 adds them in order
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) O2[dt][r] = 2.0f * O2[dt][r] + OL[dt][r];
+  __syncthreads();
+  if (w > 0) {
+    float* o = lds + (w - 1) * NRED * 64 + lane;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      o[r * 64] = G[r];
+      o[(4 + r) * 64] = X[r];
+      o[(8 + r) * 64] = u[r];
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[(12 + 4 * dt + r) * 64] = O2[dt][r];
+  }
+  __syncthreads();
+  if (w > 0) return;
+  for (int i = 0; i < W - 1; ++i) {
+    const float* o = lds + i * NRED * 64 + lane;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      G[r] += o[r * 64];
+      X[r] += o[(4 + r) * 64];
+      u[r] += o[(8 + r) * 64];
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) O2[dt][r] += o[(12 + 4 * dt + r) * 64];
+  }
+  // second-order part:  [X + p * (2 G - u - rowsum(2 p G))] v + (2 O2 + first-order part)
+  floatx4 pi;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float ur = sum16(u[r]);
+    const float rs = sum16(pc[r] * 2.0f * G[r]);
+    pi[r] = X[r] + pc[r] * (2.0f * G[r] - ur - rs);
+  }
+  // the tile of this wavefront may alias sums that it has read: same wavefront, LDS in order
+  const float4 pia = to_a(pi);
+  float vb[DT][4];
+  v_rows(vb);
+  pv(pia, vb, O2);
+  store(a.ol, O2);
+}
+
+// W wavefronts per pair: twelve fit a CU, three workgroups of four; eight share the rows where a CU gets one pair at most.
+template <int DT>
+int launch_mhsa_small(hipStream_t st, const MhsaArgs& a) {
+  const int64_t pairs = a.B * a.H;
+  if (pairs > 0x7ffffff0LL) return FOLX_HIP_ENOTSUP;
+  const int W = a.P < 8 ? 1 : (pairs <= 192 && a.P >= 16 ? 8 : 4);
+  const size_t tiles = (size_t)W * 16 * 20, sums = (size_t)(W - 1) * (12 + 4 * DT) * 64;
+  const size_t shm = 4 * (tiles > sums ? tiles : sums);
+  const dim3 grid((unsigned)((pairs + NXCD - 1) / NXCD * NXCD)), block((unsigned)(FOLX_WAVE * W));
+  const bool masked = a.mask != nullptr || a.imask != nullptr;
+  if (a.e != nullptr) {
+    if (masked) mhsa_small_kernel<DT, true, true><<<grid, block, shm, st>>>(a);
+    else mhsa_small_kernel<DT, true, false><<<grid, block, shm, st>>>(a);
+  } else {
+    if (masked) mhsa_small_kernel<DT, false, true><<<grid, block, shm, st>>>(a);
+    else mhsa_small_kernel<DT, false, false><<<grid, block, shm, st>>>(a);
+  }
+  return folx_launch_status();
+}
+
 template <int NW, int DT>
 int launch_mhsa(hipStream_t st, const MhsaArgs& a) {
   const int64_t blocks = a.B * a.H;
@@ -425,7 +787,14 @@ static int mhsa_entry(void* stream, const float* q, const float* q_jac, const fl
   hipStream_t st = (hipStream_t)stream;
   const int nw = (n + 15) / 16;
   switch (nw) {
-    case 1: return launch_mhsa_d<1>(st, a);
+    case 1:
+      // the buffer descriptors of the small form span a walker's (n, H, d) block with 32-bit offsets
+      if ((int64_t)n * H * d * 4 >= (int64_t)FAR) return launch_mhsa_d<2>(st, a);
+      switch ((d + 15) / 16) {
+        case 1: return launch_mhsa_small<1>(st, a);
+        case 2: return launch_mhsa_small<2>(st, a);
+        default: return launch_mhsa_small<4>(st, a);
+      }
     case 2: return launch_mhsa_d<2>(st, a);
     case 3: return launch_mhsa_d<3>(st, a);
     default: return launch_mhsa_d<4>(st, a);
