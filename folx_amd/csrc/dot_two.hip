@@ -19,6 +19,8 @@
 // loop body as one more row (p = P) that is left out of the second-order sum.  Inside a group of
 // 16 values of k the order is permuted (lane (l16, lg), step r <-> k = 4 lg + r), so the A
 // operand is one 128-bit LDS read per four MFMAs.
+//
+// Up to 32 x 32 x 32 nothing has to be shared: dot_two_small_kernel (its mapping stands there).
 #include <atomic>
 
 #include "common.h"
@@ -192,6 +194,179 @@ __global__ __launch_bounds__(DT_NT) void dot_two_kernel(DotTwoArgs g) {
   }
 }
 
+// I, J, Kc <= 32: one wavefront covers a whole batch element (TI x TJ blocks of 16 x 16, KT groups of 16 k), so nothing is
+// shared: operands go from memory straight into MFMA operand registers and the W wavefronts of a workgroup take the Jacobian
+// rows p = w, w + W, ..., the next row's operands requested before this row's products; the sums over rows meet in LDS once
+// at the end.  The product is formed transposed (b in the A operand), so a lane ends with four consecutive columns of a row
+// of y: 128-bit stores.  Padding is lanes whose buffer offset lies past the descriptor's end (zeros; dropped stores).
+// a_vec / b_vec: the contracted axis has unit stride and every piece of four is whole and aligned: 128-bit loads.
+// Bound by HBM.  The tiled form above left three of its four wavefronts without a block and paid two barriers and an LDS
+// round trip per row at these sizes: 2048 products q k^T of 16 x 16 x 16, P = 48 (0.31 GB): 323 -> 66 us (4.8 TB/s); of
+// 32 x 32 x 32, P = 96: 1446 -> 528 us (4.7 TB/s); 64 of 16 x 16 x 16, P = 48: 99 -> 22 us.
+constexpr int NXCD = 8;
+constexpr uint32_t FAR = 0x40000000u;      // past every descriptor's end
+constexpr int64_t EXTENT_MAX = 0x0fffffff;  // elements of an operand's tile from its first to its last: below FAR in bytes
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+template <int TI, int TJ, int KT, bool CONSTB>
+__global__ __launch_bounds__(512) void dot_two_small_kernel(DotTwoArgs g, int a_vec, int b_vec, int y_vec) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];  // [W - 1][TI * TJ * 4][64] sums
+  const int W = blockDim.x / FOLX_WAVE;
+  const int lane = threadIdx.x % FOLX_WAVE, w = folx_wave_id();
+  const int l16 = lane % 16, lg = lane / 16;
+  // ids are dealt round-robin to the XCDs: consecutive batch elements (heads of a walker share cache lines) go to one
+  const int64_t per = (g.NB + NXCD - 1) / NXCD;
+  const int64_t bt = (int64_t)(blockIdx.x % NXCD) * per + blockIdx.x / NXCD;
+  if (bt >= g.NB) return;
+  const int64_t b0 = bt / g.NB1, b1 = bt % g.NB1;
+  const int I = g.I, J = g.J, Kc = g.Kc, P = g.P;
+  const int64_t a_off = b0 * g.a_sb0 + b1 * g.a_sb1, b_off = b0 * g.b_sb0 + b1 * g.b_sb1;
+  const uint32_t a_si = (uint32_t)g.a_si, a_sk = (uint32_t)g.a_sk, b_sj = (uint32_t)g.b_sj, b_sk = (uint32_t)g.b_sk;
+  const uint32_t a_bytes = Kc > 0 ? 4u * ((uint32_t)(I - 1) * a_si + (uint32_t)(Kc - 1) * a_sk + 1u) : 0u;
+  const uint32_t b_bytes = Kc > 0 ? 4u * ((uint32_t)(J - 1) * b_sj + (uint32_t)(Kc - 1) * b_sk + 1u) : 0u;
+
+  // element (row / column l16 of block i, k = 16 t + 4 lg + r)
+  auto load = [&](const float* src, uint32_t bytes, int n, uint32_t s, uint32_t sk, int vec, int blk,
+                  floatx4 (&reg)[KT]) __attribute__((always_inline)) {
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, bytes, 0x00027000);
+    const int row = 16 * blk + l16;
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      const int k = 16 * t + 4 * lg;
+      const uint32_t base = 4u * ((uint32_t)row * s + (uint32_t)k * sk);
+      if (vec) {
+        reg[t] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, row < n && k < Kc ? base : FAR, 0, 0));
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          reg[t][r] = __uint_as_float(
+              __builtin_amdgcn_raw_buffer_load_b32(rs, row < n && k + r < Kc ? base + 4u * r * sk : FAR, 0, 0));
+      }
+    }
+  };
+  auto load_a = [&](const float* src, floatx4 (&reg)[TI][KT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i) load(src + a_off, a_bytes, I, a_si, a_sk, a_vec, i, reg[i]);
+  };
+  auto load_b = [&](const float* src, floatx4 (&reg)[TJ][KT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) load(src + b_off, b_bytes, J, b_sj, b_sk, b_vec, j, reg[j]);
+  };
+  auto store = [&](float* dst, const floatx4 (&c)[TI][TJ]) __attribute__((always_inline)) {
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(dst + bt * I * J, 0, (uint32_t)(I * J) * 4u, 0x00027000);
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) {
+        const int row = 16 * i + l16, col = 16 * j + 4 * lg;
+        const uint32_t off = (uint32_t)(row * J + col) * 4u;
+        if (y_vec) {
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uintx4, c[i][j]), rs, row < I && col < J ? off : FAR, 0, 0);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float v = c[i][j][r];
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rs, row < I && col + r < J ? off + 4u * r : FAR, 0, 0);
+          }
+        }
+      }
+  };
+  auto mul = [&](const floatx4 (&x)[TI][KT], const floatx4 (&y)[TJ][KT], floatx4 (&acc)[TI][TJ]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < KT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+          for (int j = 0; j < TJ; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j][t][r], x[i][t][r], acc[i][j], 0, 0, 0);
+  };
+  auto zero = [&](floatx4 (&acc)[TI][TJ]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  };
+
+  // pass p < P: Jacobian row p; pass p == P: the Laplacians take the place of the row
+  floatx4 an[TI][KT], bn[TJ][KT];
+  auto fetch = [&](int p) __attribute__((always_inline)) {
+    load_a(p == P ? g.al : g.aj + (int64_t)p * g.a_sp, an);
+    if constexpr (!CONSTB) load_b(p == P ? g.bl : g.bj + (int64_t)p * g.b_sp, bn);
+  };
+  floatx4 a[TI][KT], b[TJ][KT], cross[TI][TJ], lap[TI][TJ];
+  load_a(g.a, a);
+  load_b(g.b, b);
+  if (w <= P) fetch(w);
+  if (w == 0) {
+    floatx4 acc[TI][TJ];
+    zero(acc);
+    mul(a, b, acc);
+    store(g.y, acc);
+  }
+  zero(cross);
+  zero(lap);
+  for (int p = w; p <= P; p += W) {
+    floatx4 aj[TI][KT], bj[TJ][KT], acc[TI][TJ];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i) aj[i][t] = an[i][t];
+      if constexpr (!CONSTB)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) bj[j][t] = bn[j][t];
+    }
+    if (p + W <= P) fetch(p + W);
+    zero(acc);
+    mul(aj, b, acc);
+    if constexpr (!CONSTB) {
+      mul(a, bj, acc);
+      if (p < P) mul(aj, bj, cross);
+    }
+    if (p < P) {
+      store(g.yj + (int64_t)p * g.y_sp, acc);
+    } else {
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) lap[i][j] = acc[i][j];
+    }
+  }
+
+  // sums over rows: wavefronts 1 .. W - 1 leave theirs in LDS, wavefront 0 adds them in order
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) lap[i][j][r] += 2.0f * cross[i][j][r];
+  if (w > 0) {
+    float* o = sm + (w - 1) * (TI * TJ * 4 * FOLX_WAVE) + lane;
+#pragma unroll
+    for (int e = 0; e < TI * TJ * 4; ++e) o[e * FOLX_WAVE] = lap[e / 4 / TJ][e / 4 % TJ][e % 4];
+  }
+  __syncthreads();
+  if (w > 0) return;
+  for (int v = 0; v < W - 1; ++v) {
+    const float* o = sm + v * (TI * TJ * 4 * FOLX_WAVE) + lane;
+#pragma unroll
+    for (int e = 0; e < TI * TJ * 4; ++e) lap[e / 4 / TJ][e / 4 % TJ][e % 4] += o[e * FOLX_WAVE];
+  }
+  store(g.yl, lap);
+}
+
+template <int TI, int TJ, int KT>
+int launch_small(hipStream_t st, const DotTwoArgs& g, bool constb, int a_vec, int b_vec, int y_vec) {
+  // fewer than eight rows are not worth sharing; eight wavefronts where a CU gets one batch element at most
+  const int W = g.P < 8 ? 1 : (g.NB <= 192 && g.P >= 16 ? 8 : 4);
+  const size_t lds = sizeof(float) * (W - 1) * TI * TJ * 4 * FOLX_WAVE;
+  const dim3 grid((unsigned)((g.NB + NXCD - 1) / NXCD * NXCD)), block((unsigned)(FOLX_WAVE * W));
+  if (constb) dot_two_small_kernel<TI, TJ, KT, true><<<grid, block, lds, st>>>(g, a_vec, b_vec, y_vec);
+  else dot_two_small_kernel<TI, TJ, KT, false><<<grid, block, lds, st>>>(g, a_vec, b_vec, y_vec);
+  return folx_launch_status();
+}
+
 }  // namespace
 
 extern "C" int folx_hip_dot_two_fwdlap(void* stream, const float* a, const float* a_jac, const float* a_lap,
@@ -214,6 +389,27 @@ extern "C" int folx_hip_dot_two_fwdlap(void* stream, const float* a, const float
     if (strides[i] < 0) return FOLX_HIP_EINVAL;
   g.NB = NB; g.NB1 = NB1; g.I = I; g.J = J; g.Kc = Kc; g.P = P;
   g.y_sp = NB * (int64_t)I * J;
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t a_ext = (I - 1) * g.a_si + (Kc > 0 ? Kc - 1 : 0) * g.a_sk, b_ext = (J - 1) * g.b_sj + (Kc > 0 ? Kc - 1 : 0) * g.b_sk;
+  if (I <= 32 && J <= 32 && Kc <= 32 && a_ext < EXTENT_MAX && b_ext < EXTENT_MAX && NB <= 0x7ffffff0LL) {
+    const bool whole = Kc % 4 == 0;
+    const int a_vec = whole && g.a_sk == 1 && ((g.a_si | g.a_sb0 | g.a_sb1 | g.a_sp) & 3) == 0 && folx_aligned16(a) &&
+                      folx_aligned16(a_jac) && folx_aligned16(a_lap);
+    const int b_vec = whole && g.b_sk == 1 && ((g.b_sj | g.b_sb0 | g.b_sb1 | g.b_sp) & 3) == 0 && folx_aligned16(b) &&
+                      folx_aligned16(b_jac) && folx_aligned16(b_lap);
+    const int y_vec = J % 4 == 0 && folx_aligned16(y) && folx_aligned16(y_jac) && folx_aligned16(y_lap);
+    const int form = (I > 16 ? 4 : 0) + (J > 16 ? 2 : 0) + (Kc > 16 ? 1 : 0);
+    switch (form) {
+      case 0: return launch_small<1, 1, 1>(st, g, constb, a_vec, b_vec, y_vec);
+      case 1: return launch_small<1, 1, 2>(st, g, constb, a_vec, b_vec, y_vec);
+      case 2: return launch_small<1, 2, 1>(st, g, constb, a_vec, b_vec, y_vec);
+      case 3: return launch_small<1, 2, 2>(st, g, constb, a_vec, b_vec, y_vec);
+      case 4: return launch_small<2, 1, 1>(st, g, constb, a_vec, b_vec, y_vec);
+      case 5: return launch_small<2, 1, 2>(st, g, constb, a_vec, b_vec, y_vec);
+      case 6: return launch_small<2, 2, 1>(st, g, constb, a_vec, b_vec, y_vec);
+      default: return launch_small<2, 2, 2>(st, g, constb, a_vec, b_vec, y_vec);
+    }
+  }
   g.tiles_i = (I + DT_TILE - 1) / DT_TILE;
   g.tiles_j = (J + DT_TILE - 1) / DT_TILE;
   const int64_t blocks = NB * g.tiles_i * g.tiles_j;
@@ -221,7 +417,6 @@ extern "C" int folx_hip_dot_two_fwdlap(void* stream, const float* a, const float
   const int Kp = (Kc + 15) / 16 * 16 > 0 ? (Kc + 15) / 16 * 16 : 16;
   g.Kc = Kc;
   const size_t lds = sizeof(float) * (2 * DT_TILE * (Kp + 4) + 2 * Kp * DT_BS);
-  hipStream_t st = (hipStream_t)stream;
   const int nld = DT_TILE * Kp / DT_NT;  // 2, 4, ..., 16
   const dim3 grid((unsigned)blocks), block(DT_NT);
   if (nld <= 4) {

@@ -50,3 +50,39 @@ def test_mhsa_short_sequences(B, n, H, d, P, edge, masked):
     assert_val(got[1][:, :, m], ref[1][:, :, m], 'o_jac')
     assert_lap(got[2][:, m], ref[2][:, m], 'o_lap')
     assert all(bool(torch.isfinite(t).all()) for t in got)
+
+
+# up to 32 x 32 x 32 one wavefront per batch element (1 / 4 / 8 sharing the Jacobian rows), 33: the tiled form; pieces of
+# four k whole and aligned or not, rows of y whole or not
+@pytest.mark.parametrize('NB0,NB1,I,J,Kc,P', [(3, 2, 16, 16, 16, 39), (1, 1, 17, 32, 20, 8), (2, 3, 32, 17, 32, 9),
+                                              (200, 1, 4, 16, 30, 17), (2, 2, 15, 5, 31, 16), (1, 3, 32, 32, 1, 0),
+                                              (2, 1, 1, 1, 17, 7), (2, 2, 33, 8, 8, 9), (5, 2, 24, 12, 4, 12)])
+@pytest.mark.parametrize('layout', ['contiguous', 'interleaved', 'offset'])
+def test_dot_two_small_products(NB0, NB1, I, J, Kc, P, layout):
+    from folx_amd import kernels as K
+
+    print(f'case dot_two NB=({NB0},{NB1}) I={I} J={J} K={Kc} P={P} {layout}', flush=True)
+    rng = np.random.default_rng(I * 100 + J)
+    a = [rand(rng, *s, NB0, NB1, I, Kc) for s in ((), (P,), ())]
+    b = [rand(rng, *s, NB0, NB1, Kc, J) for s in ((), (P,), ())]
+    ref = rules.dot_two_rule(*f64(*a, *b))
+
+    def lay(t, transposed):
+        if layout == 'contiguous':
+            return dev(t)
+        if layout == 'offset':  # rows that start off the 16-byte boundary
+            return torch.nn.functional.pad(dev(t), (1, 2))[..., 1:-2]
+        t = np.swapaxes(t, -1, -2) if transposed else t  # (walker, position, head, feature), b as k^T
+        t = dev(np.swapaxes(t, -3, -2)).transpose(-3, -2)
+        return t.transpose(-1, -2) if transposed else t
+
+    got = K.dot_two(*[lay(t, False) for t in a], *[lay(t, True) for t in b])
+    assert_val(got[0], ref[0], 'y')
+    assert_val(got[1], ref[1], 'y_jac')
+    assert_lap(got[2], ref[2], 'y_lap')
+    W = rand(rng, NB1, Kc, J)
+    ref = rules.dot_const_rule(*f64(*a, W))
+    got = K.dot_const(*[lay(t, False) for t in a], dev(W))
+    assert_val(got[0], ref[0], 'y')
+    assert_val(got[1], ref[1], 'y_jac')
+    assert_lap(got[2], ref[2], 'y_lap')
