@@ -57,26 +57,64 @@ __global__ __launch_bounds__(256) void reduce_mid_v4_kernel(const float* __restr
   *reinterpret_cast<float4*>(out + o4 * 4) = acc;
 }
 
-// inner == 1: one wavefront per output element, lanes stride over the reduced axis.
-template <bool MAX>
-__global__ __launch_bounds__(256) void reduce_last_kernel(const float* __restrict__ in,
-                                                          float* __restrict__ out, int64_t total,
-                                                          int64_t red, int64_t span, int64_t lo, float alpha) {
-  const int lane = threadIdx.x % FOLX_WAVE;
-  const int64_t o = (int64_t)blockIdx.x * (256 / FOLX_WAVE) + threadIdx.x / FOLX_WAVE;
-  if (o >= total) return;
-  const float* src = in + o * span + lo;
-  float acc = MAX ? -INFINITY : 0.0f;
-  for (int64_t r = lane; r < red; r += FOLX_WAVE) {
-    const float v = src[r];
-    acc = MAX ? fmaxf(acc, v) : acc + v;
-  }
+// inner == 1: G lanes (a power of two) per output element, each taking pieces of VEC consecutive values, U outputs of a
+// group in flight.  Bound by HBM: G is the least that covers the reduced axis in one piece per lane, so that a wavefront
+// reads one contiguous stretch (64 / G outputs side by side).  A whole wavefront per output left 48 of 64 lanes idle on
+// the softmax sums of 16 particles: 1.6 M outputs of 16: 182 -> 17 us (6.6 TB/s); 5.7 M of 30: 826 -> 193 us.
+template <bool MAX, int VEC, int U>
+__global__ __launch_bounds__(256) void reduce_last_kernel(const float* __restrict__ in, float* __restrict__ out,
+                                                          int64_t total, int64_t red, int64_t span, int64_t lo,
+                                                          int32_t G, float alpha) {
+  const int per = 256 / G, g = threadIdx.x / G, l = threadIdx.x % G;
+  const int64_t o0 = (int64_t)blockIdx.x * (per * U) + g;
+  const int64_t pieces = red / VEC;
+  float acc[U];
 #pragma unroll
-  for (int off = FOLX_WAVE / 2; off > 0; off >>= 1) {
-    const float v = __shfl_xor(acc, off, FOLX_WAVE);
-    acc = MAX ? fmaxf(acc, v) : acc + v;
+  for (int u = 0; u < U; ++u) acc[u] = MAX ? -INFINITY : 0.0f;
+  for (int64_t r = l; r < pieces; r += G) {
+    float v[U][VEC];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // outputs past the end read the last one's values
+      const int64_t o = o0 + u * per < total ? o0 + u * per : total - 1;
+      const float* p = in + o * span + lo + r * VEC;
+      if constexpr (VEC == 4) {
+        const float4 q = folx_ld_stream4(p);
+        v[u][0] = q.x; v[u][1] = q.y; v[u][2] = q.z; v[u][3] = q.w;
+      } else {
+        v[u][0] = *p;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) acc[u] = MAX ? fmaxf(acc[u], v[u][i]) : acc[u] + v[u][i];
   }
-  if (lane == 0) out[o] = MAX ? acc : alpha * acc;
+  for (int off = G / 2; off > 0; off >>= 1)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float v = __shfl_xor(acc[u], off, FOLX_WAVE);
+      acc[u] = MAX ? fmaxf(acc[u], v) : acc[u] + v;
+    }
+  if (l == 0)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (o0 + u * per < total) out[o0 + u * per] = MAX ? acc[u] : alpha * acc[u];
+}
+
+template <bool MAX, int VEC>
+int launch_reduce_last(hipStream_t st, const float* in, float* out, int64_t total, int64_t red, int64_t span, int64_t lo,
+                       float alpha) {
+  int G = 1;
+  while (G < FOLX_WAVE && G < red / VEC) G *= 2;
+  const int64_t per = 256 / G;
+  // four outputs per group once that still leaves every CU several workgroups
+  const int U = total >= 4 * per * 2048 ? 4 : 1;
+  const int64_t blocks = (total + per * U - 1) / (per * U);
+  if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
+  if (U == 4) reduce_last_kernel<MAX, VEC, 4><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(in, out, total, red, span, lo, G, alpha);
+  else reduce_last_kernel<MAX, VEC, 1><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(in, out, total, red, span, lo, G, alpha);
+  return folx_launch_status();
 }
 
 template <bool MAX>
@@ -87,9 +125,9 @@ int launch_reduce(hipStream_t st, const float* in, float* out, int64_t rows, int
   if (total == 0) return FOLX_HIP_OK;
   if (!in || !out) return FOLX_HIP_EINVAL;
   if (inner == 1 && red >= 16) {
-    const int64_t blocks = (total + 3) / 4;
-    if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
-    reduce_last_kernel<MAX><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(in, out, total, red, span, lo, alpha);
+    if (red % 4 == 0 && span % 4 == 0 && lo % 4 == 0 && folx_aligned16(in))
+      return launch_reduce_last<MAX, 4>(st, in, out, total, red, span, lo, alpha);
+    return launch_reduce_last<MAX, 1>(st, in, out, total, red, span, lo, alpha);
   } else if (inner % 4 == 0 && folx_aligned16(in) && folx_aligned16(out)) {
     const int64_t blocks = (total / 4 + 255) / 256;
     if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;

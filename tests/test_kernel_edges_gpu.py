@@ -86,3 +86,21 @@ def test_dot_two_small_products(NB0, NB1, I, J, Kc, P, layout):
     assert_val(got[0], ref[0], 'y')
     assert_val(got[1], ref[1], 'y_jac')
     assert_lap(got[2], ref[2], 'y_lap')
+
+
+# groups of 1 .. 64 lanes per output, 128-bit pieces or single values, one or four outputs per group in flight
+@pytest.mark.parametrize('total,span,lo,hi', [(5, 16, 0, 16), (7, 17, 0, 17), (3, 40, 4, 36), (3, 40, 3, 36), (1, 1000, 0, 1000),
+                                              (9, 999, 1, 998), (524288 + 3, 16, 0, 16), (33000, 260, 0, 260), (131072, 19, 1, 18)])
+def test_reduce_last_axis(total, span, lo, hi):
+    from folx_amd import kernels as K
+
+    print(f'case reduce_last total={total} span={span} window=({lo},{hi})', flush=True)
+    x = rand(np.random.default_rng(span), 1, total, span, 1)
+    got = K.reduce_sum(dev(x), 1, total, span, 1, 0.5, (lo, hi)).reshape(total)
+    ref = 0.5 * x[0, :, lo:hi, 0].astype(np.float64).sum(axis=1)
+    # each addend passes at most (hi - lo) rounded additions
+    bound = (hi - lo) * 2.0 ** -24 * 0.5 * np.abs(x[0, :, lo:hi, 0].astype(np.float64)).sum(axis=1) + 1e-30
+    assert (np.abs(got.cpu().numpy() - ref) <= bound).all()
+    if (lo, hi) == (0, span):
+        m = K.reduce_max(dev(x), total, span, 1)
+        assert torch.equal(m.reshape(total).cpu(), torch.as_tensor(x[0, :, :, 0].max(axis=1)))
