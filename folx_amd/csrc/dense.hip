@@ -8,7 +8,8 @@
 // double-buffered LDS tiles, one barrier per chunk.  For N > 128 the tile is 128 x 256 on 8
 // wavefronts (each 64 x 64), so a layer of width 256 reads its A rows from HBM exactly once
 // and two workgroups share a CU; narrower layers use 128 x {128, 64, 32} tiles on 4
-// wavefronts.
+// wavefronts, and so do launches that such tiles would spread unevenly over the CUs, as 64 x 64 (the rule stands at the
+// entry point).
 //
 // Main path (K a multiple of 16, 16-byte aligned operands): the chunks go from global memory
 // straight into LDS (global_load_lds_dwordx4), no staging registers and no LDS store
@@ -737,6 +738,22 @@ __global__ __launch_bounds__(256) void dense_n1_flat_kernel(Segs sg, const float
   }
 }
 
+// Main path.  Requires K % 16 == 0, N % 4 == 0 and 16-byte aligned operands.
+template <int BM, int BN, int WM, int WN>
+int launch_dma(hipStream_t st, Segs& sg, const float* W, const float* bias, int32_t K, int32_t N, bool has_res) {
+  int64_t row_tiles = 0;
+  for (int s = 0; s < 3; ++s) { sg.tiles[s] = (sg.rows[s] + BM - 1) / BM; row_tiles += sg.tiles[s]; }
+  const int32_t col_tiles = (N + BN - 1) / BN;
+  const int64_t blocks = (row_tiles + NXCD - 1) / NXCD * NXCD * col_tiles;
+  if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
+  const dim3 grid((unsigned)blocks), block(64 * WM * WN);
+  if (has_res)
+    dense_dma_kernel<BM, BN, WM, WN, true><<<grid, block, 0, st>>>(sg, W, bias, K, N, row_tiles, col_tiles);
+  else
+    dense_dma_kernel<BM, BN, WM, WN, false><<<grid, block, 0, st>>>(sg, W, bias, K, N, row_tiles, col_tiles);
+  return folx_launch_status();
+}
+
 template <int BM, int BN, int WM, int WN, int MINB>
 int launch_cfg(hipStream_t st, Segs& sg, const float* W, const float* bias, int32_t K, int32_t N,
                bool vec, bool has_res) {
@@ -756,13 +773,7 @@ int launch_cfg(hipStream_t st, Segs& sg, const float* W, const float* bias, int3
       return folx_launch_status();
     }
   }
-  if (vec && K % BK == 0 && N >= 4) {
-    if (has_res)
-      dense_dma_kernel<BM, BN, WM, WN, true><<<grid, block, 0, st>>>(sg, W, bias, K, N, row_tiles, col_tiles);
-    else
-      dense_dma_kernel<BM, BN, WM, WN, false><<<grid, block, 0, st>>>(sg, W, bias, K, N, row_tiles, col_tiles);
-    return folx_launch_status();
-  }
+  if (vec && K % BK == 0 && N >= 4) return launch_dma<BM, BN, WM, WN>(st, sg, W, bias, K, N, has_res);
   if (vec && has_res)
     dense_kernel<BM, BN, WM, WN, MINB, true, true><<<grid, block, 0, st>>>(sg, W, bias, K, N, row_tiles, col_tiles);
   else if (vec)
@@ -812,6 +823,20 @@ extern "C" int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const fl
     const int64_t blocks = std::min<int64_t>((total + 31) / 32, 256 * 32);
     dense_n1_kernel<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(sg, W, bias, K, total);
     return folx_launch_status();
+  }
+  // A CU works through its share of 128 x 256 tiles (8 units of 64 x 64; 128 x 128: 4) at the rate of the matrix pipe,
+  // however many share it, so a launch takes ceil(tiles / 256) tile times; 64 x 64 tiles divide finer, also the columns
+  // (N = 160 is 192 instead of 256), at an eighth less rate (twice the LDS reads per product).  K = N = 256: 1280 rows
+  // 36 -> 10 us, 20 480 rows (160 tiles) 40 -> 30, 47 104 (368) 73 -> 62, 82 432 (644) 105 -> 101; 159 900 rows
+  // (1249 tiles) would go 173 -> 191.  The opt-in products have the 128 x 256 tile only.
+  if (N > 64 && vec && K % BK == 0 && (N <= 128 || folx_gemm_mode() != FOLX_HIP_GEMM_BF16X3)) {
+    int64_t big = 0, small = 0;
+    for (int s = 0; s < 3; ++s) { big += (sg.rows[s] + 127) / 128; small += (sg.rows[s] + 63) / 64; }
+    const double units = N > 128 ? 8.0 : 4.0;
+    big *= N > 128 ? (N + 255) / 256 : 1;
+    small *= (N + 63) / 64;
+    if (1.16 * (double)small < units * (double)((big + 255) / 256 * 256))
+      return launch_dma<64, 64, 2, 2>(st, sg, W, bias, K, N, has_res);
   }
   if (N > 128) return launch_cfg<128, 256, 2, 4, 2>(st, sg, W, bias, K, N, vec, has_res);
   if (N > 64) return launch_cfg<128, 128, 2, 2, 3>(st, sg, W, bias, K, N, vec, has_res);

@@ -104,3 +104,23 @@ def test_reduce_last_axis(total, span, lo, hi):
     if (lo, hi) == (0, span):
         m = K.reduce_max(dev(x), total, span, 1)
         assert torch.equal(m.reshape(total).cpu(), torch.as_tensor(x[0, :, :, 0].max(axis=1)))
+
+
+# 64 x 64 tiles where larger ones would leave CUs idle: cut row and column tiles in every segment, one chunk of K, skip connection
+@pytest.mark.parametrize('rows,P,Kd,N', [((1, 1), 1, 16, 68), ((3, 21), 2, 48, 100), ((1, 64), 3, 32, 128), ((5, 13), 9, 256, 132),
+                                         ((2, 65), 7, 64, 300), ((40, 10), 30, 256, 256)])
+def test_dense_small_tiles(rows, P, Kd, N):
+    from folx_amd import kernels as K
+
+    print(f'case dense rows={rows} P={P} K={Kd} N={N}', flush=True)
+    rng = np.random.default_rng(N)
+    t = [rand(rng, *rows, Kd), rand(rng, P, *rows, Kd), rand(rng, *rows, Kd)]
+    W, b = (rand(rng, Kd, N) / np.sqrt(Kd)).astype(np.float32), rand(rng, N)
+    res = [rand(rng, *rows, N), rand(rng, P, *rows, N), rand(rng, *rows, N)]
+    ref = rules.dense_rule(*f64(*t, W, b))
+    for skip in (None, tuple(dev(r) for r in res)):
+        got = K.dense(*[dev(v) for v in t], dev(W), dev(b), skip)
+        want = ref if skip is None else [a + r for a, r in zip(ref, res)]
+        assert_val(got[0], want[0], 'y')
+        assert_val(got[1], want[1], 'y_jac')
+        assert_lap(got[2], want[2], 'y_lap')
