@@ -109,7 +109,10 @@ struct WideParams {
 
 // PT = Jacobian rows of a tile: 32 (4 positions per tile, one per accumulator block), or 16 for
 // the activation alone (8 positions per tile, two per block: registers 0-7 of a block belong
-// to the first, 8-15 to the second), which wastes less when P is 16 more than a multiple of 32.
+// to the first, 8-15 to the second), or 8 (four per block), whichever leaves the fewest empty rows
+// (plan_wide): P = 21 fills 24 rows instead of 32, P = 39 fills 40 instead of 48 or 64.  A 7-electron FermiNet-style step of
+// 512 walkers, whose layers went unfused with 832 instead of 320 contracted features: 2.58 -> 1.48 ms.  The activation's tiles may
+// hold more positions than are left: those past R read position R - 1 and are neither stored nor summed.
 // SPLIT: the products on the bf16 matrix pipe from operands split into three bf16 pieces, with
 // the loop of dense_split_kernel: A and W chunks come through registers and every element is
 // split once per workgroup on its way into LDS (A stage [piece][g][row][8 bf16], W stage
@@ -128,7 +131,7 @@ __global__ __launch_bounds__(NT, 4) void dense_wide_kernel(WideParams a) {
   constexpr int W_PLANE = 2 * 4 * BN * 4;  //        and of a W chunk
   constexpr int RT = BM / PT;  // positions of a tile
   constexpr int PB = 32 / PT;  // positions of a 32-row accumulator block
-  static_assert(PT == 32 || (PT == 16 && !NORM), "LayerNorm's row sums assume one position per block");
+  static_assert(PT == 32 || ((PT == 16 || PT == 8) && !NORM), "LayerNorm's row sums assume one position per block");
   __shared__ __attribute__((aligned(16))) float As0[SPLIT ? 3 * A_PLANE / 4 : BM * BK];
   __shared__ __attribute__((aligned(16))) float As1[SPLIT ? 3 * A_PLANE / 4 : BM * BK];
   __shared__ __attribute__((aligned(16))) float Ws0[SPLIT ? 3 * W_PLANE / 4 : BK * BN];
@@ -151,6 +154,7 @@ __global__ __launch_bounds__(NT, 4) void dense_wide_kernel(WideParams a) {
   const int32_t col0 = ct * BN;
   const int32_t K = a.K, N = a.N, P = a.P;
   const int64_t R = a.R;
+  auto inside = [&](int64_t pos) __attribute__((always_inline)) -> int64_t { return NORM || pos < R ? pos : R - 1; };
 
   const int tid = threadIdx.x;
   const int lane = tid % 64;
@@ -173,13 +177,13 @@ __global__ __launch_bounds__(NT, 4) void dense_wide_kernel(WideParams a) {
     int p = p0 + m % PT;
     if (p >= P) p = P - 1;  // reaches accumulator rows that are neither stored nor summed
     if constexpr (PARTS) {
-      a_pos = r0 + m / PT;
+      a_pos = inside(r0 + m / PT);
       a_posg = a_pos / a.parts.group;
       a_row = p;
       a_kc = kc * 4;
       a_p[i] = nullptr;
     } else {
-      a_p[i] = a.jac + ((int64_t)p * R + r0 + m / PT) * K + kc * 4;  // tile row m: position m / PT, row m % PT
+      a_p[i] = a.jac + ((int64_t)p * R + inside(r0 + m / PT)) * K + kc * 4;  // tile row m: position m / PT, row m % PT
     }
   }
 #pragma unroll
@@ -226,7 +230,7 @@ __global__ __launch_bounds__(NT, 4) void dense_wide_kernel(WideParams a) {
         int gc = col0 + wc + j * 32 + l32;
         if (gc >= N) gc = N - 1;
 #pragma unroll
-        for (int b = 0; b < PB; ++b) dr[i][j][b] = a.z[(r0 + (wrow * TM + i) * PB + b) * N + gc];
+        for (int b = 0; b < PB; ++b) dr[i][j][b] = a.z[inside(r0 + (wrow * TM + i) * PB + b) * N + gc];
       }
   }
   // SPLIT staging: thread t has k quarter t % 4 of tile row t / 4; wavefront w has rows 2 w and
@@ -240,12 +244,12 @@ __global__ __launch_bounds__(NT, 4) void dense_wide_kernel(WideParams a) {
     int p = p0 + m % PT;
     if (p >= P) p = P - 1;
     if constexpr (PARTS) {  // the part and the address inside it are found per chunk
-      a_pos = r0 + m / PT;
+      a_pos = inside(r0 + m / PT);
       a_posg = a_pos / a.parts.group;
       a_row = p;
       a_kc = q * 4;
     } else {
-      sa_src = a.jac + ((int64_t)p * R + r0 + m / PT) * K + q * 4;
+      sa_src = a.jac + ((int64_t)p * R + inside(r0 + m / PT)) * K + q * 4;
     }
     sa_dst = ((q / 2) * BM + m) * 16 + (q % 2) * 8;
     int wn = col0 + lane * 4;
@@ -322,7 +326,7 @@ __global__ __launch_bounds__(NT, 4) void dense_wide_kernel(WideParams a) {
             const int g = r / 4, b = g / GB;
             int prow = p0 + 4 * lh + 8 * (g % GB) + r % 4;
             if (prow >= P) prow = P - 1;  // rows past P of a ragged tile are neither stored nor summed
-            const int64_t pos = r0 + (wrow * TM + i) * PB + b;
+            const int64_t pos = inside(r0 + (wrow * TM + i) * PB + b);
             acc[i][j][r] = a.pre_jac[(int64_t)prow * pre_pstride + (pos / a.pre_group) * N + gc];
           }
         }
@@ -558,7 +562,7 @@ __global__ __launch_bounds__(NT, 4) void dense_wide_kernel(WideParams a) {
   // Register r of a block is tile row 8 (r / 4) + 4 (lane / 32) + r % 4 of the block, column
   // lane % 32: Jacobian row p0 + (that row) % PT of the block's position (that row) / PT.
   const int64_t pstride = R * N;  // floats between consecutive Jacobian rows
-  const bool full_tile = (p0 + PT <= P) && (col0 + BN <= N);
+  const bool full_tile = (p0 + PT <= P) && (col0 + BN <= N) && (NORM || r0 + RT <= R);
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int64_t pos = r0 + (wrow * TM + i) * PB;
@@ -608,7 +612,7 @@ __global__ __launch_bounds__(NT, 4) void dense_wide_kernel(WideParams a) {
           for (int rr = 0; rr < 4; ++rr) {
             const int pl = 8 * (g % GB) + rr;
             const int64_t off = (int64_t)pl * pstride + (int64_t)b * N;
-            const bool live = FULL || (p0 + 4 * lh + pl < P && gc < N);
+            const bool live = FULL || (p0 + 4 * lh + pl < P && gc < N && (NORM || pos + b < R));
             rb[rr] = 0.0f;
             if constexpr (RES) {
               if constexpr (FULL) rb[rr] = __builtin_nontemporal_load(resp + off);
@@ -645,7 +649,7 @@ __global__ __launch_bounds__(NT, 4) void dense_wide_kernel(WideParams a) {
               float w = d1[b] * v;
               if constexpr (RES) w += rbuf[g & 1][rr];
               __builtin_nontemporal_store(w, o);
-            } else if (p0 + 4 * lh + pl < P) {
+            } else if (p0 + 4 * lh + pl < P && (NORM || pos + b < R)) {
               if constexpr (ACT) ss[b] = fmaf(v, v, ss[b]);
               if (gc < N) *o = d1[b] * v + (RES ? rbuf[g & 1][rr] : 0.0f);
             }
@@ -664,7 +668,7 @@ __global__ __launch_bounds__(NT, 4) void dense_wide_kernel(WideParams a) {
 #pragma unroll
         for (int b = 0; b < PB; ++b) {
           const float t = ss[b] + __shfl_xor(ss[b], 32, FOLX_WAVE);
-          if (lh == 0 && gc < N) a.ss[so + (int64_t)b * N] = t;
+          if (lh == 0 && gc < N && (NORM || pos + b < R)) a.ss[so + (int64_t)b * N] = t;
         }
       }
       if constexpr (NORM) {
@@ -854,10 +858,13 @@ struct WidePlan {
 bool plan_wide(int64_t R, int32_t P, int32_t K, int32_t N, bool norm, bool act, WidePlan& pl) {
   if (R <= 0 || R % 4 != 0 || P < 1 || K < BK || K % BK != 0 || N <= 128 || N % 4 != 0) return false;
   if (norm && K > KMAX_NORM) return false;
-  // groups of 16 Jacobian rows where that leaves fewer empty tile rows
-  pl.PT = (!norm && R % 8 == 0 && (P + 15) / 16 * 16 < (P + 31) / 32 * 32) ? 16 : 32;
+  // the largest groups of Jacobian rows that leave the fewest empty tile rows
+  pl.PT = 32;
+  if (!norm)
+    for (int g = 16; g >= 8; g /= 2)
+      if ((P + g - 1) / g * g < (P + pl.PT - 1) / pl.PT * pl.PT) pl.PT = g;
   pl.PG = (P + pl.PT - 1) / pl.PT;
-  pl.pos_tiles = R / (BM / pl.PT);
+  pl.pos_tiles = (R + BM / pl.PT - 1) / (BM / pl.PT);
   pl.row_tiles = pl.pos_tiles * pl.PG;
   pl.col_tiles = (N + BN - 1) / BN;
   pl.blocks = (pl.row_tiles + NXCD - 1) / NXCD * NXCD * pl.col_tiles;
@@ -950,10 +957,13 @@ int run_wide(hipStream_t st, bool norm, int32_t act, float param, const float* x
     return has_act ? launch_wide<true, true, 32>(st, a, pl, y, y_lap) : launch_wide<true, false, 32>(st, a, pl, y, y_lap);
   if (parts) {
     a.parts = *parts;
-    return pl.PT == 16 ? launch_wide<false, true, 16, true>(st, a, pl, y, y_lap, res, res_lap)
-                       : launch_wide<false, true, 32, true>(st, a, pl, y, y_lap, res, res_lap);
+    return pl.PT == 8    ? launch_wide<false, true, 8, true>(st, a, pl, y, y_lap, res, res_lap)
+           : pl.PT == 16 ? launch_wide<false, true, 16, true>(st, a, pl, y, y_lap, res, res_lap)
+                         : launch_wide<false, true, 32, true>(st, a, pl, y, y_lap, res, res_lap);
   }
-  return pl.PT == 16 ? launch_wide<false, true, 16>(st, a, pl, y, y_lap) : launch_wide<false, true, 32>(st, a, pl, y, y_lap);
+  return pl.PT == 8    ? launch_wide<false, true, 8>(st, a, pl, y, y_lap)
+         : pl.PT == 16 ? launch_wide<false, true, 16>(st, a, pl, y, y_lap)
+                       : launch_wide<false, true, 32>(st, a, pl, y, y_lap);
 }
 
 }  // namespace

@@ -158,26 +158,31 @@ def dense(x, jac, lap, W, bias=None, res=None, row_slice=None):
 FUSED_ACTS = ('tanh', 'silu', 'logistic', 'sigmoid', 'softplus', 'exp', 'sin', 'cos', 'square')
 
 
-def _wide_tiles_filled(P, rows, norm):
-    """The wide fused kernels cut their tiles into groups of 32 Jacobian rows (16 for the
-    activation alone over a multiple of 8 rows, where that wastes less); a last group that is
-    mostly empty costs more MFMA work than the fusion saves."""
+def _wide_tiles_filled(P, norm, K, spared=None):
+    """Whether the wide fused kernels are the faster choice.  They cut their tiles into groups of 32 Jacobian rows (for the
+    activation alone also 16 or 8, whichever wastes least), and the empty rows of a last group are matrix work: for
+    LayerNorm up to an eighth of the rows.  For the activation the fused form contracts ``K`` features of ``padded`` rows,
+    a tenth slower than the plain product, which contracts ``spared`` (the whole concatenation, where the fused form
+    reads it in parts; else ``K``) features of P rows and is followed by a pass over the result, the time of
+    contracting 84 features more."""
     if P is None:
         return True
-    group = 16 if (not norm and rows % 8 == 0 and -(-P // 16) * 16 < -(-P // 32) * 32) else 32
-    return -(-P // group) * group <= 1.125 * P
+    if norm:
+        return -(-P // 32) * 32 <= 1.125 * P
+    padded = min(-(-P // g) * g for g in (32, 16, 8))
+    return padded <= 1.125 * P or 1.1 * padded * K <= P * ((spared or K) + 84)
 
 
-def dense_act_supported(name, K, N, rows=None, P=None):
+def dense_act_supported(name, K, N, rows=None, P=None, spared=None):
     """Shapes and functions the fused dense + activation kernels are built for: narrow layers
     (K, N <= 128), and wide ones (N > 128, K a multiple of 16) over a multiple of 4 rows.
-    With ``P`` (Jacobian rows) given, also whether the wide kernel is the faster choice."""
+    With ``P`` (Jacobian rows) given, also whether the wide kernel is the faster choice (``spared``: see there)."""
     if name not in FUSED_ACTS:
         return False
     if 4 <= K <= 128 and K % 4 == 0 and 1 <= N <= 128:
         return True
     return (rows is not None and rows > 0 and rows % 4 == 0 and K % 16 == 0 and N > 128 and N % 4 == 0
-            and _wide_tiles_filled(P, rows, False))
+            and _wide_tiles_filled(P, False, K, spared))
 
 
 def dense_act_residual_supported(K, N):
@@ -268,7 +273,7 @@ def norm_dense_supported(name, K, N, rows, P=None):
     """Shapes and functions ``norm_dense`` is built for (``name`` None: no activation); with
     ``P`` (Jacobian rows) given, also whether it is the faster choice."""
     return ((name is None or name in FUSED_ACTS) and rows > 0 and rows % 4 == 0 and K % 16 == 0 and K <= 512
-            and N > 128 and N % 4 == 0 and _wide_tiles_filled(P, rows, True))
+            and N > 128 and N % 4 == 0 and _wide_tiles_filled(P, True, K))
 
 
 def norm_dense(name, x, jac, lap, gamma, beta, eps, W, bias=None, param=0.0):

@@ -974,9 +974,11 @@ def _dot_parts(lc: LazyConcat, W, kwargs, thr: int):
         group = int(np.prod(lead, dtype=np.int64))
         Ktot = sum((t.a if isinstance(t, LazyBroadcast) else t).shape[-1] for t in lc.parts)
         srcs = [t.a if isinstance(t, LazyBroadcast) else t for t in lc.parts]
+        own = sum(t.shape[-1] for t in lc.parts if not isinstance(t, LazyBroadcast))  # features met once per position
         P = max(u.jacobian.max_n + 1 if u.jacobian.weak else u.jacobian.data.shape[0] for u in srcs)
         ok = (np.shape(W)[0] == Ktot and np.shape(W)[1] > 128 and group >= 1
-              and K.dense_act_supported(act, Ktot, np.shape(W)[1], rows=B * group, P=P))
+              and K.dense_act_supported(act, own if 0 < own < Ktot and group > 1 else Ktot, np.shape(W)[1], rows=B * group, P=P,
+                                        spared=Ktot))
     if not ok:
         kw = dict(kwargs)
         Kin = np.shape(W)[0] if np.ndim(W) == 2 else 0

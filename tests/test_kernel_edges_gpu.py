@@ -124,3 +124,31 @@ def test_dense_small_tiles(rows, P, Kd, N):
         assert_val(got[0], want[0], 'y')
         assert_val(got[1], want[1], 'y_jac')
         assert_lap(got[2], want[2], 'y_lap')
+
+
+# groups of 8 Jacobian rows (16 positions a tile, four per accumulator block): the last tile's positions and the last
+# group's rows cut, operand whole or in parts with a per-walker term and a skip connection
+@pytest.mark.parametrize('rows,P,N', [((1, 4), 6, 132), ((5, 4), 21, 256), ((2, 16), 39, 300), ((4, 13), 24, 256), ((9, 4), 8, 260)])
+def test_dense_act_groups_of_eight(rows, P, N):
+    from folx_amd import kernels as K
+
+    print(f'case dense_act rows={rows} P={P} N={N}', flush=True)
+    rng = np.random.default_rng(P)
+    B, n = rows
+    parts = [rand(rng, P, *rows, 32), rand(rng, P, *rows, 48)]
+    x, J, L = rand(rng, *rows, 80), np.concatenate(parts, -1), rand(rng, *rows, 80)
+    W, b = (rand(rng, 80, N) / np.sqrt(80)).astype(np.float32), rand(rng, N)
+    z = rules.dense_rule(*f64(x, J, L, W, b))
+    ref = rules.elementwise_rule('tanh', *z)
+    got = K.dense_act('tanh', dev(x), dev(J), dev(L), dev(W), dev(b))
+    assert_val(got[0], ref[0], 'y')
+    assert_val(got[1], ref[1], 'y_jac')
+    assert_lap(got[2], ref[2], 'y_lap')
+    pre = [rand(rng, B, N), rand(rng, P, B, N), rand(rng, B, N)]
+    res = [rand(rng, *rows, N), rand(rng, P, *rows, N), rand(rng, *rows, N)]
+    ref = rules.elementwise_rule('tanh', *[t + np.expand_dims(q, -2).astype(np.float64) for t, q in zip(z, pre)])
+    got = K.dense_act_parts('tanh', dev(x), dev(L), [dev(t) for t in parts], (32, 48), (0, 0), n, dev(W), dev(b), 0.0,
+                            tuple(dev(t) for t in res), tuple(dev(t) for t in pre))
+    assert_val(got[0], ref[0] + res[0], 'y')
+    assert_val(got[1], ref[1] + res[1], 'y_jac')
+    assert_lap(got[2], ref[2] + res[2], 'y_lap')
