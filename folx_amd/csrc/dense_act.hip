@@ -30,6 +30,7 @@
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) char gchar;    // global memory, so that stores stay global_store
 typedef __attribute__((address_space(1))) float gfloat;
 
@@ -329,6 +330,165 @@ __global__ __launch_bounds__(NTHR, 2) void dense_act_kernel(DAParams a) {
   if (odd) lap_step(As0); else lap_step(As1);
 }
 
+// Few Jacobian rows (P <= 6: networks whose Jacobian stays sparse per node, pair features of FermiNet-style layers).  The
+// kernel above walks such a layer in P + 2 dependent steps of one 32-row tile, each behind a barrier, so a small batch took
+// that chain's latency on a quarter of the CUs.  Here a workgroup owns 16 to 128 positions and asks for all P + 2 tiles at
+// once, waits once, and each wavefront forms its 16 x 16 block of every one of the P + 2 products side by side
+// (v_mfma_f32_16x16x4_f32: independent accumulators of 4 registers, one W operand for all of them, taken from L2 one group of
+// 16 k ahead), which leaves f', f'' and the sum of squares as plain register arithmetic.  The product is formed transposed, so
+// a lane holds 4 consecutive columns of one position and stores them 128 bits at a time.  LDS tiles as above, one per row s
+// of the triplet; 34 to 74 VGPRs, so LDS sets the occupancy.  A form with W in registers, a grid of the resident workgroups and
+// the next tile's loads behind the current product was no faster on large R (28 .. 40 % slower for P = 6) and 15 % slower on
+// small.
+// us, general kernel -> this: R = 2000, P = 4, 100 x 100: 18.7 -> 10.4; 300, 2, 16 x 16: 8.6 -> 4.0; 25 088, 6, 32 x 32 with a
+// skip connection: 50 -> 20 (4 TB/s); 262 144 of these: 260 -> 163 (4.9 TB/s).
+template <int NR>
+__global__ __launch_bounds__(512) void dense_act_few_kernel(DAParams a, int wc, int wr, int vec) {
+  extern __shared__ __attribute__((aligned(16))) float tile[];
+  const int tid = threadIdx.x;
+  const int lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int l16 = lane % 16;
+  const int lq = lane / 16;
+  const int K = a.K, N = a.N;
+  const int npr = K / 4;
+  const int64_t R = a.R, RK = R * K;
+  const int br = 16 * wr;
+  const int64_t r0 = (int64_t)blockIdx.x * br;
+
+  int sh = __builtin_ctz(npr);
+  if (sh > 4) sh = 4;
+  const int rshift = 4 - sh;
+  const int rmask = (1 << sh) - 1;
+
+  const int pieces = br * npr;
+  const int stride = pieces * 4;  // floats from one tile to the next
+  for (int c = wave * 64; c < pieces; c += 64 * wc * wr) {
+    const int q = c + lane;
+    if (q < pieces) {  // lane i's 16 bytes land at slot c + i
+      int m = q / npr;
+      const int piece = (q - m * npr) ^ ((m >> rshift) & rmask);
+      if (r0 + m >= R) m = (int)(R - 1 - r0);
+      const int off = m * K + 4 * piece;
+#pragma unroll
+      for (int s = 0; s < NR; ++s) {
+        const float* src = (s == 0 ? a.x : (s < NR - 1 ? a.jac + (s - 1) * RK : a.lap)) + r0 * K;
+        __builtin_amdgcn_global_load_lds(FOLX_GPTR(src + off), FOLX_LPTR(&tile[s * stride + c * 4]), 16, 0, 0);
+      }
+    }
+  }
+
+  const int col0 = wave % wc * 16;
+  const int row = wave / wc * 16 + l16;  // this lane's position in the tile
+  const float* wp = a.W + (int64_t)(4 * lq) * N + min(col0 + l16, N - 1);
+  const int groups = K / 16;
+  float w[4] = {0.f, 0.f, 0.f, 0.f};
+  auto load_w = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = wp[(int64_t)(16 * j + i) * N];
+  };
+  if (groups > 0) load_w(0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+
+  floatx4 acc[NR];
+#pragma unroll
+  for (int s = 0; s < NR; ++s) acc[s] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int sw = (row >> rshift) & rmask;
+  const float* base = tile + row * K;
+  for (int j = 0; j < groups; ++j) {
+    const float wv[4] = {w[0], w[1], w[2], w[3]};
+    if (j + 1 < groups) load_w(j + 1);
+    floatx4 av[NR];
+    const int at = ((4 * j + lq) ^ sw) * 4;
+#pragma unroll
+    for (int s = 0; s < NR; ++s) av[s] = *reinterpret_cast<const floatx4*>(base + s * stride + at);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int s = 0; s < NR; ++s) acc[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[i], av[s][i], acc[s], 0, 0, 0);
+  }
+  for (int piece = 4 * groups; piece < npr; ++piece) {  // the last K % 16 features, four a step
+    const float wv = a.W[(int64_t)(4 * piece + lq) * N + min(col0 + l16, N - 1)];
+    const int at = (piece ^ sw) * 4 + lq;
+#pragma unroll
+    for (int s = 0; s < NR; ++s) acc[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, base[s * stride + at], acc[s], 0, 0, 0);
+  }
+
+  // register r of a 16 x 16 block: position lane % 16, column 4 (lane / 16) + r
+  const int n0 = col0 + 4 * lq;
+  const int cols = min(4, N - n0);
+  if (r0 + row >= R || cols <= 0) return;
+  float d1[4], d2[4];
+  floatx4 ssq = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float o;
+    act_eval_fused(a.act, acc[0][r] + ((a.bias != nullptr && r < cols) ? a.bias[n0 + r] : 0.f), a.prm, o, d1[r], d2[r]);
+    acc[0][r] = o;
+#pragma unroll
+    for (int s = 1; s < NR - 1; ++s) {
+      ssq[r] += acc[s][r] * acc[s][r];
+      acc[s][r] *= d1[r];
+    }
+    acc[NR - 1][r] = d1[r] * acc[NR - 1][r] + d2[r] * ssq[r];
+  }
+  const int64_t at = (r0 + row) * N + n0, RN = R * N;
+  if (a.res != nullptr) {
+    floatx4 rv[NR];
+#pragma unroll
+    for (int s = 0; s < NR; ++s) {
+      const float* p = (s == 0 ? a.res : (s < NR - 1 ? a.res_jac + (s - 1) * RN : a.res_lap)) + at;
+      if (vec) rv[s] = *reinterpret_cast<const floatx4*>(p);
+      else
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rv[s][r] = r < cols ? p[r] : 0.f;
+    }
+#pragma unroll
+    for (int s = 0; s < NR; ++s)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[s][r] += rv[s][r];
+  }
+#pragma unroll
+  for (int s = 0; s < NR; ++s) {
+    float* p = (s == 0 ? a.y : (s < NR - 1 ? a.y_jac + (s - 1) * RN : a.y_lap)) + at;
+    if (vec) *reinterpret_cast<floatx4*>(p) = acc[s];
+    else
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (r < cols) p[r] = acc[s][r];
+  }
+}
+
+constexpr int FEW_ROWS = 6;
+constexpr int FEW_LDS = 40960;  // four workgroups a CU where several row blocks share one
+
+// When the few-rows kernel is the faster one (R, K, N over 6000 .. 200 000 x 4 .. 128 x 32 .. 128 and P = 1, 3, 6, both
+// measured).  The general kernel reads W into registers once for all rows of a tile and overlaps its loads with its matrix work, which
+// is worth 5 to 25 % once its tiles cover the CUs; below that the few-rows kernel took 0.52 .. 1.03 of its time (R = 6000).
+// It also wins where the general one multiplies 32-column strips past N or, for K > N, the columns of a wider plan: 48 x 48
+// 0.81 .. 0.91, 96 x 96 0.84 .. 0.92, K = 128 to N = 64 0.62 .. 0.81, but 100 x 100 0.95 .. 1.03 (112 columns for 128).  And it
+// reads a skip connection 128 bits at a time ahead of its stores: 0.4 .. 0.65 wherever measured.
+bool few_rows(const DAPlan& pl, int32_t P, int32_t N, bool has_res) {
+  if (P > FEW_ROWS) return false;
+  return has_res || pl.row_tiles <= 192 || 12 * ((N + 15) / 16 * 16) < 10 * 32 * pl.wc;
+}
+
+template <int NR>
+int launch_few(hipStream_t st, const DAParams& prm) {
+  const int wc = (prm.N + 15) / 16;
+  auto lds = [&](int wr) { return 64 * wr * prm.K * NR; };  // at most 64 KB for wr = 1
+  // 8 wavefronts where N leaves room for several row blocks, but no fewer than two workgroups per CU
+  int wr = 8 / wc;
+  while (wr > 1 && (lds(wr) > FEW_LDS || (prm.R + 16 * wr - 1) / (16 * wr) < 512)) --wr;
+  const int64_t blocks = (prm.R + 16 * wr - 1) / (16 * wr);
+  if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
+  const int vec = prm.N % 4 == 0 && folx_aligned16(prm.y) && folx_aligned16(prm.y_jac) && folx_aligned16(prm.y_lap) &&
+                  folx_aligned16(prm.res) && folx_aligned16(prm.res_jac) && folx_aligned16(prm.res_lap);
+  dense_act_few_kernel<NR><<<dim3((unsigned)blocks), dim3(64 * wc * wr), lds(wr), st>>>(prm, wc, wr, vec);
+  return folx_launch_status();
+}
+
 template <int KS, int WC>
 void launch_da(hipStream_t st, DAParams prm, const DAPlan& pl) {
   if (pl.G == 1) {
@@ -378,6 +538,16 @@ extern "C" int folx_hip_dense_act_fwdlap(void* stream, int32_t act, float param,
   prm.part = (float*)workspace;
   prm.R = R; prm.P = P; prm.K = K; prm.N = N; prm.G = pl.G; prm.PG = pl.PG; prm.act = act; prm.prm = param; prm.mode = 0;
   hipStream_t st = (hipStream_t)stream;
+  switch (few_rows(pl, P, N, res != nullptr) ? P : FEW_ROWS + 1) {
+    case 0: return launch_few<2>(st, prm);
+    case 1: return launch_few<3>(st, prm);
+    case 2: return launch_few<4>(st, prm);
+    case 3: return launch_few<5>(st, prm);
+    case 4: return launch_few<6>(st, prm);
+    case 5: return launch_few<7>(st, prm);
+    case FEW_ROWS: return launch_few<8>(st, prm);
+    default: break;
+  }
   const int code = pl.wc * 100 + pl.ks;
   switch (code) {
     case 101: launch_da<1, 1>(st, prm, pl); break;

@@ -152,3 +152,38 @@ def test_dense_act_groups_of_eight(rows, P, N):
     assert_val(got[0], ref[0] + res[0], 'y')
     assert_val(got[1], ref[1] + res[1], 'y_jac')
     assert_lap(got[2], ref[2] + res[2], 'y_lap')
+
+
+# up to six Jacobian rows: 1 .. 8 blocks of 16 columns and of 16 positions a workgroup, the last ones cut; features in whole
+# groups of 16, with a rest, or only a rest; one column short of a 128-bit store; outputs off the 16-byte boundary
+@pytest.mark.parametrize('R,P,Kd,N', [(1, 0, 4, 1), (17, 1, 12, 16), (31, 2, 16, 17), (2000, 4, 100, 100), (16, 6, 128, 128),
+                                      (9000, 3, 36, 30), (66000, 6, 32, 32), (15, 5, 20, 127), (8191, 2, 64, 48), (33, 6, 112, 64)])
+@pytest.mark.parametrize('act', ['tanh', 'silu'])
+def test_dense_act_few_jacobian_rows(R, P, Kd, N, act):
+    from folx_amd import kernels as K
+
+    print(f'case dense_act R={R} P={P} K={Kd} N={N} {act}', flush=True)
+    rng = np.random.default_rng(R + N)
+    t = [rand(rng, R, Kd), rand(rng, P, R, Kd), rand(rng, R, Kd)]
+    W, b = (rand(rng, Kd, N) / np.sqrt(Kd)).astype(np.float32), rand(rng, N)
+    res = [rand(rng, R, N), rand(rng, P, R, N), rand(rng, R, N)]
+    ref = rules.elementwise_rule(act, *rules.dense_rule(*f64(*t, W, b)))
+
+    def off_boundary(a):
+        return torch.nn.functional.pad(dev(a).reshape(-1), (1, 0))[1:].reshape(a.shape)
+
+    for skip in (None, tuple(dev(r) for r in res), tuple(off_boundary(r) for r in res)):
+        got = K.dense_act(act, *[dev(v) for v in t], dev(W), dev(b), 0.0, skip)
+        want = ref if skip is None else [a + r for a, r in zip(ref, res)]
+        assert_val(got[0], want[0], 'y')
+        if P:
+            assert_val(got[1], want[1], 'y_jac')
+        assert_lap(got[2], want[2], 'y_lap')
+    # a row holds its own position alone: infinities of one do not reach another
+    bad = [v.copy() for v in t]
+    for v in bad:
+        v[..., R // 2, :] = np.inf
+    got = K.dense_act(act, *[dev(v) for v in bad], dev(W), dev(b))
+    keep = np.arange(R) != R // 2
+    assert_val(got[0][keep], ref[0][keep], 'y')
+    assert_lap(got[2][keep], ref[2][keep], 'y_lap')
