@@ -858,15 +858,19 @@ struct WidePlan {
 bool plan_wide(int64_t R, int32_t P, int32_t K, int32_t N, bool norm, bool act, WidePlan& pl) {
   if (R <= 0 || R % 4 != 0 || P < 1 || K < BK || K % BK != 0 || N <= 128 || N % 4 != 0) return false;
   if (norm && K > KMAX_NORM) return false;
-  // the largest groups of Jacobian rows that leave the fewest empty tile rows
+  // The largest groups of Jacobian rows that leave the fewest empty tile rows.  Groups of 8, and tiles cut past the last
+  // position, only in launches of more workgroups than reside at once (two a CU): below that empty rows cost no time, while
+  // each group adds a slab of partial sums.
   pl.PT = 32;
+  pl.col_tiles = (N + BN - 1) / BN;
   if (!norm)
-    for (int g = 16; g >= 8; g /= 2)
-      if ((P + g - 1) / g * g < (P + pl.PT - 1) / pl.PT * pl.PT) pl.PT = g;
+    for (int g = 16; g >= 8; g /= 2) {
+      const int64_t groups = (P + pl.PT - 1) / pl.PT, tiles = (R + BM / pl.PT - 1) / (BM / pl.PT) * groups * pl.col_tiles;
+      if ((P + g - 1) / g * g < groups * pl.PT && ((g == 16 && R % 8 == 0) || tiles > 512)) pl.PT = g;
+    }
   pl.PG = (P + pl.PT - 1) / pl.PT;
   pl.pos_tiles = (R + BM / pl.PT - 1) / (BM / pl.PT);
   pl.row_tiles = pl.pos_tiles * pl.PG;
-  pl.col_tiles = (N + BN - 1) / BN;
   pl.blocks = (pl.row_tiles + NXCD - 1) / NXCD * NXCD * pl.col_tiles;
   if (pl.blocks > 0x7fffffffLL) return false;
   if (R * (int64_t)N / 4 / 256 + 1 > 0x7fffffffLL) return false;

@@ -126,9 +126,10 @@ def test_dense_small_tiles(rows, P, Kd, N):
         assert_lap(got[2], want[2], 'y_lap')
 
 
-# groups of 8 Jacobian rows (16 positions a tile, four per accumulator block): the last tile's positions and the last
-# group's rows cut, operand whole or in parts with a per-walker term and a skip connection
-@pytest.mark.parametrize('rows,P,N', [((1, 4), 6, 132), ((5, 4), 21, 256), ((2, 16), 39, 300), ((4, 13), 24, 256), ((9, 4), 8, 260)])
+# groups of 8 Jacobian rows (16 positions a tile, four per accumulator block) in launches of more than 512 tiles, of 16 or 32 in
+# smaller ones: the last tile's positions and the last group's rows cut, operand whole or in parts with a per-walker term and a skip connection
+@pytest.mark.parametrize('rows,P,N', [((1, 4), 6, 132), ((515, 4), 21, 256), ((66, 16), 39, 300), ((164, 13), 24, 256), ((1030, 4), 8, 260),
+                                      ((60, 4), 33, 256), ((521, 4), 13, 256)])
 def test_dense_act_groups_of_eight(rows, P, N):
     from folx_amd import kernels as K
 
