@@ -334,14 +334,15 @@ __global__ __launch_bounds__(NTHR, 2) void dense_act_kernel(DAParams a) {
 // kernel above walks such a layer in P + 2 dependent steps of one 32-row tile, each behind a barrier, so a small batch took
 // that chain's latency on a quarter of the CUs.  Here a workgroup owns 16 to 128 positions and asks for all P + 2 tiles at
 // once, waits once, and each wavefront forms its 16 x 16 block of every one of the P + 2 products side by side
-// (v_mfma_f32_16x16x4_f32: independent accumulators of 4 registers, one W operand for all of them, taken from L2 one group of
-// 16 k ahead), which leaves f', f'' and the sum of squares as plain register arithmetic.  The product is formed transposed, so
+// (v_mfma_f32_16x16x4_f32: independent accumulators of 4 registers, one W operand for all of them, taken from L2 16 k
+// ahead), which leaves f', f'' and the sum of squares as plain register arithmetic.  The product is formed transposed, so
 // a lane holds 4 consecutive columns of one position and stores them 128 bits at a time.  LDS tiles as above, one per row s
-// of the triplet; 34 to 74 VGPRs, so LDS sets the occupancy.  A form with W in registers, a grid of the resident workgroups and
+// of the triplet; 34 to 74 VGPRs, so LDS sets the occupancy.  The products of a column are added in the order of the kernel above (128-bit reads of 16 k in
+// another order took 1 us less a layer and stood further from 64 bits on a small FermiNet-style function).  A form with W in registers, a grid of the resident workgroups and
 // the next tile's loads behind the current product was no faster on large R (28 .. 40 % slower for P = 6) and 15 % slower on
 // small.
-// us, general kernel -> this: R = 2000, P = 4, 100 x 100: 18.7 -> 10.4; 300, 2, 16 x 16: 8.6 -> 4.0; 25 088, 6, 32 x 32 with a
-// skip connection: 50 -> 20 (4 TB/s); 262 144 of these: 260 -> 163 (4.9 TB/s).
+// us, general kernel -> this: R = 2000, P = 4, 100 x 100: 18.7 -> 11.7; 300, 2, 16 x 16: 8.6 -> 4.0; 25 088, 6, 32 x 32 with a
+// skip connection: 50 -> 20 (4 TB/s); 262 144 of these: 260 -> 167 (4.8 TB/s).
 template <int NR>
 __global__ __launch_bounds__(512) void dense_act_few_kernel(DAParams a, int wc, int wr, int vec) {
   extern __shared__ __attribute__((aligned(16))) float tile[];
@@ -380,14 +381,20 @@ __global__ __launch_bounds__(512) void dense_act_few_kernel(DAParams a, int wc, 
 
   const int col0 = wave % wc * 16;
   const int row = wave / wc * 16 + l16;  // this lane's position in the tile
-  const float* wp = a.W + (int64_t)(4 * lq) * N + min(col0 + l16, N - 1);
-  const int groups = K / 16;
-  float w[4] = {0.f, 0.f, 0.f, 0.f};
-  auto load_w = [&](int j) __attribute__((always_inline)) {
+  const float* wp = a.W + min(col0 + l16, N - 1);
+  const int groups = (K + 7) / 8;
+  // k of this lane in step e of group j: 8 j + 4 (lane / 16 % 2) + 2 e + lane / 32, so that a column's products are added in the
+  // general kernel's order (two of its steps in one)
+  const int k0 = 4 * (lq & 1) + (lq >> 1);
+  float w[4];
+  auto load_w = [&](int j) __attribute__((always_inline)) {  // groups j and j + 1
 #pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = wp[(int64_t)(16 * j + i) * N];
+    for (int i = 0; i < 4; ++i) {
+      const int k = 8 * j + k0 + 8 * (i / 2) + 2 * (i % 2);
+      w[i] = k < K ? wp[(int64_t)k * N] : 0.f;
+    }
   };
-  if (groups > 0) load_w(0);
+  load_w(0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
@@ -396,23 +403,25 @@ __global__ __launch_bounds__(512) void dense_act_few_kernel(DAParams a, int wc, 
   for (int s = 0; s < NR; ++s) acc[s] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int sw = (row >> rshift) & rmask;
   const float* base = tile + row * K;
-  for (int j = 0; j < groups; ++j) {
+  auto group = [&](int j, float w0, float w1) __attribute__((always_inline)) {
+    // past K a lane meets zeros of W and the last piece of its own row
+    const int at = ((min(2 * j + (lq & 1), npr - 1) ^ sw) * 4) + (lq >> 1);
+    float v0[NR], v1[NR];
+#pragma unroll
+    for (int s = 0; s < NR; ++s) {
+      v0[s] = base[s * stride + at];
+      v1[s] = base[s * stride + at + 2];
+    }
+#pragma unroll
+    for (int s = 0; s < NR; ++s) acc[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(w0, v0[s], acc[s], 0, 0, 0);
+#pragma unroll
+    for (int s = 0; s < NR; ++s) acc[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(w1, v1[s], acc[s], 0, 0, 0);
+  };
+  for (int j = 0; j < groups; j += 2) {
     const float wv[4] = {w[0], w[1], w[2], w[3]};
-    if (j + 1 < groups) load_w(j + 1);
-    floatx4 av[NR];
-    const int at = ((4 * j + lq) ^ sw) * 4;
-#pragma unroll
-    for (int s = 0; s < NR; ++s) av[s] = *reinterpret_cast<const floatx4*>(base + s * stride + at);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int s = 0; s < NR; ++s) acc[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[i], av[s][i], acc[s], 0, 0, 0);
-  }
-  for (int piece = 4 * groups; piece < npr; ++piece) {  // the last K % 16 features, four a step
-    const float wv = a.W[(int64_t)(4 * piece + lq) * N + min(col0 + l16, N - 1)];
-    const int at = (piece ^ sw) * 4 + lq;
-#pragma unroll
-    for (int s = 0; s < NR; ++s) acc[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, base[s * stride + at], acc[s], 0, 0, 0);
+    if (j + 2 < groups) load_w(j + 2);
+    group(j, wv[0], wv[1]);
+    if (j + 1 < groups) group(j + 1, wv[2], wv[3]);
   }
 
   // register r of a 16 x 16 block: position lane % 16, column 4 (lane / 16) + r
