@@ -389,20 +389,24 @@ __global__ __launch_bounds__(FOLX_WAVE * NW) void mhsa_kernel(MhsaArgs a) {
 // n <= 16: one wavefront covers all query rows of a (walker, head) pair, so its rows c need nothing from its neighbours:
 // q'_c, k'_c and v'_c go from memory straight into MFMA operand registers and the W wavefronts of a workgroup take the rows
 // c = w, w + W, ... with every sum over rows in registers, added through LDS once at the end (k and v wait in LDS, the same
-// for all of them: 168 registers, twelve wavefronts on a CU).  Rows and columns of the padding are lanes whose buffer offset
+// for all of them: 168 registers, twelve wavefronts on a CU; with a bias or masks and four blocks of features 182 to 194,
+// eight wavefronts).  Rows and columns of the padding are lanes whose buffer offset
 // lies past the descriptor's end: they read zeros and their stores are dropped, so no access is tested.  DT = 1, 2 or 4
 // blocks of 16 features.
 // Bound by HBM (16 n d bytes per pair and row, at 4.7-5.1 TB/s), for few pairs by the latency of a wavefront's rows.  One
 // wavefront per pair with the tiles of mhsa_kernel (two barriers and an LDS copy of k', v' per row) was bound by that chain:
 // 1200 pairs of 13 x 64, P = 39: 300 -> 139 us; 256 of 10 x 64, P = 30: 112 -> 24 us; 2048 of 16 x 16, P = 48: 146 -> 94 us;
-// 16000 of 16 x 64, P = 48: 2.69 -> 2.56 ms.
+// 16000 of 16 x 64, P = 48: 2.69 -> 2.56 ms.  With a bias, masks, both (former kernel -> this; in parentheses held to 168
+// registers, 15 to 32 of them spilled, and the bias loaded where it is added): 1200 pairs of 13 x 64, P = 39: 414 -> 150 us
+// (202), 742 -> 153 (210), 847 -> 158 (286); 2048 of 12 x 36, P = 36: 202 -> 162 (275), 503 -> 189 (280), 368 -> 192 (392);
+// 4096 of 16 x 64, P = 48: 752 -> 690 (844), 2053 -> 617 (832), 2324 -> 685 (1163).
 constexpr int NXCD = 8;
 constexpr uint32_t FAR = 0x40000000u;  // past every descriptor's end, also with the row and piece offsets added
 typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
 
 template <int DT, bool EDGE, bool MASKED>
-__global__ __launch_bounds__(512, 3) void mhsa_small_kernel(MhsaArgs a) {
+__global__ __launch_bounds__(512, DT == 4 && (EDGE || MASKED) ? 2 : 3) void mhsa_small_kernel(MhsaArgs a) {
   constexpr float BIG = 1e20f;
   constexpr int NS = 20;           // LDS row stride of a 16 x 16 tile
   constexpr int NRED = 12 + 4 * DT;
@@ -500,10 +504,16 @@ __global__ __launch_bounds__(512, 3) void mhsa_small_kernel(MhsaArgs a) {
     }
   };
   const int64_t etok = (int64_t)H * n, ebase = (b * n) * etok + (int64_t)h * n, eslice = B * n * etok;
-  auto edge_add = [&](const float* src, floatx4& acc) __attribute__((always_inline)) {
+  const uint32_t ebytes = (uint32_t)(((int64_t)n * etok - (int64_t)h * n) * 4);
+  uint32_t eo[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (4 * lg + r < n && l16 < n) acc[r] += src[ebase + (int64_t)(4 * lg + r) * etok + l16];
+  for (int r = 0; r < 4; ++r) eo[r] = 4 * lg + r < n && l16 < n ? (uint32_t)((4 * lg + r) * (int32_t)etok + l16) * 4u : FAR;
+  auto load_e = [&](const float* src) __attribute__((always_inline)) -> floatx4 {
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src) + ebase, 0, ebytes, 0x00027000);
+    floatx4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, eo[r], 0, 0));
+    return v;
   };
   auto qk = [&](const float4 (&x)[DT], const float4 (&y)[DT], floatx4& acc) __attribute__((always_inline)) {
 #pragma unroll
@@ -541,18 +551,23 @@ __global__ __launch_bounds__(512, 3) void mhsa_small_kernel(MhsaArgs a) {
   auto src_of = [&](const float* jac, const float* lap, int c) __attribute__((always_inline)) -> const float* {
     return c == P ? lap : jac + (int64_t)c * slice;
   };
-  // The next row's q', k' are asked for as soon as the products that read this row's are issued, and its v' behind the
-  // other three: half a row of matrix work ahead in the same registers, the rest of the latency is other wavefronts' time.
+  // The next row's q', k' (and bias) are asked for as soon as the products that read this row's are issued, and its v'
+  // behind the other three: half a row of matrix work ahead in the same registers, the rest of the latency is other
+  // wavefronts' time.  (Loads complete in order: a bias loaded where it is added would wait for the next row's operands.)
   float4 qj[DT], kj[DT];
+  floatx4 ej;
   float vj[DT][4];
   auto fetch_qk = [&](int c) __attribute__((always_inline)) {
     load_rows(src_of(a.qj, a.ql, c), aoj, qj);
     load_rows(src_of(a.kj, a.kl, c), aoj, kj);
+    if constexpr (EDGE) ej = load_e(c == P ? a.el : a.ej + (int64_t)c * eslice);
   };
   auto fetch_v = [&](int c) __attribute__((always_inline)) { load_v(src_of(a.vj, a.vl, c), voj, vj); };
 
   float4 qa[DT];
   load_rows(a.q, ao, qa);
+  floatx4 e0;
+  if constexpr (EDGE) e0 = load_e(a.e);
   if (w == 0) {
     float4 kr[DT];
     float vr[DT][4];
@@ -595,7 +610,7 @@ __global__ __launch_bounds__(512, 3) void mhsa_small_kernel(MhsaArgs a) {
     k_rows(kb);
     qk(qa, kb, pc);
   }
-  if constexpr (EDGE) edge_add(a.e, pc);
+  if constexpr (EDGE) pc += e0;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     float sv = pc[r];
@@ -635,8 +650,8 @@ __global__ __launch_bounds__(512, 3) void mhsa_small_kernel(MhsaArgs a) {
       }
       qk(qa, kj, sj);
       if (!is_lap) qk(qj, kj, G);
+      if constexpr (EDGE) sj += ej;
       if (next) fetch_qk(c + W);
-      if constexpr (EDGE) edge_add(is_lap ? a.el : a.ej + (int64_t)c * eslice, sj);
       floatx4 pj;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -788,8 +803,8 @@ static int mhsa_entry(void* stream, const float* q, const float* q_jac, const fl
   const int nw = (n + 15) / 16;
   switch (nw) {
     case 1:
-      // the buffer descriptors of the small form span a walker's (n, H, d) block with 32-bit offsets
-      if ((int64_t)n * H * d * 4 >= (int64_t)FAR) return launch_mhsa_d<2>(st, a);
+      // the buffer descriptors of the small form span a walker's (n, H, d) and (n, H, n) blocks with 32-bit offsets
+      if ((int64_t)n * H * (e && n > d ? n : d) * 4 >= (int64_t)FAR) return launch_mhsa_d<2>(st, a);
       switch ((d + 15) / 16) {
         case 1: return launch_mhsa_small<1>(st, a);
         case 2: return launch_mhsa_small<2>(st, a);

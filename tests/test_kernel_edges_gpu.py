@@ -52,6 +52,13 @@ def test_mhsa_short_sequences(B, n, H, d, P, edge, masked):
     assert all(bool(torch.isfinite(t).all()) for t in got)
 
 
+# both together, every block count of features; 48: three blocks on the instance for four
+@pytest.mark.parametrize('B,n,H,d,P', [(2, 13, 4, 64, 39), (3, 16, 2, 48, 7), (1, 16, 1, 36, 17), (5, 3, 3, 20, 9), (70, 9, 3, 8, 12),
+                                       (2, 5, 2, 64, 0), (2, 17, 2, 64, 5)])
+def test_mhsa_short_sequences_bias_and_masks(B, n, H, d, P):
+    test_mhsa_short_sequences(B, n, H, d, P, True, True)
+
+
 # up to 32 x 32 x 32 one wavefront per batch element (1 / 4 / 8 sharing the Jacobian rows), 33: the tiled form; pieces of
 # four k whole and aligned or not, rows of y whole or not
 @pytest.mark.parametrize('NB0,NB1,I,J,Kc,P', [(3, 2, 16, 16, 16, 39), (1, 1, 17, 32, 20, 8), (2, 3, 32, 17, 32, 9),
