@@ -803,8 +803,11 @@ static int mhsa_entry(void* stream, const float* q, const float* q_jac, const fl
   const int nw = (n + 15) / 16;
   switch (nw) {
     case 1:
-      // the buffer descriptors of the small form span a walker's (n, H, d) and (n, H, n) blocks with 32-bit offsets
-      if ((int64_t)n * H * (e && n > d ? n : d) * 4 >= (int64_t)FAR) return launch_mhsa_d<2>(st, a);
+      // The buffer descriptors of the small form span a walker's (n, H, d) and (n, H, n) blocks with 32-bit offsets, and
+      // beyond 16 features it stores two or four floats at a time; mhsa_kernel stores single ones.
+      if ((int64_t)n * H * (e && n > d ? n : d) * 4 >= (int64_t)FAR ||
+          (d > 16 && !(folx_aligned16(o) && folx_aligned16(o_jac) && folx_aligned16(o_lap))))
+        return launch_mhsa_d<2>(st, a);
       switch ((d + 15) / 16) {
         case 1: return launch_mhsa_small<1>(st, a);
         case 2: return launch_mhsa_small<2>(st, a);

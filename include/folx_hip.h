@@ -555,7 +555,8 @@ int folx_hip_solve_fwdlap(void* stream, const float* A, const float* A_jac, cons
  *   (1 = active coordinate) or NULL.
  * Replaces mhsa_forward_laplacian and its Pallas kernel
  * (folx/experimental/pallas/attention/forward_laplacian.py:27-179, :349-487).
- * Supported: n <= 64, d <= 64, d % 4 == 0.
+ * Supported: n <= 64, d <= 64, d % 4 == 0, q, k, v and their derivatives 16-byte aligned
+ * (FOLX_HIP_ENOTSUP otherwise); the outputs may start at any float.
  */
 int folx_hip_mhsa_fwdlap(void* stream, const float* q, const float* q_jac, const float* q_lap,
                          const float* k, const float* k_jac, const float* k_lap,

@@ -59,6 +59,34 @@ def test_mhsa_short_sequences_bias_and_masks(B, n, H, d, P):
     test_mhsa_short_sequences(B, n, H, d, P, True, True)
 
 
+# outputs that start at any float: single stores for 16 features, the general kernel beyond; what lies around them is kept
+@pytest.mark.parametrize('n,H,d,P', [(16, 2, 64, 5), (13, 3, 32, 9), (7, 2, 20, 3), (5, 1, 16, 8), (20, 2, 64, 3)])
+@pytest.mark.parametrize('edge', [False, True])
+def test_mhsa_outputs_off_the_16_byte_boundary(n, H, d, P, edge):
+    from folx_amd import _lib
+
+    print(f'case mhsa unaligned outputs n={n} H={H} d={d} P={P} edge={edge}', flush=True)
+    rng = np.random.default_rng(d)
+    B = 2
+    args = []
+    for s in (1 / np.sqrt(d), 1.0, 1.0):
+        args += [s * rand(rng, B, n, H, d), s * rand(rng, P, B, n, H, d), s * rand(rng, B, n, H, d)]
+    e = [rand(rng, B, n, H, n), rand(rng, P, B, n, H, n), rand(rng, B, n, H, n)] if edge else []
+    ref = rules.mhsa_rule(*f64(*args), np.ones((B, n), dtype=bool), np.ones((P, B), dtype=bool), *f64(*(e or [None] * 3)))
+    ins = [dev(t) for t in args[:6] + e + args[6:]]
+    size = B * n * H * d
+    outs = [torch.full((m + 8,), 7.0, device='cuda') for m in (size, P * size, size)]
+    fn = _lib.load().folx_hip_mhsea_fwdlap if edge else _lib.load().folx_hip_mhsa_fwdlap
+    _lib.check(fn(torch.cuda.current_stream().cuda_stream, *[t.data_ptr() for t in ins], None, None,
+                  *[t.data_ptr() + 4 * (i + 1) for i, t in enumerate(outs)], B, n, H, d, P), 'mhsa')
+    got = [t[i + 1:i + 1 + m] for i, (t, m) in enumerate(zip(outs, (size, P * size, size)))]
+    assert_val(got[0].reshape(ref[0].shape), ref[0], 'o')
+    assert_val(got[1].reshape(ref[1].shape), ref[1], 'o_jac')
+    assert_lap(got[2].reshape(ref[2].shape), ref[2], 'o_lap')
+    for i, (t, m) in enumerate(zip(outs, (size, P * size, size))):
+        assert bool((t[:i + 1] == 7.0).all()) and bool((t[i + 1 + m:] == 7.0).all())
+
+
 # up to 32 x 32 x 32 one wavefront per batch element (1 / 4 / 8 sharing the Jacobian rows), 33: the tiled form; pieces of
 # four k whole and aligned or not, rows of y whole or not
 @pytest.mark.parametrize('NB0,NB1,I,J,Kc,P', [(3, 2, 16, 16, 16, 39), (1, 1, 17, 32, 20, 8), (2, 3, 32, 17, 32, 9),

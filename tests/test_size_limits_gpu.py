@@ -120,6 +120,30 @@ def test_attention_at_shapes_the_kernels_do_not_take():
     masked_attention_beyond_kernel_sizes(run, to_np, n=1, H=1, d=1, valid=1, B=1)
 
 
+def test_attention_on_a_walker_whose_heads_take_a_gigabyte():
+    """16 positions, 2^18 heads of 64: one walker's q is 2^30 bytes, past the 32-bit offsets of the kernel for short sequences.  The heads
+    are independent, so the same heads as 256 walkers of 1024 (which that kernel takes) give the same result up to the order
+    of the sums: at most 64 products of O(1) numbers, 64 * 2^-24 of the sum of their magnitudes (up to 64) at the very worst."""
+    from folx_amd import kernels as K
+
+    n, H, d, parts = 16, 1 << 18, 64, 256
+    g = torch.Generator(device='cuda').manual_seed(9)
+    print('case attention n=16 H=2^18 d=64', flush=True)
+    ins = []
+    for s in (0.125, 1.0, 1.0):
+        ins += [s * torch.randn(*lead, 1, n, H, d, device='cuda', generator=g) for lead in ((), (1,), ())]
+
+    def as_walkers(t):  # (.., 1, n, H, d) -> (.., parts, n, H / parts, d)
+        v = t.reshape(*t.shape[:-4], n, parts, H // parts, d).movedim(-3, -4)
+        return v.contiguous()
+
+    whole = K.mhsa(*ins)
+    split = K.mhsa(*[as_walkers(t) for t in ins])
+    for w, s in zip(whole, split):
+        assert bool(torch.isfinite(w).all())
+        assert (as_walkers(w) - s).abs().max().item() < 64 * 64 * 2.0 ** -24
+
+
 def test_masked_attention_on_more_than_64_positions():
     """70 electrons of which 50 are real (the coordinates of the others inactive), 2 heads of 8: beyond the attention
     kernels' n <= 64, so the rule runs through the product and softmax rules with the masks applied; valid rows equal
