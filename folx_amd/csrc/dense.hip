@@ -8,8 +8,8 @@
 // double-buffered LDS tiles, one barrier per chunk.  For N > 128 the tile is 128 x 256 on 8
 // wavefronts (each 64 x 64), so a layer of width 256 reads its A rows from HBM exactly once
 // and two workgroups share a CU; narrower layers use 128 x {128, 64, 32} tiles on 4
-// wavefronts, and so do launches that such tiles would spread unevenly over the CUs, as 64 x 64 (the rule stands at the
-// entry point).
+// wavefronts, and so do launches that such tiles would spread unevenly over the CUs, as 64 x 64 (the rule stands in
+// dense_tiles.h).
 //
 // Main path (K a multiple of 16, 16-byte aligned operands): the chunks go from global memory
 // straight into LDS (global_load_lds_dwordx4), no staging registers and no LDS store
@@ -41,6 +41,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "dense_tiles.h"
 #include "split_bf16.h"
 
 namespace {
@@ -824,19 +825,10 @@ extern "C" int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const fl
     dense_n1_kernel<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(sg, W, bias, K, total);
     return folx_launch_status();
   }
-  // A CU works through its share of 128 x 256 tiles (8 units of 64 x 64; 128 x 128: 4) at the rate of the matrix pipe,
-  // however many share it, so a launch takes ceil(tiles / 256) tile times; 64 x 64 tiles divide finer, also the columns
-  // (N = 160 is 192 instead of 256), at an eighth less rate (twice the LDS reads per product).  K = N = 256: 1280 rows
-  // 36 -> 10 us, 20 480 rows (160 tiles) 40 -> 30, 47 104 (368) 73 -> 62, 82 432 (644) 105 -> 101; 159 900 rows
-  // (1249 tiles) would go 173 -> 191.  The opt-in products have the 128 x 256 tile only.
-  if (N > 64 && vec && K % BK == 0 && (N <= 128 || folx_gemm_mode() != FOLX_HIP_GEMM_BF16X3)) {
-    int64_t big = 0, small = 0;
-    for (int s = 0; s < 3; ++s) { big += (sg.rows[s] + 127) / 128; small += (sg.rows[s] + 63) / 64; }
-    const double units = N > 128 ? 8.0 : 4.0;
-    big *= N > 128 ? (N + 255) / 256 : 1;
-    small *= (N + 63) / 64;
-    if (1.16 * (double)small < units * (double)((big + 255) / 256 * 256))
-      return launch_dma<64, 64, 2, 2>(st, sg, W, bias, K, N, has_res);
+  if (N > 64 && vec && K % BK == 0) {
+    bool small;
+    folx_dense_units(sg.rows, N, folx_gemm_mode() == FOLX_HIP_GEMM_BF16X3, small);
+    if (small) return launch_dma<64, 64, 2, 2>(st, sg, W, bias, K, N, has_res);
   }
   if (N > 128) return launch_cfg<128, 256, 2, 4, 2>(st, sg, W, bias, K, N, vec, has_res);
   if (N > 64) return launch_cfg<128, 128, 2, 2, 3>(st, sg, W, bias, K, N, vec, has_res);

@@ -520,6 +520,20 @@ extern "C" int64_t folx_hip_dense_act_workspace_bytes(int64_t R, int32_t P, int3
   return pl.ws_bytes;
 }
 
+extern "C" int folx_hip_dense_act_form(int64_t R, int32_t P, int32_t K, int32_t N, int32_t has_res) {
+  DAPlan pl;
+  if (R <= 0 || P < 0) return FOLX_HIP_EINVAL;
+  if (plan_dense_act(R, P, K, N, pl)) return few_rows(pl, P, N, has_res != 0) ? FOLX_HIP_FORM_FEW : FOLX_HIP_FORM_TILES;
+  return folx_dense_act_wide_group(R, P, K, N);
+}
+
+extern "C" int folx_hip_dense_act_faster(int64_t R, int32_t P, int32_t K, int32_t N, int32_t plain_K) {
+  DAPlan pl;
+  if (R <= 0 || P < 0 || plain_K <= 0) return FOLX_HIP_EINVAL;
+  if (plan_dense_act(R, P, K, N, pl)) return 1;
+  return folx_dense_act_wide_faster(R, P, K, N, plain_K);
+}
+
 extern "C" int folx_hip_dense_act_fwdlap(void* stream, int32_t act, float param, const float* x, const float* jac,
                                          const float* lap, const float* W, const float* bias, const float* res,
                                          const float* res_jac, const float* res_lap, float* y,

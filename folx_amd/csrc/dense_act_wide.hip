@@ -46,11 +46,13 @@
 // (lane l, register j of group t <-> k = 8 t + 4 (l / 32) + j), piece c of an A row stored at
 // slot c ^ ((row / 2) % 4).  Only the address a lane asks for differs: tile row m is
 // Jacobian row p0 + m % 32 of position r0 + m / 32.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
 #include "activations.h"
 #include "dense_act_wide.h"
+#include "dense_tiles.h"
 #include "split_bf16.h"
 
 namespace {
@@ -109,8 +111,8 @@ struct WideParams {
 
 // PT = Jacobian rows of a tile: 32 (4 positions per tile, one per accumulator block), or 16 for
 // the activation alone (8 positions per tile, two per block: registers 0-7 of a block belong
-// to the first, 8-15 to the second), or 8 (four per block), whichever leaves the fewest empty rows
-// (plan_wide): P = 21 fills 24 rows instead of 32, P = 39 fills 40 instead of 48 or 64.  A 7-electron FermiNet-style step of
+// to the first, 8-15 to the second), or 8 (four per block): fewer empty rows (P = 21 fills 24 instead of 32, P = 39 fills 40
+// instead of 48 or 64) for more epilogue work per row (act_group).  A 7-electron FermiNet-style step of
 // 512 walkers, whose layers went unfused with 832 instead of 320 contracted features: 2.58 -> 1.48 ms.  The activation's tiles may
 // hold more positions than are left: those past R read position R - 1 and are neither stored nor summed.
 // SPLIT: the products on the bf16 matrix pipe from operands split into three bf16 pieces, with
@@ -855,26 +857,77 @@ struct WidePlan {
   int32_t PG, PT, col_tiles;
 };
 
+// What the forms of a dense + activation layer cost: times in us of a 64 x 64 tile and contracted feature on one CU (140
+// TFLOP/s over the chip; 233 of fp32 products from bf16 pieces), the work around the K loop in features of that cost, the
+// launches, and a MB of a streaming pass.  Fitted to 183 layers per mode (R = 500 .. 40 000, P = 3 .. 183, K = 16 .. 512,
+// N = 132 .. 512, all four forms timed): 6 and 7 % rms.
+struct WideRates {
+  double feature, plain, group8, group16, group32, plain_launches, fused_launches, mb;
+};
+constexpr WideRates RATES[2] = {{0.015, 46, 50, 36, 29, 9, 13, 0.14}, {0.009, 51, 103, 74, 55, 8, 9, 0.19}};
+
+double wide_time(bool split, int64_t R, int32_t P, int32_t K, int32_t N, int PT) {
+  const WideRates& c = RATES[split];
+  const int64_t groups = (P + PT - 1) / PT, tiles = (R + BM / PT - 1) / (BM / PT) * groups * ((N + BN - 1) / BN);
+  const int64_t rows[3] = {R, 0, R};
+  bool small;
+  const double around = PT == 8 ? c.group8 : (PT == 16 ? c.group16 : c.group32);
+  return c.fused_launches + folx_dense_units(rows, N, split, small) * c.feature * (K + c.plain) +
+         8.0 * (double)((tiles + 255) / 256) * c.feature * (K + around) + c.mb * 4e-6 * (double)R * N * (double)(groups + 4);
+}
+
+double plain_time(bool split, int64_t R, int32_t P, int32_t K, int32_t N) {
+  const WideRates& c = RATES[split];
+  const int64_t rows[3] = {R, P * R, R};
+  bool small;
+  return c.plain_launches + folx_dense_units(rows, N, split, small) * c.feature * (K + c.plain) +
+         c.mb * 4e-6 * (double)R * N * 2.0 * (P + 2);
+}
+
+// A form replaces the one that needs no estimate (groups of 16 where they divide the positions and leave fewer empty rows than
+// 32; the plain product where those leave more than an eighth of the rows empty) only for this much less time: the
+// estimate's own error.
+constexpr double GAIN = 0.95;
+
+int base_group(int64_t R, int32_t P) { return R % 8 == 0 && (P + 15) / 16 * 16 < (P + 31) / 32 * 32 ? 16 : 32; }
+
+// Jacobian rows of a group for the activation alone.  One group of 8 (P <= 8) would be a layer of short launches, where the
+// plain product was as fast.  Of the 183 layers none is more than 5 % slower than in the form that needs no estimate; the
+// fewest empty rows alone were 6 to 52 % slower on 30 of them (R = 1788, P = 21, K = 64, N = 300: plain 45 us, groups
+// of 8 65; R = 6000, P = 117, K = 64, N = 256: groups of 32 297 us, of 8 329; bf16x3, R = 1968, P = 87, K = 16, N = 256: 50 and 71).
+// 180 other layers (R = 250 .. 60 000, P = 2 .. 120): 0.88 of the time of the forms without an estimate in the mean, 0.90 with bf16x3
+// (the fewest empty rows: 0.92 and 0.94, more than 3 % slower on 33); four 4 to 6 % slower, among them calls of the same
+// form, so within the noise of 20 us.
+int act_group(bool split, int64_t R, int32_t P, int32_t K, int32_t N) {
+  const int base = base_group(R, P);
+  int best = base;
+  double least = GAIN * wide_time(split, R, P, K, N, base);
+  for (int g = 32; g >= (P > 8 ? 8 : 16); g /= 2) {
+    const double t = wide_time(split, R, P, K, N, g);
+    if (t < least) { best = g; least = t; }
+  }
+  return best;
+}
+
 bool plan_wide(int64_t R, int32_t P, int32_t K, int32_t N, bool norm, bool act, WidePlan& pl) {
   if (R <= 0 || R % 4 != 0 || P < 1 || K < BK || K % BK != 0 || N <= 128 || N % 4 != 0) return false;
   if (norm && K > KMAX_NORM) return false;
-  // The largest groups of Jacobian rows that leave the fewest empty tile rows.  Groups of 8, and tiles cut past the last
-  // position, only in launches of more workgroups than reside at once (two a CU): below that empty rows cost no time, while
-  // each group adds a slab of partial sums.
   pl.PT = 32;
-  pl.col_tiles = (N + BN - 1) / BN;
-  if (!norm)
-    for (int g = 16; g >= 8; g /= 2) {
-      const int64_t groups = (P + pl.PT - 1) / pl.PT, tiles = (R + BM / pl.PT - 1) / (BM / pl.PT) * groups * pl.col_tiles;
-      if ((P + g - 1) / g * g < groups * pl.PT && ((g == 16 && R % 8 == 0) || tiles > 512)) pl.PT = g;
+  int32_t slabs = 0;
+  if (!norm)  // the workspace serves both product modes: the query and the launch may meet different ones
+    for (bool split : {false, true}) {
+      const int g = act_group(split, R, P, K, N);
+      slabs = std::max(slabs, (P + g - 1) / g);
+      if (split == (folx_gemm_mode() == FOLX_HIP_GEMM_BF16X3)) pl.PT = g;
     }
+  pl.col_tiles = (N + BN - 1) / BN;
   pl.PG = (P + pl.PT - 1) / pl.PT;
   pl.pos_tiles = (R + BM / pl.PT - 1) / (BM / pl.PT);
   pl.row_tiles = pl.pos_tiles * pl.PG;
   pl.blocks = (pl.row_tiles + NXCD - 1) / NXCD * NXCD * pl.col_tiles;
   if (pl.blocks > 0x7fffffffLL) return false;
   if (R * (int64_t)N / 4 / 256 + 1 > 0x7fffffffLL) return false;
-  const int64_t slab = (int64_t)pl.PG * R * N;
+  const int64_t slab = (int64_t)std::max(pl.PG, slabs) * R * N;
   int64_t o = 0;
   auto take = [&](int64_t n) { const int64_t at = o; o += (n + 3) / 4 * 4; return at; };
   pl.o_ss = act ? take(slab) : 0;
@@ -971,6 +1024,20 @@ int run_wide(hipStream_t st, bool norm, int32_t act, float param, const float* x
 }
 
 }  // namespace
+
+int folx_dense_act_wide_group(int64_t R, int32_t P, int32_t K, int32_t N) {
+  WidePlan pl;
+  return plan_wide(R, P, K, N, false, true, pl) ? pl.PT : FOLX_HIP_ENOTSUP;
+}
+
+int folx_dense_act_wide_faster(int64_t R, int32_t P, int32_t K, int32_t N, int32_t plain) {
+  WidePlan pl;
+  if (!plan_wide(R, P, K, N, false, true, pl)) return FOLX_HIP_ENOTSUP;
+  const int base = base_group(R, P);
+  if ((P + base - 1) / base * base <= 1.125 * P) return 1;
+  const bool split = folx_gemm_mode() == FOLX_HIP_GEMM_BF16X3;
+  return wide_time(split, R, P, K, N, pl.PT) < GAIN * plain_time(split, R, P, plain, N);
+}
 
 int64_t folx_dense_act_wide_ws_bytes(int64_t R, int32_t P, int32_t K, int32_t N) {
   WidePlan pl;

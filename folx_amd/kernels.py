@@ -158,36 +158,18 @@ def dense(x, jac, lap, W, bias=None, res=None, row_slice=None):
 FUSED_ACTS = ('tanh', 'silu', 'logistic', 'sigmoid', 'softplus', 'exp', 'sin', 'cos', 'square')
 
 
-def _wide_tiles_filled(P, norm, K, N, rows, spared=None):
-    """Whether the wide fused kernels are the faster choice.  They cut their tiles into groups of 32 Jacobian rows (for the
-    activation alone also 16 or 8, whichever wastes least, as in the kernels' plan), and the empty rows of a last group are matrix work: for
-    LayerNorm up to an eighth of the rows.  For the activation the fused form contracts ``K`` features of ``padded`` rows,
-    a tenth slower than the plain product, which contracts ``spared`` (the whole concatenation, where the fused form
-    reads it in parts; else ``K``) features of P rows and is followed by a pass over the result, the time of
-    contracting 84 features more."""
-    if P is None:
-        return True
-    if norm:
-        return -(-P // 32) * 32 <= 1.125 * P
-    PT = 32
-    for g in (16, 8):
-        groups = -(-P // PT)
-        if -(-P // g) * g < groups * PT and ((g == 16 and rows % 8 == 0) or -(-rows * PT // 128) * groups * -(-N // 256) > 512):
-            PT = g
-    padded = -(-P // PT) * PT
-    return padded <= 1.125 * P or 1.1 * padded * K <= P * ((spared or K) + 84)
-
-
 def dense_act_supported(name, K, N, rows=None, P=None, spared=None):
     """Shapes and functions the fused dense + activation kernels are built for: narrow layers
     (K, N <= 128), and wide ones (N > 128, K a multiple of 16) over a multiple of 4 rows.
-    With ``P`` (Jacobian rows) given, also whether the wide kernel is the faster choice (``spared``: see there)."""
+    With ``P`` (Jacobian rows) given, also whether the wide kernel is expected to be faster than the plain product over
+    ``spared`` features (the whole concatenation, where the fused form reads it in parts; else ``K``) and the activation
+    after it: the library knows the tiles of both (folx_hip_dense_act_faster)."""
     if name not in FUSED_ACTS:
         return False
     if 4 <= K <= 128 and K % 4 == 0 and 1 <= N <= 128:
         return True
     return (rows is not None and rows > 0 and rows % 4 == 0 and K % 16 == 0 and N > 128 and N % 4 == 0
-            and _wide_tiles_filled(P, False, K, N, rows, spared))
+            and (P is None or _lib.load().folx_hip_dense_act_faster(rows, P, K, N, spared or K) == 1))
 
 
 def dense_act_residual_supported(K, N):
@@ -276,9 +258,10 @@ def dense_act_parts(name, x, lap, jac_parts, widths, broadcast, group, W, bias=N
 
 def norm_dense_supported(name, K, N, rows, P=None):
     """Shapes and functions ``norm_dense`` is built for (``name`` None: no activation); with
-    ``P`` (Jacobian rows) given, also whether it is the faster choice."""
+    ``P`` (Jacobian rows) given, also whether it is the faster choice: its tiles hold groups of 32 Jacobian rows, and the
+    empty rows of a last group are matrix work, more than the fusion saves beyond an eighth."""
     return ((name is None or name in FUSED_ACTS) and rows > 0 and rows % 4 == 0 and K % 16 == 0 and K <= 512
-            and N > 128 and N % 4 == 0 and _wide_tiles_filled(P, True, K, N, rows))
+            and N > 128 and N % 4 == 0 and (P is None or -(-P // 32) * 32 <= 1.125 * P))
 
 
 def norm_dense(name, x, jac, lap, gamma, beta, eps, W, bias=None, param=0.0):

@@ -199,6 +199,21 @@ int folx_hip_dense_act_fwdlap(void* stream, int32_t act, float param, const floa
                               int64_t workspace_bytes);
 
 /*
+ * Host-only questions about a shape, answered for the current product mode; nothing is launched.
+ * folx_hip_dense_act_form: the form that folx_hip_dense_act_fwdlap takes (`has_res`: with a skip
+ * connection): FOLX_HIP_FORM_TILES or FOLX_HIP_FORM_FEW for a narrow layer, the Jacobian rows of a
+ * tile group (8, 16 or 32) for a wide one.
+ * folx_hip_dense_act_faster: 1 where the fused rule is expected to be faster than
+ * folx_hip_dense_fwdlap over plain_K features (K, or the whole concatenation whose parts the fused rule
+ * reads) followed by folx_hip_elementwise_fwdlap, 0 where it is not.
+ * FOLX_HIP_ENOTSUP for shapes that the rule does not take.
+ */
+#define FOLX_HIP_FORM_TILES 1
+#define FOLX_HIP_FORM_FEW 2
+int folx_hip_dense_act_form(int64_t R, int32_t P, int32_t K, int32_t N, int32_t has_res);
+int folx_hip_dense_act_faster(int64_t R, int32_t P, int32_t K, int32_t N, int32_t plain_K);
+
+/*
  * folx_hip_dense_act_fwdlap for a wide layer whose input is a concatenation along the feature
  * axis that is never formed: part i contributes widths[i] consecutive features (multiples of
  * 16, at most 8 parts, K = their sum), jac_parts[i] is its Jacobian [P][rows_i][widths[i]]

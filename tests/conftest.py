@@ -11,6 +11,13 @@ sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
 
 def pytest_configure(config):
     config.addinivalue_line('markers', 'gpu: test needs a real MI355X (run with -m gpu)')
+    # rules ask the kernel library about shapes, on the host too
+    from folx_amd import _lib
+
+    if not os.path.exists(_lib.LIBPATH) and not hasattr(config, 'workerinput'):
+        from folx_amd import build
+
+        build.build(verbose=False)
 
 
 def pytest_collection_modifyitems(config, items):

@@ -171,3 +171,56 @@ def test_product_fails_loudly_without_gpu():
         pytest.skip('GPU present')
     with pytest.raises(_lib.FolxHipError):
         folx_amd.forward_laplacian(lambda x: fnp.tanh(x), 0)(np.zeros(3, np.float32))
+
+
+# us (plain product + activation, groups of 8, 16, 32) of a dense + activation layer, measured in both product modes: a form whose
+# estimate is not well ahead must not displace the faster one
+MEASURED_LAYERS = [
+    # mode, R, P, K, N, times, Jacobian rows of a group, whether the fused rule is the faster one
+    ('f32', 5376, 8, 512, 256, (152, 176, 237, 419), None, 0),
+    ('f32', 1788, 21, 64, 300, (45, 65, 63, 61), None, 0),
+    ('f32', 6000, 117, 64, 256, (518, 329, 319, 297), 32, 1),
+    ('f32', 3584, 39, 256, 256, (230, 209, 231, 263), 8, 1),
+    ('f32', 5376, 24, 512, 256, (380, 321, 441, 436), 8, 1),
+    ('bf16x3', 5376, 21, 512, 256, (218, 244, 304, 294), None, 0),
+    ('bf16x3', 3584, 8, 256, 256, (55, 65, 76, 112), None, 0),
+    ('bf16x3', 6000, 117, 64, 256, (453, 310, 286, 261), 32, 1),
+    ('bf16x3', 1968, 87, 16, 256, (104, 71, 57, 50), 32, 1),
+]
+
+
+@pytest.mark.parametrize('mode,R,P,K,N,times,group,faster', MEASURED_LAYERS)
+def test_wide_dense_act_takes_the_form_that_was_measured_faster(lib, mode, R, P, K, N, times, group, faster):
+    before = lib.folx_hip_get_gemm_mode()
+    lib.folx_hip_set_gemm_mode(_lib.GEMM_MODE[mode])
+    try:
+        assert lib.folx_hip_dense_act_faster(R, P, K, N, K) == faster
+        if group is not None:
+            assert lib.folx_hip_dense_act_form(R, P, K, N, 0) == group
+            assert dict(zip((8, 16, 32), times[1:]))[group] <= 1.05 * min(times)
+        else:
+            assert times[0] == min(times)
+        # read in parts, the fused rule contracts 320 of 832 features
+        assert lib.folx_hip_dense_act_faster(3584, 21, 320, 256, 832) == 1
+    finally:
+        lib.folx_hip_set_gemm_mode(before)
+
+
+def test_one_workspace_serves_both_product_modes(lib):
+    before = lib.folx_hip_get_gemm_mode()
+    forms, sizes = [], []
+    for mode in _lib.GEMM_MODE.values():
+        lib.folx_hip_set_gemm_mode(mode)
+        forms.append(lib.folx_hip_dense_act_form(2060, 21, 80, 256, 0))
+        sizes.append(lib.folx_hip_dense_act_workspace_bytes(2060, 21, 80, 256))
+    lib.folx_hip_set_gemm_mode(before)
+    assert forms == [8, 32] and sizes == [3 * 2060 * 256 * 4] * 2
+
+
+def test_questions_about_a_shape(lib):
+    form, faster = lib.folx_hip_dense_act_form, lib.folx_hip_dense_act_faster
+    assert form(2000, 4, 100, 100, 0) == 2 and form(1 << 20, 4, 100, 100, 0) == 1 and form(1 << 20, 4, 100, 100, 1) == 2
+    assert faster(2000, 4, 100, 100, 100) == 1
+    assert form(64, 33, 200, 256, 0) == faster(64, 33, 200, 256, 200) == _lib.ENOTSUP   # K % 16
+    assert form(64, 0, 256, 256, 0) == faster(64, 0, 256, 256, 256) == _lib.ENOTSUP     # no Jacobian row
+    assert form(-1, 4, 100, 100, 0) == faster(64, 33, 256, 256, 0) == _lib.EINVAL

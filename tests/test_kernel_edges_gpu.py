@@ -161,8 +161,8 @@ def test_dense_small_tiles(rows, P, Kd, N):
         assert_lap(got[2], want[2], 'y_lap')
 
 
-# groups of 8 Jacobian rows (16 positions a tile, four per accumulator block) in launches of more than 512 tiles, of 16 or 32 in
-# smaller ones: the last tile's positions and the last group's rows cut, operand whole or in parts with a per-walker term and a skip connection
+# wide dense + activation: the last tile's positions and the last group's rows cut, operand whole or in parts with a per-walker term
+# and a skip connection (which form each size takes is pinned below)
 @pytest.mark.parametrize('rows,P,N', [((1, 4), 6, 132), ((515, 4), 21, 256), ((66, 16), 39, 300), ((164, 13), 24, 256), ((1030, 4), 8, 260),
                                       ((60, 4), 33, 256), ((521, 4), 13, 256)])
 def test_dense_act_groups_of_eight(rows, P, N):
@@ -188,6 +188,26 @@ def test_dense_act_groups_of_eight(rows, P, N):
     assert_val(got[0], ref[0] + res[0], 'y')
     assert_val(got[1], ref[1] + res[1], 'y_jac')
     assert_lap(got[2], ref[2] + res[2], 'y_lap')
+
+
+# groups of 8 Jacobian rows (16 positions a tile, four per accumulator block), of 16 (8 positions, two per block) and of 32, each
+# with and without a cut last tile and a cut last group, in both product modes
+@pytest.mark.parametrize('mode', ['f32', 'bf16x3'])
+@pytest.mark.parametrize('rows,P,N,form', [((257, 4), 21, 132, 8), ((130, 4), 24, 260, 8), ((66, 8), 21, 260, 8), ((257, 4), 21, 256, 8),
+                                           ((129, 4), 9, 260, 16), ((63, 8), 9, 132, 16), ((271, 4), 45, 260, 16), ((125, 4), 9, 132, 32),
+                                           ((64, 16), 96, 256, 32)])
+def test_dense_act_group_forms(mode, rows, P, N, form):
+    from folx_amd import _lib
+    from folx_amd import kernels as K
+
+    before = K.get_gemm_mode()
+    K.set_gemm_mode(mode)
+    try:
+        assert _lib.load().folx_hip_dense_act_form(rows[0] * rows[1], P, 80, N, 0) == form
+        print(f'mode {mode}', flush=True)
+        test_dense_act_groups_of_eight(rows, P, N)
+    finally:
+        K.set_gemm_mode(before)
 
 
 # up to six Jacobian rows: 1 .. 8 blocks of 16 columns and of 16 positions a workgroup, the last ones cut; features in whole
