@@ -337,7 +337,7 @@ __global__ __launch_bounds__(NTHR, 2) void dense_act_kernel(DAParams a) {
 // (v_mfma_f32_16x16x4_f32: independent accumulators of 4 registers, one W operand for all of them, taken from L2 16 k
 // ahead), which leaves f', f'' and the sum of squares as plain register arithmetic.  The product is formed transposed, so
 // a lane holds 4 consecutive columns of one position and stores them 128 bits at a time.  LDS tiles as above, one per row s
-// of the triplet; 34 to 74 VGPRs, so LDS sets the occupancy.  The products of a column are added in the order of the kernel above (128-bit reads of 16 k in
+// of the triplet; 40 to 88 VGPRs (P = 0 .. 6).  The products of a column are added in the order of the kernel above (128-bit reads of 16 k in
 // another order took 1 us less a layer and stood further from 64 bits on a small FermiNet-style function).  A form with W in registers, a grid of the resident workgroups and
 // the next tile's loads behind the current product was no faster on large R (28 .. 40 % slower for P = 6) and 15 % slower on
 // small.
@@ -472,15 +472,29 @@ __global__ __launch_bounds__(512) void dense_act_few_kernel(DAParams a, int wc, 
 constexpr int FEW_ROWS = 6;
 constexpr int FEW_LDS = 40960;  // four workgroups a CU where several row blocks share one
 
-// When the few-rows kernel is the faster one (R, K, N over 6000 .. 200 000 x 4 .. 128 x 32 .. 128 and P = 1, 3, 6, both
-// measured).  The general kernel reads W into registers once for all rows of a tile and overlaps its loads with its matrix work, which
-// is worth 5 to 25 % once its tiles cover the CUs; below that the few-rows kernel took 0.52 .. 1.03 of its time (R = 6000).
-// It also wins where the general one multiplies 32-column strips past N or, for K > N, the columns of a wider plan: 48 x 48
-// 0.81 .. 0.91, 96 x 96 0.84 .. 0.92, K = 128 to N = 64 0.62 .. 0.81, but 100 x 100 0.95 .. 1.03 (112 columns for 128).  And it
-// reads a skip connection 128 bits at a time ahead of its stores: 0.4 .. 0.65 wherever measured.
-bool few_rows(const DAPlan& pl, int32_t P, int32_t N, bool has_res) {
+// When the few-rows kernel is the faster one (both timed over 2100 shapes: R = 55 .. 240 000, K = 4 .. 128, N = 1 .. 128, P = 0 .. 6).
+// The general kernel reads W into registers once for all rows of a tile and overlaps its loads with its matrix work, which
+// is worth 5 to 25 % once its tiles cover the CUs; below that (160 tiles) the few-rows kernel took 0.43 .. 0.95 of its time, up to 192
+// 0.74 .. 0.98 unless all of the general kernel's matrix work is for columns and features that exist (its K comes in five sizes, its
+// columns in strips of 32, 64 or 128): 128 x 128 1.04, 1.07, 1.14 for P = 1, 4, 6.  In larger launches it wins where enough of that
+// work is padding: 48 x 48 0.81 .. 0.91, 96 x 96 0.84 .. 0.92, K = 128 to N = 64 0.62 .. 0.81, but 100 x 100 0.95 .. 1.03 (112 columns for
+// 128).  Its six rows with a share above 0.7 did not (N = 48, K = 32: 1.11 .. 1.20; 84 of 128 columns, K = 64: 1.04 .. 1.14), nor did
+// K <= 8, where there is little matrix work to save (96 of 128 columns: P = 2 1.02 .. 1.12, P = 6 1.15 .. 1.26; 48 of 64: P = 1, 3
+// 0.85 .. 1.04, P = 6 1.06 .. 1.21).  And it reads a skip connection ahead of its stores, 128 bits at a time where N allows: 0.4 .. 1.0
+// (once 1.2).  For N not a multiple of 4 its lanes store four single floats, 16 bytes apart from lane to lane: in launches that cover the CUs
+// it needs so much more padded work saved per column, the more rows are stored (K, N, P = 20, 42, 5: 1.67; 24, 87, 4: 1.56; 16, 43,
+// 1: 1.37; but 124, 41, 6: 0.84; 80, 85, 1: 0.77).
+// Of 2100 shapes, skip connections and any N among them, its choice was more than 3 % slower than the general kernel on 28, at most 20 %.
+// 300 others without one: 0.69 of the general kernel's time in the mean, 4 to 7 % more on three.
+bool few_rows(const DAPlan& pl, int32_t P, int32_t K, int32_t N, bool has_res) {
   if (P > FEW_ROWS) return false;
-  return has_res || pl.row_tiles <= 192 || 12 * ((N + 15) / 16 * 16) < 10 * 32 * pl.wc;
+  if (has_res) return true;
+  const int cols = (N + 15) / 16 * 16;
+  const double share = (K + 7) / 8 * cols / (32.0 * pl.ks * pl.wc);  // of the general kernel's matrix work that this one does
+  if (N % 4 != 0 && N > 16 && pl.row_tiles > 120 && 256 * pl.ks * pl.wc * (1 - share) < (45 + 9 * P) * N) return false;
+  if (pl.row_tiles <= 192) return K <= 8 || pl.wc < 4 || pl.row_tiles <= 160 || share <= (P == FEW_ROWS ? 0.9 : 0.95);
+  if (12 * cols >= 10 * 32 * pl.wc) return false;
+  return share <= 0.7 || (K <= 8 ? pl.wc == 2 && P <= 3 : P < FEW_ROWS);
 }
 
 template <int NR>
@@ -523,7 +537,7 @@ extern "C" int64_t folx_hip_dense_act_workspace_bytes(int64_t R, int32_t P, int3
 extern "C" int folx_hip_dense_act_form(int64_t R, int32_t P, int32_t K, int32_t N, int32_t has_res) {
   DAPlan pl;
   if (R <= 0 || P < 0) return FOLX_HIP_EINVAL;
-  if (plan_dense_act(R, P, K, N, pl)) return few_rows(pl, P, N, has_res != 0) ? FOLX_HIP_FORM_FEW : FOLX_HIP_FORM_TILES;
+  if (plan_dense_act(R, P, K, N, pl)) return few_rows(pl, P, K, N, has_res != 0) ? FOLX_HIP_FORM_FEW : FOLX_HIP_FORM_TILES;
   return folx_dense_act_wide_group(R, P, K, N);
 }
 
@@ -561,7 +575,7 @@ extern "C" int folx_hip_dense_act_fwdlap(void* stream, int32_t act, float param,
   prm.part = (float*)workspace;
   prm.R = R; prm.P = P; prm.K = K; prm.N = N; prm.G = pl.G; prm.PG = pl.PG; prm.act = act; prm.prm = param; prm.mode = 0;
   hipStream_t st = (hipStream_t)stream;
-  switch (few_rows(pl, P, N, res != nullptr) ? P : FEW_ROWS + 1) {
+  switch (few_rows(pl, P, K, N, res != nullptr) ? P : FEW_ROWS + 1) {
     case 0: return launch_few<2>(st, prm);
     case 1: return launch_few<3>(st, prm);
     case 2: return launch_few<4>(st, prm);

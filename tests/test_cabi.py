@@ -206,6 +206,19 @@ def test_wide_dense_act_takes_the_form_that_was_measured_faster(lib, mode, R, P,
         lib.folx_hip_set_gemm_mode(before)
 
 
+# narrow layers without a skip connection: time of the few-rows kernel over the general one's
+@pytest.mark.parametrize('R,P,K,N,ratio', [
+    (2000, 4, 100, 100, 0.63), (6000, 6, 128, 128, 1.14), (6000, 4, 128, 128, 1.07), (4091, 6, 128, 128, 0.71), (6000, 6, 4, 128, 0.92),
+    (5115, 3, 64, 64, 0.67), (60000, 1, 20, 48, 0.85), (60000, 6, 64, 48, 1.07), (60000, 6, 4, 48, 1.16), (60000, 4, 128, 100, 1.06),
+    (32763, 6, 8, 96, 1.26), (28795, 2, 8, 96, 1.08), (140795, 6, 32, 48, 1.20), (60000, 4, 128, 48, 0.64), (187472, 0, 128, 48, 0.52),
+    (195179, 5, 20, 42, 1.67), (21110, 4, 24, 87, 1.56), (74292, 1, 16, 43, 1.37), (27965, 6, 124, 41, 0.84), (68104, 1, 80, 85, 0.77),
+    (105354, 0, 44, 11, 0.50), (49595, 3, 124, 11, 0.46), (3299, 1, 20, 78, 0.79),
+])
+def test_narrow_dense_act_takes_the_kernel_that_was_measured_faster(lib, R, P, K, N, ratio):
+    assert lib.folx_hip_dense_act_form(R, P, K, N, 0) == (2 if ratio < 1 else 1)
+    assert lib.folx_hip_dense_act_form(R, P, K, N, 1) == 2
+
+
 def test_one_workspace_serves_both_product_modes(lib):
     before = lib.folx_hip_get_gemm_mode()
     forms, sizes = [], []
