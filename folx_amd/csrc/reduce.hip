@@ -61,10 +61,13 @@ __global__ __launch_bounds__(256) void reduce_mid_v4_kernel(const float* __restr
 // group in flight.  Bound by HBM: G is the least that covers the reduced axis in one piece per lane, so that a wavefront
 // reads one contiguous stretch (64 / G outputs side by side).  A whole wavefront per output left 48 of 64 lanes idle on
 // the softmax sums of 16 particles: 1.6 M outputs of 16: 182 -> 17 us (6.6 TB/s); 5.7 M of 30: 826 -> 193 us.
-template <bool MAX, int VEC, int U>
+// WAVE: G = 64 as a constant; a long axis read in single values is bound by its instructions (23 317 sums of 206: 7.6 -> 6.6 us,
+// 29 035 of 434: 15.5 -> 14.4 us).
+template <bool MAX, int VEC, int U, bool WAVE>
 __global__ __launch_bounds__(256) void reduce_last_kernel(const float* __restrict__ in, float* __restrict__ out,
                                                           int64_t total, int64_t red, int64_t span, int64_t lo,
-                                                          int32_t G, float alpha) {
+                                                          int32_t group, float alpha) {
+  const int G = WAVE ? FOLX_WAVE : group;
   const int per = 256 / G, g = threadIdx.x / G, l = threadIdx.x % G;
   const int64_t o0 = (int64_t)blockIdx.x * (per * U) + g;
   const int64_t pieces = red / VEC;
@@ -112,8 +115,14 @@ int launch_reduce_last(hipStream_t st, const float* in, float* out, int64_t tota
   const int U = total >= 4 * per * 2048 ? 4 : 1;
   const int64_t blocks = (total + per * U - 1) / (per * U);
   if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
-  if (U == 4) reduce_last_kernel<MAX, VEC, 4><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(in, out, total, red, span, lo, G, alpha);
-  else reduce_last_kernel<MAX, VEC, 1><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(in, out, total, red, span, lo, G, alpha);
+  const dim3 grid((unsigned)blocks), block(256);
+  if (G == FOLX_WAVE) {
+    if (U == 4) reduce_last_kernel<MAX, VEC, 4, true><<<grid, block, 0, st>>>(in, out, total, red, span, lo, G, alpha);
+    else reduce_last_kernel<MAX, VEC, 1, true><<<grid, block, 0, st>>>(in, out, total, red, span, lo, G, alpha);
+  } else {
+    if (U == 4) reduce_last_kernel<MAX, VEC, 4, false><<<grid, block, 0, st>>>(in, out, total, red, span, lo, G, alpha);
+    else reduce_last_kernel<MAX, VEC, 1, false><<<grid, block, 0, st>>>(in, out, total, red, span, lo, G, alpha);
+  }
   return folx_launch_status();
 }
 
