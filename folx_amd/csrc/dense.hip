@@ -788,6 +788,15 @@ int launch_cfg(hipStream_t st, Segs& sg, const float* W, const float* bias, int3
 
 }  // namespace
 
+extern "C" int folx_hip_dense_form(int64_t R, int32_t P, int32_t K, int32_t N) {
+  if (R <= 0 || P < 0 || K <= 0 || N <= 0) return FOLX_HIP_EINVAL;
+  if (N <= 64 || N % 4 != 0 || K % BK != 0) return FOLX_HIP_ENOTSUP;
+  const int64_t rows[3] = {R, P * R, R};
+  bool small;
+  folx_dense_units(rows, N, folx_gemm_mode() == FOLX_HIP_GEMM_BF16X3, small);
+  return small ? 64 : 128;
+}
+
 extern "C" int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const float* jac,
                                           const float* lap, const float* W, const float* bias,
                                           const float* res, const float* res_jac, const float* res_lap,

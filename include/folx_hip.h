@@ -206,12 +206,15 @@ int folx_hip_dense_act_fwdlap(void* stream, int32_t act, float param, const floa
  * folx_hip_dense_act_faster: 1 where the fused rule is expected to be faster than
  * folx_hip_dense_fwdlap over plain_K features (K, or the whole concatenation whose parts the fused rule
  * reads) followed by folx_hip_elementwise_fwdlap, 0 where it is not.
- * FOLX_HIP_ENOTSUP for shapes that the rule does not take.
+ * folx_hip_dense_form: rows of the tiles (64 or 128) that folx_hip_dense_fwdlap cuts 16-byte aligned operands with N > 64,
+ * N % 4 == 0 and K % 16 == 0 into.
+ * FOLX_HIP_ENOTSUP for shapes that the rule does not take (folx_hip_dense_form: for any other).
  */
 #define FOLX_HIP_FORM_TILES 1
 #define FOLX_HIP_FORM_FEW 2
 int folx_hip_dense_act_form(int64_t R, int32_t P, int32_t K, int32_t N, int32_t has_res);
 int folx_hip_dense_act_faster(int64_t R, int32_t P, int32_t K, int32_t N, int32_t plain_K);
+int folx_hip_dense_form(int64_t R, int32_t P, int32_t K, int32_t N);
 
 /*
  * folx_hip_dense_act_fwdlap for a wide layer whose input is a concatenation along the feature

@@ -236,4 +236,10 @@ def test_questions_about_a_shape(lib):
     assert faster(2000, 4, 100, 100, 100) == 1
     assert form(64, 33, 200, 256, 0) == faster(64, 33, 200, 256, 200) == _lib.ENOTSUP   # K % 16
     assert form(64, 0, 256, 256, 0) == faster(64, 0, 256, 256, 256) == _lib.ENOTSUP     # no Jacobian row
+    tile = lib.folx_hip_dense_form
+    # R, P, K, N of tests/test_kernel_edges_gpu.py::test_dense_small_tiles, then the line between the two
+    for shape in ((1, 1, 16, 68), (63, 2, 48, 100), (64, 3, 32, 128), (65, 9, 256, 132), (130, 7, 64, 300), (400, 30, 256, 256), (1280, 62, 256, 256)):
+        assert tile(*shape) == 64
+    assert tile(1550, 100, 256, 256) == 128 and tile(3000, 98, 512, 100) == 128
+    assert tile(64, 3, 32, 64) == tile(64, 3, 40, 128) == tile(64, 3, 32, 130) == _lib.ENOTSUP
     assert form(-1, 4, 100, 100, 0) == faster(64, 33, 256, 256, 0) == _lib.EINVAL

@@ -210,7 +210,8 @@ def test_dense_act_group_forms(mode, rows, P, N, form):
         K.set_gemm_mode(before)
 
 
-# up to six Jacobian rows: 1 .. 8 blocks of 16 columns and of 16 positions a workgroup, the last ones cut; features in whole
+# up to six Jacobian rows (with a skip connection always the kernel for them, without one where it is the faster):
+# 1 .. 8 blocks of 16 columns and of 16 positions a workgroup, the last ones cut; features in whole
 # groups of 16, with a rest, or only a rest; one column short of a 128-bit store; outputs off the 16-byte boundary
 @pytest.mark.parametrize('R,P,Kd,N', [(1, 0, 4, 1), (17, 1, 12, 16), (31, 2, 16, 17), (2000, 4, 100, 100), (16, 6, 128, 128),
                                       (9000, 3, 36, 30), (66000, 6, 32, 32), (15, 5, 20, 127), (8191, 2, 64, 48), (33, 6, 112, 64)])
