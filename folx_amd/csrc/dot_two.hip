@@ -200,9 +200,11 @@ __global__ __launch_bounds__(DT_NT) void dot_two_kernel(DotTwoArgs g) {
 // at the end.  The product is formed transposed (b in the A operand), so a lane ends with four consecutive columns of a row
 // of y: 128-bit stores.  Padding is lanes whose buffer offset lies past the descriptor's end (zeros; dropped stores).
 // a_vec / b_vec: the contracted axis has unit stride and every piece of four is whole and aligned: 128-bit loads.
-// Bound by HBM.  The tiled form above left three of its four wavefronts without a block and paid two barriers and an LDS
-// round trip per row at these sizes: 2048 products q k^T of 16 x 16 x 16, P = 48 (0.31 GB): 323 -> 66 us (4.8 TB/s); of
-// 32 x 32 x 32, P = 96: 1446 -> 528 us (4.7 TB/s); 64 of 16 x 16 x 16, P = 48: 99 -> 22 us.
+// Bound by HBM (5.2 TB/s for 16 384 of 16 x 16 x 16, P = 48, 5.1 for 4096 of 32 x 32 x 32, P = 96), for few batch elements by the
+// latency of a wavefront's rows.  The tiled form above left three of its four wavefronts without a block and paid two
+// barriers and an LDS round trip per row at these sizes: 2048 products of 16 x 16 x 16, P = 48: 336 -> 55 us for b = k^T, 355 -> 55 for
+// b row by row; of 32 x 32 x 32, P = 96: 1445 -> 491; 64 of 16 x 16 x 16, P = 48: 102 -> 8; with a constant b 78 -> 34, 387 -> 346, 35 -> 6.
+// 300 random sizes up to the limit: 0.08 .. 0.85 of the tiled form's time.
 constexpr int NXCD = 8;
 constexpr uint32_t FAR = 0x40000000u;      // past every descriptor's end
 constexpr int64_t EXTENT_MAX = 0x0fffffff;  // elements of an operand's tile from its first to its last: below FAR in bytes
@@ -358,7 +360,10 @@ __global__ __launch_bounds__(512) void dot_two_small_kernel(DotTwoArgs g, int a_
 
 template <int TI, int TJ, int KT>
 int launch_small(hipStream_t st, const DotTwoArgs& g, bool constb, int a_vec, int b_vec, int y_vec) {
-  // fewer than eight rows are not worth sharing; eight wavefronts where a CU gets one batch element at most
+  // Fewer than eight rows are not worth sharing in launches that fill the chip; eight wavefronts where a CU gets one batch element
+  // at most.  us for W = 1, 4, 8, 16 x 16 x 16: 192, P = 16: 11.0, 6.3, 6.0; P = 48: 25.2, 10.3, 9.0; 512, P = 48: 26.9, 14.1, 13.1.  32 x 32 x 32:
+  // 192, P = 16: 37.5, 16.9, 17.0; P = 48: 98, 34.5, 32.4; 512, P = 48: 102, 55.2, 59.5; few elements with few rows would be
+  // faster with four (64, P = 6: 17.8, 9.6).
   const int W = g.P < 8 ? 1 : (g.NB <= 192 && g.P >= 16 ? 8 : 4);
   const size_t lds = sizeof(float) * (W - 1) * TI * TJ * 4 * FOLX_WAVE;
   const dim3 grid((unsigned)((g.NB + NXCD - 1) / NXCD * NXCD)), block((unsigned)(FOLX_WAVE * W));

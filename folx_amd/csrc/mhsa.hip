@@ -26,7 +26,8 @@ namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Sum and maximum over the 16 lanes of a row, by DPP: quad permutes (lane ^ 1, lane ^ 2), then the two mirrors, which
-// meet equal values in every quad (half of 8) by then.  Vector instructions only, where a shuffle is a trip through LDS.
+// meet equal values in every quad (half of 8) by then.  Vector instructions only, where a shuffle is a trip through LDS:
+// mhsa_kernel on 1200 pairs of 17 x 64, P = 51: 797 -> 766 us, on 1024 of 32 x 64, P = 96: 745 -> 725 us.
 template <int CTRL>
 __device__ __forceinline__ float dpp16(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
@@ -393,10 +394,10 @@ __global__ __launch_bounds__(FOLX_WAVE * NW) void mhsa_kernel(MhsaArgs a) {
 // eight wavefronts).  Rows and columns of the padding are lanes whose buffer offset
 // lies past the descriptor's end: they read zeros and their stores are dropped, so no access is tested.  DT = 1, 2 or 4
 // blocks of 16 features.
-// Bound by HBM (16 n d bytes per pair and row, at 4.7-5.1 TB/s), for few pairs by the latency of a wavefront's rows.  One
+// Bound by HBM (16 n d bytes per pair and row, at 4.6-5.3 TB/s), for few pairs by the latency of a wavefront's rows.  One
 // wavefront per pair with the tiles of mhsa_kernel (two barriers and an LDS copy of k', v' per row) was bound by that chain:
 // 1200 pairs of 13 x 64, P = 39: 300 -> 139 us; 256 of 10 x 64, P = 30: 112 -> 24 us; 2048 of 16 x 16, P = 48: 146 -> 94 us;
-// 16000 of 16 x 64, P = 48: 2.69 -> 2.56 ms.  With a bias, masks, both (former kernel -> this; in parentheses held to 168
+// 16000 of 16 x 64, P = 48: 2.69 -> 2.56 ms; 33 to 48 features run as four blocks: 1200 of 13 x 48, P = 39: 232 -> 108 us.  With a bias, masks, both (former kernel -> this; in parentheses held to 168
 // registers, 15 to 32 of them spilled, and the bias loaded where it is added): 1200 pairs of 13 x 64, P = 39: 414 -> 150 us
 // (202), 742 -> 153 (210), 847 -> 158 (286); 2048 of 12 x 36, P = 36: 202 -> 162 (275), 503 -> 189 (280), 368 -> 192 (392);
 // 4096 of 16 x 64, P = 48: 752 -> 690 (844), 2053 -> 617 (832), 2324 -> 685 (1163).
@@ -734,6 +735,9 @@ __global__ __launch_bounds__(512, DT == 4 && (EDGE || MASKED) ? 2 : 3) void mhsa
 }
 
 // W wavefronts per pair: twelve fit a CU, three workgroups of four; eight share the rows where a CU gets one pair at most.
+// us for W = 1, 4, 8, pairs of 16 x 16: 192, P = 16: 16.6, 8.3, 7.8; P = 48: 41.7, 16.5, 13.0; 512, P = 48: 45.9, 21.8, 20.7.  Of 10 x 64:
+// 192, P = 16: 34.8, 15.6, 16.7; P = 48: 96, 32.1, 29.7; 384, P = 48: 98, 49.0, 53.1.  Below eight rows the copies and sums are
+// most of what four wavefronts do: 8192 pairs of 10 x 64, P = 7: 154, 172 (W = 4); few pairs would still be faster with four (64, P = 6: 17, 10).
 template <int DT>
 int launch_mhsa_small(hipStream_t st, const MhsaArgs& a) {
   const int64_t pairs = a.B * a.H;
