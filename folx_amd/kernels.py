@@ -81,6 +81,45 @@ class _timed:
             lt.records.append((self.name, self.key, self.e0, e1))
 
 
+class _Share:
+    """The start of a launch that evaluates several rules, as one of them sees it: its share of the time."""
+
+    __slots__ = ('e0', 'share')
+
+    def __init__(self, e0, share):
+        self.e0, self.share = e0, share
+
+    def elapsed_time(self, e1):
+        return self.share * self.e0.elapsed_time(e1)
+
+
+class _timed_chain:
+    """``_timed`` for one launch that evaluates several rules, ``[(name, key, work), ...]``: each is on record with its
+    share of the launch's time by work."""
+
+    __slots__ = ('rules', 'e0')
+
+    def __init__(self, rules):
+        self.rules = rules
+
+    def __enter__(self):
+        lt = LaunchTimer.active
+        self.e0 = None
+        if lt is not None and (lt.only is None or any(r[0] in lt.only for r in self.rules)):
+            self.e0 = torch.cuda.Event(enable_timing=True)
+            self.e0.record()
+
+    def __exit__(self, *exc):
+        lt = LaunchTimer.active
+        if lt is not None and self.e0 is not None:
+            e1 = torch.cuda.Event(enable_timing=True)
+            e1.record()
+            total = sum(w for _, _, w in self.rules)
+            for name, key, w in self.rules:
+                if lt.only is None or name in lt.only:
+                    lt.records.append((name, key, _Share(self.e0, w / total), e1))
+
+
 def set_gemm_mode(mode: str):
     """How the wide dense rules form their fp32 products: ``'f32'`` (FP32 matrix instructions, the
     default) or ``'bf16x3'`` (operands split exactly into three bf16 pieces, six exact piece
@@ -207,6 +246,58 @@ def dense_act(name, x, jac, lap, W, bias=None, param=0.0, res=None):
             f'dense_act_fwdlap[{name}]',
         )
     return y, yj, yl
+
+
+CHAIN_MAX_LAYERS = 16
+CHAIN_MAX_WIDTH = 128
+
+
+def _chain_args(layers):
+    """(number of layers, function codes, widths) of ``dense_chain``'s layers as the library takes them."""
+    n = len(layers)
+    acts = (ctypes.c_int32 * n)(*[-1 if name is None else ACT[name] for name, _, _, _ in layers])
+    widths = (ctypes.c_int32 * (n + 1))(layers[0][1].shape[0], *[W.shape[1] for _, W, _, _ in layers])
+    return n, acts, widths
+
+
+def dense_chain_faster(layers, R, P):
+    """Whether one launch (``dense_chain``) is the way to evaluate these layers over R positions and P Jacobian rows;
+    the library knows (folx_hip_dense_chain_faster)."""
+    n, acts, widths = _chain_args(layers)
+    return _lib.load().folx_hip_dense_chain_faster(n, acts, widths, R, P) == 1
+
+
+def dense_chain(layers, x, jac, lap, keep_hidden=False):
+    """Several narrow layers ``h <- f(h @ W + bias)`` in one launch: ``layers`` = [(name, W (K, N), bias or None, param), ...],
+    the last with ``name`` None if it is a plain matrix-vector product.  Returns the last layer's triplet and, with
+    ``keep_hidden``, the triplet that goes into that product (else None)."""
+    n, acts, widths = _chain_args(layers)
+    _chk(x, jac, lap, *[t for _, W, b, _ in layers for t in (W, b)])
+    P = jac.shape[0]
+    lead = tuple(x.shape[:-1])
+    R = int(np.prod(lead, dtype=np.int64))
+    assert x.shape[-1] == widths[0] and all(W.shape[0] == k for (_, W, _, _), k in zip(layers, widths))
+
+    def triplet(N):
+        y = torch.empty((*lead, N), device=x.device, dtype=torch.float32)
+        return y, torch.empty((P, *lead, N), device=x.device, dtype=torch.float32), torch.empty_like(y)
+
+    out = triplet(widths[n])
+    hidden = triplet(widths[n - 1]) if keep_hidden else None
+    params = (ctypes.c_float * n)(*[float(prm) for _, _, _, prm in layers])
+    Ws = (ctypes.c_void_p * n)(*[W.data_ptr() for _, W, _, _ in layers])
+    bs = (ctypes.c_void_p * n)(*[None if b is None else b.data_ptr() for _, _, b, _ in layers])
+    rules = [('dense_act_fwdlap', (name, R, P, *W.shape), W.numel()) if name is not None else
+             ('dense_fwdlap', (R, P, *W.shape, False), W.numel()) for name, W, _, _ in layers]
+    with _timed_chain(rules):
+        check(
+            _lib.load().folx_hip_dense_chain_fwdlap(
+                _stream(), n, acts, params, Ws, bs, widths, _p(x), _p(jac), _p(lap), *[_p(t) for t in out],
+                *[_p(t) for t in hidden or (None, None, None)], R, P
+            ),
+            'dense_chain_fwdlap',
+        )
+    return out, hidden
 
 
 def dense_act_parts(name, x, lap, jac_parts, widths, broadcast, group, W, bias=None, param=0.0, res=None, pre=None):

@@ -162,10 +162,13 @@ def dot(h, W, b=None, residual=None, row_slice=None, act=None, norm=None):
         h, norm = h.h, h
     elif isinstance(h, LazySlice) and row_slice is None and h.ndim >= 2 and h.axis == h.ndim - 2:
         h, row_slice = h.a, (h.lo, h.hi)
-    elif not isinstance(h, LazyConcat):
+    elif not isinstance(h, LazyConcat) and not (isinstance(h, LazyDot) and norm is None and row_slice is None
+                                                and h.opens_chain(W)):
         h = force(h)
     kwargs = {'bias': b, 'row_slice': row_slice, 'act': act, 'norm': norm}
     explicit = residual is not None or act is not None
+    if explicit and isinstance(h, LazyDot):
+        h = force(h)
     if explicit or not _is_triplet(h) or _is_triplet(W) or np.ndim(W) != 2:
         return _call_keep('dot_general', (h, force(W)), {**kwargs, 'residual': force(residual)})
     lead = tuple(h.shape[:-1])
@@ -509,7 +512,7 @@ def reshape(a, shape):
     from .wrapped_functions import LazyDot
 
     if (isinstance(a, LazyDot) and a._value is None and len(shape) >= 1 and shape[-1] == a.shape[-1]
-            and isinstance(a.h, FwdLaplArray) and a.kwargs.get('row_slice') is None and a.kwargs.get('norm') is None):
+            and isinstance(a.h, (FwdLaplArray, LazyDot)) and a.kwargs.get('row_slice') is None and a.kwargs.get('norm') is None):
         # only the leading axes change: the same product on the input with those leading axes, its epilogue
         # (bias, activation, skip connection) still open -- e.g. `(h.reshape(-1, K) @ W).reshape(n, n, N) + b`
         h = _call('reshape', (a.h,), {'new_sizes': (*shape[:-1], a.h.shape[-1])})

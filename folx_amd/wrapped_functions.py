@@ -17,6 +17,7 @@ rule raises ``KeyError`` in ``get_laplacian``.
 from __future__ import annotations
 
 import logging
+import sys
 from typing import Any, Callable
 
 import numpy as np
@@ -888,16 +889,25 @@ class LazyDot(Deferred):
     of its shape added to it the skip connection.  ``kwargs`` are those of the ``dot_general``
     rule (bias, act, norm, row_slice); evaluation is that rule."""
 
-    __slots__ = ('h', 'W', 'kwargs', 'shape')
+    __slots__ = ('h', 'W', 'kwargs', 'shape', 'depth')
 
     def __init__(self, h, W, kwargs, shape, thr=0):
         super().__init__(thr)
         self.h, self.W, self.kwargs, self.shape = h, W, dict(kwargs), tuple(shape)
+        self.depth = 1 + h.depth if isinstance(h, LazyDot) else 1   # unevaluated layers up to this one
 
     def with_(self, **kw):
         return LazyDot(self.h, self.W, {**self.kwargs, **kw}, self.shape, self.thr)
 
+    def opens_chain(self, W):
+        """Whether this may stay unevaluated as the operand of a product with ``W``: a Dense + activation layer in front of
+        another narrow one (``_evaluate_chain``)."""
+        return (self._value is None and self.depth < K.CHAIN_MAX_LAYERS and _chain_layer(self) and isinstance(W, (np.ndarray, torch.Tensor)) and np.ndim(W) == 2
+                and np.shape(W)[0] == self.shape[-1] and np.shape(W)[1] <= K.CHAIN_MAX_WIDTH)
+
     def _evaluate(self, residual=None):
+        if isinstance(self.h, LazyDot):
+            return _evaluate_chain(self, residual)
         return dot_general((self.h, self.W), {**self.kwargs, 'residual': residual}, self.thr)
 
     def value_with_residual(self, residual):
@@ -906,6 +916,102 @@ class LazyDot(Deferred):
 
         with fnp.sparsity_threshold(self.thr):
             return self._evaluate(residual)
+
+
+def _chain_layer(d) -> bool:
+    """A plain Dense + activation layer narrow enough for ``kernels.dense_chain``."""
+    kw = d.kwargs
+    return (kw.get('act') in K.FUSED_ACTS and kw.get('norm') is None and kw.get('row_slice') is None
+            and isinstance(d.W, (np.ndarray, torch.Tensor)) and np.ndim(d.W) == 2
+            and 1 <= np.shape(d.W)[0] <= K.CHAIN_MAX_WIDTH and 1 <= np.shape(d.W)[1] <= K.CHAIN_MAX_WIDTH)
+
+
+def _references(owner):
+    """References to ``owner.h``; compared with what this returns for an object that nothing else refers to."""
+    h = owner.h
+    return sys.getrefcount(h)
+
+
+def _single_reference():
+    class Owner:
+        pass
+
+    owner = Owner()
+    owner.h = Owner()
+    return _references(owner)
+
+
+_ONE_OWNER = _single_reference()
+
+
+def _evaluate_chain(last, residual):
+    """Products whose operand is itself an unevaluated Dense + activation layer, and so on down to a triplet: narrow layers
+    over few Jacobian rows run as one launch (``kernels.dense_chain``), anything else layer by layer, which is also what
+    defines the result.  A layer's handle that something besides the next layer refers to is evaluated for itself (it may be
+    read again) and the chain starts behind it; a matrix-vector product at the end hands its operand's triplet back."""
+    ends_in_vector = (residual is None and last.kwargs.get('act') is None and last.kwargs.get('norm') is None
+                      and last.kwargs.get('row_slice') is None and not _is(last.W) and np.shape(last.W)[1] == 1)
+    nodes, hidden, cur = [last], None, last
+    while isinstance(cur.h, LazyDot) and cur.h._value is None:
+        if _references(cur) != _ONE_OWNER:
+            if cur is not last or not ends_in_vector:
+                break
+            hidden = cur.h
+        cur = cur.h
+        nodes.append(cur)
+    h = force(cur.h) if isinstance(cur.h, Deferred) and not isinstance(cur.h, LazyConcat) else cur.h
+    nodes.reverse()
+    fit = len(nodes) if ends_in_vector or (residual is None and _chain_layer(last)) else len(nodes) - 1
+    from . import numpy as fnp
+
+    i = 0
+    while i < len(nodes):
+        if i == 0 and fit > 1 and _is(h):
+            got = _chain_launch(h, nodes[:fit], hidden is not None)
+            if got is not None:
+                h, kept = got
+                if hidden is not None:
+                    hidden._value = kept
+                i = fit
+                continue
+        node = nodes[i]
+        with fnp.sparsity_threshold(node.thr):
+            h = dot_general((h, node.W), {**node.kwargs, 'residual': residual if node is last else None}, node.thr)
+        if node is hidden:
+            node._value = h
+        i += 1
+    return h
+
+
+def _chain_launch(h: FwdLaplArray, nodes, keep: bool):
+    """``nodes`` over ``h`` in one launch: (last triplet, the one in front of it if ``keep``), or None where the layers go
+    one by one."""
+    if not h.x.is_cuda or any(np.shape(d.W)[0] != k for d, k in zip(nodes, (h.shape[-1], *[d.shape[-1] for d in nodes[:-1]]))):
+        return None
+    J, mask = h.jacobian.data, h.jacobian.x0_idx
+    proj, aligned = None, False
+    if mask is not None:
+        proj, aligned = ia.dot_projection(mask, -1, nodes[0].thr)
+        if proj is not None and ia.has_duplicates(proj):
+            return None
+    P = h.jacobian.max_n + 1 if mask is not None and proj is None else (J.shape[0] if proj is None else proj.shape[0])
+    R = h.x.numel() // max(h.x.shape[-1], 1)
+    layers = [(d.kwargs.get('act'), d.W, d.kwargs.get('bias'), d.kwargs.get('act_param', 0.0)) for d in nodes]
+    if R < 1 or not K.dense_chain_faster(layers, R, P):
+        return None
+    if mask is not None and proj is None:
+        J = h.jacobian.dense_array
+    elif aligned:
+        J = so.materialize(J, ia.get_index_mask(mask, proj), P)
+    dev = h.x.device
+    layers = [(act, so.device_const(W, dev), None if b is None else so.device_const(b, dev), prm) for act, W, b, prm in layers]
+    out, kept = K.dense_chain(layers, h.x, J, h.laplacian, keep)
+
+    def wrap(t):
+        new_mask = None if proj is None else np.broadcast_to(proj, (proj.shape[0], *h.shape[:-1], t[0].shape[-1]))
+        return FwdLaplArray(t[0], FwdJacobian(t[1], new_mask), t[2])
+
+    return wrap(out), None if kept is None else wrap(kept)
 
 
 class LazyMul(Deferred):
