@@ -17,8 +17,16 @@
 // one half take what they need from the other by a rotation inside 16 lanes.
 // A column's products are added in the order of dense_act.hip (two of its steps in one instruction: k = 8 j + 4 (q % 2) +
 // 2 e + q / 2 for lane group q of step e), and the matrix-vector product at the end in that of dense_n1_flat_kernel, so a chain
-// returns the bits of its layers run one by one.  Inside a run of 16 k the tile is stored in the order in which the lanes take
-// it, so that they read 128 bits at a time.
+// returns the bits of its layers run one by one in dense_act_few_kernel (the general kernel rounds d1 z_lap + d2 ssq the other
+// way round).  Inside a run of 16 k the tile is stored in the order in which the lanes take it, so that they read 128 bits at a
+// time.
+//
+// What bounds it: the matrix pipe together with the other instructions of its wavefronts (442 vector instructions a layer and
+// wavefront beside 156 matrix ones at 100 x 100, P = 4; the pipe busy 47 % of the time, and 16 % of the time CUs without work at
+// the end), and for 100 features the four SIMDs' unequal shares of seven wavefronts: 70 TFLOP/s there, 100 at 128 x 128, P = 6.
+// Weights through a descriptor and operands one chunk ahead: 8 to 14 % of the time.  80 registers for a third workgroup a
+// CU spilled 70 of them (429 -> 631 us).  us, layers one by one -> chain: ten layers of 100, P = 4: 2000 positions
+// 101 -> 43, 25 600 503 -> 390; four of 50, P = 3, 15 750: 106 -> 31; six of 128, P = 6, 100 000: 1408 -> 1156.
 #include "activations.h"
 
 namespace {
@@ -56,21 +64,34 @@ __device__ __forceinline__ float other_half(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false));
 }
 
-// W[k][col] for the four k of this lane in chunk j (16 k); past K zero
-__device__ __forceinline__ void chain_weights(const ChainLayer& ly, int col, int lq, int j, float (&w)[4]) {
-  const int c = min(col, ly.N - 1);
+// A lane's weights of one column: chunk j (16 k) gives it k = 16 j + 4 (lq % 2) + lq / 2 + {0, 2, 8, 10}.  Loads through a
+// descriptor of the K N floats, chunk after chunk: past K they bring zero.  (Past N, too wide a wavefront's columns are those
+// of the next row: never stored.)
+struct ChainW {
+  __amdgpu_buffer_rsrc_t rsrc;
+  int chunk;   // bytes from one chunk to the next
+  int off[4];  // bytes, of the next chunk
+  __device__ __forceinline__ void layer(const ChainLayer& ly, int col, int lq) {
+    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ly.W), 0, ly.K * ly.N * 4, 0x00027000);
+    chunk = 64 * ly.N;
+    const int k0 = 4 * (lq & 1) + (lq >> 1);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = 16 * j + 8 * (i / 2) + 4 * (lq & 1) + 2 * (i % 2) + (lq >> 1);
-    const float v = ly.W[min(k, ly.K - 1) * ly.N + c];
-    w[i] = k < ly.K ? v : 0.f;
+    for (int i = 0; i < 4; ++i) off[i] = 4 * ((k0 + 8 * (i / 2) + 2 * (i % 2)) * ly.N + col);
   }
-}
+  __device__ __forceinline__ void next(float (&w)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      w[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, off[i], 0, 0));
+      off[i] += chunk;
+    }
+  }
+};
 
 template <int NR, int PB>
 __global__ __launch_bounds__(512, 4) void dense_chain_kernel(ChainParams a) {
   constexpr bool HALF = PB == 8;
   constexpr int NB = HALF ? (NR + 1) / 2 : NR;
+  constexpr bool AHEAD = NB <= 6;  // operands from LDS one chunk ahead of their products: 4 NB registers, and 128 are to be had
   extern __shared__ __attribute__((aligned(16))) float tile[];
   const int tid = threadIdx.x;
   const int nthr = blockDim.x;
@@ -85,8 +106,10 @@ __global__ __launch_bounds__(512, 4) void dense_chain_kernel(ChainParams a) {
   const int col = 16 * wave + l16;  // as the product's W operand
 
   float wA[4], wB[4];
-  chain_weights(a.layer[0], col, lq, 0, wA);
-  chain_weights(a.layer[0], col, lq, 1, wB);
+  ChainW weights;
+  weights.layer(a.layer[0], col, lq);
+  weights.next(wA);
+  weights.next(wB);
 
   {  // the input triplet, zero from K to the next multiple of 16
     const int K = a.layer[0].K, Kp = (K + 15) / 16 * 16;
@@ -142,52 +165,81 @@ __global__ __launch_bounds__(512, 4) void dense_chain_kernel(ChainParams a) {
       }
       const int chunks = (K + 15) / 16;
       const float* base = tile + l16 * ld + 4 * lq;
-      auto chunk = [&](int j, float (&w)[4]) __attribute__((always_inline)) {
-        floatx4 v[NB];
+      floatx4 vA[NB], vB[NB];
+      auto read = [&](int j, floatx4 (&v)[NB]) __attribute__((always_inline)) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) v[b] = *reinterpret_cast<const floatx4*>(base + b * bs + 16 * j);
+      };
+      // the products of chunk j, while chunk j + 1 comes from LDS and the weights of chunk j + 2 from memory
+      auto chunk = [&](int j, float (&w)[4], floatx4 (&v)[NB], floatx4 (&next)[NB]) __attribute__((always_inline)) {
+        if constexpr (AHEAD) {
+          if (j + 1 < chunks) read(j + 1, next);
+        } else {
+          read(j, v);
+        }
         const float wv[4] = {w[0], w[1], w[2], w[3]};
-        chain_weights(ly, col, lq, j + 2, w);
+        weights.next(w);
+        if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[i], v[b][i], acc[b], 0, 0, 0);
+        if (16 * j + 8 < K)
+#pragma unroll
+          for (int i = 2; i < 4; ++i)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[i], v[b][i], acc[b], 0, 0, 0);
       };
+      if constexpr (AHEAD) read(0, vA);
       for (int j = 0; j < chunks; j += 2) {
-        chunk(j, wA);
-        if (j + 1 < chunks) chunk(j + 1, wB);
+        chunk(j, wA, vA, AHEAD ? vB : vA);
+        if (j + 1 < chunks) chunk(j + 1, wB, AHEAD ? vB : vA, vA);
       }
     }
     const bool last = l + 1 == L;
     const bool store = last || (l + 2 == L && a.h != nullptr);
     if (!last) {
-      chain_weights(a.layer[l + 1], col, lq, 0, wA);
-      chain_weights(a.layer[l + 1], col, lq, 1, wB);
+      weights.layer(a.layer[l + 1], col, lq);
+      weights.next(wA);
+      weights.next(wB);
     }
     if (active) {
+      if constexpr (HALF) {
+        // rows 2 b and 2 b + 1 of the triplet are in the two halves of a group of 16 lanes: one half evaluates the function of
+        // columns 0 and 2, the other that of 1 and 3, and they exchange the results
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float o, d1, d2, ssq = 0.f;
-        if constexpr (HALF) {
-          const float zo = other_half(acc[0][r]);
-          act_eval_fused(ly.act, (half == 0 ? acc[0][r] : zo) + bias[r], ly.prm, o, d1, d2);
+        for (int r2 = 0; r2 < 4; r2 += 2) {
+          const float z0 = acc[0][r2], z1 = other_half(acc[0][r2 + 1]);  // half 0: column r2; half 1: column r2 + 1
+          float e, e1, e2;
+          act_eval_fused(ly.act, (half == 0 ? z0 : z1) + (half == 0 ? bias[r2] : bias[r2 + 1]), ly.prm, e, e1, e2);
+          const float f = other_half(e), f1 = other_half(e1), f2 = other_half(e2);
 #pragma unroll
-          for (int b = 0; b < NB; ++b) {
-            const float mine = acc[b][r], theirs = other_half(mine);
-            const float lo = half == 0 ? mine : theirs, hi = half == 0 ? theirs : mine;
-            if (b > 0 && 2 * b < NR - 1) ssq += lo * lo;
-            if (2 * b + 1 < NR - 1) ssq += hi * hi;
+          for (int r = r2; r < r2 + 2; ++r) {
+            const bool own = half == r - r2;
+            const float o = own ? e : f, d1 = own ? e1 : f1, d2 = own ? e2 : f2;
+            float ssq = 0.f;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+              const float mine = acc[b][r], theirs = other_half(mine);
+              const float lo = half == 0 ? mine : theirs, hi = half == 0 ? theirs : mine;
+              if (b > 0 && 2 * b < NR - 1) ssq += lo * lo;
+              if (2 * b + 1 < NR - 1) ssq += hi * hi;
+            }
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+              const float v = d1 * acc[b][r];
+              const float with_lap = d1 * acc[b][r] + d2 * ssq;
+              // row of the triplet: 2 b (half 0) or 2 b + 1
+              const float lo = b == 0 ? o : (2 * b == NR - 1 ? with_lap : v);
+              const float hi = 2 * b + 1 == NR - 1 ? with_lap : v;
+              acc[b][r] = half == 0 ? lo : hi;
+            }
           }
+        }
+      } else {
 #pragma unroll
-          for (int b = 0; b < NB; ++b) {
-            const float v = d1 * acc[b][r];
-            const float with_lap = d1 * acc[b][r] + d2 * ssq;
-            // row of the triplet: 2 b (half 0) or 2 b + 1
-            const float lo = b == 0 ? o : (2 * b == NR - 1 ? with_lap : v);
-            const float hi = 2 * b + 1 == NR - 1 ? with_lap : v;
-            acc[b][r] = half == 0 ? lo : hi;
-          }
-        } else {
+        for (int r = 0; r < 4; ++r) {
+          float o, d1, d2, ssq = 0.f;
           act_eval_fused(ly.act, acc[0][r] + bias[r], ly.prm, o, d1, d2);
           acc[0][r] = o;
 #pragma unroll
@@ -257,7 +309,10 @@ bool plan_chain(int32_t L, const int32_t* act, const int32_t* widths, int64_t R,
   pl.waves = (nmax + 15) / 16;
   if (pl.waves < 1) pl.waves = 1;
   pl.ld = (kmax + 15) / 16 * 16 + 4;
-  pl.pb = (R + 15) / 16 <= 256 ? 8 : 16;
+  // 8 positions give the shorter chain per workgroup, 16 the better use of the weights and fewer idle lanes.  us, 8 / 16: four
+  // layers of 100, P = 4: R = 2000 17.9 / 25.8, 3000 27.2 / 26.3, 6000 40.5 / 42.9, 8000 50.8 / 43.6, 50 000 288 / 260; three of 32,
+  // P = 6: 2000 8.5 / 10.8, 6000 11.0 / 13.9, 12 000 16.4 / 15.0; three of 128, P = 6: 4100 40.1 / 42.8, 8000 53.8 / 46.5.
+  pl.pb = R <= 6144 ? 8 : 16;
   const int nr = P + 2, nb = pl.pb == 8 ? (nr + 1) / 2 : nr;
   pl.lds = (int64_t)nb * 16 * pl.ld * 4;
   pl.blocks = (R + pl.pb - 1) / pl.pb;

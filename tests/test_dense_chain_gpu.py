@@ -47,13 +47,13 @@ def assert_same(got, want, few):
             assert float((a - b).abs().max()) <= 2.0 ** -18 * float(b.abs().max())
 
 
-# 8 and 16 positions a workgroup (up to 4096 positions and above), a last workgroup that is not full, every number of rows,
+# 8 and 16 positions a workgroup (up to 6144 positions and above), a last workgroup that is not full, every number of rows,
 # widths at and off the multiples of 16, the widest layer (a tile of more than 64 KB at P = 6)
 @pytest.mark.parametrize('R,P,widths,vector', [
     (1, 0, (4, 4, 8), False), (7, 1, (4, 100, 100), True), (40, 2, (128, 16, 128), False), (333, 3, (20, 52, 36, 60), True),
     (2000, 4, (4, 100, 100, 100), True), (77, 5, (8, 12, 100), False), (500, 6, (32, 128, 128, 32), True),
-    (4096, 4, (4, 40, 24), True), (4097, 4, (4, 40, 24), True), (4101, 0, (16, 64, 64), False), (5003, 1, (4, 20, 112), True),
-    (4100, 2, (4, 100, 28), False), (4099, 3, (12, 32, 32), True), (4111, 5, (8, 96, 4), True), (6001, 6, (128, 128, 128), True),
+    (6144, 4, (4, 40, 24), True), (6145, 4, (4, 40, 24), True), (6149, 0, (16, 64, 64), False), (7003, 1, (4, 20, 112), True),
+    (6148, 2, (4, 100, 28), False), (6147, 3, (12, 32, 32), True), (6159, 5, (8, 96, 4), True), (6401, 6, (128, 128, 128), True),
 ])
 def test_chain_returns_the_bits_of_its_layers(R, P, widths, vector):
     acts = (['silu', 'tanh', 'softplus', 'sin'] * 4)[:len(widths) - 1]
@@ -71,7 +71,7 @@ def test_chain_returns_the_bits_of_its_layers(R, P, widths, vector):
         assert hidden is None and all(torch.equal(a, b) for a, b in zip(got, want))
 
 
-@pytest.mark.parametrize('R,P,widths', [(63, 3, (3, 50, 50, 1)), (4200, 6, (5, 7, 17, 33)), (300, 2, (1, 1, 1)), (90, 4, (127, 127, 3, 1))])
+@pytest.mark.parametrize('R,P,widths', [(63, 3, (3, 50, 50, 1)), (6200, 6, (5, 7, 17, 33)), (300, 2, (1, 1, 1)), (90, 4, (127, 127, 3, 1))])
 def test_chain_of_any_width(R, P, widths):
     acts = ['silu', 'tanh', 'cos'][:len(widths) - 1]
     if widths[-1] == 1:
