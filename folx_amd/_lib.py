@@ -73,6 +73,7 @@ ACT = {
     'log1p': 12, 'reciprocal': 13, 'expm1': 14, 'integer_pow': 15,
     'sinh': 16, 'cosh': 17, 'tan': 18, 'asin': 19, 'acos': 20, 'atan': 21, 'asinh': 22, 'acosh': 23,
     'atanh': 24, 'erf': 25, 'erfc': 26, 'erf_inv': 27, 'cbrt': 28, 'pow': 29, 'lgamma': 30, 'digamma': 31,
+    'gelu': 32, 'gelu_tanh': 33,
 }
 GEMM_MODE = {'f32': 0, 'bf16x3': 1}
 BINOP = {'mul': 0, 'div': 1, 'add': 2, 'sub': 3, 'min': 4, 'max': 5}

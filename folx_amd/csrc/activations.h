@@ -132,6 +132,17 @@ __device__ __forceinline__ void act_eval(float x, float prm, float& y, float& d1
   } else if constexpr (ACT == FOLX_ACT_POW) {
     float pm2 = powf(x, prm - 2.0f);
     y = pm2 * x * x; d1 = prm * pm2 * x; d2 = prm * (prm - 1.0f) * pm2;
+  } else if constexpr (ACT == FOLX_ACT_GELU) {
+    const float c = 0.5f * (1.0f + erff(0.70710678118654752f * x));       // Phi(x)
+    const float g = 0.39894228040143268f * expf(-0.5f * x * x);           // Phi'(x)
+    y = x * c; d1 = c + x * g; d2 = g * (2.0f - x * x);
+  } else if constexpr (ACT == FOLX_ACT_GELU_TANH) {
+    // x (1 + tanh u) / 2 with u = a (x + b x^3)
+    const float a = 0.79788456080286536f, b = 0.044715f, xx = x * x;
+    const float t = tanhf(a * x * (1.0f + b * xx)), u1 = a * (1.0f + 3.0f * b * xx), s = 1.0f - t * t;
+    y = 0.5f * x * (1.0f + t);
+    d1 = 0.5f * (1.0f + t) + 0.5f * x * s * u1;
+    d2 = s * (u1 + x * (3.0f * a * b * x - t * u1 * u1));
   } else {  // FOLX_ACT_INTEGER_POW
     int n = (int)prm;
     // x^(n-2) by repeated multiplication on |n-2|, then one or two more factors
@@ -149,7 +160,8 @@ __device__ __forceinline__ void act_eval(float x, float prm, float& y, float& d1
 inline bool act_fused(int act) {
   switch (act) {
     case FOLX_ACT_TANH: case FOLX_ACT_SILU: case FOLX_ACT_LOGISTIC: case FOLX_ACT_SOFTPLUS:
-    case FOLX_ACT_EXP: case FOLX_ACT_SIN: case FOLX_ACT_COS: case FOLX_ACT_SQUARE:
+    case FOLX_ACT_EXP: case FOLX_ACT_SIN: case FOLX_ACT_COS: case FOLX_ACT_SQUARE: case FOLX_ACT_GELU:
+    case FOLX_ACT_GELU_TANH:
       return true;
   }
   return false;
@@ -164,6 +176,8 @@ __device__ __forceinline__ void act_eval_fused(int act, float x, float prm, floa
     case FOLX_ACT_EXP: act_eval<FOLX_ACT_EXP>(x, prm, y, d1, d2); break;
     case FOLX_ACT_SIN: act_eval<FOLX_ACT_SIN>(x, prm, y, d1, d2); break;
     case FOLX_ACT_COS: act_eval<FOLX_ACT_COS>(x, prm, y, d1, d2); break;
+    case FOLX_ACT_GELU: act_eval<FOLX_ACT_GELU>(x, prm, y, d1, d2); break;
+    case FOLX_ACT_GELU_TANH: act_eval<FOLX_ACT_GELU_TANH>(x, prm, y, d1, d2); break;
     default: act_eval<FOLX_ACT_SQUARE>(x, prm, y, d1, d2); break;
   }
 }

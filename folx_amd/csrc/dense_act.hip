@@ -293,7 +293,7 @@ __global__ __launch_bounds__(NTHR, 2) void dense_act_kernel(DAParams a) {
     switch (a.act) {
       FOLX_DA_CASE(FOLX_ACT_TANH) FOLX_DA_CASE(FOLX_ACT_SILU) FOLX_DA_CASE(FOLX_ACT_LOGISTIC)
       FOLX_DA_CASE(FOLX_ACT_SOFTPLUS) FOLX_DA_CASE(FOLX_ACT_EXP) FOLX_DA_CASE(FOLX_ACT_SIN)
-      FOLX_DA_CASE(FOLX_ACT_COS)
+      FOLX_DA_CASE(FOLX_ACT_COS) FOLX_DA_CASE(FOLX_ACT_GELU) FOLX_DA_CASE(FOLX_ACT_GELU_TANH)
       default:
         _Pragma("unroll") for (int t = 0; t < TM; ++t) _Pragma("unroll") for (int r = 0; r < 16; ++r)
             act_eval<FOLX_ACT_SQUARE>(acc[t][r] + bcol, a.prm, o[t][r], d1[t][r], d2[t][r]);

@@ -194,7 +194,8 @@ def dense(x, jac, lap, W, bias=None, res=None, row_slice=None):
     return y, yj, yl
 
 
-FUSED_ACTS = ('tanh', 'silu', 'logistic', 'sigmoid', 'softplus', 'exp', 'sin', 'cos', 'square')
+FUSED_ACTS = ('tanh', 'silu', 'logistic', 'sigmoid', 'softplus', 'exp', 'sin', 'cos', 'square', 'gelu',
+              'gelu_tanh')
 
 
 def dense_act_supported(name, K, N, rows=None, P=None, spared=None):

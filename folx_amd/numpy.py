@@ -90,6 +90,7 @@ arcsin, arccos, arctan = _u('asin'), _u('acos'), _u('atan')
 arcsinh, arccosh, arctanh = _u('asinh'), _u('acosh'), _u('atanh')
 erf, erfc, erf_inv, cbrt = _u('erf'), _u('erfc'), _u('erf_inv'), _u('cbrt')
 lgamma, digamma = _u('lgamma'), _u('digamma')
+_gelu, _gelu_tanh = _u('gelu'), _u('gelu_tanh')
 reciprocal, negative, sign, stop_gradient = _u('reciprocal'), _u('neg'), _u('sign'), _u('stop_gradient')
 
 
@@ -901,10 +902,7 @@ def elu(a, alpha=1.0):
 
 def gelu(a, approximate=True):
     """``jax.nn.gelu``: the tanh form by default, ``approximate=False`` the erf form (test/test_layers.py:709)."""
-    if approximate:
-        inner = multiply(add(a, multiply(integer_pow(a, 3), 0.044715)), float(np.sqrt(2.0 / np.pi)))
-        return multiply(multiply(a, 0.5), add(tanh(inner), 1.0))
-    return multiply(multiply(a, 0.5), add(erf(multiply(a, float(1.0 / np.sqrt(2.0)))), 1.0))
+    return (_gelu_tanh if approximate else _gelu)(a)
 
 
 def log_softmax(a, axis=-1):

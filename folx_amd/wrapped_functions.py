@@ -142,6 +142,7 @@ _NP_UNARY = {
     'softplus': lambda x: np.logaddexp(x, 0), 'neg': np.negative,
     'sinh': np.sinh, 'cosh': np.cosh, 'tan': np.tan, 'asin': np.arcsin, 'acos': np.arccos, 'atan': np.arctan,
     'asinh': np.arcsinh, 'acosh': np.arccosh, 'atanh': np.arctanh, 'cbrt': np.cbrt,
+    'gelu_tanh': lambda x: 0.5 * x * (1 + np.tanh(np.sqrt(2.0 / np.pi) * (x + 0.044715 * x**3))),
 }
 
 
@@ -161,10 +162,10 @@ def _unary_rule(name: str) -> ForwardLaplacian:
                 return np.asarray(a) ** int(param)
             if name == 'pow':
                 return np.asarray(a) ** float(param)
-            if name in ('erf', 'erfc', 'erf_inv', 'lgamma', 'digamma'):
+            if name in ('erf', 'erfc', 'erf_inv', 'lgamma', 'digamma', 'gelu'):
                 import scipy.special as sp
 
-                return {'erf': sp.erf, 'erfc': sp.erfc, 'erf_inv': sp.erfinv, 'lgamma': sp.gammaln,
+                return {'gelu': lambda v: 0.5 * v * (1 + sp.erf(v / np.sqrt(2.0))), 'erf': sp.erf, 'erfc': sp.erfc, 'erf_inv': sp.erfinv, 'lgamma': sp.gammaln,
                         'digamma': sp.digamma}[name](np.asarray(a))
             return _NP_UNARY[name](np.asarray(a))
         mask = a.jacobian.x0_idx
@@ -2048,7 +2049,7 @@ def mhsea_forward_laplacian(args, kwargs, sparsity_threshold):
 
 for _n in ['tanh', 'exp', 'log', 'sqrt', 'rsqrt', 'square', 'logistic', 'sin', 'cos', 'abs', 'log1p',
            'expm1', 'integer_pow', 'silu', 'softplus', 'reciprocal', 'sinh', 'cosh', 'tan', 'asin', 'acos', 'atan',
-           'asinh', 'acosh', 'atanh', 'erf', 'erfc', 'erf_inv', 'cbrt', 'pow', 'lgamma', 'digamma']:
+           'asinh', 'acosh', 'atanh', 'erf', 'erfc', 'erf_inv', 'cbrt', 'pow', 'lgamma', 'digamma', 'gelu', 'gelu_tanh']:
     register_function(_n, _unary_rule(_n))
 register_function('sigmoid', _unary_rule('logistic'))  # string key, folx/wrapped_functions.py:554
 register_function('neg', neg_rule)

@@ -197,6 +197,20 @@ def _digamma(x):
     return digamma(x), p1, p2
 
 
+def _gelu(x):
+    from scipy.special import erf
+
+    c, g = 0.5 * (1 + erf(x / np.sqrt(2.0))), np.exp(-0.5 * x * x) / np.sqrt(2 * np.pi)
+    return x * c, c + x * g, g * (2 - x * x)
+
+
+def _gelu_tanh(x):
+    a, b = np.sqrt(2 / np.pi), 0.044715
+    t, u1, u2 = np.tanh(a * (x + b * x**3)), a * (1 + 3 * b * x * x), 6 * a * b * x
+    s = 1 - t * t
+    return 0.5 * x * (1 + t), 0.5 * (1 + t) + 0.5 * x * s * u1, s * u1 + 0.5 * x * (s * u2 - 2 * t * s * u1 * u1)
+
+
 def _identity(x):
     return x, np.ones_like(x), np.zeros_like(x)
 
@@ -225,6 +239,7 @@ ACTIVATIONS = {
     'asinh': _asinh, 'acosh': _acosh, 'atanh': _atanh, 'erf': _erf, 'erfc': _erfc, 'erf_inv': _erf_inv,
     'cbrt': _cbrt, 'lgamma': _lgamma, 'digamma': _digamma,
 }
+_GELU = {'gelu': _gelu, 'gelu_tanh': _gelu_tanh}
 
 
 def integer_pow(x, n: int):
@@ -243,6 +258,8 @@ def elementwise_rule(name, x, J, lap, param=None):
         y, d1, d2 = integer_pow(x, int(param))
     elif name == 'pow':  # x^param, x > 0, constant real exponent (jax.lax.pow_p)
         y, d1, d2 = x**param, param * x ** (param - 1), param * (param - 1) * x ** (param - 2)
+    elif name in _GELU:  # compositions of the reference's primitives, one function here
+        y, d1, d2 = _GELU[name](x)
     elif name == 'scale':  # y = param * x, linear
         y, d1, d2 = param * x, np.full_like(x, param), np.zeros_like(x)
     else:

@@ -1,0 +1,43 @@
+"""GELU (both forms) as one function: the elementwise rule and the fused dense + activation rules against the float64 oracle,
+for arguments from the flat tail to the linear range."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import rules
+from tolerances import assert_lap, assert_val
+
+from folx_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+dev = lambda v: torch.as_tensor(np.asarray(v, dtype=np.float32)).cuda()
+
+
+def compare(got, ref, what):
+    assert_val(got[0], ref[0], what + ' x')
+    assert_val(got[1], ref[1], what + ' jacobian')
+    assert_lap(got[2], ref[2], what + ' laplacian')
+
+
+@pytest.mark.parametrize('name', ['gelu', 'gelu_tanh'])
+@pytest.mark.parametrize('shape,P', [((1, 1), 0), ((3, 5), 2), ((7, 64), 48)])
+def test_elementwise_gelu(name, shape, P):
+    print(f'case {name} {shape} P={P}', flush=True)
+    g = np.random.default_rng(0)
+    x = g.uniform(-7, 7, size=shape).astype(np.float32)
+    J, L = g.normal(size=(P, *shape)).astype(np.float32), g.normal(size=shape).astype(np.float32)
+    ref = rules.elementwise_rule(name, *[v.astype(np.float64) for v in (x, J, L)])
+    compare(K.elementwise(name, dev(x), dev(J), dev(L)), ref, name)
+
+
+# narrow general and few-rows kernels, the wide kernel
+@pytest.mark.parametrize('name', ['gelu', 'gelu_tanh'])
+@pytest.mark.parametrize('rows,P,k,n', [((2, 40), 30, 64, 128), ((3, 7), 4, 20, 36), ((4, 8), 32, 64, 256)])
+def test_dense_gelu(name, rows, P, k, n):
+    print(f'case dense {name} {rows} P={P} {k} x {n}', flush=True)
+    g = np.random.default_rng(1)
+    t = [g.normal(size=s).astype(np.float32) for s in ((*rows, k), (P, *rows, k), (*rows, k))]
+    W, b = (g.normal(size=(k, n)) / np.sqrt(k)).astype(np.float32), g.normal(size=n).astype(np.float32)
+    z = rules.dense_rule(*[v.astype(np.float64) for v in (*t, W, b)])
+    compare(K.dense_act(name, *[dev(v) for v in t], dev(W), dev(b)), rules.elementwise_rule(name, *z), name)
