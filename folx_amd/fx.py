@@ -21,6 +21,7 @@ import torch
 
 from . import numpy as fnp
 from .api import BatchedArray, FwdLaplArray
+from .fx_attention import attention, fuse_attention
 from .interpreter import ForwardLaplacianFn
 
 aten = torch.ops.aten
@@ -580,6 +581,15 @@ def _identity(a, *_, **__):
     return a
 
 
+def _attention(q, k, v):
+    """A group that ``fuse_attention`` found; an operand without derivatives takes the two products."""
+    if all(_is_t(t) and not isinstance(t, BatchedArray) for t in (q, k, v)):
+        return fnp.multi_head_self_attention(q, k, v)
+    heads_first = lambda t: fnp.transpose(t, (1, 0, 2))    # noqa: E731
+    p = fnp.softmax(fnp.matmul(heads_first(q), fnp.swapaxes(heads_first(k), -1, -2)), axis=-1)
+    return heads_first(fnp.matmul(p, heads_first(v)))
+
+
 # ATen operation -> the function of the same meaning (which finds its rule in the registry)
 RULES = {
     aten.add.Tensor: lambda a, b, alpha=1: fnp.add(a, _scaled(b, alpha)),
@@ -719,6 +729,7 @@ RULES = {
         dropout_mask=None, scale=None, enable_gqa=False: (_sdpa(q, k, v, dropout_p, is_causal, attn_mask, scale), None),
     aten._cdist_forward.default: _cdist,
     torch.ops.folx_amd.multi_head_self_attention.default: fnp.multi_head_self_attention,
+    attention: _attention,
 }
 
 
@@ -862,14 +873,33 @@ _WEIGHT_READERS = {aten.mm.default, aten.addmm.default, aten.bmm.default, aten.m
 _DEVICE_CONST_MIN = 256   # constants of at least this many floats live on the device between evaluations
 
 
+def _reading_order(gm: torch.fx.GraphModule):
+    """(position of each node, {node: the nodes it is the last to read}); worked out once per graph."""
+    got = gm.meta.get('folx_reading_order')
+    if got is None:
+        order = {n: i for i, n in enumerate(gm.graph.nodes)}
+        last_read = {}
+        for n in order:
+            if n.users and n.op != 'output':
+                last_read.setdefault(max(n.users, key=order.__getitem__), []).append(n)
+        got = gm.meta['folx_reading_order'] = (order, last_read)
+    return got
+
+
 def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None):
     """One pass over the equations of a traced graph (folx/interpreter.py:218-264): constant equations come from
     ``fold_constants``, the others go through ``RULES``."""
     env = dict(fold_constants(gm) if consts is None else consts)
     it = iter(inputs)
     look = lambda a: env[a] if isinstance(a, torch.fx.Node) else a
-    order = {n: i for i, n in enumerate(gm.graph.nodes)}
+    order, last_read = _reading_order(gm)
+    done = None
     for node in gm.graph.nodes:
+        if done is not None:   # what nobody reads any more: its memory serves the next equation, and a deferred value is free
+            args = kwargs = None
+            for n in last_read.get(done, ()):
+                env.pop(n, None)
+        done = node
         if node in env:
             continue
         if node.op == 'placeholder':
@@ -983,6 +1013,8 @@ class TracedForwardLaplacian(ForwardLaplacianFn):
                 finally:
                     _TRACING[0] = False
             self.constants[shapes] = fold_constants(gm)
+            if fuse_attention(gm, self.constants[shapes]):
+                self.constants[shapes] = fold_constants(gm)
         return gm
 
     def _constants(self, shapes, device):

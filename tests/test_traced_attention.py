@@ -1,0 +1,110 @@
+"""Attention spelled with products and a softmax in a traced torch function: which spellings become the attention rule, and
+that they give what the two products and the softmax give (on the CPU stand-ins for the kernels)."""
+
+import math
+
+import cpu_kernels
+import pytest
+import torch
+
+from folx_amd import fx
+from folx_amd.fx_attention import attention
+
+N, H, D = 6, 2, 4
+g = torch.Generator().manual_seed(0)
+W = [torch.randn(3, H * D, generator=g) for _ in range(3)]
+SINGLE = [torch.randn(3, D, generator=g) for _ in range(3)]
+heads = lambda x: [(x @ w).view(N, H, D).permute(1, 0, 2) for w in W]
+softmax = lambda s: torch.softmax(s, dim=-1)
+
+
+def matmul(x):
+    q, k, v = heads(x)
+    return (softmax(q @ k.transpose(-1, -2) / math.sqrt(D)) @ v).permute(1, 0, 2).reshape(N, H * D).sum(0)
+
+
+def einsum(x):
+    q, k, v = [(x @ w).view(N, H, D) for w in W]
+    return torch.einsum('hij,jhd->ihd', softmax(torch.einsum('ihd,jhd->hij', q, k) * 0.5), v)
+
+
+def one_head(x):
+    q, k, v = [x @ w for w in SINGLE]
+    return softmax(q @ k.T) @ v
+
+
+def leading_axis(x):
+    q, k, v = [t.unsqueeze(0) for t in heads(x)]
+    return softmax(q @ k.mT * 0.3) @ v
+
+
+def same_operand(x):
+    q = x @ SINGLE[0]
+    return softmax(q @ q.T / 2) @ q
+
+
+def permuted_values(x):
+    q, k, v = heads(x)
+    return softmax(q @ k.transpose(-1, -2) * torch.tensor(0.7)) @ v.flip(0)
+
+
+def chunked(x):
+    q, k, v = [t.reshape(N, H, D).transpose(0, 1) for t in (x @ torch.cat(W, 1)).chunk(3, -1)]
+    return (softmax(q @ k.transpose(-1, -2) / 2) @ v).transpose(0, 1).flatten(1)
+
+
+def two_layers(x):
+    h = einsum(x).reshape(N, H * D)[:, :3]
+    return matmul(h)
+
+
+def scores_read_twice(x):
+    q, k, v = heads(x)
+    s = q @ k.transpose(-1, -2) / 2
+    return (softmax(s) @ v).sum() + s.sum()
+
+
+def masked(x):
+    q, k, v = heads(x)
+    s = (q @ k.transpose(-1, -2)).masked_fill(torch.ones(N, N).triu(1).bool(), -1e9)
+    return softmax(s) @ v
+
+
+def over_queries(x):
+    q, k, v = heads(x)
+    return torch.softmax(q @ k.transpose(-1, -2), dim=-2) @ v
+
+
+def transposed_scores(x):
+    q, k, v = heads(x)
+    return softmax((q @ k.transpose(-1, -2)).transpose(-1, -2)) @ v
+
+
+def constant_values(x):
+    q, k, _ = heads(x)
+    return softmax(q @ k.transpose(-1, -2)) @ torch.ones(H, N, D)
+
+
+def feature_axis_in_front(x):
+    q, k, v = [(x @ w).view(N, D, H).permute(2, 0, 1) for w in W]
+    return (softmax(q @ k.transpose(-1, -2) / 2) @ v).permute(1, 2, 0).reshape(N, H * D)
+
+
+FUSED = {matmul: 1, einsum: 1, one_head: 1, leading_axis: 1, same_operand: 1, permuted_values: 1, chunked: 1, two_layers: 2}
+LEFT = [scores_read_twice, masked, over_queries, transposed_scores, constant_values, feature_axis_in_front]
+
+
+@pytest.mark.parametrize('thr', [0, 3])
+@pytest.mark.parametrize('fn', [*FUSED, *LEFT], ids=lambda f: f.__name__)
+def test_attention_in_a_traced_function(monkeypatch, fn, thr):
+    cpu_kernels.install(monkeypatch)
+    x = torch.randn(3, N, 3, generator=torch.Generator().manual_seed(1))
+    traced = fx.forward_laplacian_torch(fn, thr)
+    got = traced.batched(x)
+    (graph,) = [gm.graph for gm in traced.graphs.values()]
+    assert sum(n.target is attention for n in graph.nodes) == FUSED.get(fn, 0)
+    monkeypatch.setattr(fx, 'fuse_attention', lambda gm, consts: 0)
+    want = fx.forward_laplacian_torch(fn, thr).batched(x)
+    for a, b in ((got.x, want.x), (got.jacobian.dense_array, want.jacobian.dense_array), (got.laplacian, want.laplacian)):
+        # stand-ins compute in 64 bits and round every rule's result to 32: a few roundings on either side
+        torch.testing.assert_close(a, b, rtol=2e-5, atol=2e-5 * float(b.abs().max()))
