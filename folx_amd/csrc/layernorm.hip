@@ -31,22 +31,61 @@ __device__ __forceinline__ float wave_sum1(float a) {
   return a;
 }
 
+// Sums over LW lanes.  Below a wavefront: quad permutes, the two mirrors (which meet equal values in every quad, every half of
+// 8 by then) and a swap of neighbouring rows of 16, all vector instructions, where a shuffle is a trip through LDS.
+template <int CTRL>
+__device__ __forceinline__ float ln_dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+template <int LW>
+__device__ __forceinline__ float group_sum(float v) {
+  if constexpr (LW == FOLX_WAVE) {
+    return wave_sum1(v);
+  } else {
+    v += ln_dpp<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+    v += ln_dpp<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+    v += ln_dpp<0x141>(v);  // row_half_mirror
+    if constexpr (LW > 8) v += ln_dpp<0x140>(v);  // row_mirror
+    if constexpr (LW > 16) {
+      const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+      v = __uint_as_float(both[0]) + __uint_as_float(both[1]);
+    }
+    return v;
+  }
+}
+template <int LW>
+__device__ __forceinline__ void group_sum3(float& a, float& b, float& c) {
+  if constexpr (LW == FOLX_WAVE) {
+    wave_sum3(a, b, c);
+  } else {
+    a = group_sum<LW>(a); b = group_sum<LW>(b); c = group_sum<LW>(c);
+  }
+}
+
 constexpr int PSPLIT = 4;
 
 // PER_WAVE: for a few Jacobian rows (sparse storage, P <= 8) a whole workgroup per row of features would
 // mostly wait at its barrier: each WAVEFRONT owns a row of features then and walks all P Jacobian rows
 // itself (four in flight), no LDS and no barrier.
-template <int NV, bool PER_WAVE>
+// LW < 64 lanes to a row of features (F <= 4 LW): the wavefront holds 64 / LW consecutive rows side by side, so that it reads
+// and writes up to 1 KB of a Jacobian row at a time whatever F is.  With one row to a wavefront F = 64 left three quarters of
+// the lanes idle.  us, one row -> 64 / LW rows: 8192 rows, P = 48: F = 32 85 -> 20, 64 87 -> 41 (5.2 TB/s), 96 91 -> 60,
+// 128 95 -> 82; 1000 rows, P = 96, F = 64: 27 -> 13.5; 32 768 rows, P = 3, F = 64: 42 -> 17; 100 rows, P = 12: 5.6 -> 4.8.
+template <int NV, bool PER_WAVE, int LW = FOLX_WAVE>
 __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void layernorm_kernel(
     const float* __restrict__ x, const float* __restrict__ jac, const float* __restrict__ lap,
     const float* __restrict__ gamma, const float* __restrict__ beta, float* __restrict__ y,
     float* __restrict__ y_jac, float* __restrict__ y_lap, int64_t R, int32_t F, int32_t P, float eps) {
   __shared__ float4 redT[PSPLIT][NV * FOLX_WAVE];
-  __shared__ float reds[PSPLIT][2];
-  const int lane = threadIdx.x % FOLX_WAVE;
+  constexpr int ROWS = FOLX_WAVE / LW;  // of features, per wavefront
+  __shared__ float reds[PSPLIT][ROWS][2];
+  const int wlane = threadIdx.x % FOLX_WAVE;
+  const int lane = wlane % LW, sub = wlane / LW;
   const int w = threadIdx.x / FOLX_WAVE;
-  const int64_t row = PER_WAVE ? (int64_t)blockIdx.x * PSPLIT + w : (int64_t)blockIdx.x;
-  if (PER_WAVE && row >= R) return;
+  const int64_t first = (PER_WAVE ? (int64_t)blockIdx.x * PSPLIT + w : (int64_t)blockIdx.x) * ROWS;
+  if (PER_WAVE && first >= R) return;
+  const bool live = ROWS == 1 || first + sub < R;
+  const int64_t row = live ? first + sub : R - 1;
   constexpr int PS = PER_WAVE ? 1 : PSPLIT;  // distance between the Jacobian rows of a wavefront
   const int F4 = F / 4;
   const float invF = 1.0f / (float)F;
@@ -58,8 +97,8 @@ __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void layernorm_kernel(
   float sx = 0.0f;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int i4 = lane + FOLX_WAVE * v;
-    ok[v] = i4 < F4;
+    const int i4 = lane + LW * v;
+    ok[v] = live && i4 < F4;
     c[v] = make_float4(0.f, 0.f, 0.f, 0.f);
     g[v] = c[v];
     if (ok[v]) {
@@ -68,7 +107,7 @@ __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void layernorm_kernel(
       sx += c[v].x + c[v].y + c[v].z + c[v].w;
     }
   }
-  const float mu = wave_sum1(sx) * invF;
+  const float mu = group_sum<LW>(sx) * invF;
   float sv = 0.0f;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
@@ -77,7 +116,7 @@ __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void layernorm_kernel(
       sv += c[v].x * c[v].x + c[v].y * c[v].y + c[v].z * c[v].z + c[v].w * c[v].w;
     }
   }
-  const float var = wave_sum1(sv) * invF;
+  const float var = group_sum<LW>(sv) * invF;
   const float r = 1.0f / sqrtf(var + eps);
   const float r2 = r * r, r3 = r2 * r, r5 = r3 * r2;
 
@@ -90,7 +129,7 @@ __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void layernorm_kernel(
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       u[v] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (ok[v]) u[v] = folx_ld_stream4(jac + (int64_t)p * S + off + 4 * (lane + FOLX_WAVE * v));
+      if (ok[v]) u[v] = folx_ld_stream4(jac + (int64_t)p * S + off + 4 * (lane + LW * v));
     }
   };
   auto partial = [&](const float4* u, float& s1, float& s2, float& s3) {
@@ -117,7 +156,7 @@ __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void layernorm_kernel(
         o.y = g[v].y * r * (dy - c[v].y * cb);
         o.z = g[v].z * r * (dz - c[v].z * cb);
         o.w = g[v].w * r * (dw - c[v].w * cb);
-        folx_st_stream4(y_jac + (int64_t)p * S + off + 4 * (lane + FOLX_WAVE * v), o);
+        folx_st_stream4(y_jac + (int64_t)p * S + off + 4 * (lane + LW * v), o);
       }
     }
   };
@@ -134,10 +173,10 @@ __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void layernorm_kernel(
     partial(u1, b1, b2, b3);
     partial(u2, c1, c2, c3);
     partial(u3, e1, e2, e3);
-    wave_sum3(a1, a2, a3);
-    wave_sum3(b1, b2, b3);
-    wave_sum3(c1, c2, c3);
-    wave_sum3(e1, e2, e3);
+    group_sum3<LW>(a1, a2, a3);
+    group_sum3<LW>(b1, b2, b3);
+    group_sum3<LW>(c1, c2, c3);
+    group_sum3<LW>(e1, e2, e3);
     finish_row(p, u0, a1, a2, a3);
     finish_row(p + PS, u1, b1, b2, b3);
     finish_row(p + 2 * PS, u2, c1, c2, c3);
@@ -148,7 +187,7 @@ __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void layernorm_kernel(
     load_row(p, u0);
     float a1, a2, a3;
     partial(u0, a1, a2, a3);
-    wave_sum3(a1, a2, a3);
+    group_sum3<LW>(a1, a2, a3);
     finish_row(p, u0, a1, a2, a3);
   }
 
@@ -156,17 +195,17 @@ __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void layernorm_kernel(
   // wavefront's read of x before the write of y, which makes in-place use safe)
   if constexpr (!PER_WAVE) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v) redT[w][v * FOLX_WAVE + lane] = T[v];
-    if (lane == 0) { reds[w][0] = sb2; reds[w][1] = ss; }
+    for (int v = 0; v < NV; ++v) redT[w][v * FOLX_WAVE + wlane] = T[v];
+    if (lane == 0) { reds[w][sub][0] = sb2; reds[w][sub][1] = ss; }
     __syncthreads();
     if (w != 0) return;
-    sb2 = reds[0][0]; ss = reds[0][1];
+    sb2 = reds[0][sub][0]; ss = reds[0][sub][1];
 #pragma unroll
     for (int ww = 1; ww < PSPLIT; ++ww) {
-      sb2 += reds[ww][0]; ss += reds[ww][1];
+      sb2 += reds[ww][sub][0]; ss += reds[ww][sub][1];
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        const float4 t = redT[ww][v * FOLX_WAVE + lane];
+        const float4 t = redT[ww][v * FOLX_WAVE + wlane];
         T[v].x += t.x; T[v].y += t.y; T[v].z += t.z; T[v].w += t.w;
       }
     }
@@ -179,19 +218,19 @@ __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void layernorm_kernel(
   for (int v = 0; v < NV; ++v) {
     l[v] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (ok[v]) {
-      l[v] = *reinterpret_cast<const float4*>(lap + off + 4 * (lane + FOLX_WAVE * v));
+      l[v] = *reinterpret_cast<const float4*>(lap + off + 4 * (lane + LW * v));
       sl += l[v].x + l[v].y + l[v].z + l[v].w;
       scl += c[v].x * l[v].x + c[v].y * l[v].y + c[v].z * l[v].z + c[v].w * l[v].w;
     }
   }
   float dummy = 0.0f;
-  wave_sum3(sl, scl, dummy);
+  group_sum3<LW>(sl, scl, dummy);
   const float ml = sl * invF, mcl = scl * invF;
   const float k2 = 3.0f * r5 * sb2 - r3 * ss;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     if (ok[v]) {
-      const int i4 = lane + FOLX_WAVE * v;
+      const int i4 = lane + LW * v;
       const float4 bt = beta ? *reinterpret_cast<const float4*>(beta + 4 * i4) : make_float4(0.f, 0.f, 0.f, 0.f);
       float4 yo, lo;
       yo.x = g[v].x * r * c[v].x + bt.x; yo.y = g[v].y * r * c[v].y + bt.y;
@@ -220,19 +259,24 @@ extern "C" int folx_hip_layernorm_fwdlap(void* stream, const float* x, const flo
   for (const void* p : ptrs)
     if (p && !folx_aligned16(p)) return FOLX_HIP_ENOTSUP;
   const bool per_wave = P <= 8;
-  const int64_t blocks = per_wave ? (R + PSPLIT - 1) / PSPLIT : R;
+  const int lw = F <= 32 ? 8 : (F <= 64 ? 16 : (F <= 128 ? 32 : FOLX_WAVE));
+  const int64_t rows = (int64_t)(FOLX_WAVE / lw) * (per_wave ? PSPLIT : 1);  // of features, per workgroup
+  const int64_t blocks = (R + rows - 1) / rows;
   if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
   hipStream_t st = (hipStream_t)stream;
   dim3 grid((unsigned)blocks), block(FOLX_WAVE * PSPLIT);
   const int nv = (F / 4 + FOLX_WAVE - 1) / FOLX_WAVE;
-#define FOLX_LN(NV)                                                                                               \
-  if (per_wave) layernorm_kernel<NV, true><<<grid, block, 0, st>>>(x, jac, lap, gamma, beta, y, y_jac, y_lap, R, F, P, eps); \
-  else layernorm_kernel<NV, false><<<grid, block, 0, st>>>(x, jac, lap, gamma, beta, y, y_jac, y_lap, R, F, P, eps);
-  switch (nv) {
-    case 1: FOLX_LN(1) break;
-    case 2: FOLX_LN(2) break;
-    case 3: FOLX_LN(3) break;
-    default: FOLX_LN(4) break;
+#define FOLX_LN(NV, LW)                                                                                               \
+  if (per_wave) layernorm_kernel<NV, true, LW><<<grid, block, 0, st>>>(x, jac, lap, gamma, beta, y, y_jac, y_lap, R, F, P, eps); \
+  else layernorm_kernel<NV, false, LW><<<grid, block, 0, st>>>(x, jac, lap, gamma, beta, y, y_jac, y_lap, R, F, P, eps);
+  switch (lw < FOLX_WAVE ? -lw : nv) {
+    case -8: FOLX_LN(1, 8) break;
+    case -16: FOLX_LN(1, 16) break;
+    case -32: FOLX_LN(1, 32) break;
+    case 1: FOLX_LN(1, FOLX_WAVE) break;
+    case 2: FOLX_LN(2, FOLX_WAVE) break;
+    case 3: FOLX_LN(3, FOLX_WAVE) break;
+    default: FOLX_LN(4, FOLX_WAVE) break;
   }
 #undef FOLX_LN
   return folx_launch_status();
