@@ -143,8 +143,28 @@ __global__ __launch_bounds__(FOLX_WAVE * PSPLIT) void mul_sparse_kernel(
   }
 }
 
-__global__ __launch_bounds__(256) void rows_affine_kernel(const float* __restrict__ in,
-                                                          float* __restrict__ out, int64_t rows,
+// Row stacks of up to three arrays (a triplet's value, Jacobian rows and Laplacian) in one launch, numbered through: end[a]
+// is the first row behind array a.  Rows below `shifted` get beta d added.
+struct RowArrays {
+  const float* in[3];
+  float* out[3];
+  int64_t end[3];
+  int64_t shifted;
+  // row r's start in both, given the row lengths
+  __device__ __forceinline__ void find(int64_t r, int64_t in_S, int64_t S, const float*& src, float*& dst) const {
+    src = in[0]; dst = out[0];
+    if (r >= end[0]) {
+      const bool third = r >= end[1];
+      src = third ? in[2] : in[1];
+      dst = third ? out[2] : out[1];
+      r -= third ? end[1] : end[0];
+    }
+    src += r * in_S;
+    dst += r * S;
+  }
+};
+
+__global__ __launch_bounds__(256) void rows_affine_kernel(RowArrays arrays, int64_t rows,
                                                           int64_t in_S, int64_t S,
                                                           const float* __restrict__ c,
                                                           const float* __restrict__ d, float alpha,
@@ -156,15 +176,19 @@ __global__ __launch_bounds__(256) void rows_affine_kernel(const float* __restric
   const float cv = c ? alpha * c[ic.off(i)] : alpha;
   const float dv = d ? beta * d[id.off(i)] : 0.0f;
   // blockIdx.y strides over rows so that very tall stacks need no 64-bit grid
-  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) out[r * S + i] = in[r * in_S + oi] * cv + dv;
+  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
+    const float* in;
+    float* out;
+    arrays.find(r, in_S, S, in, out);
+    out[i] = in[oi] * cv + (r < arrays.shifted ? dv : 0.0f);
+  }
 }
 
 // The same map for index spaces whose inner extent is a multiple of 4 and whose operands are contiguous
 // (stride 1) or constant (stride 0) along it, all 16-byte aligned: a thread owns four consecutive
 // elements, one 128-bit streaming load and store per row, and its three offsets are computed once --
 // in 32-bit arithmetic (S < 2^31), without any division when the index space is flat.
-__global__ __launch_bounds__(256) void rows_affine_v4_kernel(const float* __restrict__ in,
-                                                             float* __restrict__ out, int64_t rows,
+__global__ __launch_bounds__(256) void rows_affine_v4_kernel(RowArrays arrays, int64_t rows,
                                                              int64_t in_S, int64_t S,
                                                              const float* __restrict__ c,
                                                              const float* __restrict__ d, float alpha,
@@ -194,11 +218,15 @@ __global__ __launch_bounds__(256) void rows_affine_v4_kernel(const float* __rest
     dv = make_float4(beta * v.x, beta * v.y, beta * v.z, beta * v.w);
   }
   for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-    const float* p = in + r * in_S + oi;
+    const float* in;
+    float* out;
+    arrays.find(r, in_S, S, in, out);
+    const float* p = in + oi;
     float4 v;
     if (iin.s2) v = folx_ld_stream4(p);
     else v = make_float4(*p, *p, *p, *p);
-    folx_st_stream4(out + r * S + i, make_float4(v.x * cv.x + dv.x, v.y * cv.y + dv.y, v.z * cv.z + dv.z, v.w * cv.w + dv.w));
+    const float4 e = r < arrays.shifted ? dv : make_float4(0.f, 0.f, 0.f, 0.f);
+    folx_st_stream4(out + i, make_float4(v.x * cv.x + e.x, v.y * cv.y + e.y, v.z * cv.z + e.z, v.w * cv.w + e.w));
   }
 }
 
@@ -239,37 +267,68 @@ extern "C" int folx_hip_binary_fwdlap(void* stream, int32_t op, const float* a, 
   return folx_launch_status();
 }
 
-extern "C" int folx_hip_rows_affine(void* stream, const float* in, float* out, int64_t rows,
-                                    int64_t in_S, const float* c, const float* d, float alpha,
-                                    float beta, const int64_t* dims) {
-  if (!dims || rows < 0 || in_S < 0) return FOLX_HIP_EINVAL;
+namespace {
+
+int launch_affine(hipStream_t st, int n, const float* const* in, float* const* out, const int64_t* rows_of, int64_t shifted,
+                  int64_t in_S, const float* c, const float* d, float alpha, float beta, const int64_t* dims) {
+  if (!dims || in_S < 0) return FOLX_HIP_EINVAL;
   if (dims[0] < 0 || dims[1] < 0 || dims[2] < 0) return FOLX_HIP_EINVAL;
   const int64_t S = dims[0] * dims[1] * dims[2];
-  if (S == 0 || rows == 0) return FOLX_HIP_OK;
-  if (!in || !out) return FOLX_HIP_EINVAL;
+  RowArrays a;
+  int64_t rows = 0;
+  bool in16 = true, out16 = true;
+  int used = 0;
+  for (int k = 0; k < n; ++k) {
+    if (rows_of[k] < 0) return FOLX_HIP_EINVAL;
+    if (S == 0 || rows_of[k] == 0) continue;
+    if (!in[k] || !out[k]) return FOLX_HIP_EINVAL;
+    rows += rows_of[k];
+    a.in[used] = in[k]; a.out[used] = out[k]; a.end[used++] = rows;
+    in16 = in16 && folx_aligned16(in[k]);
+    out16 = out16 && folx_aligned16(out[k]);
+  }
+  if (rows == 0) return FOLX_HIP_OK;
+  for (int k = used; k < 3; ++k) { a.in[k] = a.in[used - 1]; a.out[k] = a.out[used - 1]; a.end[k] = rows; }
+  a.shifted = shifted;
   const int64_t blocks = (S + 255) / 256;
   if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
   Bcast3 iin = mk(dims, 1), ic = mk(dims, 2), id = mk(dims, 3);
   const unsigned gy = (unsigned)(rows < 1024 ? rows : 1024);
   // 128-bit form: inner extent a multiple of 4, every operand contiguous or constant along it, every other
   // stride and the row pitch multiples of 4 floats, 16-byte aligned pointers, 32-bit element index
-  auto vec_ok = [&](const Bcast3& b, const float* p) {
-    if (!p) return true;
+  auto vec_ok = [&](const Bcast3& b, bool aligned) {
     if (b.s2 != 0 && b.s2 != 1) return false;
     if (b.s2 == 0) return true;
-    return folx_aligned16(p) && (dims[1] == 1 || b.s1 % 4 == 0) && (dims[0] == 1 || b.s0 % 4 == 0);
+    return aligned && (dims[1] == 1 || b.s1 % 4 == 0) && (dims[0] == 1 || b.s0 % 4 == 0);
   };
-  const bool v4 = dims[2] % 4 == 0 && S < 0x7fffffffLL && folx_aligned16(out) && vec_ok(iin, in) && vec_ok(ic, c) &&
-                  vec_ok(id, d) && (rows == 1 || iin.s2 == 0 || in_S % 4 == 0);
+  const bool v4 = dims[2] % 4 == 0 && S < 0x7fffffffLL && out16 && vec_ok(iin, in16) && (!c || vec_ok(ic, folx_aligned16(c))) &&
+                  (!d || vec_ok(id, folx_aligned16(d))) && (rows == 1 || iin.s2 == 0 || in_S % 4 == 0);
   if (v4) {
     const int64_t blocks4 = (S / 4 + 255) / 256;
-    rows_affine_v4_kernel<<<dim3((unsigned)blocks4, gy), dim3(256), 0, (hipStream_t)stream>>>(
-        in, out, rows, in_S, S, c, d, alpha, beta, iin, ic, id);
+    rows_affine_v4_kernel<<<dim3((unsigned)blocks4, gy), dim3(256), 0, st>>>(a, rows, in_S, S, c, d, alpha, beta, iin, ic, id);
   } else {
-    rows_affine_kernel<<<dim3((unsigned)blocks, gy), dim3(256), 0, (hipStream_t)stream>>>(
-        in, out, rows, in_S, S, c, d, alpha, beta, iin, ic, id);
+    rows_affine_kernel<<<dim3((unsigned)blocks, gy), dim3(256), 0, st>>>(a, rows, in_S, S, c, d, alpha, beta, iin, ic, id);
   }
   return folx_launch_status();
+}
+
+}  // namespace
+
+extern "C" int folx_hip_rows_affine(void* stream, const float* in, float* out, int64_t rows,
+                                    int64_t in_S, const float* c, const float* d, float alpha,
+                                    float beta, const int64_t* dims) {
+  if (rows < 0) return FOLX_HIP_EINVAL;
+  return launch_affine((hipStream_t)stream, 1, &in, &out, &rows, rows, in_S, c, d, alpha, beta, dims);
+}
+
+extern "C" int folx_hip_affine_fwdlap(void* stream, const float* x, const float* jac, const float* lap, float* y,
+                                      float* y_jac, float* y_lap, int32_t P, int64_t in_S, const float* c, const float* d,
+                                      float alpha, float beta, const int64_t* dims) {
+  if (P < 0) return FOLX_HIP_EINVAL;
+  const float* in[3] = {x, jac, lap};
+  float* out[3] = {y, y_jac, y_lap};
+  const int64_t rows[3] = {1, P, 1};
+  return launch_affine((hipStream_t)stream, 3, in, out, rows, 1, in_S, c, d, alpha, beta, dims);
 }
 
 extern "C" int folx_hip_mul_sparse_fwdlap(void* stream, const float* a, const float* a_jac, const float* a_lap,

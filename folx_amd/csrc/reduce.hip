@@ -6,15 +6,35 @@
 
 namespace {
 
+// Up to three arrays (a triplet's value, Jacobian rows and Laplacian) in one launch: outputs are numbered through, end[a] is
+// the first number behind array a.  On small batches a launch of its own for each cost more than its work (7 electrons, 512
+// walkers: a spin-wise mean of the value 4.7 us where its Jacobian rows take 8).
+struct Arrays {
+  const float* in[3];
+  float* out[3];
+  int64_t end[3];
+  // the array of output o, which becomes its number inside that array
+  __device__ __forceinline__ void find(int64_t& o, const float*& src, float*& dst) const {
+    src = in[0]; dst = out[0];
+    if (o >= end[0]) {
+      const bool third = o >= end[1];
+      src = third ? in[2] : in[1];
+      dst = third ? out[2] : out[1];
+      o -= third ? end[1] : end[0];
+    }
+  }
+};
+
 // inner >= 2: one thread per output element, consecutive threads on consecutive `inner`
 // positions so every step of the loop over `red` is a coalesced read.
 template <bool MAX>
-__global__ __launch_bounds__(256) void reduce_mid_kernel(const float* __restrict__ in,
-                                                         float* __restrict__ out, int64_t total,
-                                                         int64_t red, int64_t inner, int64_t span, int64_t lo,
-                                                         float alpha) {
-  const int64_t o = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(256) void reduce_mid_kernel(Arrays arrays, int64_t total, int64_t red,
+                                                         int64_t inner, int64_t span, int64_t lo, float alpha) {
+  int64_t o = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (o >= total) return;
+  const float* in;
+  float* out;
+  arrays.find(o, in, out);
   const int64_t ii = o % inner;
   const int64_t ro = o / inner;  // (row, outer) flattened
   const float* src = in + (ro * span + lo) * inner + ii;
@@ -30,12 +50,14 @@ __global__ __launch_bounds__(256) void reduce_mid_kernel(const float* __restrict
 // four of them in flight per thread (the scalar form above keeps one 4-byte load per thread in
 // flight and reaches 3 TB/s on the spin-wise means of a 16-electron layer; this one 5).
 template <bool MAX>
-__global__ __launch_bounds__(256) void reduce_mid_v4_kernel(const float* __restrict__ in,
-                                                            float* __restrict__ out, int64_t total4,
+__global__ __launch_bounds__(256) void reduce_mid_v4_kernel(Arrays arrays /* numbered by four outputs */, int64_t total4,
                                                             int64_t red, int64_t inner, int64_t span, int64_t lo,
                                                             float alpha) {
-  const int64_t o4 = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  int64_t o4 = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (o4 >= total4) return;
+  const float* in;
+  float* out;
+  arrays.find(o4, in, out);
   const int64_t inner4 = inner / 4;
   const int64_t ii = (o4 % inner4) * 4;
   const int64_t ro = o4 / inner4;  // (row, outer) flattened
@@ -64,23 +86,30 @@ __global__ __launch_bounds__(256) void reduce_mid_v4_kernel(const float* __restr
 // WAVE: G = 64 as a constant; a long axis read in single values is bound by its instructions (23 317 sums of 206: 7.6 -> 6.6 us,
 // 29 035 of 434: 15.5 -> 14.4 us).
 template <bool MAX, int VEC, int U, bool WAVE>
-__global__ __launch_bounds__(256) void reduce_last_kernel(const float* __restrict__ in, float* __restrict__ out,
-                                                          int64_t total, int64_t red, int64_t span, int64_t lo,
-                                                          int32_t group, float alpha) {
+__global__ __launch_bounds__(256) void reduce_last_kernel(Arrays arrays, int64_t total, int64_t red, int64_t span,
+                                                          int64_t lo, int32_t group, float alpha) {
   const int G = WAVE ? FOLX_WAVE : group;
   const int per = 256 / G, g = threadIdx.x / G, l = threadIdx.x % G;
   const int64_t o0 = (int64_t)blockIdx.x * (per * U) + g;
   const int64_t pieces = red / VEC;
   float acc[U];
+  const float* src[U];
+  float* dst[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) acc[u] = MAX ? -INFINITY : 0.0f;
+  for (int u = 0; u < U; ++u) {
+    acc[u] = MAX ? -INFINITY : 0.0f;
+    // outputs past the end read the last one's values
+    int64_t o = o0 + u * per < total ? o0 + u * per : total - 1;
+    const float* in;
+    arrays.find(o, in, dst[u]);
+    src[u] = in + o * span + lo;
+    dst[u] += o;
+  }
   for (int64_t r = l; r < pieces; r += G) {
     float v[U][VEC];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      // outputs past the end read the last one's values
-      const int64_t o = o0 + u * per < total ? o0 + u * per : total - 1;
-      const float* p = in + o * span + lo + r * VEC;
+      const float* p = src[u] + r * VEC;
       if constexpr (VEC == 4) {
         const float4 q = folx_ld_stream4(p);
         v[u][0] = q.x; v[u][1] = q.y; v[u][2] = q.z; v[u][3] = q.w;
@@ -102,12 +131,11 @@ __global__ __launch_bounds__(256) void reduce_last_kernel(const float* __restric
   if (l == 0)
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (o0 + u * per < total) out[o0 + u * per] = MAX ? acc[u] : alpha * acc[u];
+      if (o0 + u * per < total) *dst[u] = MAX ? acc[u] : alpha * acc[u];
 }
 
 template <bool MAX, int VEC>
-int launch_reduce_last(hipStream_t st, const float* in, float* out, int64_t total, int64_t red, int64_t span, int64_t lo,
-                       float alpha) {
+int launch_reduce_last(hipStream_t st, const Arrays& a, int64_t total, int64_t red, int64_t span, int64_t lo, float alpha) {
   int G = 1;
   while (G < FOLX_WAVE && G < red / VEC) G *= 2;
   const int64_t per = 256 / G;
@@ -117,37 +145,58 @@ int launch_reduce_last(hipStream_t st, const float* in, float* out, int64_t tota
   if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
   const dim3 grid((unsigned)blocks), block(256);
   if (G == FOLX_WAVE) {
-    if (U == 4) reduce_last_kernel<MAX, VEC, 4, true><<<grid, block, 0, st>>>(in, out, total, red, span, lo, G, alpha);
-    else reduce_last_kernel<MAX, VEC, 1, true><<<grid, block, 0, st>>>(in, out, total, red, span, lo, G, alpha);
+    if (U == 4) reduce_last_kernel<MAX, VEC, 4, true><<<grid, block, 0, st>>>(a, total, red, span, lo, G, alpha);
+    else reduce_last_kernel<MAX, VEC, 1, true><<<grid, block, 0, st>>>(a, total, red, span, lo, G, alpha);
   } else {
-    if (U == 4) reduce_last_kernel<MAX, VEC, 4, false><<<grid, block, 0, st>>>(in, out, total, red, span, lo, G, alpha);
-    else reduce_last_kernel<MAX, VEC, 1, false><<<grid, block, 0, st>>>(in, out, total, red, span, lo, G, alpha);
+    if (U == 4) reduce_last_kernel<MAX, VEC, 4, false><<<grid, block, 0, st>>>(a, total, red, span, lo, G, alpha);
+    else reduce_last_kernel<MAX, VEC, 1, false><<<grid, block, 0, st>>>(a, total, red, span, lo, G, alpha);
+  }
+  return folx_launch_status();
+}
+
+// array k: outer[k] x (window of span) x inner
+template <bool MAX>
+int launch_reduce(hipStream_t st, int n, const float* const* in, float* const* out, const int64_t* outer, int64_t red,
+                  int64_t inner, float alpha, int64_t span, int64_t lo) {
+  if (red < 0 || inner < 0 || lo < 0 || lo + red > span) return FOLX_HIP_EINVAL;
+  Arrays a;
+  int64_t total = 0;
+  bool in16 = true, out16 = true;
+  int used = 0;
+  for (int k = 0; k < n; ++k) {
+    if (outer[k] < 0) return FOLX_HIP_EINVAL;
+    if (outer[k] * inner == 0) continue;
+    if (!in[k] || !out[k]) return FOLX_HIP_EINVAL;
+    total += outer[k] * inner;
+    a.in[used] = in[k]; a.out[used] = out[k]; a.end[used++] = total;
+    in16 = in16 && folx_aligned16(in[k]);
+    out16 = out16 && folx_aligned16(out[k]);
+  }
+  if (total == 0) return FOLX_HIP_OK;
+  for (int k = used; k < 3; ++k) { a.in[k] = a.in[used - 1]; a.out[k] = a.out[used - 1]; a.end[k] = total; }
+  if (inner == 1 && red >= 16) {
+    if (red % 4 == 0 && span % 4 == 0 && lo % 4 == 0 && in16)
+      return launch_reduce_last<MAX, 4>(st, a, total, red, span, lo, alpha);
+    return launch_reduce_last<MAX, 1>(st, a, total, red, span, lo, alpha);
+  } else if (inner % 4 == 0 && in16 && out16) {
+    const int64_t blocks = (total / 4 + 255) / 256;
+    if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
+    for (int64_t& e : a.end) e /= 4;
+    reduce_mid_v4_kernel<MAX><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(a, total / 4, red, inner, span, lo, alpha);
+  } else {
+    const int64_t blocks = (total + 255) / 256;
+    if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
+    reduce_mid_kernel<MAX><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(a, total, red, inner, span, lo, alpha);
   }
   return folx_launch_status();
 }
 
 template <bool MAX>
-int launch_reduce(hipStream_t st, const float* in, float* out, int64_t rows, int64_t outer,
-                  int64_t red, int64_t inner, float alpha, int64_t span, int64_t lo) {
-  if (rows < 0 || outer < 0 || red < 0 || inner < 0 || lo < 0 || lo + red > span) return FOLX_HIP_EINVAL;
-  const int64_t total = rows * outer * inner;
-  if (total == 0) return FOLX_HIP_OK;
-  if (!in || !out) return FOLX_HIP_EINVAL;
-  if (inner == 1 && red >= 16) {
-    if (red % 4 == 0 && span % 4 == 0 && lo % 4 == 0 && folx_aligned16(in))
-      return launch_reduce_last<MAX, 4>(st, in, out, total, red, span, lo, alpha);
-    return launch_reduce_last<MAX, 1>(st, in, out, total, red, span, lo, alpha);
-  } else if (inner % 4 == 0 && folx_aligned16(in) && folx_aligned16(out)) {
-    const int64_t blocks = (total / 4 + 255) / 256;
-    if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
-    reduce_mid_v4_kernel<MAX><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(in, out, total / 4, red, inner, span, lo,
-                                                                          alpha);
-  } else {
-    const int64_t blocks = (total + 255) / 256;
-    if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
-    reduce_mid_kernel<MAX><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(in, out, total, red, inner, span, lo, alpha);
-  }
-  return folx_launch_status();
+int launch_reduce(hipStream_t st, const float* in, float* out, int64_t rows, int64_t outer, int64_t red, int64_t inner,
+                  float alpha, int64_t span, int64_t lo) {
+  if (rows < 0 || outer < 0) return FOLX_HIP_EINVAL;
+  const int64_t ro = rows * outer;
+  return launch_reduce<MAX>(st, 1, &in, &out, &ro, red, inner, alpha, span, lo);
 }
 
 }  // namespace
@@ -167,4 +216,11 @@ extern "C" int folx_hip_reduce_sum_window(void* stream, const float* in, float* 
 extern "C" int folx_hip_reduce_max(void* stream, const float* in, float* out, int64_t outer,
                                    int64_t red, int64_t inner) {
   return launch_reduce<true>((hipStream_t)stream, in, out, 1, outer, red, inner, 1.0f, red, 0);
+}
+
+extern "C" int folx_hip_reduce_sum_arrays(void* stream, int32_t n, const float* const* in, float* const* out,
+                                          const int64_t* outer, int64_t span, int64_t lo, int64_t hi, int64_t inner,
+                                          float alpha) {
+  if (n < 1 || n > 3 || !in || !out || !outer || hi < lo) return FOLX_HIP_EINVAL;
+  return launch_reduce<false>((hipStream_t)stream, n, in, out, outer, hi - lo, inner, alpha, span, lo);
 }

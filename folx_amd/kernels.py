@@ -8,6 +8,7 @@ contiguous and on the GPU.  Layout: x (B, *s), jac (P, B, *s), lap (B, *s).
 from __future__ import annotations
 
 import ctypes
+import math
 
 import numpy as np
 import torch
@@ -700,16 +701,19 @@ def mul_sparse(a, aj, al, b, bj, bl, index):
     return y, yj, yl
 
 
-def rows_affine(inp, rows, row_shape, out_shape, c=None, d=None, alpha=1.0, beta=1.0):
-    """out[r] = alpha * in[r] * c + beta * d with broadcasting to ``out_shape``.
-    ``inp`` holds ``rows`` rows of shape ``row_shape``; c / d are arrays broadcastable to
-    ``out_shape``.  Returns a tensor (rows, *out_shape)."""
-    _chk(inp, c, d)
+def _affine_space(row_shape, out_shape, c, d):
+    """The index space of ``alpha * in * c + beta * d`` over ``out_shape``: (c, d, dims), with c and d spelled out over more
+    axes where three index dimensions do not cover their broadcasts, or None if the input's do not fit."""
     sin = bstrides(row_shape, out_shape)
-    sc = bstrides(c.shape, out_shape) if c is not None else [0] * len(out_shape)
-    sd = bstrides(d.shape, out_shape) if d is not None else [0] * len(out_shape)
-    col = collapse3(out_shape, sin, sc, sd)
-    if col is None:
+
+    def space(c, d):
+        sc = bstrides(c.shape, out_shape) if c is not None else [0] * len(out_shape)
+        sd = bstrides(d.shape, out_shape) if d is not None else [0] * len(out_shape)
+        col = collapse3(out_shape, sin, sc, sd)
+        return None if col is None else (c, d, [*col[0], *col[1][0], *col[1][1], *col[1][2]])
+
+    got = space(c, d)
+    if got is None:
         # a coefficient array that is broadcast along inner axes (e.g. a per-matrix identity against
         # (walker, row, determinant, column)): spell its broadcast out over all axes but the first,
         # then over all axes, until the index space collapses to three dimensions
@@ -720,14 +724,19 @@ def rows_affine(inp, rows, row_shape, out_shape, c=None, d=None, alpha=1.0, beta
                 full = (1,) * (len(out_shape) - t.dim()) + tuple(t.shape)
                 tgt = tuple(full[:lead]) + tuple(out_shape[lead:])
                 return t.reshape(full).expand(tgt).contiguous()
-            c2, d2 = spelled(c), spelled(d)
-            sc = bstrides(c2.shape, out_shape) if c2 is not None else [0] * len(out_shape)
-            sd = bstrides(d2.shape, out_shape) if d2 is not None else [0] * len(out_shape)
-            col = collapse3(out_shape, sin, sc, sd)
-            if col is not None:
-                c, d = c2, d2
+            got = space(spelled(c), spelled(d))
+            if got is not None:
                 break
-    if col is None:
+    return got
+
+
+def rows_affine(inp, rows, row_shape, out_shape, c=None, d=None, alpha=1.0, beta=1.0):
+    """out[r] = alpha * in[r] * c + beta * d with broadcasting to ``out_shape``.
+    ``inp`` holds ``rows`` rows of shape ``row_shape``; c / d are arrays broadcastable to
+    ``out_shape``.  Returns a tensor (rows, *out_shape)."""
+    _chk(inp, c, d)
+    got = _affine_space(row_shape, out_shape, c, d)
+    if got is None:
         # the INPUT is broadcast along several separate groups of axes: spell the first group out in a pass of its own
         # (a plain broadcast copy, three index dimensions), then come back with one group fewer
         rs = (1,) * (len(out_shape) - len(row_shape)) + tuple(int(v) for v in row_shape)
@@ -743,18 +752,39 @@ def rows_affine(inp, rows, row_shape, out_shape, c=None, d=None, alpha=1.0, beta
         raise NotImplementedError(
             f'rows_affine: the input of shape {tuple(row_shape)} broadcast to {tuple(out_shape)} needs more than '
             'three index dimensions; broadcast it with broadcast_to first')
-    n, (s_in, s_c, s_d) = col
+    c, d, dims = got
     out = torch.empty((rows, *out_shape), device=inp.device, dtype=torch.float32)
     in_S = int(np.prod(row_shape, dtype=np.int64))
     with _timed('rows_affine', (rows, int(np.prod(out_shape, dtype=np.int64)))):
         check(
             _lib.load().folx_hip_rows_affine(
-                _stream(), _p(inp), _p(out), rows, in_S, _p(c), _p(d), float(alpha), float(beta),
-                _dims(*n, *s_in, *s_c, *s_d),
+                _stream(), _p(inp), _p(out), rows, in_S, _p(c), _p(d), float(alpha), float(beta), _dims(*dims),
             ),
             'rows_affine',
         )
     return out
+
+
+def affine(x, jac, lap, row_shape, out_shape, c=None, d=None, alpha=1.0, beta=1.0):
+    """``rows_affine`` of a triplet in one launch: ``alpha * x * c + beta * d``, and ``alpha * (.) * c`` of the Jacobian rows and
+    the Laplacian; None where the input's broadcast does not fit one launch."""
+    _chk(x, jac, lap, c, d)
+    got = _affine_space(row_shape, out_shape, c, d)
+    if got is None:
+        return None
+    c, d, dims = got
+    P = jac.shape[0]
+    y = torch.empty(out_shape, device=x.device, dtype=torch.float32)
+    yj, yl = torch.empty((P, *out_shape), device=x.device, dtype=torch.float32), torch.empty_like(y)
+    with _timed('rows_affine', (P + 2, y.numel())):
+        check(
+            _lib.load().folx_hip_affine_fwdlap(
+                _stream(), _p(x), _p(jac), _p(lap), _p(y), _p(yj), _p(yl), P, x.numel(), _p(c), _p(d), float(alpha),
+                float(beta), _dims(*dims),
+            ),
+            'affine_fwdlap',
+        )
+    return y, yj, yl
 
 
 def reduce_sum(inp, rows, outer, red, inner, alpha=1.0, window=None):
@@ -771,6 +801,29 @@ def reduce_sum(inp, rows, outer, red, inner, alpha=1.0, window=None):
                                                         inner, float(alpha))
         check(rc, 'reduce_sum')
     return out
+
+
+def reduce_sum_arrays(arrays, axes, alpha=1.0, window=None):
+    """The sum over one axis of up to three arrays in one launch: array i over its axis ``axes[i]``, the axes and everything
+    behind them of one shape (a triplet's value, Jacobian rows and Laplacian)."""
+    _chk(*arrays)
+    red, inner = arrays[0].shape[axes[0]], math.prod(arrays[0].shape[axes[0] + 1:])
+    lo, hi = (0, red) if window is None else window
+    outs, n = [], len(arrays)
+    for t, ax in zip(arrays, axes):
+        assert t.shape[ax] == red and math.prod(t.shape[ax + 1:]) == inner
+        outs.append(torch.empty((*t.shape[:ax], *t.shape[ax + 1:]), device=t.device, dtype=torch.float32))
+    outer = [math.prod(t.shape[:ax]) for t, ax in zip(arrays, axes)]
+    with _timed('reduce_sum', (1, sum(outer), red, inner)):
+        check(
+            _lib.load().folx_hip_reduce_sum_arrays(
+                _stream(), n, (ctypes.c_void_p * n)(*[t.data_ptr() for t in arrays]),
+                (ctypes.c_void_p * n)(*[t.data_ptr() for t in outs]), (ctypes.c_int64 * n)(*outer), red, int(lo), int(hi),
+                inner, float(alpha)
+            ),
+            'reduce_sum_arrays',
+        )
+    return outs
 
 
 def reduce_max(inp, outer, red, inner):

@@ -245,8 +245,12 @@ def _affine_const(t: FwdLaplArray, c, *, mul: bool, alpha: float, beta: float) -
         if not mul:
             ct = None
     full = (B, *out_shape)
-    x = K.rows_affine(t.x, 1, (B, *t.shape), full, ct, d_t, a_x, b_x).reshape(full)
     same = out_shape == t.shape and ct is None and a_j == 1.0
+    if not same and t.x.is_cuda:   # value, Jacobian rows and Laplacian in one launch
+        got = K.affine(t.x, t.jacobian.data, t.laplacian, (B, *t.shape), full, ct, d_t, a_x, b_x)
+        if got is not None:
+            return FwdLaplArray(got[0], FwdJacobian(got[1], _bmask(t.jacobian.x0_idx, k, out_shape)), got[2])
+    x = K.rows_affine(t.x, 1, (B, *t.shape), full, ct, d_t, a_x, b_x).reshape(full)
     if same:
         J, lap = t.jacobian.data, t.laplacian
     else:
@@ -1232,6 +1236,16 @@ def _reduce_tensor(t: torch.Tensor, lead: int, axes, alpha=1.0, window=None) -> 
     return t
 
 
+def _reduce_tensors(ts, leads, axes, alpha=1.0, window=None):
+    """``_reduce_tensor`` of several arrays with the same logical axes, on the GPU in one launch an axis."""
+    if not ts[0].is_cuda:
+        return [_reduce_tensor(t, lead, axes, alpha, window) for t, lead in zip(ts, leads)]
+    for ax in sorted(axes, reverse=True):
+        ts = K.reduce_sum_arrays([t.contiguous() for t in ts], [ax + lead for lead in leads], alpha, window)
+        alpha = 1.0
+    return ts
+
+
 def reduce_sum(args, kwargs, sparsity_threshold):
     """``reduce_sum`` (SUMMATION, folx/wrapped_functions.py:388-392).  Dense: the same sum
     on x, rows and lap.  Sparse (``sparse_sum_jvp``, folx/jvp.py:89-176): static output
@@ -1256,11 +1270,10 @@ def reduce_sum(args, kwargs, sparsity_threshold):
         assert len(axes) == 1
         window = (int(window[0]), int(window[1]))
         assert 0 <= window[0] <= window[1] <= a.shape[axes[0]]
-    x = _reduce_tensor(a.x, 1, axes, scale, window)
-    lap = _reduce_tensor(a.laplacian, 1, axes, scale, window)
     J, mask = a.jacobian.data, a.jacobian.x0_idx
     if mask is None:
-        return FwdLaplArray(x, FwdJacobian(_reduce_tensor(J, 2, axes, scale, window), None), lap)
+        x, Jr, lap = _reduce_tensors((a.x, J, a.laplacian), (1, 2, 1), axes, scale, window)
+        return FwdLaplArray(x, FwdJacobian(Jr, None), lap)
 
     k = mask.shape[0]
     mask = np.broadcast_to(mask, (k, *a.shape))
@@ -1287,11 +1300,13 @@ def reduce_sum(args, kwargs, sparsity_threshold):
     kept_shape = [n for i, n in enumerate(a.shape) if i not in axes]
     if (slot == first).all():
         # every row keeps one slot along the reduced axes: reduce rows, then re-slot
-        Jr = _reduce_tensor(J, 2, axes, scale, window)
+        x, Jr, lap = _reduce_tensors((a.x, J, a.laplacian), (1, 2, 1), axes, scale, window)
         slot_c = first.reshape(k, *kept_shape)
         ident = n_out == k and (slot_c == np.arange(k).reshape(k, *([1] * (slot_c.ndim - 1)))).all()
         Jo = Jr if ident else so.materialize(Jr, slot_c, n_out)
-    elif len(axes) == 1:
+        return FwdLaplArray(x, FwdJacobian(Jo, out_mask), lap)
+    x, lap = _reduce_tensors((a.x, a.laplacian), (1, 1), axes, scale, window)
+    if len(axes) == 1:
         # slots vary along the reduced axis: gather (row, entry of the axis) pairs into their slots, the
         # data read where it lies (no slice of the window, no permuted copy)
         Jo = so.materialize_reduced(J, slot, n_out, axes[0], a.shape, window, scale)

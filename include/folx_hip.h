@@ -396,6 +396,11 @@ int folx_hip_layernorm_fwdlap(void* stream, const float* x, const float* jac, co
 int folx_hip_rows_affine(void* stream, const float* in, float* out, int64_t rows,
                          int64_t in_S, const float* c, const float* d, float alpha,
                          float beta, const int64_t* dims);
+/* The same for a triplet: y = alpha x c + beta d, and alpha (.) c on the P Jacobian rows and the Laplacian, which are never
+ * shifted (LINEAR against a constant, folx/wrapped_functions.py:361-376), in one launch; dims and in_S as above. */
+int folx_hip_affine_fwdlap(void* stream, const float* x, const float* jac, const float* lap, float* y, float* y_jac,
+                           float* y_lap, int32_t P, int64_t in_S, const float* c, const float* d, float alpha, float beta,
+                           const int64_t* dims);
 
 /*
  * Sum over the middle axis: in [rows][outer][red][inner] -> out [rows][outer][inner],
@@ -414,6 +419,10 @@ int folx_hip_reduce_sum(void* stream, const float* in, float* out, int64_t rows,
 int folx_hip_reduce_sum_window(void* stream, const float* in, float* out, int64_t rows,
                                int64_t outer, int64_t span, int64_t lo, int64_t hi,
                                int64_t inner, float alpha);
+/* The same window sum of up to three arrays (a triplet's value, Jacobian rows and Laplacian) in one launch: array k is
+ * [outer[k]][span][inner] -> [outer[k]][inner]; in, out and outer are host arrays of n entries. */
+int folx_hip_reduce_sum_arrays(void* stream, int32_t n, const float* const* in, float* const* out, const int64_t* outer,
+                               int64_t span, int64_t lo, int64_t hi, int64_t inner, float alpha);
 
 /* max over the middle axis of a value array (no derivatives): [outer][red][inner] ->
  * [outer][inner].  Used for the stop-gradient shift of logsumexp. */
