@@ -14,6 +14,7 @@ shape ``(k, *shape)`` shared by all walkers, as in the reference under ``vmap``.
 
 from __future__ import annotations
 
+import math
 from enum import IntFlag
 from typing import Any, NamedTuple, Protocol
 
@@ -206,7 +207,7 @@ class FwdLaplArray:
 
     @property
     def size(self):
-        return int(np.prod(self.shape, dtype=int))
+        return int(math.prod(self.shape))
 
     @property
     def B(self):

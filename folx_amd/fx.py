@@ -14,6 +14,7 @@ LayerNorm in front of it and the activation behind it exactly as in a model writ
 from __future__ import annotations
 
 import logging
+import math
 import operator
 
 import numpy as np
@@ -91,8 +92,8 @@ def _reduce(fn):
 def _view(a, shape):
     shape = [int(n) for n in shape]
     if -1 in shape:
-        known = int(np.prod([n for n in shape if n != -1], dtype=int))
-        shape[shape.index(-1)] = int(np.prod(_shape(a), dtype=int)) // max(known, 1)
+        known = int(math.prod([n for n in shape if n != -1]))
+        shape[shape.index(-1)] = int(math.prod(_shape(a))) // max(known, 1)
     return fnp.reshape(a, tuple(shape))
 
 
@@ -224,7 +225,7 @@ def _var(root):
     def rule(a, dim=None, correction=1, keepdim=False):
         nd = len(_shape(a))
         axes = _dims(dim, nd)
-        n = int(np.prod([_shape(a)[i] for i in axes], dtype=int))
+        n = int(math.prod([_shape(a)[i] for i in axes]))
         c = 1 if correction is None else correction
         centred = fnp.subtract(a, fnp.mean(a, axis=axes, keepdims=True))
         v = fnp.multiply(fnp.sum(fnp.square(centred), axis=axes, keepdims=bool(keepdim)), 1.0 / max(n - float(c), 1e-30))
@@ -544,9 +545,9 @@ def _index_dynamic(a, indices):
     ishape = tuple(flat.shape[1:])
     flat = flat.expand(B, *ishape)
     # (lead..., N, tail...) -> pick along N for every index entry
-    src = fnp.reshape(a, (*s[:lo], int(np.prod(dims, dtype=int)), *s[hi:]))
+    src = fnp.reshape(a, (*s[:lo], int(math.prod(dims)), *s[hi:]))
     lead, tail = s[:lo], s[hi:]
-    k = int(np.prod(ishape, dtype=int))
+    k = int(math.prod(ishape))
     idx = flat.reshape(B, *([1] * len(lead)), k, *([1] * len(tail))).expand(B, *lead, k, *tail)
     out = _select_along(src, BatchedArray(idx), lo)
     return fnp.reshape(out, (*lead, *ishape, *tail))
@@ -868,21 +869,48 @@ def fold_constants(gm: torch.fx.GraphModule):
     return {n: _tree(v, _const) for n, v in env.items()}
 
 
+_OPERAND_READERS = {aten.add.Tensor, aten.mul.Tensor}   # their rules take a device tensor as the constant operand
 _WEIGHT_READERS = {aten.mm.default, aten.addmm.default, aten.bmm.default, aten.matmul.default, aten.mv.default,
                    aten.native_layer_norm.default}
 _DEVICE_CONST_MIN = 256   # constants of at least this many floats live on the device between evaluations
 
 
-def _reading_order(gm: torch.fx.GraphModule):
-    """(position of each node, {node: the nodes it is the last to read}); worked out once per graph."""
-    got = gm.meta.get('folx_reading_order')
+class _Step:
+    """What does not change from one evaluation of an equation to the next: where its operands come from (an argument that
+    holds no node, or one node, is taken as it is), the keyword values a rule sees, and which values nobody reads after it."""
+
+    __slots__ = ('node', 'op', 'target', 'args', 'kwargs', 'drop')
+
+    def __init__(self, node, drop):
+        self.node, self.op, self.target, self.drop = node, node.op, node.target, drop
+        nested = lambda a: not isinstance(a, torch.fx.Node) and any(True for _ in _nodes_in(a))   # noqa: E731
+        self.args = [(2 if nested(a) else (1 if isinstance(a, torch.fx.Node) else 0), a) for a in node.args]
+        kept = {k: v for k, v in node.kwargs.items() if k not in ('dtype', 'device', 'layout', 'pin_memory', 'memory_format')}
+        self.kwargs = [(k, 2 if nested(v) else (1 if isinstance(v, torch.fx.Node) else 0), v) for k, v in kept.items()]
+
+
+def _nodes_in(a):
+    if isinstance(a, torch.fx.Node):
+        yield a
+    elif isinstance(a, (list, tuple)):
+        for t in a:
+            yield from _nodes_in(t)
+    elif isinstance(a, dict):
+        yield from _nodes_in(tuple(a.values()))
+    elif isinstance(a, slice):
+        yield from _nodes_in((a.start, a.stop, a.step))
+
+
+def _steps(gm: torch.fx.GraphModule):
+    """(position of each node, its ``_Step``s in order); worked out once per graph."""
+    got = gm.meta.get('folx_steps')
     if got is None:
         order = {n: i for i, n in enumerate(gm.graph.nodes)}
         last_read = {}
         for n in order:
             if n.users and n.op != 'output':
                 last_read.setdefault(max(n.users, key=order.__getitem__), []).append(n)
-        got = gm.meta['folx_reading_order'] = (order, last_read)
+        got = gm.meta['folx_steps'] = (order, [_Step(n, tuple(last_read.get(n, ()))) for n in order])
     return got
 
 
@@ -892,23 +920,22 @@ def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None):
     env = dict(fold_constants(gm) if consts is None else consts)
     it = iter(inputs)
     look = lambda a: env[a] if isinstance(a, torch.fx.Node) else a
-    order, last_read = _reading_order(gm)
-    done = None
-    for node in gm.graph.nodes:
-        if done is not None:   # what nobody reads any more: its memory serves the next equation, and a deferred value is free
-            args = kwargs = None
-            for n in last_read.get(done, ()):
-                env.pop(n, None)
-        done = node
+    take = lambda kind, a: a if kind == 0 else (env[a] if kind == 1 else torch.fx.node.map_arg(a, look))   # noqa: E731
+    order, steps = _steps(gm)
+    done = ()
+    for step in steps:
+        args = kwargs = None
+        for n in done:   # what nobody reads any more: its memory serves the next equation, and a deferred value is free
+            env.pop(n, None)
+        done, node = step.drop, step.node
         if node in env:
             continue
-        if node.op == 'placeholder':
+        if step.op == 'placeholder':
             env[node] = next(it)
-        elif node.op == 'call_function':
-            args = torch.fx.node.map_arg(node.args, look)
-            kwargs = torch.fx.node.map_arg(node.kwargs, look)
-            kwargs = {k: v for k, v in kwargs.items() if k not in ('dtype', 'device', 'layout', 'pin_memory', 'memory_format')}
-            rule = RULES.get(node.target)
+        elif step.op == 'call_function':
+            args = [take(kind, a) for kind, a in step.args]
+            kwargs = {k: take(kind, a) for k, kind, a in step.kwargs}
+            rule = RULES.get(step.target)
             functional = _functional_form(node.target) if rule is None else None
             if functional is not None:
                 # an in-place update of an intermediate (inside a library function: ``tmp.add_(eps)``): the functional
@@ -933,7 +960,7 @@ def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None):
             except Exception:
                 logging.error(f'forward Laplacian of {node.format_node()} failed')   # folx/interpreter.py:254-257
                 raise
-        elif node.op == 'output':
+        elif step.op == 'output':
             return torch.fx.node.map_arg(node.args[0], look)
         else:
             raise NotImplementedError(f'graph node {node.op}')
@@ -1028,7 +1055,15 @@ class TracedForwardLaplacian(ForwardLaplacianFn):
                 return v
             # only what the product rules read (weights): they take device tensors as they are, and every other
             # rule keeps seeing host arrays, whatever the size of its constants
-            hit = self.constants[key] = {n: (_tree(v, place) if n.users and all(u.target in _WEIGHT_READERS for u in n.users) else v)
+            def read_by(n, readers):
+                return n.users and all(u.target in readers for u in n.users)
+
+            def small(v):
+                if isinstance(v, np.ndarray) and v.dtype == np.float32 and v.ndim >= 1 and device.type != 'cpu':
+                    return torch.as_tensor(np.ascontiguousarray(v)).to(device)
+                return v
+            hit = self.constants[key] = {n: (_tree(v, place) if read_by(n, _WEIGHT_READERS) else
+                                             small(v) if read_by(n, _OPERAND_READERS) else v)
                                          for n, v in self.constants[shapes].items()}
         return hit
 

@@ -9,6 +9,7 @@ lines it follows.  Nothing here touches the GPU.
 
 from __future__ import annotations
 
+import math
 from typing import Sequence
 
 import numpy as np
@@ -123,7 +124,7 @@ def init_mask(shape, offset: int = 0) -> np.ndarray:
 
 @_memo
 def _init_mask(shape, offset):
-    n = int(np.prod(shape, dtype=int))
+    n = int(math.prod(shape))
     return (np.arange(n, dtype=np.int32) + np.int32(offset)).reshape(1, *shape)
 
 
@@ -212,7 +213,7 @@ def gather_table(idx: np.ndarray, n_out: int):
     """
     k = idx.shape[0]
     s = idx.shape[1:]
-    S = int(np.prod(s, dtype=int))
+    S = int(math.prod(s))
     flat = idx.reshape(k, S).T  # (S, k)
     if k == 0 or S == 0:
         return np.full((n_out, 1, *s), -1, dtype=np.int32)
@@ -381,7 +382,7 @@ def slogdet_entry_mask(x0_idx, k: int, x_shape, transposed: bool):
             return None
         idx = idx.swapaxes(-1, -2)
         shape = shape[:-2] + (shape[-1], shape[-2])
-    if k * int(np.prod(shape, dtype=np.int64)) > SLOGDET_MAX_MASK_ENTRIES:
+    if k * int(math.prod(shape)) > SLOGDET_MAX_MASK_ENTRIES:
         return None
     n, m = shape[-2:]
     full = np.broadcast_to(idx, (k, *shape)).reshape(k, -1, n, m)
@@ -501,7 +502,7 @@ def index_positions(shape, idx) -> np.ndarray:
             new_idx.append(np.where((arr < 0) | (arr >= size), size, arr))
             padded_axes.append(axis)
             axis += 1
-    pos = np.arange(int(np.prod(shape, dtype=np.int64)), dtype=INT).reshape(shape)
+    pos = np.arange(int(math.prod(shape)), dtype=INT).reshape(shape)
     for ax in padded_axes:
         pad = [(0, 0)] * len(shape)
         pad[ax] = (0, 1)
@@ -534,7 +535,7 @@ def scatter_out_mask(op_mask, upd_mask, tpos: np.ndarray, op_shape, is_set: bool
     union of the operand's dependencies (none where a 'set' overwrites the position) and of
     those of the update elements landing there, ``-1`` padded at the end; at least one row."""
     op_shape = tuple(int(d) for d in op_shape)
-    op_size = int(np.prod(op_shape, dtype=np.int64))
+    op_size = int(math.prod(op_shape))
     tflat = np.asarray(tpos).reshape(-1)
     pos_parts, dep_parts = [], []
     if upd_mask is not None:

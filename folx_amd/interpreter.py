@@ -9,6 +9,7 @@ gets from an outer ``jax.vmap``, is built into the data layout and switched on w
 
 from __future__ import annotations
 
+import math
 import numpy as np
 import torch
 
@@ -37,7 +38,7 @@ def init_forward_laplacian_state(x: torch.Tensor, sparsity: bool, weights=None, 
     coordinates are ``offset .. offset + n`` of ``total``."""
     B = x.shape[0]
     shape = tuple(x.shape[1:])
-    n = int(np.prod(shape, dtype=int))
+    n = int(math.prod(shape))
     total = n if total is None else int(total)
     dev = x.device
     w = np.ones(shape, dtype=np.float32) if weights is None else np.broadcast_to(
@@ -86,12 +87,12 @@ class ForwardLaplacianFn:
         size = 0
         for a in args:
             if isinstance(a, (FwdLaplArray, BatchedArray)):
-                size += int(np.prod(a.shape, dtype=int))
+                size += int(math.prod(a.shape))
             elif isinstance(a, (torch.Tensor, np.ndarray)):
-                size += int(np.prod(a.shape[1:], dtype=int))
+                size += int(math.prod(a.shape[1:]))
         thr = self._threshold(size)
         # several array arguments are differentiated together: one index space, numbered in argument order
-        sizes = [int(np.prod(a.shape[1:], dtype=int)) if isinstance(a, (torch.Tensor, np.ndarray)) else 0 for a in args]
+        sizes = [int(math.prod(a.shape[1:])) if isinstance(a, (torch.Tensor, np.ndarray)) else 0 for a in args]
         total, offset = int(np.sum(sizes)), 0
         if isinstance(weights, (tuple, list)):
             assert len(weights) == len(args), 'weights: one entry per argument'

@@ -25,8 +25,8 @@ def _stream():
     caller may have switched streams.  The raw getter costs a tenth of ``torch.cuda.current_stream()``,
     which matters for workloads of many short launches."""
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return _raw_stream(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 class LaunchTimer:
@@ -138,9 +138,8 @@ def get_gemm_mode() -> str:
 
 
 def _p(t):
-    if t is None:
-        return None
-    return ctypes.c_void_p(t.data_ptr())
+    """A tensor's address for a ``c_void_p`` argument (ctypes takes the number as it is)."""
+    return None if t is None else t.data_ptr()
 
 
 def _chk(*ts):
@@ -179,8 +178,8 @@ def dense(x, jac, lap, W, bias=None, res=None, row_slice=None):
         lead = (*lead[:-1], hi - lo)
         group, gstride = hi - lo, n
         off = lo * K * 4  # bytes from the first row of a group of n to row lo
-        xp, jp, lp = (ctypes.c_void_p(t.data_ptr() + off) for t in (x, jac, lap))
-    R = int(np.prod(lead, dtype=np.int64))
+        xp, jp, lp = (t.data_ptr() + off for t in (x, jac, lap))
+    R = int(math.prod(lead))
     y = torch.empty((*lead, N), device=x.device, dtype=torch.float32)
     yj = torch.empty((P, *lead, N), device=x.device, dtype=torch.float32)
     yl = torch.empty_like(y)
@@ -227,7 +226,7 @@ def dense_act(name, x, jac, lap, W, bias=None, param=0.0, res=None):
     K, N = W.shape
     P = jac.shape[0]
     lead = tuple(x.shape[:-1])
-    R = int(np.prod(lead, dtype=np.int64))
+    R = int(math.prod(lead))
     lib = _lib.load()
     nbytes = int(lib.folx_hip_dense_act_workspace_bytes(R, P, K, N))
     if nbytes < 0:
@@ -277,7 +276,7 @@ def dense_chain(layers, x, jac, lap, keep_hidden=False):
     _chk(x, jac, lap, *[t for _, W, b, _ in layers for t in (W, b)])
     P = jac.shape[0]
     lead = tuple(x.shape[:-1])
-    R = int(np.prod(lead, dtype=np.int64))
+    R = int(math.prod(lead))
     assert x.shape[-1] == widths[0] and all(W.shape[0] == k for (_, W, _, _), k in zip(layers, widths))
 
     def triplet(N):
@@ -314,7 +313,7 @@ def dense_act_parts(name, x, lap, jac_parts, widths, broadcast, group, W, bias=N
     assert sum(widths) == K and x.shape[-1] == K
     P = jac_parts[0].shape[0]
     lead = tuple(x.shape[:-1])
-    R = int(np.prod(lead, dtype=np.int64))
+    R = int(math.prod(lead))
     n = len(jac_parts)
     for J, w, bc in zip(jac_parts, widths, broadcast):
         assert J.is_contiguous() and J.shape[0] == P and J.numel() == P * (R // group if bc else R) * w
@@ -364,7 +363,7 @@ def norm_dense(name, x, jac, lap, gamma, beta, eps, W, bias=None, param=0.0):
     K, N = W.shape
     P = jac.shape[0]
     lead = tuple(x.shape[:-1])
-    R = int(np.prod(lead, dtype=np.int64))
+    R = int(math.prod(lead))
     act = -1 if name is None else ACT[name]
     lib = _lib.load()
     nbytes = int(lib.folx_hip_norm_dense_workspace_bytes(R, P, K, N, act))
@@ -512,7 +511,7 @@ def slogdet_any(A, AJ, AL):
     lap = tr(A^-1 lap_A) - sum_c tr(M_c M_c) with M_c = A^-1 dA_c from the batched product kernel."""
     _chk(A, AJ, AL)
     n, P, lead = A.shape[-1], AJ.shape[0], tuple(A.shape[:-2])
-    NM = int(np.prod(lead, dtype=np.int64))
+    NM = int(math.prod(lead))
     _, sign, ld, Mt, Lt = _inverse_times_rows(A.contiguous().reshape(NM, n, n), AJ.contiguous().reshape(P, NM, n, n),
                                               AL.contiguous().reshape(NM, n, n))
     trl, _ = trace_pair(Lt)
@@ -529,7 +528,7 @@ def inv_any(A, AJ, AL):
     C_jac[c] = -M_c C, C_lap = (2 sum_c M_c M_c - C lap_A) C with M_c = C dA_c.  Same shapes as ``inv``."""
     _chk(A, AJ, AL)
     n, P, lead = A.shape[-1], AJ.shape[0], tuple(A.shape[:-2])
-    NM = int(np.prod(lead, dtype=np.int64))
+    NM = int(math.prod(lead))
     C, _, _, Mt, Lt = _inverse_times_rows(A.contiguous().reshape(NM, n, n), AJ.contiguous().reshape(P, NM, n, n),
                                           AL.contiguous().reshape(NM, n, n))
     four = lambda v: v.unsqueeze(-3)                     # (.., NM, 1, n, n)
@@ -581,7 +580,7 @@ def exp_envelope(d, dj, dl, sigma, pi):
     assert d.shape[-1] == nI and tuple(pi.shape) == (nI, O)
     P = dj.shape[0]
     lead = tuple(d.shape[:-1])
-    R = int(np.prod(lead, dtype=np.int64))
+    R = int(math.prod(lead))
     y = torch.empty((*lead, O), device=d.device, dtype=torch.float32)
     yj = torch.empty((P, *lead, O), device=d.device, dtype=torch.float32)
     yl = torch.empty_like(y)
@@ -659,7 +658,10 @@ def binary(op, a, aj, al, b, bj, bl):
     if tuple(bj.shape[1:]) != tuple(b.shape):
         assert tuple(bj.shape[1:]) == tuple(out_shape), (bj.shape, b.shape, out_shape)
         b, bl = b.expand(out_shape).contiguous(), bl.expand(out_shape).contiguous()
-    col = collapse3(out_shape, bstrides(a.shape, out_shape), bstrides(b.shape, out_shape))
+    if a.shape == b.shape:
+        col = (1, 1, a.numel()), ((0, 0, 1), (0, 0, 1))
+    else:
+        col = collapse3(out_shape, bstrides(a.shape, out_shape), bstrides(b.shape, out_shape))
     if col is None:
         a, aj, al = (t.expand(*t.shape[: t.dim() - a.dim()], *out_shape).contiguous() for t in (a, aj, al))
         b, bj, bl = (t.expand(*t.shape[: t.dim() - b.dim()], *out_shape).contiguous() for t in (b, bj, bl))
@@ -704,6 +706,8 @@ def mul_sparse(a, aj, al, b, bj, bl, index):
 def _affine_space(row_shape, out_shape, c, d):
     """The index space of ``alpha * in * c + beta * d`` over ``out_shape``: (c, d, dims), with c and d spelled out over more
     axes where three index dimensions do not cover their broadcasts, or None if the input's do not fit."""
+    if tuple(row_shape) == tuple(out_shape) and (c is None or c.numel() == 1) and (d is None or d.numel() == 1):
+        return c, d, (1, 1, math.prod(out_shape), 0, 0, 1, 0, 0, 0, 0, 0, 0)
     sin = bstrides(row_shape, out_shape)
 
     def space(c, d):
@@ -754,8 +758,8 @@ def rows_affine(inp, rows, row_shape, out_shape, c=None, d=None, alpha=1.0, beta
             'three index dimensions; broadcast it with broadcast_to first')
     c, d, dims = got
     out = torch.empty((rows, *out_shape), device=inp.device, dtype=torch.float32)
-    in_S = int(np.prod(row_shape, dtype=np.int64))
-    with _timed('rows_affine', (rows, int(np.prod(out_shape, dtype=np.int64)))):
+    in_S = int(math.prod(row_shape))
+    with _timed('rows_affine', (rows, int(math.prod(out_shape)))):
         check(
             _lib.load().folx_hip_rows_affine(
                 _stream(), _p(inp), _p(out), rows, in_S, _p(c), _p(d), float(alpha), float(beta), _dims(*dims),
@@ -920,8 +924,8 @@ def slogdet(A, AJ, AL, row_axis=None, factor=None):
     ra = nd - 2 if row_axis is None else row_axis % nd
     assert ra < nd - 1 and A.shape[ra] == n, 'slogdet needs square matrices'
     outer, mid = tuple(A.shape[:ra]), tuple(A.shape[ra + 1:-1])
-    NB = int(np.prod(outer, dtype=np.int64))
-    ND = int(np.prod(mid, dtype=np.int64))
+    NB = int(math.prod(outer))
+    ND = int(math.prod(mid))
     lead = (*outer, *mid)
     sign = torch.empty(lead, device=A.device, dtype=torch.float32)
     ld = torch.empty_like(sign)
@@ -961,7 +965,7 @@ def sparse_slogdet(A, AJ, AL, take, cols, rows, transposed):
     k = AJ.shape[0]
     C, rank, width = take.shape
     lead = A.shape[:-2]
-    NM = int(np.prod(lead, dtype=np.int64)) if len(lead) else 1
+    NM = int(math.prod(lead)) if len(lead) else 1
     sign = torch.empty(lead, device=A.device, dtype=torch.float32)
     ld = torch.empty_like(sign)
     ldj = torch.empty((C, *lead), device=A.device, dtype=torch.float32)
@@ -983,7 +987,7 @@ def inv(A, AJ, AL):
     n = A.shape[-1]
     P = AJ.shape[0]
     lead = A.shape[:-2]
-    NM = int(np.prod(lead, dtype=np.int64)) if len(lead) else 1
+    NM = int(math.prod(lead)) if len(lead) else 1
     C, CJ, CL = torch.empty_like(A), torch.empty_like(AJ), torch.empty_like(AL)
     with _timed('inv_fwdlap', (NM, n, P)):
         check(_lib.load().folx_hip_inv_fwdlap(_stream(), _p(A), _p(AJ), _p(AL), _p(C), _p(CJ), _p(CL), NM, n, P),
@@ -998,7 +1002,7 @@ def solve(A, AJ, AL, b, bJ, bL, P):
     n, m = b.shape[-2:]
     lead = A.shape[:-2]
     assert tuple(b.shape[:-2]) == tuple(lead) and A.shape[-1] == n and A.shape[-2] == n
-    NM = int(np.prod(lead, dtype=np.int64)) if len(lead) else 1
+    NM = int(math.prod(lead)) if len(lead) else 1
     y = torch.empty_like(b)
     yJ = torch.empty((P, *b.shape), device=b.device, dtype=torch.float32)
     yL = torch.empty_like(b)

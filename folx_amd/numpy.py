@@ -10,12 +10,15 @@ sparsity_threshold)``.  Shapes and axes are per walker, as inside ``jax.vmap``.
 from __future__ import annotations
 
 import contextlib
+import math
 import threading
 
 import numpy as np
 
 from .api import BatchedArray, FwdLaplArray
-from .wrapped_functions import get_laplacian, register_function
+from .kernels import FUSED_ACTS
+from .wrapped_functions import (Deferred, LazyBroadcast, LazyConcat, LazyDot, LazyLayerNorm, LazyMul, LazySlice, LazyTranspose,
+                                force, get_laplacian, register_function)
 
 _state = threading.local()
 
@@ -38,8 +41,6 @@ def _call(name, args, kwargs=None):
     """Look the rule up and call it.  Deferred values among the arguments are evaluated first
     (also one level inside tuples and among the keyword values): only the functions below that
     know how to absorb one hand it on, through ``_call_keep``."""
-    from .wrapped_functions import force
-
     kwargs = {k: force(v) for k, v in (kwargs or {}).items()}
     return get_laplacian(name, wrap_if_missing=True)(tuple(force(a) for a in args), kwargs, current_threshold())
 
@@ -57,8 +58,6 @@ def _call_keep(name, args, kwargs=None):
 
 
 def _is_triplet(a):
-    from .wrapped_functions import Deferred
-
     return isinstance(a, (FwdLaplArray, Deferred))
 
 
@@ -71,9 +70,6 @@ def _shape(a):
 # elementwise -------------------------------------------------------------------------------
 def _u(name):
     def fn(a):
-        from .kernels import FUSED_ACTS
-        from .wrapped_functions import LazyDot
-
         if isinstance(a, LazyDot) and name in FUSED_ACTS and a.kwargs.get('act') is None:
             return a.with_(act=name)  # Dense + activation: one rule where the kernels take the shape
         return _call(name, (a,))
@@ -111,8 +107,6 @@ def power(a, c):
 
 
 def add(a, b):
-    from .wrapped_functions import LazyDot, force
-
     for d, o in ((b, a), (a, b)):
         if not isinstance(d, LazyDot) or d._value is not None:  # an evaluated product is an ordinary triplet
             continue
@@ -132,8 +126,6 @@ def subtract(a, b):
 
 
 def multiply(a, b):
-    from .wrapped_functions import LazyMul, force
-
     if _is_triplet(a) and _is_triplet(b) and tuple(a.shape) == tuple(b.shape) and len(a.shape) >= 2:
         return LazyMul(force(a), force(b), current_threshold())  # slogdet can take the factor on load
     return _call('mul', (a, b))
@@ -156,8 +148,6 @@ def dot(h, W, b=None, residual=None, row_slice=None, act=None, norm=None):
     ``residual`` a triplet of the output shape, ``row_slice = (lo, hi)`` for
     ``h[..., lo:hi, :] @ W``, ``act`` a scalar function applied to ``h @ W + b`` (the residual is
     added to the activated result), ``norm = (gamma, beta, eps)`` a LayerNorm of ``h``."""
-    from .wrapped_functions import LazyConcat, LazyDot, LazyLayerNorm, LazySlice, force
-
     if isinstance(h, LazyLayerNorm):
         assert norm is None, 'dot: the operand already is a layer_norm'
         h, norm = h.h, h
@@ -182,8 +172,6 @@ def layer_norm(h, gamma=None, beta=None, eps=1e-5, lazy=True):
     """LayerNorm over the last axis (one fused rule; same result as the primitive chain).  The
     result is deferred: products that can take LayerNorm into their own rule never evaluate it,
     all other consumers share one evaluation."""
-    from .wrapped_functions import LazyLayerNorm, force
-
     del lazy
     h = force(h)
     if isinstance(h, FwdLaplArray):
@@ -234,7 +222,7 @@ def dot_general(lhs, rhs, dimension_numbers):
         f'dot_general: {sl} and {sr} do not match under {dimension_numbers}'
     lf = [i for i in range(len(sl)) if i not in lc and i not in lb]
     rf = [i for i in range(len(sr)) if i not in rc and i not in rb]
-    size = lambda shp, idx: int(np.prod([shp[i] for i in idx], dtype=np.int64))
+    size = lambda shp, idx: int(math.prod([shp[i] for i in idx]))
     bshape = [sl[i] for i in lb]
     lshape, rshape = [sl[i] for i in lf], [sr[i] for i in rf]
     Bt, I, J, Kc = size(sl, lb), size(sl, lf), size(sr, rf), size(sl, lc)
@@ -389,8 +377,6 @@ def slogdet(A, row_axis=None, factor=None):
     in place.  ``factor`` (same shape as ``A``): the matrices are ``A * factor``; orbitals times
     envelopes are then multiplied while the matrices are loaded.  Same result as
     ``slogdet(multiply(A, factor))``."""
-    from .wrapped_functions import LazyMul, LazyTranspose
-
     if isinstance(A, LazyTranspose) and row_axis is None and factor is None:
         A, row_axis = A.a, A.row_axis       # matrix rows on another axis: read in place
     if isinstance(A, LazyMul) and factor is None:
@@ -453,8 +439,6 @@ def sum(a, axis=None, keepdims=False, window=None, scale=None):
     """``window = (lo, hi)`` with a single ``axis``: the sum of ``a[..., lo:hi, ...]`` along that
     axis, without forming the slice (what ``sum(a[..., lo:hi, ...], axis)`` becomes by itself).
     ``scale``: a constant factor applied in the same rule (the ``1 / n`` of ``mean``)."""
-    from .wrapped_functions import LazySlice
-
     if isinstance(a, LazySlice) and window is None and _axes(axis, a.ndim) == (a.axis,):
         a, window = a.a, (a.lo, a.hi)       # the sum of a slice along the reduced axis: read in place
     shape = _shape(a)
@@ -476,7 +460,7 @@ def sum(a, axis=None, keepdims=False, window=None, scale=None):
 def mean(a, axis=None, keepdims=False, window=None):
     shape = _shape(a)
     axes = _axes(axis, len(shape))
-    n = int(np.prod([shape[i] for i in axes], dtype=int)) if window is None else int(window[1] - window[0])
+    n = int(math.prod([shape[i] for i in axes])) if window is None else int(window[1] - window[0])
     return sum(a, axis, keepdims, window, scale=1.0 / n)
 
 
@@ -507,11 +491,9 @@ def logsumexp(a, axis=-1, b=None):
 def reshape(a, shape):
     shape = tuple(int(s) for s in shape)
     if -1 in shape:
-        tot = int(np.prod(_shape(a), dtype=int))
-        rest = -int(np.prod(shape, dtype=int))
+        tot = int(math.prod(_shape(a)))
+        rest = -int(math.prod(shape))
         shape = tuple(tot // rest if s == -1 else s for s in shape)
-    from .wrapped_functions import LazyDot
-
     if (isinstance(a, LazyDot) and a._value is None and len(shape) >= 1 and shape[-1] == a.shape[-1]
             and isinstance(a.h, (FwdLaplArray, LazyDot)) and a.kwargs.get('row_slice') is None and a.kwargs.get('norm') is None):
         # only the leading axes change: the same product on the input with those leading axes, its epilogue
@@ -522,8 +504,6 @@ def reshape(a, shape):
 
 
 def transpose(a, axes=None):
-    from .wrapped_functions import LazyMul, LazyTranspose
-
     nd = len(_shape(a))
     axes = tuple(range(nd))[::-1] if axes is None else tuple(ax % nd for ax in axes)
     if nd >= 3 and isinstance(a, (FwdLaplArray, LazyMul)) and axes[-1] == nd - 1 and axes[-2] != nd - 2 \
@@ -557,8 +537,6 @@ def squeeze(a, axis):
 def broadcast_to(a, shape, lazy=True):
     """A vector broadcast along new leading axes is deferred: a concatenation that a product
     reads in parts takes it as it is, everything else evaluates it."""
-    from .wrapped_functions import LazyBroadcast, force
-
     del lazy
     shape = tuple(int(n) for n in shape)
     a = force(a)
@@ -570,8 +548,6 @@ def broadcast_to(a, shape, lazy=True):
 
 
 def getitem(a, idx):
-    from .wrapped_functions import LazySlice, force
-
     a = force(a)
     if isinstance(a, FwdLaplArray):
         # a contiguous window along ONE axis, everything else taken whole: deferred, so that the product
@@ -588,8 +564,6 @@ def getitem(a, idx):
 def concatenate(arrs, axis=-1, lazy=True):
     """Along the last axis of triplets the result is deferred: a product that can read its operand
     in parts never forms the concatenation (nor the broadcasts among the parts)."""
-    from .wrapped_functions import LazyBroadcast, LazyConcat, force
-
     del lazy
     arrs = tuple(t if isinstance(t, LazyBroadcast) else force(t) for t in arrs)
     nd = len(_shape(arrs[0]))
@@ -926,7 +900,7 @@ def norm(a, axis=None, keepdims=False):
 
 def vdot(a, b):
     """``jnp.vdot`` on real data: both arguments flattened, one number."""
-    n = int(np.prod(_shape(a), dtype=int))
+    n = int(math.prod(_shape(a)))
     return sum(multiply(reshape(a, (n,)), reshape(b, (n,))))
 
 
@@ -935,7 +909,7 @@ def inner(a, b):
 
 
 def outer(a, b):
-    na, nb = int(np.prod(_shape(a), dtype=int)), int(np.prod(_shape(b), dtype=int))
+    na, nb = int(math.prod(_shape(a))), int(math.prod(_shape(b)))
     return multiply(reshape(a, (na, 1)), reshape(b, (1, nb)))
 
 
@@ -965,7 +939,7 @@ def take(a, indices, axis=None):
     """``jnp.take`` with static integer indices (out-of-range entries are an error, as under ``mode='raise'``)."""
     idx = np.asarray(indices)
     if axis is None:
-        return getitem(reshape(a, (int(np.prod(_shape(a), dtype=int)),)), idx)
+        return getitem(reshape(a, (int(math.prod(_shape(a))),)), idx)
     axis = axis % len(_shape(a))
     return getitem(a, (*([slice(None)] * axis), idx))
 
@@ -1063,8 +1037,6 @@ def convert_element_type(a, new_dtype):              # jax.lax.convert_element_t
 
 def allclose(a, b, rtol=1e-5, atol=1e-8):
     """``numpy.allclose`` on values (triplets contribute their ``x``)."""
-    from .wrapped_functions import force
-
     val = lambda v: force(v).x.detach().cpu().numpy() if _is_triplet(v) else (  # noqa: E731
         v.data.detach().cpu().numpy() if isinstance(v, BatchedArray) else np.asarray(v))
     return bool(np.allclose(val(a), val(b), rtol=rtol, atol=atol))

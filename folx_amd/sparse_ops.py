@@ -7,6 +7,7 @@ model that is evaluated repeatedly (or replayed from a HIP graph) never re-uploa
 from __future__ import annotations
 
 import hashlib
+import math
 
 import numpy as np
 import torch
@@ -100,6 +101,16 @@ def device_const(arr, device) -> torch.Tensor:
     return t
 
 
+def scalar_const(value: float, device) -> torch.Tensor:
+    """One float32 number on the device, cached by its value."""
+    key = ('scalar', float(value), math.copysign(1.0, value), str(device))   # 0.0 and -0.0 are one dictionary key
+    t = _CONST_CACHE.get(key)
+    if t is None:
+        t = torch.as_tensor(np.full((1,), value, dtype=np.float32)).to(device)
+        _CONST_CACHE[key] = t
+    return t
+
+
 def cached_tensors() -> list:
     """Every device tensor the caches hold right now (what a captured graph must keep alive)."""
     out = []
@@ -139,8 +150,8 @@ def materialize(data: torch.Tensor, idx: np.ndarray, n_out: int) -> torch.Tensor
     n_inner = ia.split_inner(idx)
     n_outer_axes = len(s) - n_inner
     s_outer, s_inner = s[:n_outer_axes], s[n_outer_axes:]
-    S_outer = int(np.prod(s_outer, dtype=np.int64))
-    S_inner = int(np.prod(s_inner, dtype=np.int64))
+    S_outer = int(math.prod(s_outer))
+    S_inner = int(math.prod(s_inner))
     idx_c = idx[(slice(None), *([slice(None)] * n_outer_axes), *([0] * n_inner))]
     data = data.contiguous().reshape(k, B, S_outer * S_inner)
     key = _key(idx_c, 'take', n_out)
@@ -186,9 +197,9 @@ def materialize_reduced(data: torch.Tensor, slot: np.ndarray, n_out: int, axis: 
     sp = np.moveaxis(full, axis + 1, 1).reshape(k * RED, *before, *after)
     n_const = min(ia.split_inner(sp), len(after))  # trailing kept axes along which the map is constant
     n_var = len(after) - n_const
-    O = int(np.prod(before, dtype=np.int64))
-    IV = int(np.prod(after[:n_var], dtype=np.int64))
-    IC = int(np.prod(after[n_var:], dtype=np.int64))
+    O = int(math.prod(before))
+    IV = int(math.prod(after[:n_var]))
+    IC = int(math.prod(after[n_var:]))
     idx_c = sp[(slice(None), *([slice(None)] * (len(before) + n_var)), *([0] * n_const))]
     key = _key(np.ascontiguousarray(idx_c), 'take_reduced', n_out)
     cached = _TABLE_CACHE.get((key, str(data.device)))
@@ -243,8 +254,8 @@ def add_sparse_rows_(dense: torch.Tensor, data: torch.Tensor, idx: np.ndarray) -
     idx = np.broadcast_to(idx, (k, *s))
     n_inner = ia.split_inner(idx)
     n_outer_axes = len(s) - n_inner
-    S_outer = int(np.prod(s[:n_outer_axes], dtype=np.int64))
-    S_inner = int(np.prod(s[n_outer_axes:], dtype=np.int64))
+    S_outer = int(math.prod(s[:n_outer_axes]))
+    S_inner = int(math.prod(s[n_outer_axes:]))
     idx_c = idx[(slice(None), *([slice(None)] * n_outer_axes), *([0] * n_inner))]
     assert int(idx_c.max(initial=-1)) < dense.shape[0]
     table = device_table(idx_c.reshape(k, S_outer), data.device)

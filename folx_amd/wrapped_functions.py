@@ -17,6 +17,7 @@ rule raises ``KeyError`` in ``get_laplacian``.
 from __future__ import annotations
 
 import logging
+import math
 import sys
 from typing import Any, Callable
 
@@ -236,7 +237,7 @@ def _affine_const(t: FwdLaplArray, c, *, mul: bool, alpha: float, beta: float) -
             d_t, b_x = None, 0.0
         else:
             a_x = a_j = alpha
-            d_t = so.device_const(np.full((1,) * (nd + 1), cval, dtype=np.float32), dev)
+            d_t = so.scalar_const(cval, dev).reshape((1,) * (nd + 1))
             b_x = beta
     else:
         ct = _const_tensor(c, nd, dev)
@@ -706,8 +707,8 @@ def _dot_two_operands(lhs: FwdLaplArray, rhs: FwdLaplArray, thr: int) -> FwdLapl
     same_batch = la[:-2] == rb[:-2]
     use_mul_sum = not same_batch or la[-1] > K.DOT_TWO_KMAX
     if same_batch and lhs.jacobian.weak and rhs.jacobian.weak:
-        inter = int(np.prod((*la, rb[-1]), dtype=np.int64))
-        in_size = max(int(np.prod(la, dtype=np.int64)), int(np.prod(rb, dtype=np.int64)))
+        inter = int(math.prod((*la, rb[-1])))
+        in_size = max(int(math.prod(la)), int(math.prod(rb)))
         k_mul = lhs.jacobian.data.shape[0] + rhs.jacobian.data.shape[0]
         n_dense = max(lhs.jacobian.max_n, rhs.jacobian.max_n) + 1
         use_mul_sum = use_mul_sum or inter == in_size or k_mul * inter < n_dense * in_size
@@ -717,7 +718,7 @@ def _dot_two_operands(lhs: FwdLaplArray, rhs: FwdLaplArray, thr: int) -> FwdLapl
     P = max(Ja.shape[0], Jb.shape[0])
     Ja, Jb = so.pad_rows(Ja, P), so.pad_rows(Jb, P)
     B = lhs.B
-    NB0 = B * int(np.prod(la[:-2], dtype=np.int64))
+    NB0 = B * int(math.prod(la[:-2]))
     va = lambda t, lead: t.reshape(*lead, NB0, 1, la[-2], la[-1])
     vb = lambda t, lead: t.reshape(*lead, NB0, 1, rb[-2], rb[-1])
     y, Jy, lapy = K.dot_two(va(lhs.x.contiguous(), ()), va(Ja.contiguous(), (P,)), va(lhs.laplacian.contiguous(), ()),
@@ -730,8 +731,6 @@ def _dot_two_operands(lhs: FwdLaplArray, rhs: FwdLaplArray, thr: int) -> FwdLapl
 def _dot_mul_sum(lhs: FwdLaplArray, rhs: FwdLaplArray, a_vec: bool, b_vec: bool) -> FwdLaplArray:
     """Both operands are rearranged so that the contracted axis is last and broadcast against
     each other, then multiplied and summed (folx/wrapped_functions.py:47-68, :263-286)."""
-    from . import numpy as fnp
-
     a, b = lhs, rhs
     if a_vec:
         a = fnp.expand_dims(a, 0)
@@ -772,8 +771,6 @@ class Deferred:
 
     def value(self, sparsity_threshold=None) -> FwdLaplArray:
         if self._value is None:
-            from . import numpy as fnp
-
             with fnp.sparsity_threshold(self.thr if sparsity_threshold is None else sparsity_threshold):
                 self._value = self._evaluate()
         return self._value
@@ -785,7 +782,7 @@ class Deferred:
 
     @property
     def size(self):
-        return int(np.prod(self.shape, dtype=int))
+        return int(math.prod(self.shape))
 
     x = property(lambda self: self.value().x)
     jacobian = property(lambda self: self.value().jacobian)
@@ -917,8 +914,6 @@ class LazyDot(Deferred):
 
     def value_with_residual(self, residual):
         """``residual + (this product)`` as one rule; the handle itself stays unevaluated."""
-        from . import numpy as fnp
-
         with fnp.sparsity_threshold(self.thr):
             return self._evaluate(residual)
 
@@ -967,8 +962,6 @@ def _evaluate_chain(last, residual):
     h = force(cur.h) if isinstance(cur.h, Deferred) and not isinstance(cur.h, LazyConcat) else cur.h
     nodes.reverse()
     fit = len(nodes) if ends_in_vector or (residual is None and _chain_layer(last)) else len(nodes) - 1
-    from . import numpy as fnp
-
     i = 0
     while i < len(nodes):
         if i == 0 and fit > 1 and _is(h):
@@ -1082,7 +1075,7 @@ def _dot_parts(lc: LazyConcat, W, kwargs, thr: int):
     if ok:
         first = lc.parts[0].a if isinstance(lc.parts[0], LazyBroadcast) else lc.parts[0]
         B, dev = first.B, first.x.device
-        group = int(np.prod(lead, dtype=np.int64))
+        group = int(math.prod(lead))
         Ktot = sum((t.a if isinstance(t, LazyBroadcast) else t).shape[-1] for t in lc.parts)
         srcs = [t.a if isinstance(t, LazyBroadcast) else t for t in lc.parts]
         own = sum(t.shape[-1] for t in lc.parts if not isinstance(t, LazyBroadcast))  # features met once per position
@@ -1162,8 +1155,6 @@ def layer_norm_rule(args, kwargs, sparsity_threshold):
         first = np.take(mask, [0], axis=-1)
         fusable = bool((mask == first).all()) and not ia.has_duplicates(mask)
     if not fusable:
-        from . import numpy as fnp
-
         mu = fnp.mean(h, axis=-1, keepdims=True)
         c = fnp.subtract(h, mu)
         var = fnp.mean(fnp.square(c), axis=-1, keepdims=True)
@@ -1192,8 +1183,6 @@ def exp_envelope_rule(args, kwargs, sparsity_threshold):
         first = np.take(mask, [0], axis=-1)
         fusable = bool((mask == first).all()) and not ia.has_duplicates(mask)
     if not fusable:
-        from . import numpy as fnp
-
         e = fnp.exp(fnp.negative(fnp.multiply(fnp.expand_dims(d, -1), sigma)))
         return fnp.sum(fnp.multiply(e, pi), axis=-2)
     dev = d.x.device
@@ -1226,9 +1215,9 @@ def _reduce_tensor(t: torch.Tensor, lead: int, axes, alpha=1.0, window=None) -> 
     assert window is None or len(axes) == 1
     for ax in sorted(axes, reverse=True):
         full_ax = ax + lead
-        outer = int(np.prod(shape[:full_ax], dtype=np.int64))
+        outer = int(math.prod(shape[:full_ax]))
         red = shape[full_ax]
-        inner = int(np.prod(shape[full_ax + 1 :], dtype=np.int64))
+        inner = int(math.prod(shape[full_ax + 1 :]))
         t = K.reduce_sum(t.contiguous().reshape(-1), 1, outer, red, inner, alpha, window)
         alpha = 1.0
         del shape[full_ax]
@@ -1315,7 +1304,7 @@ def reduce_sum(args, kwargs, sparsity_threshold):
         nd = a.ndim
         kept = [i for i in range(nd) if i not in axes]
         perm = [0] + [ax + 2 for ax in axes] + [1] + [i + 2 for i in kept]
-        R = int(np.prod([a.shape[ax] for ax in axes], dtype=np.int64))
+        R = int(math.prod([a.shape[ax] for ax in axes]))
         Jp = J.permute(*perm).contiguous().reshape(k * R, a.B, *[a.shape[i] for i in kept])
         sp = np.transpose(slot, [0] + [ax + 1 for ax in axes] + [i + 1 for i in kept])
         sp = sp.reshape(k * R, *[a.shape[i] for i in kept])
@@ -1458,7 +1447,7 @@ def _take_positions(a, idx):
         return np.asarray(a).reshape(-1)[pos]
     B, dev = a.B, a.x.device
     k = a.jacobian.data.shape[0]
-    S = int(np.prod(shape, dtype=np.int64))
+    S = int(math.prod(shape))
     t = so.device_table(pos.reshape(-1, 1), dev)
     x = K.gather_cols(a.x.reshape(B, S), t).reshape(B, *pos.shape)
     J = K.gather_cols(a.jacobian.data.reshape(k * B, S), t).reshape(k, B, *pos.shape)
@@ -1568,8 +1557,8 @@ def _scatter_rule(mode: str) -> ForwardLaplacian:
         op_shape = _logical_shape(operand)
         tpos = ia.index_positions(op_shape, kwargs['idx'])
         upd_shape = tuple(tpos.shape)
-        op_size = int(np.prod(op_shape, dtype=np.int64))
-        upd_size = int(np.prod(upd_shape, dtype=np.int64))
+        op_size = int(math.prod(op_shape))
+        upd_size = int(math.prod(upd_shape))
         if not _is(operand) and not _is(updates):
             raise NotImplementedError('scatter of constants into constants needs no derivative rule')
         like = operand if _is(operand) else updates
@@ -1728,8 +1717,8 @@ def reduce_max_values(args, kwargs, sparsity_threshold):
     t = data
     for ax in sorted(axes, reverse=True):
         f = ax + 1
-        outer = int(np.prod(shape[:f], dtype=np.int64))
-        inner = int(np.prod(shape[f + 1 :], dtype=np.int64))
+        outer = int(math.prod(shape[:f]))
+        inner = int(math.prod(shape[f + 1 :]))
         t = K.reduce_max(t.contiguous().reshape(-1), outer, shape[f], inner)
         del shape[f]
         t = t.reshape(shape)
@@ -1864,8 +1853,6 @@ def solve_wrapper(args, kwargs, sparsity_threshold):
     if n_ > K.SMALL_MATRIX_MAX or m_ > K.SMALL_MATRIX_MAX:
         # beyond the one-system-per-wavefront kernel: y = A^-1 b through the inverse rule (any size) and the
         # product rules; b of rank 1 is a vector, as numpy.matmul has it
-        from . import numpy as fnp
-
         with fnp.sparsity_threshold(sparsity_threshold):
             if _is(A):
                 Ainv = inv_wrapper((A,), {}, sparsity_threshold)
@@ -1990,8 +1977,6 @@ def mhsa_forward_laplacian(args, kwargs, sparsity_threshold):
         # Masks (reference_mhsa_kernel, folx/experimental/pallas/attention/mhsa.py:79-94): a score whose
         # query or key is padding is replaced by -1e20 in front of the softmax; Jacobian rows of inactive
         # input coordinates are zero (the kernel never forms them, .../forward_laplacian.py:483-485).
-        from . import numpy as fnp
-
         if input_mask is not None:
             im = input_mask.data if isinstance(input_mask, BatchedArray) else input_mask
             im = im.to(dev) if isinstance(im, torch.Tensor) else torch.as_tensor(np.asarray(im)).to(dev)
@@ -2002,7 +1987,7 @@ def mhsa_forward_laplacian(args, kwargs, sparsity_threshold):
                 J = t.jacobian.dense_array
                 assert im.shape[0] >= J.shape[0], 'input_mask must have one entry per Jacobian row'
                 J = so.pad_rows(J, im.shape[0])
-                PB, S = J.shape[0] * B, int(np.prod(t.shape, dtype=np.int64))
+                PB, S = J.shape[0] * B, int(math.prod(t.shape))
                 Jz = K.rows_affine(J.contiguous().reshape(PB, S), 1, (PB, S), (PB, S), im.reshape(PB, 1).contiguous(), None)
                 return FwdLaplArray(t.x, FwdJacobian(Jz.reshape(J.shape), None), t.laplacian)
 
@@ -2115,3 +2100,5 @@ register_function('inv', inv_wrapper)      # string keys, folx/wrapped_functions
 register_function('solve', solve_wrapper)
 register_function('_multi_head_self_attention', mhsa_forward_laplacian)
 register_function('_multi_head_self_edge_attention', mhsea_forward_laplacian)
+
+from . import numpy as fnp  # noqa: E402  (it imports this module; the rules above call it)
