@@ -738,44 +738,55 @@ __global__ __launch_bounds__(256) void dense_wide_finish(float* __restrict__ y, 
   reinterpret_cast<float4*>(y_lap)[i] = zl;
 }
 
-// Wg = diag(gamma) W and per column the pair (w1, c0) = (1^T Wg, bias + beta @ W).  A block
-// takes 64 columns; its 16 wavefronts split the K rows.
-__global__ __launch_bounds__(1024) void norm_fold_kernel(const float* __restrict__ W, const float* __restrict__ bias,
-                                                         const float* __restrict__ gamma,
-                                                         const float* __restrict__ beta, float* __restrict__ Wg,
-                                                         float2* __restrict__ wc, int32_t K, int32_t N) {
-  __shared__ float ps[16][64], pc[16][64];
-  const int c = threadIdx.x % 64, sl = threadIdx.x / 64;
-  const int n = blockIdx.x * 64 + c;
+// Wg = diag(gamma) W and per column the pair (w1, c0) = (1^T Wg, bias + beta @ W).  A block takes 16 columns; its 16 groups of
+// 16 lanes split the K rows, eight of them requested at a time, and the partial sums meet within a wavefront first.
+constexpr int FOLD_COLS = 16;
+
+__device__ __forceinline__ void norm_fold(const float* __restrict__ W, const float* __restrict__ bias,
+                                          const float* __restrict__ gamma, const float* __restrict__ beta,
+                                          float* __restrict__ Wg, float2* __restrict__ wc, int32_t K, int32_t N, int block) {
+  __shared__ float ps[4][FOLD_COLS], pc[4][FOLD_COLS];
+  const int c = threadIdx.x % FOLD_COLS, sl = threadIdx.x / FOLD_COLS;
+  const int n = block * FOLD_COLS + c;
   float s = 0.0f, cc = 0.0f;
   if (n < N) {
-    for (int k = sl; k < K; k += 16) {
-      const float w = W[(int64_t)k * N + n];
-      const float wg = gamma ? gamma[k] * w : w;
-      Wg[(int64_t)k * N + n] = wg;
-      s += wg;
-      if (beta) cc = fmaf(beta[k], w, cc);
+    for (int k0 = sl; k0 < K; k0 += 8 * 16) {
+      float w[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) w[u] = W[(int64_t)min(k0 + 16 * u, K - 1) * N + n];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int k = k0 + 16 * u;
+        if (k < K) {
+          const float wg = gamma ? gamma[k] * w[u] : w[u];
+          Wg[(int64_t)k * N + n] = wg;
+          s += wg;
+          if (beta) cc = fmaf(beta[k], w[u], cc);
+        }
+      }
     }
   }
-  ps[sl][c] = s;
-  pc[sl][c] = cc;
+#pragma unroll
+  for (int off = 32; off >= 16; off /= 2) {
+    s += __shfl_xor(s, off, FOLX_WAVE);
+    cc += __shfl_xor(cc, off, FOLX_WAVE);
+  }
+  if (sl % 4 == 0) { ps[sl / 4][c] = s; pc[sl / 4][c] = cc; }
   __syncthreads();
   if (sl == 0 && n < N) {
-    float ts = 0.0f, tc = bias ? bias[n] : 0.0f;
-    for (int i = 0; i < 16; ++i) { ts += ps[i][c]; tc += pc[i][c]; }
-    wc[n] = make_float2(ts, tc);
+    const float tc = bias ? bias[n] : 0.0f;
+    wc[n] = make_float2((ps[0][c] + ps[1][c]) + (ps[2][c] + ps[3][c]), tc + ((pc[0][c] + pc[1][c]) + (pc[2][c] + pc[3][c])));
   }
 }
 
 // One wavefront per position: xh, rs, LN(x) and the part of LN's lap row that is linear in the
 // input's lap row, gamma rs (lap - mean(lap) - xh mean(xh lap)).  K <= 512: two float4 per lane.
-__global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict__ x, const float* __restrict__ lap,
-                                                        const float* __restrict__ gamma,
-                                                        const float* __restrict__ beta, float* __restrict__ xhat,
-                                                        float* __restrict__ rs, float* __restrict__ nx,
-                                                        float* __restrict__ nlap, int64_t R, int32_t K, float eps) {
+__device__ __forceinline__ void norm_rows(const float* __restrict__ x, const float* __restrict__ lap,
+                                          const float* __restrict__ gamma, const float* __restrict__ beta,
+                                          float* __restrict__ xhat, float* __restrict__ rs, float* __restrict__ nx,
+                                          float* __restrict__ nlap, int64_t R, int32_t K, float eps, int64_t block) {
   const int lane = threadIdx.x % 64;
-  const int64_t pos = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;
+  const int64_t pos = block * 4 + threadIdx.x / 64;
   if (pos >= R) return;
   auto wsum = [](float v) __attribute__((always_inline)) {
 #pragma unroll
@@ -832,6 +843,17 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict_
   }
 }
 
+// Both in one launch, the blocks of the weights first: neither reads what the other writes.  K = N = 256: 16.5 us for the weights
+// (64 columns a block, 16 requests in a row each) and 4.9 us for the rows of 640 positions, each its own launch, became 6 us.
+__global__ __launch_bounds__(256) void norm_prepare_kernel(const float* x, const float* lap, const float* W, const float* bias,
+                                                           const float* gamma, const float* beta, float* xhat, float* rs,
+                                                           float* nx, float* nlap, float* Wg, float2* wc, int64_t R, int32_t K,
+                                                           int32_t N, float eps) {
+  const int fold = (N + FOLD_COLS - 1) / FOLD_COLS;
+  if ((int)blockIdx.x < fold) norm_fold(W, bias, gamma, beta, Wg, wc, K, N, (int)blockIdx.x);
+  else norm_rows(x, lap, gamma, beta, xhat, rs, nx, nlap, R, K, eps, (int64_t)blockIdx.x - fold);
+}
+
 // y[r][c] += pre[r / group][c], y_lap likewise: the per-walker pre-activation term on the x and lap
 // rows (one float4 per thread).
 __global__ __launch_bounds__(256) void wide_add_pre_kernel(float* __restrict__ y, float* __restrict__ y_lap,
@@ -855,7 +877,21 @@ struct WidePlan {
   int64_t row_tiles, pos_tiles, blocks, ws_bytes;
   int64_t o_ss, o_s1, o_sc, o_xhat, o_rs, o_nx, o_nlap, o_wg, o_wc;
   int32_t PG, PT, col_tiles;
+  bool apart;  // LayerNorm as a launch of its own in front of the product
 };
+
+// Small LayerNorm + Dense calls run as the two rules one after the other, the normalised triplet in the workspace: the fused
+// form's launches on the positions (prepare, x / lap product, finish) and its 128 x 256 tiles cost 45 to 100 us whatever the size,
+// where the plain product has 64 x 64 tiles.  us, fused / apart, K = N = 256: P = 30, R = 64 56 / 16, 640 62 / 41, 1920 102 / 98; P = 96,
+// R = 64 56 / 28, 256 62 / 54, 480 97 / 83, 640 98 / 99; 512: P = 32, R = 64 97 / 31, 640 172 / 128, 960 175 / 167, 1920 318 / 322; 192: P = 60,
+// R = 640 78 / 50, 1920 137 / 127.  The two meet at 60 000 rows of 256, 50 000 of 512 and 150 000 of 192 features; the line keeps the
+// workspace within the library's own scratch array, so that every call the entry point without a workspace took it still
+// takes.  With an activation the comparison is with the fused dense + activation rule, which has the same tiles: 59 / 55 at
+// P = 30, R = 64, 100 / 92 at P = 32, R = 64 of 512, even at 8000 rows, and 63 against 60 at P = 96, R = 128.
+bool norm_apart(int64_t R, int32_t P, int32_t K, bool act) {
+  const int64_t rows = (int64_t)(P + 2) * R;
+  return act ? P <= 64 && rows <= 8192 : rows * K <= (int64_t)14 << 20;
+}
 
 // What the forms of a dense + activation layer cost: times in us of a 64 x 64 tile and contracted feature on one CU (140
 // TFLOP/s over the chip; 233 of fp32 products from bf16 pieces), the work around the K loop in features of that cost, the
@@ -941,6 +977,14 @@ bool plan_wide(int64_t R, int32_t P, int32_t K, int32_t N, bool norm, bool act, 
     pl.o_wg = take((int64_t)K * N);
     pl.o_wc = take(2 * (int64_t)N);
   }
+  pl.apart = norm && norm_apart(R, P, K, act);
+  if (pl.apart) {  // the normalised triplet, then what the rule behind it needs
+    int64_t need = (int64_t)(P + 2) * R * K;
+    WidePlan behind;
+    if (act && plan_wide(R, P, K, N, false, true, behind)) need += behind.ws_bytes / 4;
+    pl.apart = need * 4 <= FOLX_HIP_STATIC_SCRATCH_BYTES;
+    if (pl.apart) o = need;
+  }
   pl.ws_bytes = o * 4;
   return true;
 }
@@ -977,6 +1021,16 @@ int run_wide(hipStream_t st, bool norm, int32_t act, float param, const float* x
     return FOLX_HIP_ENOTSUP;
   if (!workspace || workspace_bytes < pl.ws_bytes || !folx_aligned16(workspace)) return FOLX_HIP_EINVAL;
   float* ws = (float*)workspace;
+  if (pl.apart) {
+    const int64_t RK = R * (int64_t)K;
+    float *nx = ws, *nj = nx + RK, *nl = nj + P * RK, *rest = nl + RK;
+    const int rc = folx_hip_layernorm_fwdlap(st, x, jac, lap, gamma, beta, nx, nj, nl, R, K, P, eps);
+    if (rc != FOLX_HIP_OK) return rc;
+    if (!has_act)
+      return folx_hip_dense_fwdlap(st, nx, nj, nl, W, bias, nullptr, nullptr, nullptr, y, y_jac, y_lap, R, P, K, N);
+    return run_wide(st, false, act, param, nx, nj, nl, nullptr, nullptr, 0.0f, W, bias, y, y_jac, y_lap, R, P, K, N, rest,
+                    workspace_bytes - (int64_t)(rest - ws) * 4);
+  }
   WideParams a;
   a.jac = jac; a.W = W; a.z = y; a.y_jac = y_jac; a.res_jac = res_jac;
   a.pre_jac = pre_jac; a.pre_group = pre_group;
@@ -987,13 +1041,12 @@ int run_wide(hipStream_t st, bool norm, int32_t act, float param, const float* x
   const float* in_x = x;
   const float* in_lap = lap;
   if (norm) {
-    norm_fold_kernel<<<dim3((unsigned)((N + 63) / 64)), dim3(1024), 0, st>>>(W, bias, gamma, beta, ws + pl.o_wg,
-                                                                          (float2*)(ws + pl.o_wc), K, N);
-    int rc = folx_launch_status();
-    if (rc != FOLX_HIP_OK) return rc;
-    norm_rows_kernel<<<dim3((unsigned)((R + 3) / 4)), dim3(256), 0, st>>>(
-        x, lap, gamma, beta, ws + pl.o_xhat, ws + pl.o_rs, ws + pl.o_nx, ws + pl.o_nlap, R, K, eps);
-    rc = folx_launch_status();
+    const int64_t blocks = (N + FOLD_COLS - 1) / FOLD_COLS + (R + 3) / 4;
+    if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
+    norm_prepare_kernel<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(
+        x, lap, W, bias, gamma, beta, ws + pl.o_xhat, ws + pl.o_rs, ws + pl.o_nx, ws + pl.o_nlap, ws + pl.o_wg,
+        (float2*)(ws + pl.o_wc), R, K, N, eps);
+    const int rc = folx_launch_status();
     if (rc != FOLX_HIP_OK) return rc;
     a.W = ws + pl.o_wg; a.xhat = ws + pl.o_xhat; a.rs = ws + pl.o_rs; a.wc = (const float2*)(ws + pl.o_wc);
     a.s1 = ws + pl.o_s1; a.sc = ws + pl.o_sc;
