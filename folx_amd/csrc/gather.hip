@@ -5,49 +5,6 @@
 
 namespace {
 
-// out[t][b][so][si] = sum_s data[take[t][s][so]][b][so][si]   (take < 0: no source)
-// Threads run along (so, si) in units of VEC floats so reads and writes are coalesced
-// 128-bit accesses when S_inner allows; the table entries are read once per thread and
-// reused for the WPT walkers the thread loops over (blockIdx.y selects the walker group).
-constexpr int GATHER_WPT = 8;
-
-template <int VEC>
-__global__ __launch_bounds__(256) void gather_rows_kernel(const float* __restrict__ data,
-                                                          const int32_t* __restrict__ take,
-                                                          float* __restrict__ out, int32_t n_slots,
-                                                          int64_t B, int64_t S_outer, int64_t S_inner) {
-  const int64_t S = S_outer * S_inner;
-  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
-  if (e >= S) return;
-  const int64_t so = e / S_inner;
-  const int32_t t = blockIdx.z;
-  int32_t src[8];
-  const int32_t ns = n_slots < 8 ? n_slots : 8;
-  for (int s = 0; s < ns; ++s) src[s] = take[((int64_t)t * n_slots + s) * S_outer + so];
-  const int64_t b0 = (int64_t)blockIdx.y * GATHER_WPT;
-  const int64_t b1 = b0 + GATHER_WPT < B ? b0 + GATHER_WPT : B;
-  for (int64_t b = b0; b < b1; ++b) {
-    float acc[VEC];
-#pragma unroll
-    for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
-    for (int s = 0; s < n_slots; ++s) {
-      const int32_t r = s < 8 ? src[s] : take[((int64_t)t * n_slots + s) * S_outer + so];
-      if (r >= 0) {
-        const float* p = data + ((int64_t)r * B + b) * S + e;
-        if constexpr (VEC == 4) {
-          const float4 v = *reinterpret_cast<const float4*>(p);
-          acc[0] += v.x; acc[1] += v.y; acc[2] += v.z; acc[3] += v.w;
-        } else {
-          acc[0] += *p;
-        }
-      }
-    }
-    float* q = out + ((int64_t)t * B + b) * S + e;
-    if constexpr (VEC == 4) *reinterpret_cast<float4*>(q) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-    else *q = acc[0];
-  }
-}
-
 // The same re-indexing with a SUM OVER AN AXIS of the data folded in: the sources of a target
 // row are (row r, entry j of the reduced axis) pairs, encoded r * RED + j, and the data keeps its
 // own layout [k][B][O][RED][IV][IC] (the reduced axis in the middle, the table constant along
@@ -105,37 +62,86 @@ __global__ __launch_bounds__(256) void gather_reduce_rows_kernel(const float* __
   else *dst = alpha * acc[0];
 }
 
-// Flat form of gather_rows_kernel: a thread owns VEC consecutive floats of the (walker, so, si)
-// space of one output row, so that consecutive workgroups write consecutive memory.
-template <int VEC>
-__global__ __launch_bounds__(256) void gather_rows_flat_kernel(const float* __restrict__ data,
-                                                               const int32_t* __restrict__ take,
-                                                               float* __restrict__ out, int32_t n_slots,
-                                                               int64_t B, int64_t S_outer, int64_t S_inner) {
-  const int64_t S = S_outer * S_inner;
-  const int64_t f = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
+// out[t][b][so][si] = sum_s data[take[t][s][so]][b][so][si]   (take < 0: no source)
+// A thread owns VEC consecutive floats of the (walker, so, si) space, so that consecutive workgroups
+// write consecutive memory whatever the extents are, for ROWS output rows; IDX is the type of that
+// space's indices, 32 bits wherever it fits.
+//
+// Large calls are bound by the stores, small ones by the chain table entry -> load -> store, which each
+// thread walks once (a loop over walkers and slots walked it 8 * n_slots times: 63 rows of 750 x 21
+// values 10.5 -> 4.5 us, 3 rows of 100 slots 189 -> 12 us).  Four rows to a thread from k_out = 4 on: the
+// position is found once for them and four loads are in flight whatever the slots are (one row of odd
+// S_inner spends its time in divisions: 96 rows of 4096 x 32 x 33 in 1113 us, four rows 452, 3.7 TB/s).
+template <int VEC, int ROWS, typename IDX>
+__global__ __launch_bounds__(256) void gather_rows_kernel(const float* __restrict__ data,
+                                                          const int32_t* __restrict__ take,
+                                                          float* __restrict__ out, int32_t k_out, int32_t n_slots,
+                                                          IDX B, IDX S_outer, IDX S_inner) {
+  constexpr int SLOTS = 4 / ROWS;
+  const IDX S = S_outer * S_inner;
+  const IDX f = ((IDX)blockIdx.x * 256 + threadIdx.x) * VEC;
   if (f >= B * S) return;
-  const int64_t b = f / S, e = f - b * S;
-  const int64_t so = e / S_inner;
-  const int32_t t = blockIdx.y;
-  float acc[VEC];
+  const IDX so = f % S / S_inner;
+  const int32_t t0 = blockIdx.y * ROWS;
+  const int64_t row = (int64_t)B * S;
+  float acc[ROWS][VEC];
 #pragma unroll
-  for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
-  for (int s = 0; s < n_slots; ++s) {
-    const int32_t r = take[((int64_t)t * n_slots + s) * S_outer + so];
-    if (r >= 0) {
-      const float* p = data + ((int64_t)r * B + b) * S + e;
-      if constexpr (VEC == 4) {
-        const float4 v = folx_ld_stream4(p);
-        acc[0] += v.x; acc[1] += v.y; acc[2] += v.z; acc[3] += v.w;
-      } else {
-        acc[0] += *p;
+  for (int t = 0; t < ROWS; ++t)
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) acc[t][v] = 0.0f;
+  // Four sources at a time: first their table entries, then their loads, then the sums in slot order
+  // -- one by one, each would wait for a table entry and then for its load.
+  for (int s0 = 0; s0 < n_slots; s0 += SLOTS) {
+    int32_t r[ROWS][SLOTS];
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t)
+#pragma unroll
+      for (int u = 0; u < SLOTS; ++u)
+        r[t][u] = t0 + t < k_out && s0 + u < n_slots
+                      ? take[((int64_t)(t0 + t) * n_slots + s0 + u) * S_outer + so] : -1;
+    float val[ROWS][SLOTS][VEC];
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t)
+#pragma unroll
+      for (int u = 0; u < SLOTS; ++u) {
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) val[t][u][v] = 0.0f;
+        if (r[t][u] >= 0) {
+          const float* p = data + r[t][u] * row + f;
+          if constexpr (VEC == 4) {
+            const float4 v = folx_ld_stream4(p);
+            val[t][u][0] = v.x; val[t][u][1] = v.y; val[t][u][2] = v.z; val[t][u][3] = v.w;
+          } else {
+            val[t][u][0] = *p;
+          }
+        }
       }
-    }
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t)
+#pragma unroll
+      for (int u = 0; u < SLOTS; ++u)
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) acc[t][v] += val[t][u][v];
   }
-  float* q = out + ((int64_t)t * B + b) * S + e;
-  if constexpr (VEC == 4) folx_st_stream4(q, make_float4(acc[0], acc[1], acc[2], acc[3]));
-  else *q = acc[0];
+#pragma unroll
+  for (int t = 0; t < ROWS; ++t) {
+    if (t0 + t >= k_out) return;
+    float* q = out + (t0 + t) * row + f;
+    if constexpr (VEC == 4) folx_st_stream4(q, make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]));
+    else *q = acc[t][0];
+  }
+}
+
+template <int VEC, int ROWS>
+void launch_gather_rows(void* stream, int64_t blocks, const float* data, const int32_t* take, float* out, int32_t k_out,
+                        int32_t n_slots, int64_t B, int64_t S_outer, int64_t S_inner) {
+  const dim3 grid((unsigned)blocks, (unsigned)((k_out + ROWS - 1) / ROWS));
+  if (B * S_outer * S_inner <= 0x7fffffffLL)
+    gather_rows_kernel<VEC, ROWS, uint32_t><<<grid, dim3(256), 0, (hipStream_t)stream>>>(
+        data, take, out, k_out, n_slots, (uint32_t)B, (uint32_t)S_outer, (uint32_t)S_inner);
+  else
+    gather_rows_kernel<VEC, ROWS, int64_t><<<grid, dim3(256), 0, (hipStream_t)stream>>>(
+        data, take, out, k_out, n_slots, B, S_outer, S_inner);
 }
 
 // out[idx[r][so]][b][so][si] += data[r][b][so][si]   (idx < 0: the entry is skipped)
@@ -237,24 +243,14 @@ extern "C" int folx_hip_gather_rows(void* stream, const float* data, const int32
   if (k_out == 0 || B == 0 || S == 0) return FOLX_HIP_OK;
   if (!out || (n_slots > 0 && (!take || (k_in > 0 && !data)))) return FOLX_HIP_EINVAL;
   if (k_out > 65535) return FOLX_HIP_ENOTSUP;
-  const int64_t gy = (B + GATHER_WPT - 1) / GATHER_WPT;
-  if (gy > 65535) return FOLX_HIP_ENOTSUP;
+  if (B > 8 * 65535LL) return FOLX_HIP_ENOTSUP;
   const bool vec = (S_inner % 4 == 0) && folx_aligned16(data) && folx_aligned16(out);
-  const int64_t blocks = vec ? (S / 4 + 255) / 256 : (S + 255) / 256;
+  const int64_t blocks = (B * S + (vec ? 1023 : 255)) / (vec ? 1024 : 256);
   if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
-  if (vec) {  // 128-bit accesses: the flat form streams at 5.9 TB/s where the strided one reaches 5.2-5.4
-    const int64_t fb = (B * S / 4 + 255) / 256;
-    if (fb <= 0x7fffffffLL) {
-      gather_rows_flat_kernel<4><<<dim3((unsigned)fb, (unsigned)k_out), dim3(256), 0, (hipStream_t)stream>>>(
-          data, take, out, n_slots, B, S_outer, S_inner);
-      return folx_launch_status();
-    }
-  }
-  dim3 grid((unsigned)blocks, (unsigned)gy, (unsigned)k_out);
-  if (vec)
-    gather_rows_kernel<4><<<grid, dim3(256), 0, (hipStream_t)stream>>>(data, take, out, n_slots, B, S_outer, S_inner);
-  else
-    gather_rows_kernel<1><<<grid, dim3(256), 0, (hipStream_t)stream>>>(data, take, out, n_slots, B, S_outer, S_inner);
+  const bool rows4 = k_out >= 4;
+  const auto launch = vec ? (rows4 ? launch_gather_rows<4, 4> : launch_gather_rows<4, 1>)
+                          : (rows4 ? launch_gather_rows<1, 4> : launch_gather_rows<1, 1>);
+  launch(stream, blocks, data, take, out, k_out, n_slots, B, S_outer, S_inner);
   return folx_launch_status();
 }
 
