@@ -18,7 +18,7 @@
 // That is O(n^2 d) work per (walker, head) instead of O(P n^2 d); the kernel is bound by
 // writing the dense P x n x d output rows.
 //
-// One workgroup of 512 threads per (walker, head); q, k, v, o, p and the n x n accumulators
+// One workgroup of NT threads (64 to 512) per (walker, head), RL of them along an output row, NP passes of NT / RL rows; q, k, v, o, p and the n x n accumulators
 // live in LDS (rows of d + 4 floats, so that 16 threads reading 16 bytes each from 16
 // different rows cover all banks); the n x n x d products (scores, alpha, beta, the Laplacian's
 // score term) run on the matrix cores from those rows, the sums over j on 128-bit LDS reads; the
@@ -37,9 +37,6 @@ struct SAArgs {
   int32_t n, H, d, K;
 };
 
-constexpr int SA_NT = 512;  // two workgroups per CU (LDS and 128 registers): four wavefronts per SIMD
-constexpr int SA_RP = SA_NT / 16;  // output rows per pass: 16 threads of 16 bytes cover a row of d <= 64
-
 // dot product of two 16-byte aligned LDS vectors of 4 * d4 floats
 __device__ __forceinline__ float sa_dot(const float* u, const float* m, int d4) {
   float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
@@ -51,7 +48,6 @@ __device__ __forceinline__ float sa_dot(const float* u, const float* m, int d4) 
   }
   return (s0 + s1) + (s2 + s3);
 }
-constexpr int SA_MAXPASS = 64 / SA_RP;  // n <= 64: rows i = SA_RP pass + tid / 16
 constexpr int SA_E = 4;        // sequence positions worked on together
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -96,14 +92,14 @@ __device__ __forceinline__ floatx4 sa_tile_nt(const float* X, int ldx, const flo
 // Two products at once, C0 = X0 Y0^T (rows < nr0 of X0, rows < nc0 of Y0) and C1 = X1 Y1^T, their
 // 16 x 16 tiles dealt to the workgroup's wavefronts as one list; `put(which, r, c, value)`
 // receives every element.  (One product: nr1 = 0.)
-template <class Put>
+template <int NT, class Put>
 __device__ __forceinline__ void sa_products_nt(const float* X0, int ldx0, int nr0, const float* Y0, int ldy0, int nc0,
                                                const float* X1, int ldx1, int nr1, const float* Y1, int ldy1, int nc1,
                                                int d4, int tid, Put put) {
   const int lane = tid % 64, wave = tid / 64;
   const int tc0 = (nc0 + 15) / 16, t0 = ((nr0 + 15) / 16) * tc0;
   const int tc1 = (nc1 + 15) / 16, t1 = ((nr1 + 15) / 16) * tc1;
-  for (int t = wave; t < t0 + t1; t += SA_NT / 64) {
+  for (int t = wave; t < t0 + t1; t += NT / 64) {
     const bool second = t >= t0;
     const int tt = second ? t - t0 : t, tc = second ? tc1 : tc0;
     const int r0 = (tt / tc) * 16, c0 = (tt % tc) * 16;
@@ -121,10 +117,10 @@ __device__ __forceinline__ void sa_products_nt(const float* X0, int ldx0, int nr
   }
 }
 
-template <class Put>
+template <int NT, class Put>
 __device__ __forceinline__ void sa_product_nt(const float* X, int ldx, int nr, const float* Y, int ldy, int nc,
                                               int d4, int tid, Put put) {
-  sa_products_nt(X, ldx, nr, Y, ldy, nc, X, ldx, 0, Y, ldy, 0, d4, tid,
+  sa_products_nt<NT>(X, ldx, nr, Y, ldy, nc, X, ldx, 0, Y, ldy, 0, d4, tid,
                  [&](bool, int r, int c, float v) { put(r, c, v); });
 }
 
@@ -134,7 +130,9 @@ __host__ __device__ inline int64_t sa_lds_floats(int n, int d, int K) {
          (int64_t)K * n;
 }
 
-__global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
+template <int NT, int RL, int NP>
+__global__ __launch_bounds__(NT, 4) void mhsa_sparse_kernel(SAArgs a) {
+  constexpr int RP = NT / RL;  // output rows of a pass
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int n = a.n, d = a.d, K = a.K, H = a.H;
   const int dp = d + 4, np1 = n + 1, d4 = d / 4;
@@ -167,7 +165,7 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
   const int64_t Srow = a.B * n * (int64_t)H * d;  // elements per Jacobian row
   auto grow = [&](int i) -> int64_t { return ((b * n + i) * (int64_t)H + h) * d; };
   auto load_tile = [&](const float* src, float* dst) {
-    for (int it = tid; it < n * d4; it += SA_NT) {
+    for (int it = tid; it < n * d4; it += NT) {
       const int i = it / d4, t4 = it - i * d4;
       const float4 t = *reinterpret_cast<const float4*>(src + grow(i) + 4 * t4);
       *reinterpret_cast<float4*>(dst + i * dp + 4 * t4) = t;
@@ -177,12 +175,12 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
   load_tile(a.q, qS);
   load_tile(a.k, kS);
   load_tile(a.v, vS);
-  for (int it = tid; it < 3 * n * np1; it += SA_NT) AA[it] = 0.0f;  // AA, BB, AR are contiguous
-  for (int it = tid; it < K * n; it += SA_NT) idxS[it] = a.index[it];
+  for (int it = tid; it < 3 * n * np1; it += NT) AA[it] = 0.0f;  // AA, BB, AR are contiguous
+  for (int it = tid; it < K * n; it += NT) idxS[it] = a.index[it];
   sa_barrier();
 
   // p = softmax(q k^T)
-  sa_product_nt(qS, dp, n, kS, dp, n, d4, tid, [&](int i, int j, float v) { pS[i * np1 + j] = v; });
+  sa_product_nt<NT>(qS, dp, n, kS, dp, n, d4, tid, [&](int i, int j, float v) { pS[i * np1 + j] = v; });
   sa_barrier();
   if (tid < n) {
     float* row = pS + tid * np1;
@@ -195,7 +193,7 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
   }
   sa_barrier();
   // o = p v
-  for (int it = tid; it < n * d4; it += SA_NT) {
+  for (int it = tid; it < n * d4; it += NT) {
     const int i = it / d4, t4 = it - i * d4;
     // four partial sums (keys j % 4), added pairwise: a quarter as many roundings in a row, which
     // the Jacobian rows feel through v - o
@@ -250,12 +248,12 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
   float4 pf[SA_E];
   fetch(0, pf);
 
-  float4 t2acc[SA_MAXPASS], oreg[SA_MAXPASS];
-  const int orow = tid / 16, ot4 = tid % 16;
+  float4 t2acc[NP], oreg[NP];
+  const int orow = tid / RL, ot4 = tid % RL;
 #pragma unroll
-  for (int ps = 0; ps < SA_MAXPASS; ++ps) {
+  for (int ps = 0; ps < NP; ++ps) {
     t2acc[ps] = make_float4(0.f, 0.f, 0.f, 0.f);
-    const int i = ps * SA_RP + orow;
+    const int i = ps * RP + orow;
     oreg[ps] = (i < n && ot4 < d4) ? *reinterpret_cast<const float4*>(oS + i * dp + 4 * ot4)
                                    : make_float4(0.f, 0.f, 0.f, 0.f);
   }
@@ -273,15 +271,15 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
     if (e0 + SA_E < n) fetch(e0 + SA_E, pf);
 
     // alpha[e][s][j] = a_es . k[j],  beta[e][s][i] = q[i] . b_es,  gp[e][s] = a_es . b_es
-    sa_products_nt(aS, dp, ne * K, kS, dp, n, bS, dp, ne * K, qS, dp, n, d4, tid,
+    sa_products_nt<NT>(aS, dp, ne * K, kS, dp, n, bS, dp, ne * K, qS, dp, n, d4, tid,
                    [&](bool beta, int es, int x, float v) { (beta ? beS : alS)[es * n + x] = v; });
-    if (tid >= SA_NT - ne * K) {  // the last wavefront has no tile when n <= 48
-      const int es = SA_NT - 1 - tid;
+    if (tid >= NT - ne * K) {  // the last wavefront has no tile when n <= 48
+      const int es = NT - 1 - tid;
       gpS[es] = sa_dot(aS + es * dp, bS + es * dp, d4);
     }
     sa_barrier();
     // rho[e][s] = sum_j p[e][j] alpha[e][s][j],  gamma[e][s] = sum_j p[e][j] alpha[e][s][j] (v[j] - o[e])
-    for (int it = tid; it < ne * K * d4; it += SA_NT) {
+    for (int it = tid; it < ne * K * d4; it += NT) {
       const int es = it / d4, t4 = it - es * d4;
       const int e = e0 + es / K;
       float rho = 0.0f;
@@ -306,9 +304,9 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
       for (int ee = 0; ee < ne; ++ee) {
         const int e = e0 + ee;
         const float4 v4 = *reinterpret_cast<const float4*>(vS + e * dp + 4 * ot4);
-        float pie[SA_MAXPASS];
+        float pie[NP];
 #pragma unroll
-        for (int ps = 0; ps < SA_MAXPASS; ++ps) pie[ps] = (ps * SA_RP + orow < n) ? pS[(ps * SA_RP + orow) * np1 + e] : 0.0f;
+        for (int ps = 0; ps < NP; ++ps) pie[ps] = (ps * RP + orow < n) ? pS[(ps * RP + orow) * np1 + e] : 0.0f;
         for (int sl = 0; sl < K; ++sl) {
           const int c = idxS[sl * n + e];
           if (c < 0) continue;
@@ -319,8 +317,8 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
           const float4 g4 = *reinterpret_cast<const float4*>(gamS + es * d + 4 * ot4);
           float* dst = a.oj + (int64_t)c * Srow + 4 * ot4;
 #pragma unroll
-          for (int ps = 0; ps < SA_MAXPASS; ++ps) {
-            const int i = ps * SA_RP + orow;
+          for (int ps = 0; ps < NP; ++ps) {
+            const int i = ps * RP + orow;
             if (i < n) {
               const float bi = beS[es * n + i];
               const float4 oi = oreg[ps];
@@ -343,7 +341,7 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
       }
     }
     // n x n sums over the slots of each position of the group
-    for (int it = tid; it < ne * n; it += SA_NT) {
+    for (int it = tid; it < ne * n; it += NT) {
       const int ee = it / n, j = it - ee * n;
       const int e = e0 + ee;
       const float pee = pS[e * np1 + e];
@@ -360,8 +358,8 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
       AR[e * np1 + j] = ar;
       BB[j * np1 + e] = bb;
     }
-    if (tid >= SA_NT - ne) {
-      const int ee = SA_NT - 1 - tid;
+    if (tid >= NT - ne) {
+      const int ee = NT - 1 - tid;
       const int e = e0 + ee;
       const float pee = pS[e * np1 + e];
       float d1 = 0.0f, d2 = 0.0f, r2 = 0.0f, g = 0.0f;
@@ -386,7 +384,7 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
     R2a[i] = r2;
   }
   sa_barrier();
-  for (int it = tid; it < n * n; it += SA_NT) {
+  for (int it = tid; it < n * n; it += NT) {
     const int i = it / n, j = it - i * n;
     const int x = i * np1 + j;
     float s2 = AA[x] + BB[x], sr = AR[x] + pS[x] * BB[x];
@@ -402,9 +400,9 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
     rsum[i] = s;
   }
   // sL = lap_q k^T (into BB, whose sums of beta^2 are used up)
-  sa_product_nt(oS, dp, n, kS, dp, n, d4, tid, [&](int i, int j, float v) { BB[i * np1 + j] = v; });
+  sa_product_nt<NT>(oS, dp, n, kS, dp, n, d4, tid, [&](int i, int j, float v) { BB[i * np1 + j] = v; });
   sa_barrier();
-  for (int it = tid; it < n * n; it += SA_NT) {
+  for (int it = tid; it < n * n; it += NT) {
     const int i = it / n, j = it - i * n;
     const int x = i * np1 + j;
     const float pij = pS[x];
@@ -412,7 +410,7 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
   }
   load_tile(a.kl, oS);  // lap_q has been consumed; k itself is not needed any more
   sa_barrier();
-  sa_product_nt(qS, dp, n, oS, dp, n, d4, tid, [&](int i, int j, float v) { BB[i * np1 + j] += v; });
+  sa_product_nt<NT>(qS, dp, n, oS, dp, n, d4, tid, [&](int i, int j, float v) { BB[i * np1 + j] += v; });
   sa_barrier();
   if (tid < n) {
     const int i = tid;
@@ -422,7 +420,7 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
   }
   load_tile(a.vl, qS);  // q is not needed any more
   sa_barrier();
-  for (int it = tid; it < n * n; it += SA_NT) {
+  for (int it = tid; it < n * n; it += NT) {
     const int i = it / n, j = it - i * n;
     const int x = i * np1 + j;
     AA[x] += pS[x] * (BB[x] - rsum[i]);  // pL + M
@@ -431,8 +429,8 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
   // lap_o = p lap_v + (pL + M) v + 2 sum_c p'_c[:, e] w_c
   if (ot4 < d4) {
 #pragma unroll
-    for (int ps = 0; ps < SA_MAXPASS; ++ps) {
-      const int i = ps * SA_RP + orow;
+    for (int ps = 0; ps < NP; ++ps) {
+      const int i = ps * RP + orow;
       if (i < n) {
         float r[4] = {2.0f * t2acc[ps].x, 2.0f * t2acc[ps].y, 2.0f * t2acc[ps].z, 2.0f * t2acc[ps].w};
 #pragma unroll 4
@@ -449,6 +447,23 @@ __global__ __launch_bounds__(SA_NT, 4) void mhsa_sparse_kernel(SAArgs a) {
   }
 }
 
+template <int NT, int RL, int NP>
+int launch_sa(hipStream_t st, const SAArgs& a, size_t lds) {
+  if (lds > 64 * 1024) {
+    // raised once per process to the largest size asked for so far (not a stream operation,
+    // and then never issued again inside a stream capture)
+    static std::atomic<size_t> granted{0};
+    if (lds > granted.load()) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(mhsa_sparse_kernel<NT, RL, NP>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+        return FOLX_HIP_ENOTSUP;
+      granted.store(160 * 1024);
+    }
+  }
+  mhsa_sparse_kernel<NT, RL, NP><<<dim3((unsigned)(a.B * a.H)), dim3(NT), lds, st>>>(a);
+  return folx_launch_status();
+}
+
 }  // namespace
 
 extern "C" int folx_hip_mhsa_sparse_fwdlap(void* stream, const float* q, const float* q_jac, const float* q_lap,
@@ -460,28 +475,29 @@ extern "C" int folx_hip_mhsa_sparse_fwdlap(void* stream, const float* q, const f
   if (B == 0) return FOLX_HIP_OK;
   if (!q || !q_jac || !q_lap || !k || !k_jac || !k_lap || !v || !v_jac || !v_lap || !index || !o || !o_jac || !o_lap)
     return FOLX_HIP_EINVAL;
-  if (n > SA_RP * SA_MAXPASS || d > 64 || d % 4 != 0 || k_rows > 8 || 3 * k_rows * (d / 4) > SA_NT)
-    return FOLX_HIP_ENOTSUP;
+  if (n > 64 || d > 64 || d % 4 != 0 || k_rows > 8 || 3 * k_rows * (d / 4) > 512) return FOLX_HIP_ENOTSUP;
   const void* ptrs[] = {q, q_jac, q_lap, k, k_jac, k_lap, v, v_jac, v_lap, o, o_jac, o_lap};
   for (const void* p : ptrs)
     if (!folx_aligned16(p)) return FOLX_HIP_ENOTSUP;
   if (B * H > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
   const size_t lds = (size_t)sa_lds_floats(n, d, k_rows) * sizeof(float);
   if (lds > 160 * 1024) return FOLX_HIP_ENOTSUP;
-  if (lds > 64 * 1024) {
-    // raised once per process to the largest size asked for so far (not a stream operation,
-    // and then never issued again inside a stream capture)
-    static std::atomic<size_t> granted{0};
-    if (lds > granted.load()) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(mhsa_sparse_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
-        return FOLX_HIP_ENOTSUP;
-      granted.store(160 * 1024);
-    }
-  }
   SAArgs a;
   a.q = q; a.qs = q_jac; a.ql = q_lap; a.k = k; a.ks = k_jac; a.kl = k_lap; a.v = v; a.vs = v_jac; a.vl = v_lap;
   a.index = index; a.o = o; a.oj = o_jac; a.ol = o_lap; a.B = B; a.n = n; a.H = H; a.d = d; a.K = k_rows;
-  mhsa_sparse_kernel<<<dim3((unsigned)(B * H)), dim3(SA_NT), lds, (hipStream_t)stream>>>(a);
-  return folx_launch_status();
+  // Threads of a workgroup.  The steps between two barriers have n d / 4, n^2 or a few 16 x 16 tiles of work: 512
+  // threads suit n = 32, d = 64, and for less most of them wait at barriers while only two workgroups fit a CU.  With more
+  // workgroups than those (B H > 512; fewer: 36 us, with 64 threads 39) a workgroup gets what its steps can use.  us with 512 ->
+  // fewer, B H = 2048, K = 3: n = 16, d = 16 152 -> 49 (64; 128 53, 256 86); n = 16, d = 32 155 -> 92 (128; 256 95); n = 16,
+  // d = 64 175 -> 117, n = 13 156 -> 103 (256; 128 cannot fetch 3 K d / 4 vectors); n = 24, d = 32 236 -> 156, n = 32, d = 16
+  // 310 -> 185 (256; 128 181, 212); n = 32, d = 64 447 and 443.
+  const int nvec = 3 * k_rows * (d / 4);
+  const hipStream_t st = (hipStream_t)stream;
+  if (B * H > 512) {
+    if (n <= 16 && d <= 16 && nvec <= 64) return launch_sa<64, 4, 1>(st, a, lds);
+    if (n <= 16 && d <= 32 && nvec <= 128) return launch_sa<128, 8, 1>(st, a, lds);
+    if (n <= 16 && nvec <= 256) return launch_sa<256, 16, 1>(st, a, lds);
+    if (n <= 32 && d <= 32 && nvec <= 256) return launch_sa<256, 8, 1>(st, a, lds);
+  }
+  return launch_sa<512, 16, 2>(st, a, lds);
 }
