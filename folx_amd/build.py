@@ -25,7 +25,6 @@ SOURCES = [
     'dense_act.hip',
     'dense_act_wide.hip',
     'dense_chain.hip',
-    'dense_chain_many.hip',
     'dot_two.hip',
     'pointwise.hip',
     'reduce.hip',

@@ -28,16 +28,28 @@
 // CU spilled 70 of them (429 -> 631 us).  us, layers one by one -> chain: ten layers of 100, P = 4: 2000 positions
 // 101 -> 43, 25 600 503 -> 390; four of 50, P = 3, 15 750: 106 -> 31; six of 128, P = 6, 100 000: 1408 -> 1156.
 #include "activations.h"
-#include "dense_chain.h"
 
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-using folx_chain::MAXL;
-using ChainLayer = folx_chain::Layer;
-using ChainParams = folx_chain::Params;
-constexpr int MAXP = 6;  // more rows: dense_chain_many.hip
+constexpr int MAXL = FOLX_HIP_CHAIN_MAX_LAYERS;
+constexpr int MAXP = 6;
+
+struct ChainLayer {
+  const float *W, *bias;
+  int32_t K, N, act;  // act < 0: none (last layer, N = 1)
+  float prm;
+};
+
+struct ChainParams {
+  const float *x, *jac, *lap;
+  float *y, *y_jac, *y_lap;
+  float *h, *h_jac, *h_lap;  // what goes into a matrix-vector product at the end, where somebody else reads it too
+  int64_t R;
+  int32_t P, L, ld, vec;
+  ChainLayer layer[MAXL];
+};
 
 // where feature k of a row is kept
 __device__ __forceinline__ int chain_slot(int k) {
@@ -325,57 +337,37 @@ int launch_rows(hipStream_t st, const ChainParams& prm, const ChainPlan& pl) {
 }  // namespace
 
 extern "C" int folx_hip_dense_chain_faster(int32_t L, const int32_t* act, const int32_t* widths, int64_t R, int32_t P) {
+  ChainPlan pl;
   if (L < 1 || !act || !widths || R <= 0 || P < 0) return FOLX_HIP_EINVAL;
-  if (L == 1) return 0;
-  if (P > MAXP) {
-    bool faster;
-    int64_t bytes;
-    return folx_chain::many_plan(L, act, widths, R, P, faster, bytes) && faster ? 1 : 0;
-  }
-  ChainPlan pl;
-  return plan_chain(L, act, widths, R, P, pl) ? 1 : 0;
-}
-
-extern "C" int64_t folx_hip_dense_chain_workspace_bytes(int32_t L, const int32_t* act, const int32_t* widths, int64_t R,
-                                                        int32_t P) {
-  if (L < 1 || !act || !widths || R < 0 || P < 0) return FOLX_HIP_EINVAL;
-  bool faster;
-  int64_t bytes = 0;
-  if (P > MAXP) return folx_chain::many_plan(L, act, widths, R, P, faster, bytes) ? bytes : FOLX_HIP_ENOTSUP;
-  ChainPlan pl;
-  return plan_chain(L, act, widths, R, P, pl) ? 0 : FOLX_HIP_ENOTSUP;
+  return L > 1 && plan_chain(L, act, widths, R, P, pl) ? 1 : 0;
 }
 
 extern "C" int folx_hip_dense_chain_fwdlap(void* stream, int32_t L, const int32_t* act, const float* param,
                                            const float* const* W, const float* const* bias, const int32_t* widths,
                                            const float* x, const float* jac, const float* lap, float* y, float* y_jac,
-                                           float* y_lap, float* h, float* h_jac, float* h_lap, int64_t R, int32_t P,
-                                           void* workspace, int64_t workspace_bytes) {
+                                           float* y_lap, float* h, float* h_jac, float* h_lap, int64_t R,
+                                           int32_t P) {
   if (L < 1 || !act || !param || !W || !bias || !widths || R < 0 || P < 0) return FOLX_HIP_EINVAL;
   for (int l = 0; l <= L && l <= MAXL; ++l)
     if (widths[l] <= 0 || (l < L && l < MAXL && !W[l])) return FOLX_HIP_EINVAL;
   ChainPlan pl;
-  const int64_t need = folx_hip_dense_chain_workspace_bytes(L, act, widths, R, P);
-  if (need < 0) return (int)need;
-  if (P <= MAXP) plan_chain(L, act, widths, R, P, pl);
+  if (!plan_chain(L, act, widths, R, P, pl)) return FOLX_HIP_ENOTSUP;
   if (R == 0) return FOLX_HIP_OK;
   if (!x || !lap || !y || !y_lap || (P > 0 && (!jac || !y_jac))) return FOLX_HIP_EINVAL;
   const bool vector_last = act[L - 1] < 0;
   if ((h != nullptr) != (h_lap != nullptr) || (P > 0 && (h != nullptr) != (h_jac != nullptr)) ||
       (h != nullptr && (!vector_last || L < 2)))
     return FOLX_HIP_EINVAL;
-  if (need > 0 && (!workspace || workspace_bytes < need || !folx_aligned16(workspace))) return FOLX_HIP_EINVAL;
   ChainParams prm;
   prm.x = x; prm.jac = jac; prm.lap = lap;
   prm.y = y; prm.y_jac = y_jac; prm.y_lap = y_lap;
   prm.h = h; prm.h_jac = h_jac; prm.h_lap = h_lap;
-  prm.R = R; prm.P = P; prm.L = L; prm.ld = P > MAXP ? 0 : pl.ld;
+  prm.R = R; prm.P = P; prm.L = L; prm.ld = pl.ld;
   // the matrix-vector product stores single floats whatever the alignment
   prm.vec = vector_last ? widths[L - 1] % 4 == 0 && folx_aligned16(h) && folx_aligned16(h_jac) && folx_aligned16(h_lap)
                         : widths[L] % 4 == 0 && folx_aligned16(y) && folx_aligned16(y_jac) && folx_aligned16(y_lap);
   for (int l = 0; l < L; ++l) prm.layer[l] = {W[l], bias[l], widths[l], widths[l + 1], act[l], param[l]};
   hipStream_t st = (hipStream_t)stream;
-  if (P > MAXP) return folx_chain::many_launch(st, prm, act, widths, workspace);
   switch (P) {
     case 0: return launch_rows<2>(st, prm, pl);
     case 1: return launch_rows<3>(st, prm, pl);

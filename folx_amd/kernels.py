@@ -262,14 +262,14 @@ def _chain_args(layers):
 
 
 def dense_chain_faster(layers, R, P):
-    """Whether ``dense_chain`` is the way to evaluate these layers over R positions and P Jacobian rows;
+    """Whether one launch (``dense_chain``) is the way to evaluate these layers over R positions and P Jacobian rows;
     the library knows (folx_hip_dense_chain_faster)."""
     n, acts, widths = _chain_args(layers)
     return _lib.load().folx_hip_dense_chain_faster(n, acts, widths, R, P) == 1
 
 
 def dense_chain(layers, x, jac, lap, keep_hidden=False):
-    """Several narrow layers ``h <- f(h @ W + bias)`` in one launch (four over more than six Jacobian rows): ``layers`` = [(name, W (K, N), bias or None, param), ...],
+    """Several narrow layers ``h <- f(h @ W + bias)`` in one launch: ``layers`` = [(name, W (K, N), bias or None, param), ...],
     the last with ``name`` None if it is a plain matrix-vector product.  Returns the last layer's triplet and, with
     ``keep_hidden``, the triplet that goes into that product (else None)."""
     n, acts, widths = _chain_args(layers)
@@ -290,17 +290,11 @@ def dense_chain(layers, x, jac, lap, keep_hidden=False):
     bs = (ctypes.c_void_p * n)(*[None if b is None else b.data_ptr() for _, _, b, _ in layers])
     rules = [('dense_act_fwdlap', (name, R, P, *W.shape), W.numel()) if name is not None else
              ('dense_fwdlap', (R, P, *W.shape, False), W.numel()) for name, W, _, _ in layers]
-    lib = _lib.load()
-    nbytes = int(lib.folx_hip_dense_chain_workspace_bytes(n, acts, widths, R, P)) if P > 6 else 0
-    if nbytes < 0:
-        check(nbytes, 'dense_chain_workspace_bytes')
-    ws = torch.empty(nbytes, device=x.device, dtype=torch.uint8) if nbytes else None
     with _timed_chain(rules):
         check(
-            lib.folx_hip_dense_chain_fwdlap(
+            _lib.load().folx_hip_dense_chain_fwdlap(
                 _stream(), n, acts, params, Ws, bs, widths, _p(x), _p(jac), _p(lap), *[_p(t) for t in out],
-                *[_p(t) for t in hidden or (None, None, None)], R, P,
-                _p(ws), nbytes
+                *[_p(t) for t in hidden or (None, None, None)], R, P
             ),
             'dense_chain_fwdlap',
         )

@@ -144,7 +144,7 @@ def dot(h, W, b=None, residual=None, row_slice=None, act=None, norm=None):
     feature axis or a slice of rows in front of it, and returns a deferred value that absorbs the
     bias, the activation and the skip connection that follow (``wrapped_functions.Deferred``).
 
-    The keyword form states the same fusion explicitly: ``b`` bias,
+    The keyword form states the same fusion explicitly and evaluates at once: ``b`` bias,
     ``residual`` a triplet of the output shape, ``row_slice = (lo, hi)`` for
     ``h[..., lo:hi, :] @ W``, ``act`` a scalar function applied to ``h @ W + b`` (the residual is
     added to the activated result), ``norm = (gamma, beta, eps)`` a LayerNorm of ``h``."""
@@ -157,8 +157,7 @@ def dot(h, W, b=None, residual=None, row_slice=None, act=None, norm=None):
                                                 and h.opens_chain(W)):
         h = force(h)
     kwargs = {'bias': b, 'row_slice': row_slice, 'act': act, 'norm': norm}
-    # a Dense + activation layer alone may wait for the next one, as if written activation(dot(h, W) + b)
-    explicit = residual is not None or act is not None and (norm is not None or row_slice is not None or act not in FUSED_ACTS)
+    explicit = residual is not None or act is not None
     if explicit and isinstance(h, LazyDot):
         h = force(h)
     if explicit or not _is_triplet(h) or _is_triplet(W) or np.ndim(W) != 2:

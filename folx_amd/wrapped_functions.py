@@ -946,7 +946,7 @@ _ONE_OWNER = _single_reference()
 
 def _evaluate_chain(last, residual):
     """Products whose operand is itself an unevaluated Dense + activation layer, and so on down to a triplet: narrow layers
-    run as one rule where that is faster (``kernels.dense_chain``), anything else layer by layer, which is also what
+    over few Jacobian rows run as one launch (``kernels.dense_chain``), anything else layer by layer, which is also what
     defines the result.  A layer's handle that something besides the next layer refers to is evaluated for itself (it may be
     read again) and the chain starts behind it; a matrix-vector product at the end hands its operand's triplet back."""
     ends_in_vector = (residual is None and last.kwargs.get('act') is None and last.kwargs.get('norm') is None
@@ -982,7 +982,7 @@ def _evaluate_chain(last, residual):
 
 
 def _chain_launch(h: FwdLaplArray, nodes, keep: bool):
-    """``nodes`` over ``h`` as one rule: (last triplet, the one in front of it if ``keep``), or None where the layers go
+    """``nodes`` over ``h`` in one launch: (last triplet, the one in front of it if ``keep``), or None where the layers go
     one by one."""
     if not h.x.is_cuda or any(np.shape(d.W)[0] != k for d, k in zip(nodes, (h.shape[-1], *[d.shape[-1] for d in nodes[:-1]]))):
         return None

@@ -221,28 +221,24 @@ int folx_hip_dense_form(int64_t R, int32_t P, int32_t K, int32_t N);
 /*
  * A chain of n_layers narrow Dense + activation layers in one launch: layer l maps widths[l] to
  * widths[l + 1] features (1 .. 128), h <- act[l](h @ W[l] + bias[l]) with param[l] for the
- * function, as folx_hip_dense_act_fwdlap would layer by layer.  For P <= 6 Jacobian rows it is one launch without a
- * workspace, every sum in the order of the layers' own; above, four launches over `workspace` (16-byte aligned,
- * folx_hip_dense_chain_workspace_bytes: 0 for P <= 6).  The last act may be -1 (no function) if the last width is 1.
+ * function, as folx_hip_dense_act_fwdlap would layer by layer (same order of every sum), for
+ * P <= 6 Jacobian rows.  The last act may be -1 (no function) if the last width is 1.
  * Replaces a run of _dot_general_one_constant + elementwise rules (folx/wrapped_functions.py:71-171,
  * :400-445) whose intermediate triplets nobody else reads.
  *   x [R][widths[0]]   jac [P][R][widths[0]]   lap [R][widths[0]]
  *   W[l] [widths[l]][widths[l + 1]], bias[l] or NULL: arrays of n_layers DEVICE pointers on the host
  *   y [R][widths[n_layers]] y_jac y_lap; h, h_jac, h_lap: NULL, or with act[n_layers - 1] = -1 also the
  *   triplet in front of the last layer.
- * FOLX_HIP_ENOTSUP: more than FOLX_HIP_CHAIN_MAX_LAYERS layers, wider ones, more than 32 input features with P > 6, a function the fused
+ * FOLX_HIP_ENOTSUP: more than FOLX_HIP_CHAIN_MAX_LAYERS layers, wider ones, P > 6, a function the fused
  * rules do not take.  folx_hip_dense_chain_faster: 1 where the chain is taken to be faster than its layers one
  * by one, else 0.
  */
 #define FOLX_HIP_CHAIN_MAX_LAYERS 16
 int folx_hip_dense_chain_faster(int32_t n_layers, const int32_t* act, const int32_t* widths, int64_t R, int32_t P);
-int64_t folx_hip_dense_chain_workspace_bytes(int32_t n_layers, const int32_t* act, const int32_t* widths, int64_t R,
-                                             int32_t P);
 int folx_hip_dense_chain_fwdlap(void* stream, int32_t n_layers, const int32_t* act, const float* param,
                                 const float* const* W, const float* const* bias, const int32_t* widths,
                                 const float* x, const float* jac, const float* lap, float* y, float* y_jac,
-                                float* y_lap, float* h, float* h_jac, float* h_lap, int64_t R, int32_t P,
-                                void* workspace, int64_t workspace_bytes);
+                                float* y_lap, float* h, float* h_jac, float* h_lap, int64_t R, int32_t P);
 
 /*
  * folx_hip_dense_act_fwdlap for a wide layer whose input is a concatenation along the feature
