@@ -887,10 +887,12 @@ struct WidePlan {
 // R = 640 78 / 50, 1920 137 / 127.  The two meet at 60 000 rows of 256, 50 000 of 512 and 150 000 of 192 features; the line keeps the
 // workspace within the library's own scratch array, so that every call the entry point without a workspace took it still
 // takes.  With an activation the comparison is with the fused dense + activation rule, which has the same tiles: 59 / 55 at
-// P = 30, R = 64, 100 / 92 at P = 32, R = 64 of 512, even at 8000 rows, and 63 against 60 at P = 96, R = 128.
+// P = 30, R = 64, 100 / 92 at P = 32, R = 64 of 512, even at 8000 rows, and 63 against 60 at P = 96, R = 128.  Above 64 Jacobian rows
+// the fused form stays at every size, also where it is the slower one: the two round differently, and a determinant of 32 electrons
+// near a node turns that into 1.5e-4 of a walker's value between a batch of 4 and one of 1024.
 bool norm_apart(int64_t R, int32_t P, int32_t K, bool act) {
   const int64_t rows = (int64_t)(P + 2) * R;
-  return act ? P <= 64 && rows <= 8192 : rows * K <= (int64_t)14 << 20;
+  return P <= 64 && (act ? rows <= 8192 : rows * K <= (int64_t)14 << 20);
 }
 
 // What the forms of a dense + activation layer cost: times in us of a 64 x 64 tile and contracted feature on one CU (140

@@ -19,14 +19,15 @@ ROWS_ACT = 8192
 
 @pytest.mark.parametrize('R,P,Kd,N,act,apart', [
     (856, 33, 512, 132, None, False), (812, 33, 512, 132, None, True),        # the line at K = 512, a cut column tile
-    (572, 98, 256, 256, None, True), (576, 98, 256, 256, None, False),        # full groups but two rows
-    (44000, 5, 48, 256, None, False), (16, 1, 16, 300, None, True), (12, 193, 64, 256, None, True),
+    (896, 62, 256, 256, None, True), (900, 62, 256, 256, None, False),        # full groups but two rows
+    (44000, 5, 48, 256, None, False), (16, 1, 16, 300, None, True), (12, 193, 64, 256, None, False),
+    (40, 64, 64, 256, None, True), (40, 65, 64, 256, None, False),            # the line at 64 Jacobian rows
     (260, 30, 64, 192, 'tanh', False), (256, 30, 64, 192, 'tanh', True), (124, 64, 48, 256, 'silu', True),
     (8, 65, 80, 132, 'sin', False), (300, 40, 512, 512, 'gelu', False), (4, 2, 16, 136, 'tanh', True),
 ])
 def test_norm_dense_form(R, P, Kd, N, act, apart):
     print(f'case norm_dense R={R} P={P} K={Kd} N={N} act={act} apart={apart}', flush=True)
-    assert apart == ((P + 2) * R * Kd <= LIMIT if act is None else P <= 64 and (P + 2) * R <= ROWS_ACT)
+    assert apart == (P <= 64 and ((P + 2) * R * Kd <= LIMIT if act is None else (P + 2) * R <= ROWS_ACT))
     nbytes = _lib.load().folx_hip_norm_dense_workspace_bytes(R, P, Kd, N, -1 if act is None else _lib.ACT[act])
     triplet = 4 * (P + 2) * R * Kd
     if act is None:
