@@ -190,6 +190,9 @@ def roofline_of(dname, dkey, dn, dms, gemm):
                     f'act={act} R={R} P={P} K={Kd} N={N}')
     if dname == 'dense_act_fwdlap':
         act, R, P, Kd, N = dkey
+        if P <= 6:  # layers in a row are one launch, on record by their shares of it: the triplets between them never move
+            return mfma(2.0 * (P + 2) * R * Kd * N, f"a layer's share of dense_chain_kernel (dense_act kernels where it stands "
+                        f'alone) {act} R={R} P={P} K={Kd} N={N}')
         r = hbm(4.0 * ((P + 2) * R * (Kd + N) + Kd * N), f'dense_act_kernel {act} R={R} P={P} K={Kd} N={N}')
         r['mfma_tflops'] = 2.0 * (P + 2) * R * Kd * N / avg_s / 1e12
         r['mfma_frac'] = r['mfma_tflops'] / PEAK_FP32_MFMA_TFLOPS
