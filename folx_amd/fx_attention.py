@@ -38,7 +38,9 @@ def _shape(node):
 
 
 def _replay(node, index):
-    """The view or copy ``node`` applied to the index array of its operand; None if it repeats entries."""
+    """The view or copy ``node`` applied to the index array of its operand; None if it repeats entries.  The index is taken in
+    its own order first: whether a view exists depends on strides, and those of the array in the trace are others."""
+    index = index.contiguous()
     args = [index if a is node.args[0] else a for a in node.args]
     kwargs = {k: a for k, a in node.kwargs.items() if k != 'memory_format'}
     if any(isinstance(a, torch.fx.Node) for a in args):

@@ -90,7 +90,45 @@ def feature_axis_in_front(x):
     return (softmax(q @ k.transpose(-1, -2) / 2) @ v).permute(1, 2, 0).reshape(N, H * D)
 
 
-FUSED = {matmul: 1, einsum: 1, one_head: 1, leading_axis: 1, same_operand: 1, permuted_values: 1, chunked: 1, two_layers: 2}
+def heads_first(view):
+    """The heads-first result through a view that merges axes of it."""
+    def fn(x):
+        q, k, v = heads(x)
+        return view(softmax(q @ k.transpose(-1, -2) / 2) @ v)
+    return fn
+
+
+def flattened(x):
+    return heads_first(lambda o: o.flatten())(x)
+
+
+def one_axis(x):
+    return heads_first(lambda o: o.reshape(-1))(x)
+
+
+def rows_of_all_heads(x):
+    return heads_first(lambda o: o.reshape(H * N, D))(x)
+
+
+def rows_of_a_head(x):
+    return heads_first(lambda o: o.reshape(H, N * D))(x)
+
+
+def rows_across_heads(x):
+    return heads_first(lambda o: o.reshape(N, H * D))(x)
+
+
+def flattened_transpose(x):
+    return heads_first(lambda o: o.transpose(-1, -2).reshape(-1))(x)
+
+
+def flattened_and_multiplied(x):
+    return heads_first(lambda o: o.flatten(1) @ torch.linspace(-1, 1, 2 * N * D).reshape(N * D, 2))(x)
+
+
+FUSED = {matmul: 1, einsum: 1, one_head: 1, leading_axis: 1, same_operand: 1, permuted_values: 1, chunked: 1, two_layers: 2,
+         flattened: 1, one_axis: 1, rows_of_all_heads: 1, rows_of_a_head: 1, rows_across_heads: 1, flattened_transpose: 1,
+         flattened_and_multiplied: 1}
 LEFT = [scores_read_twice, masked, over_queries, transposed_scores, constant_values, feature_axis_in_front]
 
 
