@@ -81,7 +81,9 @@ def _scale(node, consts):
         if c is None or getattr(c, 'size', 1) != 1 or getattr(c, 'ndim', 0) != 0:
             return None
     c = float(c)
-    return 1.0 / c if node.target in (aten.div.Tensor, aten.div.Scalar) else c
+    if node.target in (aten.div.Tensor, aten.div.Scalar):
+        return 1.0 / c if c != 0.0 else None    # Python divides by no zero: left to the division itself
+    return c
 
 
 def _down(node, index, used):

@@ -146,3 +146,17 @@ def test_attention_in_a_traced_function(monkeypatch, fn, thr):
     for a, b in ((got.x, want.x), (got.jacobian.dense_array, want.jacobian.dense_array), (got.laplacian, want.laplacian)):
         # stand-ins compute in 64 bits and round every rule's result to 32: a few roundings on either side
         torch.testing.assert_close(a, b, rtol=2e-5, atol=2e-5 * float(b.abs().max()))
+
+
+def test_scores_divided_by_zero(monkeypatch):
+    """No factor of the query: the products and the softmax stay, and the result is what they make of it."""
+    cpu_kernels.install(monkeypatch)
+    x = torch.randn(3, N, 3, generator=torch.Generator().manual_seed(1))
+
+    def fn(x):
+        q, k, v = heads(x)
+        return softmax(q @ k.transpose(-1, -2) / 0.0) @ v
+
+    got = fx.forward_laplacian_torch(fn, 0).batched(x)
+    want = torch.stack([fn(t) for t in x])
+    torch.testing.assert_close(got.x, want, equal_nan=True)
