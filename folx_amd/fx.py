@@ -1036,12 +1036,15 @@ class TracedForwardLaplacian(ForwardLaplacianFn):
                 try:
                     # in-place updates and slice assignments of the function become their functional forms
                     # (add_, copy_ into a view, index_put_ ... -> add, slice_scatter, index_put ...)
-                    gm = self.graphs[shapes] = make_fx(torch.func.functionalize(self.torch_fn))(*examples)
+                    gm = make_fx(torch.func.functionalize(self.torch_fn))(*examples)
                 finally:
                     _TRACING[0] = False
-            self.constants[shapes] = fold_constants(gm)
-            if fuse_attention(gm, self.constants[shapes]):
-                self.constants[shapes] = fold_constants(gm)
+            consts = fold_constants(gm)
+            if fuse_attention(gm, consts):
+                consts = fold_constants(gm)
+            # kept once it is whole, the constants first: who finds the graph finds them too
+            self.constants[shapes] = consts
+            self.graphs[shapes] = gm
         return gm
 
     def _constants(self, shapes, device):

@@ -160,3 +160,23 @@ def test_scores_divided_by_zero(monkeypatch):
     got = fx.forward_laplacian_torch(fn, 0).batched(x)
     want = torch.stack([fn(t) for t in x])
     torch.testing.assert_close(got.x, want, equal_nan=True)
+
+
+def test_a_trace_that_fails_to_finish_is_not_kept(monkeypatch):
+    """What raises while a trace is prepared raises again at the next call: no half-rewritten graph serves it."""
+    cpu_kernels.install(monkeypatch)
+    x = torch.randn(3, N, 3, generator=torch.Generator().manual_seed(1))
+    traced = fx.forward_laplacian_torch(matmul, 0)
+
+    def broken(gm, consts):
+        raise RuntimeError('broken')
+
+    with monkeypatch.context() as m:
+        m.setattr(fx, 'fuse_attention', broken)
+        for _ in range(2):
+            with pytest.raises(RuntimeError, match='broken'):
+                traced.batched(x)
+    assert not traced.graphs
+    want = fx.forward_laplacian_torch(matmul, 0).batched(x)
+    got = traced.batched(x)
+    assert torch.equal(got.x, want.x) and torch.equal(got.laplacian, want.laplacian)
