@@ -902,28 +902,26 @@ def _nodes_in(a):
 
 
 def _steps(gm: torch.fx.GraphModule):
-    """(position of each node, its ``_Step``s in order); worked out once per graph."""
-    got = gm.meta.get('folx_steps')
-    if got is None:
-        order = {n: i for i, n in enumerate(gm.graph.nodes)}
-        last_read = {}
-        for n in order:
-            if n.users and n.op != 'output':
-                last_read.setdefault(max(n.users, key=order.__getitem__), []).append(n)
-        got = gm.meta['folx_steps'] = (order, [_Step(n, tuple(last_read.get(n, ()))) for n in order])
-    return got
+    """(position of each node, its ``_Step``s in order) of the graph as it stands."""
+    order = {n: i for i, n in enumerate(gm.graph.nodes)}
+    last_read = {}
+    for n in order:
+        if n.users and n.op != 'output':
+            last_read.setdefault(max(n.users, key=order.__getitem__), []).append(n)
+    return order, [_Step(n, tuple(last_read.get(n, ()))) for n in order]
 
 
-def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None):
+def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None, steps=None):
     """One pass over the equations of a traced graph (folx/interpreter.py:218-264): constant equations come from
-    ``fold_constants``, the others go through ``RULES``."""
+    ``fold_constants``, the others go through ``RULES``.  Who evaluates a graph often and changes it no more keeps both,
+    ``consts`` and ``steps`` (``_steps``)."""
     env = dict(fold_constants(gm) if consts is None else consts)
     it = iter(inputs)
     look = lambda a: env[a] if isinstance(a, torch.fx.Node) else a
     take = lambda kind, a: a if kind == 0 else (env[a] if kind == 1 else torch.fx.node.map_arg(a, look))   # noqa: E731
-    order, steps = _steps(gm)
+    order, listed = steps or _steps(gm)
     done = ()
-    for step in steps:
+    for step in listed:
         args = kwargs = None
         for n in done:   # what nobody reads any more: its memory serves the next equation, and a deferred value is free
             env.pop(n, None)
@@ -1022,6 +1020,7 @@ class TracedForwardLaplacian(ForwardLaplacianFn):
     def __init__(self, fn, sparsity_threshold):
         self.torch_fn = fn
         self.graphs = {}
+        self.steps = {}
         self.constants = {}
         super().__init__(self._run, sparsity_threshold)
 
@@ -1042,8 +1041,9 @@ class TracedForwardLaplacian(ForwardLaplacianFn):
             consts = fold_constants(gm)
             if fuse_attention(gm, consts):
                 consts = fold_constants(gm)
-            # kept once it is whole, the constants first: who finds the graph finds them too
+            # kept once it is whole, the graph last: who finds it finds the others too
             self.constants[shapes] = consts
+            self.steps[shapes] = _steps(gm)
             self.graphs[shapes] = gm
         return gm
 
@@ -1073,12 +1073,13 @@ class TracedForwardLaplacian(ForwardLaplacianFn):
     def _run(self, *lapl_args):
         shapes = tuple(tuple(a.shape) for a in lapl_args)
         gm = self._graph(shapes)
-        return evaluate_graph(gm, lapl_args, self._constants(shapes, lapl_args[0].x.device))
+        return evaluate_graph(gm, lapl_args, self._constants(shapes, lapl_args[0].x.device), self.steps[shapes])
 
     def invalidate(self):
         """Forget the traces (and the constants folded from them): the next call traces again, e.g. after the
         parameters of a traced module have changed."""
         self.graphs.clear()
+        self.steps.clear()
         self.constants.clear()
 
 

@@ -112,6 +112,29 @@ def test_benchmark_models_through_the_traced_front_door_on_the_gpu(thr):
         _both_front_doors(forward, make(cfg), x, thr, 'cuda')
 
 
+def test_a_copied_or_edited_graph_is_evaluated_as_it_stands(monkeypatch):
+    """``evaluate_graph`` keeps nothing about a graph: a deep copy evaluates its own nodes, an edited graph the edited ones."""
+    import copy
+
+    import cpu_kernels
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from folx_amd import fx
+    from folx_amd.interpreter import ForwardLaplacianFn
+
+    cpu_kernels.install(monkeypatch)
+    x = torch.randn(2, 5, 3, generator=torch.Generator().manual_seed(0))
+    W = torch.randn(3, 4, generator=torch.Generator().manual_seed(1))
+    gm = make_fx(lambda r: torch.tanh(r @ W).sum())(x[0])
+    evaluate = lambda g: ForwardLaplacianFn(lambda a: fx.evaluate_graph(g, (a,)), 0).batched(x)
+    first, copied = evaluate(gm), evaluate(copy.deepcopy(gm))
+    assert torch.equal(first.x, copied.x) and torch.equal(first.laplacian, copied.laplacian)
+    for node in gm.graph.nodes:
+        if node.target is torch.ops.aten.tanh.default:
+            node.target = torch.ops.aten.sin.default
+    torch.testing.assert_close(evaluate(gm).x, torch.sin(x @ W).sum((1, 2)))
+
+
 @pytest.mark.gpu
 def test_traced_model_under_graph_replay():
     """``folx_amd.jit`` around a traced model: replays return the bits of the eager evaluation."""
