@@ -137,7 +137,9 @@ def _pow_scalar(a, e):
 
 
 def _scaled(v, alpha):
-    return v if alpha == 1 else fnp.multiply(v, float(alpha))
+    if alpha == 1:
+        return v
+    return v * float(alpha) if isinstance(v, torch.Tensor) else fnp.multiply(v, float(alpha))
 
 
 def _addmm(bias, a, b, beta=1, alpha=1):
@@ -869,10 +871,12 @@ def fold_constants(gm: torch.fx.GraphModule):
     return {n: _tree(v, _const) for n, v in env.items()}
 
 
-_OPERAND_READERS = {aten.add.Tensor, aten.mul.Tensor}   # their rules take a device tensor as the constant operand
+# Rules that take a constant operand as a device tensor where another operand is a triplet: sums and products, weights
+_OPERAND_READERS = {aten.add.Tensor, aten.mul.Tensor}
 _WEIGHT_READERS = {aten.mm.default, aten.addmm.default, aten.bmm.default, aten.matmul.default, aten.mv.default,
                    aten.native_layer_norm.default}
-_DEVICE_CONST_MIN = 256   # constants of at least this many floats live on the device between evaluations
+_DEVICE_READERS = _OPERAND_READERS | _WEIGHT_READERS
+_DEVICE_CONST_MIN = 256   # weights of at least this many floats live on the device between evaluations
 
 
 class _Step:
@@ -911,10 +915,11 @@ def _steps(gm: torch.fx.GraphModule):
     return order, [_Step(n, tuple(last_read.get(n, ()))) for n in order]
 
 
-def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None, steps=None):
+def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None, steps=None, on_device=None):
     """One pass over the equations of a traced graph (folx/interpreter.py:218-264): constant equations come from
     ``fold_constants``, the others go through ``RULES``.  Who evaluates a graph often and changes it no more keeps both,
-    ``consts`` and ``steps`` (``_steps``)."""
+    ``consts`` and ``steps`` (``_steps``).  ``on_device``: device copies of some constants, for the equations in
+    ``_DEVICE_READERS`` that meet a triplet; all others take the constants as they are."""
     env = dict(fold_constants(gm) if consts is None else consts)
     it = iter(inputs)
     look = lambda a: env[a] if isinstance(a, torch.fx.Node) else a
@@ -932,6 +937,8 @@ def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None, steps=None):
             env[node] = next(it)
         elif step.op == 'call_function':
             args = [take(kind, a) for kind, a in step.args]
+            if on_device and step.target in _DEVICE_READERS and any(fnp._is_triplet(a) for a in args):
+                args = [on_device.get(a, v) if kind == 1 else v for (kind, a), v in zip(step.args, args)]
             kwargs = {k: take(kind, a) for k, kind, a in step.kwargs}
             rule = RULES.get(step.target)
             functional = _functional_form(node.target) if rule is None else None
@@ -1047,33 +1054,25 @@ class TracedForwardLaplacian(ForwardLaplacianFn):
             self.graphs[shapes] = gm
         return gm
 
-    def _constants(self, shapes, device):
+    def _on_device(self, shapes, device):
+        """Device copies of the constants that sums, products and weights read, made once per device."""
         key = (shapes, str(device))
         hit = self.constants.get(key)
         if hit is None:
-            def place(v):
-                if (isinstance(v, np.ndarray) and v.dtype == np.float32 and v.size >= _DEVICE_CONST_MIN
-                        and device.type != 'cpu'):
-                    return torch.as_tensor(np.ascontiguousarray(v)).to(device)
-                return v
-            # only what the product rules read (weights): they take device tensors as they are, and every other
-            # rule keeps seeing host arrays, whatever the size of its constants
-            def read_by(n, readers):
-                return n.users and all(u.target in readers for u in n.users)
+            def wanted(n, v):
+                if not (isinstance(v, np.ndarray) and v.dtype == np.float32 and v.ndim >= 1):
+                    return False
+                return any(u.target in _OPERAND_READERS or (u.target in _WEIGHT_READERS and v.size >= _DEVICE_CONST_MIN) for u in n.users)
 
-            def small(v):
-                if isinstance(v, np.ndarray) and v.dtype == np.float32 and v.ndim >= 1 and device.type != 'cpu':
-                    return torch.as_tensor(np.ascontiguousarray(v)).to(device)
-                return v
-            hit = self.constants[key] = {n: (_tree(v, place) if read_by(n, _WEIGHT_READERS) else
-                                             small(v) if read_by(n, _OPERAND_READERS) else v)
-                                         for n, v in self.constants[shapes].items()}
+            hit = self.constants[key] = {n: torch.as_tensor(np.ascontiguousarray(v)).to(device)
+                                         for n, v in self.constants[shapes].items() if wanted(n, v)}
         return hit
 
     def _run(self, *lapl_args):
         shapes = tuple(tuple(a.shape) for a in lapl_args)
         gm = self._graph(shapes)
-        return evaluate_graph(gm, lapl_args, self._constants(shapes, lapl_args[0].x.device), self.steps[shapes])
+        return evaluate_graph(gm, lapl_args, self.constants[shapes], self.steps[shapes],
+                              self._on_device(shapes, lapl_args[0].x.device))
 
     def invalidate(self):
         """Forget the traces (and the constants folded from them): the next call traces again, e.g. after the

@@ -135,6 +135,52 @@ def test_a_copied_or_edited_graph_is_evaluated_as_it_stands(monkeypatch):
     torch.testing.assert_close(evaluate(gm).x, torch.sin(x @ W).sum((1, 2)))
 
 
+_C = torch.linspace(-1, 1, 6)
+_LARGE = torch.linspace(-1, 1, 3 * 256).reshape(3, 256)
+# constants as operands of sums and products, where the other operand has derivatives, is a constant that is formed per call,
+# or the rule scales the constant first
+CONSTANT_OPERANDS = {
+    'alpha': lambda x: torch.add(x, _C, alpha=2.0),
+    'alpha_on_the_triplet': lambda x: torch.add(_C, x, alpha=-0.5),
+    'zeros_plus_constant': lambda x: x * (torch.zeros_like(x) + _C),
+    'ones_times_constant': lambda x: x + torch.ones_like(x) * _C,
+    'full_plus_constant': lambda x: x * (_C + torch.full_like(x, 2.0)),
+    'sign_plus_constant': lambda x: x * (torch.sign(x) + _C),
+    'sum_and_product': lambda x: (x + _C) * _C,
+    'bias_and_scale': lambda x: torch.addmm(torch.linspace(0, 1, 256), x[:, :3], _LARGE, beta=2.0, alpha=0.5),
+    'weights_of_zeros': lambda x: x.sum() + torch.zeros_like(x[:, :3]) @ _LARGE,
+}
+
+
+def _check_constant_operand(name, wrap, device):
+    fn = CONSTANT_OPERANDS[name]
+    x = torch.randn(3, 4, 6, generator=torch.Generator().manual_seed(0)) + 0.1
+    fl = wrap(folx_amd.vmap(folx_amd.forward_laplacian_torch(fn, 0)))
+    for call in range(2):
+        out = fl((x + call).to(device))
+        want = torch.stack([fn(t) for t in x + call])
+        torch.testing.assert_close(out.x.cpu(), want, rtol=1e-5, atol=1e-5)
+        J = torch.stack([torch.func.jacrev(fn)(t).reshape(*want.shape[1:], -1) for t in x + call])
+        torch.testing.assert_close(out.jacobian.dense_array.cpu().movedim(0, -1), J, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(out.laplacian.cpu(), torch.zeros_like(want), rtol=0, atol=1e-5)
+
+
+@pytest.mark.parametrize('name', CONSTANT_OPERANDS)
+def test_constant_operands(name, monkeypatch):
+    import cpu_kernels
+
+    cpu_kernels.install(monkeypatch)
+    _check_constant_operand(name, lambda f: f, 'cpu')
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('captured', [False, True], ids=['eager', 'jit'])
+@pytest.mark.parametrize('name', CONSTANT_OPERANDS)
+def test_constant_operands_on_the_gpu(name, captured):
+    print(f'constant operand {name} captured={captured}', flush=True)
+    _check_constant_operand(name, folx_amd.jit if captured else (lambda f: f), 'cuda')
+
+
 @pytest.mark.gpu
 def test_traced_model_under_graph_replay():
     """``folx_amd.jit`` around a traced model: replays return the bits of the eager evaluation."""
