@@ -135,14 +135,20 @@ __device__ __forceinline__ void act_eval(float x, float prm, float& y, float& d1
   } else if constexpr (ACT == FOLX_ACT_GELU) {
     const float c = 0.5f * (1.0f + erff(0.70710678118654752f * x));       // Phi(x)
     const float g = 0.39894228040143268f * expf(-0.5f * x * x);           // Phi'(x)
-    y = x * c; d1 = c + x * g; d2 = g * (2.0f - x * x);
+    y = x * c;
+    d1 = g != 0.0f ? c + x * g : c;              // Phi' has underflowed long before x^2 overflows
+    d2 = g != 0.0f ? g * (2.0f - x * x) : 0.0f;
   } else if constexpr (ACT == FOLX_ACT_GELU_TANH) {
     // x (1 + tanh u) / 2 with u = a (x + b x^3)
     const float a = 0.79788456080286536f, b = 0.044715f, xx = x * x;
     const float t = tanhf(a * x * (1.0f + b * xx)), u1 = a * (1.0f + 3.0f * b * xx), s = 1.0f - t * t;
     y = 0.5f * x * (1.0f + t);
-    d1 = 0.5f * (1.0f + t) + 0.5f * x * s * u1;
-    d2 = s * (u1 + x * (3.0f * a * b * x - t * u1 * u1));
+    d1 = 0.5f * (1.0f + t);
+    d2 = 0.0f;
+    if (s != 0.0f) {  // tanh is 1 in float32 long before u1^2 overflows
+      d1 += 0.5f * x * s * u1;
+      d2 = s * (u1 + x * (3.0f * a * b * x - t * u1 * u1));
+    }
   } else {  // FOLX_ACT_INTEGER_POW
     int n = (int)prm;
     // x^(n-2) by repeated multiplication on |n-2|, then one or two more factors

@@ -41,3 +41,24 @@ def test_dense_gelu(name, rows, P, k, n):
     W, b = (g.normal(size=(k, n)) / np.sqrt(k)).astype(np.float32), g.normal(size=n).astype(np.float32)
     z = rules.dense_rule(*[v.astype(np.float64) for v in (*t, W, b)])
     compare(K.dense_act(name, *[dev(v) for v in t], dev(W), dev(b)), rules.elementwise_rule(name, *z), name)
+
+
+# elementwise (no layer), narrow few-rows and general kernels, the wide kernel
+@pytest.mark.parametrize('name', ['gelu', 'gelu_tanh'])
+@pytest.mark.parametrize('P,k,n', [(2, None, None), (2, 4, 8), (9, 16, 64), (32, 16, 256)])
+def test_gelu_far_from_zero(name, P, k, n):
+    """Where the function is x or 0 in float32 its derivatives are 1 or 0 and 0, up to the largest numbers: a factor that has
+    underflowed meets no overflow."""
+    print(f'case {name} far from zero, P={P} {k} x {n}', flush=True)
+    x = np.array([s * v for v in (20.0, 1e3, 1e8, 2e9, 2e10, 1e15, 1e18, 3e19, 1e30, 3e38, 1e2, 1e12) for s in (1, -1)], np.float32)
+    y, d = np.where(x > 0, x, 0), (x > 0).astype(np.float32)
+    if k is None:
+        got = K.elementwise(name, dev(x), dev(np.ones((P, *x.shape))), dev(np.ones(x.shape)))
+    else:
+        feature = np.eye(1, k)[0]
+        t = [dev(v[..., None] * feature) for v in (x, np.ones((P, *x.shape)), np.ones(x.shape))]
+        got = K.dense_act(name, *t, dev(feature[:, None] * np.ones(n)))
+        y, d = y[:, None], d[:, None]
+    for a, want in zip(got, (y, d, d)):
+        a = a.cpu().numpy()
+        np.testing.assert_array_equal(a, np.broadcast_to(want, a.shape))
