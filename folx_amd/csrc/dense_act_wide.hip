@@ -845,6 +845,9 @@ __device__ __forceinline__ void norm_rows(const float* __restrict__ x, const flo
 
 // Both in one launch, the blocks of the weights first: neither reads what the other writes.  K = N = 256: 16.5 us for the weights
 // (64 columns a block, 16 requests in a row each) and 4.9 us for the rows of 640 positions, each its own launch, became 6 us.
+// The fused form is the one for any number of positions, also where LayerNorm and a product with 64 x 64 tiles would be faster (us, fused
+// / the two rules, K = N = 256: P = 30, R = 64 56 / 16, 640 62 / 41, 1920 102 / 98; P = 96, R = 64 56 / 28): the two round differently, and a
+// walker's Jacobian then depended on how many walkers a call has, by up to 1.5e-3 of it behind a determinant of 20 electrons.
 __global__ __launch_bounds__(256) void norm_prepare_kernel(const float* x, const float* lap, const float* W, const float* bias,
                                                            const float* gamma, const float* beta, float* xhat, float* rs,
                                                            float* nx, float* nlap, float* Wg, float2* wc, int64_t R, int32_t K,
@@ -877,23 +880,7 @@ struct WidePlan {
   int64_t row_tiles, pos_tiles, blocks, ws_bytes;
   int64_t o_ss, o_s1, o_sc, o_xhat, o_rs, o_nx, o_nlap, o_wg, o_wc;
   int32_t PG, PT, col_tiles;
-  bool apart;  // LayerNorm as a launch of its own in front of the product
 };
-
-// Small LayerNorm + Dense calls run as the two rules one after the other, the normalised triplet in the workspace: the fused
-// form's launches on the positions (prepare, x / lap product, finish) and its 128 x 256 tiles cost 45 to 100 us whatever the size,
-// where the plain product has 64 x 64 tiles.  us, fused / apart, K = N = 256: P = 30, R = 64 56 / 16, 640 62 / 41, 1920 102 / 98; P = 96,
-// R = 64 56 / 28, 256 62 / 54, 480 97 / 83, 640 98 / 99; 512: P = 32, R = 64 97 / 31, 640 172 / 128, 960 175 / 167, 1920 318 / 322; 192: P = 60,
-// R = 640 78 / 50, 1920 137 / 127.  The two meet at 60 000 rows of 256, 50 000 of 512 and 150 000 of 192 features; the line keeps the
-// workspace within the library's own scratch array, so that every call the entry point without a workspace took it still
-// takes.  With an activation the comparison is with the fused dense + activation rule, which has the same tiles: 59 / 55 at
-// P = 30, R = 64, 100 / 92 at P = 32, R = 64 of 512, even at 8000 rows, and 63 against 60 at P = 96, R = 128.  Above 64 Jacobian rows
-// the fused form stays at every size, also where it is the slower one: the two round differently, and a determinant of 32 electrons
-// near a node turns that into 1.5e-4 of a walker's value between a batch of 4 and one of 1024.
-bool norm_apart(int64_t R, int32_t P, int32_t K, bool act) {
-  const int64_t rows = (int64_t)(P + 2) * R;
-  return P <= 64 && (act ? rows <= 8192 : rows * K <= (int64_t)14 << 20);
-}
 
 // What the forms of a dense + activation layer cost: times in us of a 64 x 64 tile and contracted feature on one CU (140
 // TFLOP/s over the chip; 233 of fp32 products from bf16 pieces), the work around the K loop in features of that cost, the
@@ -979,14 +966,6 @@ bool plan_wide(int64_t R, int32_t P, int32_t K, int32_t N, bool norm, bool act, 
     pl.o_wg = take((int64_t)K * N);
     pl.o_wc = take(2 * (int64_t)N);
   }
-  pl.apart = norm && norm_apart(R, P, K, act);
-  if (pl.apart) {  // the normalised triplet, then what the rule behind it needs
-    int64_t need = (int64_t)(P + 2) * R * K;
-    WidePlan behind;
-    if (act && plan_wide(R, P, K, N, false, true, behind)) need += behind.ws_bytes / 4;
-    pl.apart = need * 4 <= FOLX_HIP_STATIC_SCRATCH_BYTES;
-    if (pl.apart) o = need;
-  }
   pl.ws_bytes = o * 4;
   return true;
 }
@@ -1023,16 +1002,6 @@ int run_wide(hipStream_t st, bool norm, int32_t act, float param, const float* x
     return FOLX_HIP_ENOTSUP;
   if (!workspace || workspace_bytes < pl.ws_bytes || !folx_aligned16(workspace)) return FOLX_HIP_EINVAL;
   float* ws = (float*)workspace;
-  if (pl.apart) {
-    const int64_t RK = R * (int64_t)K;
-    float *nx = ws, *nj = nx + RK, *nl = nj + P * RK, *rest = nl + RK;
-    const int rc = folx_hip_layernorm_fwdlap(st, x, jac, lap, gamma, beta, nx, nj, nl, R, K, P, eps);
-    if (rc != FOLX_HIP_OK) return rc;
-    if (!has_act)
-      return folx_hip_dense_fwdlap(st, nx, nj, nl, W, bias, nullptr, nullptr, nullptr, y, y_jac, y_lap, R, P, K, N);
-    return run_wide(st, false, act, param, nx, nj, nl, nullptr, nullptr, 0.0f, W, bias, y, y_jac, y_lap, R, P, K, N, rest,
-                    workspace_bytes - (int64_t)(rest - ws) * 4);
-  }
   WideParams a;
   a.jac = jac; a.W = W; a.z = y; a.y_jac = y_jac; a.res_jac = res_jac;
   a.pre_jac = pre_jac; a.pre_group = pre_group;

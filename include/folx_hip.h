@@ -279,9 +279,7 @@ int folx_hip_dense_act_parts_fwdlap(void* stream, int32_t act, float param, cons
  * nor the pre-activation Jacobian is written.  The Jacobian rows are multiplied RAW with
  * diag(gamma) W and LayerNorm's projection is applied to the product as a rank-2 correction
  * per row, so rows whose mean dwarfs their variation lose digits they would keep in the
- * three-step form.  Small calls (at most 64 Jacobian rows and a normalised triplet of 14 Mi floats,
- * with an activation 8192 rows) run as the rules one after the other, the normalised triplet in
- * the workspace.
+ * three-step form.
  *   x [R][K]  jac [P][R][K]  lap [R][K]  gamma, beta [K] or NULL  W [K][N]  bias [N] or NULL
  *   ->  y [R][N]  y_jac [P][R][N]  y_lap [R][N];  act = -1: no activation.
  * Built for N > 128 with N % 4 == 0, K % 16 == 0, K <= 512, R % 4 == 0, P >= 1, 16-byte aligned

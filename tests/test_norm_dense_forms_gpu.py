@@ -1,5 +1,5 @@
-"""LayerNorm + Dense as one kernel and as the two rules apart: on either side of the line between them, with cut tiles and partial
-groups of Jacobian rows, against the float64 oracle on the first and last positions (the rule acts on each position alone)."""
+"""LayerNorm + Dense as one rule from a few positions to many, with cut tiles and partial groups of Jacobian rows: against the
+float64 oracle on the first and last positions (the rule acts on each position alone), and independent of their number."""
 
 import numpy as np
 import pytest
@@ -9,32 +9,21 @@ from oracle import backend as ob
 from oracle import rules
 from tolerances import assert_lap, assert_val
 
-from folx_amd import _lib
 from folx_amd import kernels as K
 
 pytestmark = pytest.mark.gpu
-LIMIT = 14 << 20     # floats of the normalised triplet
-ROWS_ACT = 8192
 
 
-@pytest.mark.parametrize('R,P,Kd,N,act,apart', [
-    (856, 33, 512, 132, None, False), (812, 33, 512, 132, None, True),        # the line at K = 512, a cut column tile
-    (896, 62, 256, 256, None, True), (900, 62, 256, 256, None, False),        # full groups but two rows
-    (44000, 5, 48, 256, None, False), (16, 1, 16, 300, None, True), (12, 193, 64, 256, None, False),
-    (40, 64, 64, 256, None, True), (40, 65, 64, 256, None, False),            # the line at 64 Jacobian rows
-    (260, 30, 64, 192, 'tanh', False), (256, 30, 64, 192, 'tanh', True), (124, 64, 48, 256, 'silu', True),
-    (8, 65, 80, 132, 'sin', False), (300, 40, 512, 512, 'gelu', False), (4, 2, 16, 136, 'tanh', True),
+@pytest.mark.parametrize('R,P,Kd,N,act', [
+    (856, 33, 512, 132, None), (812, 33, 512, 132, None),        # a cut column tile, one row in the last group
+    (896, 62, 256, 256, None), (900, 62, 256, 256, None),        # full groups but two rows
+    (44000, 5, 48, 256, None), (16, 1, 16, 300, None), (12, 193, 64, 256, None),
+    (40, 64, 64, 256, None), (40, 65, 64, 256, None),
+    (260, 30, 64, 192, 'tanh'), (256, 30, 64, 192, 'tanh'), (124, 64, 48, 256, 'silu'),
+    (8, 65, 80, 132, 'sin'), (300, 40, 512, 512, 'gelu'), (4, 2, 16, 136, 'tanh'),
 ])
-def test_norm_dense_form(R, P, Kd, N, act, apart):
-    print(f'case norm_dense R={R} P={P} K={Kd} N={N} act={act} apart={apart}', flush=True)
-    assert apart == (P <= 64 and ((P + 2) * R * Kd <= LIMIT if act is None else (P + 2) * R <= ROWS_ACT))
-    nbytes = _lib.load().folx_hip_norm_dense_workspace_bytes(R, P, Kd, N, -1 if act is None else _lib.ACT[act])
-    triplet = 4 * (P + 2) * R * Kd
-    if act is None:
-        assert (nbytes == triplet) == apart
-    assert nbytes >= triplet or not apart
-    if apart:
-        assert nbytes <= _lib.STATIC_SCRATCH_BYTES
+def test_norm_dense_form(R, P, Kd, N, act):
+    print(f'case norm_dense R={R} P={P} K={Kd} N={N} act={act}', flush=True)
     g = torch.Generator(device='cuda').manual_seed(R + P)
     rn = lambda *s: torch.randn(*s, device='cuda', generator=g)
     x, J, L = rn(R, Kd) + 0.5, rn(P, R, Kd) + 0.3 * rn(P, R, 1), rn(R, Kd)
@@ -49,3 +38,19 @@ def test_norm_dense_form(R, P, Kd, N, act, apart):
     assert_val(got[0][at], ref[0], 'x')
     assert_val(got[1][:, at], ref[1], 'jacobian')
     assert_lap(got[2][at], ref[2], 'laplacian')
+
+
+@pytest.mark.parametrize('act', [None, 'tanh'])
+@pytest.mark.parametrize('P,Kd,N', [(30, 256, 256), (60, 256, 256), (64, 64, 192), (96, 512, 256)])
+def test_a_position_does_not_depend_on_how_many_there_are(P, Kd, N, act):
+    """The bits of the first positions are those of a call on them alone, from a few walkers' worth to a full chunk."""
+    print(f'case norm_dense positions P={P} K={Kd} N={N} act={act}', flush=True)
+    g = torch.Generator(device='cuda').manual_seed(P)
+    rn = lambda *s: torch.randn(*s, device='cuda', generator=g)
+    R = 4096
+    x, J, L = rn(R, Kd) + 0.5, rn(P, R, Kd) + 0.3 * rn(P, R, 1), rn(R, Kd)
+    consts = 1 + 0.3 * rn(Kd), 0.2 * rn(Kd), 1e-5, rn(Kd, N) / Kd ** 0.5, rn(N)
+    full = K.norm_dense(act, x, J, L, *consts)
+    for r in (4, 64, 640, 1024):
+        part = K.norm_dense(act, x[:r].contiguous(), J[:, :r].contiguous(), L[:r].contiguous(), *consts)
+        assert torch.equal(part[0], full[0][:r]) and torch.equal(part[1], full[1][:, :r]) and torch.equal(part[2], full[2][:r]), r
