@@ -319,6 +319,41 @@ bool plan_chain(int32_t L, const int32_t* act, const int32_t* widths, int64_t R,
   return pl.blocks <= 0x7fffffffLL;
 }
 
+// us of the chain and of its layers one by one (multiples of 4 wide): launches, a round of workgroups (per layer, and per chunk of 16
+// features and block of rows), MB moved, products; a launch's rows and the columns of its output.  Fitted to 419 chains (2 to 8
+// layers of 4 to 128 features, equal, unequal and narrow in the middle, R = 500 .. 320 000, P = 0 .. 6; 12 and 11 % rms; another
+// 607: 13 and 12 %).  A chain saves the trips through memory between its layers and nothing at its ends, where its workgroups stream
+// worse than those of one layer: 128 -> 4 -> 128 over 200 000 positions, P = 1: 160 us layer by layer, 258 in one; 4000: 13 and 8.7.
+// Of the 607, taken whenever they fit, 78 were more than 3 % slower than their layers, up to 2.7 times (0.704 of the layers' time in
+// the mean); by this rule 7 are, by at most 13 %, and 17 that
+// would gain more than 3 %, up to 25, stay apart (0.690; the faster of both each time: 0.686).
+double chain_time(const ChainPlan& pl, int32_t L, const int32_t* widths, int64_t R, int32_t P) {
+  const int nr = P + 2, nb = pl.pb == 8 ? (nr + 1) / 2 : nr;
+  const int64_t by_lds = (160 << 10) / pl.lds;
+  const double per_cu = (double)(by_lds < 16 / pl.waves ? by_lds : 16 / pl.waves);
+  double rounds = (double)pl.blocks / (256.0 * per_cu);
+  if (rounds < 1.0) rounds = 1.0;
+  int chunks = 0, tiles = 0;
+  for (int l = 0; l < L; ++l) {
+    const int c = (widths[l] + 15) / 16;
+    chunks += c;
+    tiles += c * ((widths[l + 1] + 15) / 16);
+  }
+  return 2.3 + rounds * (1.06 * L + 0.094 * nb * chunks) + 0.155 * 4e-6 * (double)R * nr * (widths[0] + widths[L]) +
+         53.5e-6 * (double)R / 16 * nr * tiles;
+}
+
+double layers_time(int32_t L, const int32_t* widths, int64_t R, int32_t P) {
+  const int nr = P + 2;
+  double t = 0.0;
+  for (int l = 0; l < L; ++l) {
+    const int K = widths[l], N = widths[l + 1];
+    t += 2.74 + 0.155 * nr + 0.033 * N +
+         (double)R * nr * (0.176 * 4e-6 * (K + N) + 13.5e-9 * ((K + 7) / 8 * 8) * ((N + 15) / 16 * 16));
+  }
+  return t;
+}
+
 template <int NR, int PB>
 int launch_chain(hipStream_t st, const ChainParams& prm, const ChainPlan& pl) {
   if (pl.lds > 65536 &&
@@ -339,7 +374,12 @@ int launch_rows(hipStream_t st, const ChainParams& prm, const ChainPlan& pl) {
 extern "C" int folx_hip_dense_chain_faster(int32_t L, const int32_t* act, const int32_t* widths, int64_t R, int32_t P) {
   ChainPlan pl;
   if (L < 1 || !act || !widths || R <= 0 || P < 0) return FOLX_HIP_EINVAL;
-  return L > 1 && plan_chain(L, act, widths, R, P, pl) ? 1 : 0;
+  if (L < 2 || !plan_chain(L, act, widths, R, P, pl)) return 0;
+  // A layer whose input is no multiple of 4 wide is a product and a function on their own, which add in another order: the chain
+  // then, for any number of positions (of 174 such chains 5 were slower than their layers, by 8 to 19 %).
+  for (int l = 0; l < L; ++l)
+    if (widths[l] % 4 != 0) return 1;
+  return chain_time(pl, L, widths, R, P) < layers_time(L, widths, R, P) ? 1 : 0;
 }
 
 extern "C" int folx_hip_dense_chain_fwdlap(void* stream, int32_t L, const int32_t* act, const float* param,

@@ -219,6 +219,21 @@ def test_narrow_dense_act_takes_the_kernel_that_was_measured_faster(lib, R, P, K
     assert lib.folx_hip_dense_act_form(R, P, K, N, 1) == 2
 
 
+# chains of narrow layers: time in one launch over that of the layers one by one
+@pytest.mark.parametrize('R,P,widths,ratio', [
+    (2000, 4, (4, *[100] * 10, 1), 0.5), (25600, 4, (4, *[100] * 10, 1), 0.77), (100000, 6, (128,) * 7, 0.82),
+    (400, 1, (128, 4, 128), 0.54), (4000, 1, (128, 4, 128), 0.68), (40000, 1, (128, 4, 128), 1.26), (200000, 3, (128, 4, 128), 1.26),
+    (200000, 1, (128, 8, 8, 128), 1.72), (4000, 6, (128, 8, 8, 128), 0.64), (180793, 3, (128, 8, 4), 2.70), (37974, 6, (100, 4, 1), 1.83),
+    (123571, 2, (100, 8, 100), 1.67), (191836, 1, (48, 48, 4, 128), 1.50), (169064, 3, (128, 8, 16, 12, 16, 20, 128), 1.39),
+    (200000, 6, (4,) * 9, 0.61), (200000, 6, (16,) * 9, 0.39), (200000, 6, (32, 128, 32), 0.77),
+    (200000, 3, (3, 64, 64, 1), 0.48), (200000, 1, (5, 127, 3, 127, 1), 0.37),
+])
+def test_a_chain_is_taken_where_it_was_measured_faster(lib, R, P, widths, ratio):
+    act = (ctypes.c_int32 * (len(widths) - 1))(*[-1 if n == 1 else _lib.ACT['tanh'] for n in widths[1:]])
+    got = lib.folx_hip_dense_chain_faster(len(widths) - 1, act, (ctypes.c_int32 * len(widths))(*widths), R, P)
+    assert got == (1 if ratio < 1 else 0)
+
+
 def test_one_workspace_serves_both_product_modes(lib):
     before = lib.folx_hip_get_gemm_mode()
     forms, sizes = [], []
