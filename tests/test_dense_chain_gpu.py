@@ -131,3 +131,23 @@ def test_front_door_chains_what_nobody_else_reads():
         assert chains == ([2, 2] if twice else [4]), chains
         assert torch.equal(got.x, want.x) and torch.equal(got.laplacian, want.laplacian)
         assert torch.equal(got.jacobian.dense_array, want.jacobian.dense_array)
+
+
+def test_chain_with_a_large_tile_under_graph_replay():
+    """More than 64 KB of LDS (P = 6, 128 features, 16 positions a workgroup): every replay returns the bits of the eager call."""
+    print('case captured chain R=6200 P=6 128 x 128 x 128', flush=True)
+    t, layers = make(6200, 6, (128, 128, 128), ['tanh', 'silu'], 4)
+    layers = [(a, dev(W), dev(b), prm) for a, W, b, prm in layers]
+    t = [dev(v) for v in t]
+    K.dense_chain(layers, *t)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, _ = K.dense_chain(layers, *t)
+    for call in range(3):
+        for v in t:
+            v.mul_(1.1)
+        graph.replay()
+        torch.cuda.synchronize()
+        want, _ = K.dense_chain(layers, *t)
+        assert all(torch.equal(a, b) for a, b in zip(out, want)), call
