@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import hashlib
 import math
+import struct
 
 import numpy as np
 import torch
@@ -102,8 +103,8 @@ def device_const(arr, device) -> torch.Tensor:
 
 
 def scalar_const(value: float, device) -> torch.Tensor:
-    """One float32 number on the device, cached by its value."""
-    key = ('scalar', float(value), math.copysign(1.0, value), str(device))   # 0.0 and -0.0 are one dictionary key
+    """One float32 number on the device, cached by its bits (0.0 and -0.0 would be one key, every NaN another)."""
+    key = ('scalar', struct.pack('d', value), str(device))
     t = _CONST_CACHE.get(key)
     if t is None:
         t = torch.as_tensor(np.full((1,), value, dtype=np.float32)).to(device)

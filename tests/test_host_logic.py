@@ -1165,3 +1165,18 @@ def test_scan_and_fori_loop_run_as_python_loops(monkeypatch):
         check_against_oracle(with_loops, x, thr)
     out, ys2 = folx_amd.vmap(folx_amd.forward_laplacian(lambda t: model(fnp, t, fnp.scan, fnp.fori_loop), 0))(x)
     assert ys2 is None and tuple(out.shape) == ()
+
+
+def test_one_number_on_the_device_is_one_entry():
+    """NaN too; zeros of both signs keep theirs."""
+    import math
+
+    from folx_amd import sparse_ops as so
+
+    cpu = torch.device('cpu')
+    so.clear_caches()
+    for _ in range(3):
+        assert math.isnan(so.scalar_const(float('nan'), cpu).item()) and so.scalar_const(2.5, cpu).item() == 2.5
+        assert math.copysign(1.0, so.scalar_const(0.0, cpu).item()) == 1.0
+        assert math.copysign(1.0, so.scalar_const(-0.0, cpu).item()) == -1.0
+    assert len(so.cached_tensors()) == 4
