@@ -43,6 +43,17 @@ def dense_act(name, x, jac, lap, W, bias=None, param=0.0, res=None):
     return tuple(_t(a) for a in out)
 
 
+def dense_chain(layers, x, jac, lap, keep_hidden=False):
+    t, hidden = (_n(x), _n(jac), _n(lap)), None
+    for i, (name, W, b, prm) in enumerate(layers):
+        if keep_hidden and i + 1 == len(layers):
+            hidden = tuple(_t(a) for a in t)
+        t = rules.dense_rule(*t, _n(W), None if b is None else _n(b))
+        if name is not None:
+            t = rules.elementwise_rule({'sigmoid': 'logistic'}.get(name, name), *t, prm)
+    return tuple(_t(a) for a in t), hidden
+
+
 def dense_act_parts(name, x, lap, jac_parts, widths, broadcast, group, W, bias=None, param=0.0, res=None, pre=None):
     P = jac_parts[0].shape[0]
     lead = tuple(x.shape[:-1])
@@ -138,11 +149,26 @@ def rows_affine(inp, rows, row_shape, out_shape, c=None, d=None, alpha=1.0, beta
     return _t(np.broadcast_to(out, (rows, *out_shape)))
 
 
+def affine(x, jac, lap, row_shape, out_shape, c=None, d=None, alpha=1.0, beta=1.0):
+    from folx_amd import kernels as K
+
+    if K._affine_space(row_shape, out_shape, c, d) is None:   # where the product goes array by array
+        return None
+    P = jac.shape[0]
+    one = lambda t, rows, d_: rows_affine(t, rows, row_shape, out_shape, c, d_, alpha, beta)
+    return one(x, 1, d).reshape(out_shape), one(jac, P, None), one(lap, 1, None).reshape(out_shape)
+
+
 def reduce_sum(inp, rows, outer, red, inner, alpha=1.0, window=None):
     v = _n(inp).reshape(rows, outer, red, inner)
     if window is not None:
         v = v[:, :, window[0]:window[1]]
     return _t(alpha * v.sum(2))
+
+
+def reduce_sum_arrays(arrays, axes, alpha=1.0, window=None):
+    lo, hi = (0, arrays[0].shape[axes[0]]) if window is None else window
+    return [_t(alpha * _n(t).take(np.arange(lo, hi), ax).sum(ax)) for t, ax in zip(arrays, axes)]
 
 
 def reduce_max(inp, outer, red, inner):
@@ -281,15 +307,41 @@ def mhsa_sparse(q, qs, ql, k, ks, kl, v, vs, vl, index, P, all_rows_named):
                                                 _n(v), dense(vs), _n(vl)))
 
 
-KERNEL_NAMES = ('dense', 'dense_act', 'dense_act_parts', 'norm_dense', 'dot_two', 'dot_const', 'exp_envelope', 'layernorm', 'elementwise', 'binary',
-                'mul_sparse', 'rows_affine', 'reduce_sum', 'reduce_max', 'gather_rows', 'gather_reduce_rows', 'gather_cols', 'scatter_add_rows',
+KERNEL_NAMES = ('dense', 'dense_act', 'dense_chain', 'dense_act_parts', 'norm_dense', 'dot_two', 'dot_const', 'exp_envelope', 'layernorm', 'elementwise', 'binary',
+                'mul_sparse', 'rows_affine', 'affine', 'reduce_sum', 'reduce_sum_arrays', 'reduce_max', 'gather_rows', 'gather_reduce_rows', 'gather_cols', 'scatter_add_rows',
                 'slogdet', 'sparse_slogdet', 'slogdet_any', 'inv', 'inv_any', 'solve', 'mhsa', 'mhsa_sparse')
 
 
-def install(monkeypatch):
+def _affine_array_by_array(x, jac, lap, row_shape, out_shape, c=None, d=None, alpha=1.0, beta=1.0):
+    from folx_amd import kernels as K
+
+    if K._affine_space(row_shape, out_shape, c, d) is None:
+        return None
+    one = lambda t, rows, d_: K.rows_affine(t, rows, row_shape, out_shape, c, d_, alpha, beta)
+    return one(x, 1, d).reshape(out_shape), one(jac, jac.shape[0], None), one(lap, 1, None).reshape(out_shape)
+
+
+def _sums_array_by_array(arrays, axes, alpha=1.0, window=None):
+    from folx_amd import kernels as K
+
+    def one(t, ax):
+        before, after = t.shape[:ax], t.shape[ax + 1:]
+        out = K.reduce_sum(t, 1, int(np.prod(before)), t.shape[ax], int(np.prod(after)), alpha, window)
+        return out.reshape(*before, *after)
+
+    return [one(t, ax) for t, ax in zip(arrays, axes)]
+
+
+def install(monkeypatch, chains=False):
+    """The stand-ins in the product's place.  Launches that serve several rules at once are taken apart into those (what the tests
+    of the front end count): triplets into their arrays and, unless ``chains``, chains of layers into layers."""
     import folx_amd.interpreter as interp
     import folx_amd.kernels as K
 
     for name in KERNEL_NAMES:
         monkeypatch.setattr(K, name, globals()[name])
+    monkeypatch.setattr(K, 'affine', _affine_array_by_array)
+    monkeypatch.setattr(K, 'reduce_sum_arrays', _sums_array_by_array)
+    if not chains:
+        monkeypatch.setattr(K, 'dense_chain_faster', lambda layers, R, P: False)
     monkeypatch.setattr(interp, '_device', lambda: torch.device('cpu'))

@@ -786,6 +786,36 @@ def test_stagecheck_runs_every_kernel_call_against_its_fp64_rule():
         K.elementwise = good
 
 
+@pytest.mark.parametrize('name', ['affine', 'reduce_sum_arrays', 'dense_chain'])
+def test_stagecheck_sees_launches_that_serve_several_rules(name):
+    import folx_amd.kernels as K
+    from stagecheck import StageCheck
+
+    g = np.random.default_rng(0)
+    t = [torch.as_tensor(g.normal(size=s).astype(np.float32)) for s in ((5, 8), (3, 5, 8), (5, 8))]
+    W = torch.as_tensor(g.normal(size=(8, 8)).astype(np.float32))
+    call = {'affine': lambda: K.affine(*t, (5, 8), (5, 8), None, None, 0.7, 0.0),
+            'reduce_sum_arrays': lambda: K.reduce_sum_arrays(t, [1, 2, 1], 0.5, (2, 7)),
+            'dense_chain': lambda: K.dense_chain([('tanh', W, None, 0.0), ('silu', W, None, 0.0), (None, W[:, :1], None, 0.0)], *t, True)}[name]
+    with StageCheck() as sc:
+        call()
+    assert sc.summary()[name][0] == 1
+    good = getattr(K, name)
+    for at in range(3):                                    # each array of the result is looked at
+        def bad(*a, **k):
+            out = good(*a, **k)
+            arrays = list(out[0] if name == 'dense_chain' else out)
+            arrays[at] = arrays[at] * (1 + 1e-3)
+            return (tuple(arrays), out[1]) if name == 'dense_chain' else arrays
+
+        setattr(K, name, bad)
+        try:
+            with pytest.raises(AssertionError, match=name), StageCheck():
+                call()
+        finally:
+            setattr(K, name, good)
+
+
 @pytest.mark.parametrize('thr', [0, 6])
 def test_forward_laplacian_of_several_arguments(thr):
     """Two differentiated array arguments share one index space, numbered in argument order

@@ -290,6 +290,21 @@ def test_full_width_well_conditioned_end_to_end_strict(name):
         np.testing.assert_allclose(g, want, rtol=rtol, atol=max(atol, floor), err_msg=f'{name} {nm}')
 
 
+def test_narrow_layers_every_rule_call_meets_the_strict_bars():
+    """The node-wise MLP with its sparse Jacobian stage by stage: sums of triplets, scalings, and its layers as one launch."""
+    from stagecheck import StageCheck
+
+    forward, p, cfg, _, _, thr = wl.build('mlp_sparse')
+    x = wl.sample_inputs('mlp_sparse', 2, seed=2)
+    print('case mlp_sparse stage by stage', flush=True)
+    with StageCheck() as sc:
+        run(lambda xp, t: xp.multiply(forward(p, t, xp), 0.5), x, thr)
+    used = sc.summary()
+    print(used, flush=True)
+    assert {'dense_chain', 'reduce_sum_arrays', 'affine'} <= set(used), used
+    assert all(w <= 1.0 for _, w, _ in used.values())
+
+
 @pytest.mark.parametrize('name,chunk', [('psiformer64', 256), ('ferminet16', 1024)])
 def test_full_batch_properties(name, chunk):
     """psiformer64 at its 1024 walkers in chunks of 256 and ferminet16 at its 4096: finite
