@@ -247,7 +247,7 @@ def _affine_const(t: FwdLaplArray, c, *, mul: bool, alpha: float, beta: float) -
             ct = None
     full = (B, *out_shape)
     same = out_shape == t.shape and ct is None and a_j == 1.0
-    if not same and t.x.is_cuda:   # value, Jacobian rows and Laplacian in one launch
+    if not same:   # value, Jacobian rows and Laplacian in one launch
         got = K.affine(t.x, t.jacobian.data, t.laplacian, (B, *t.shape), full, ct, d_t, a_x, b_x)
         if got is not None:
             return FwdLaplArray(got[0], FwdJacobian(got[1], _bmask(t.jacobian.x0_idx, k, out_shape)), got[2])
@@ -984,7 +984,7 @@ def _evaluate_chain(last, residual):
 def _chain_launch(h: FwdLaplArray, nodes, keep: bool):
     """``nodes`` over ``h`` in one launch: (last triplet, the one in front of it if ``keep``), or None where the layers go
     one by one."""
-    if not h.x.is_cuda or any(np.shape(d.W)[0] != k for d, k in zip(nodes, (h.shape[-1], *[d.shape[-1] for d in nodes[:-1]]))):
+    if any(np.shape(d.W)[0] != k for d, k in zip(nodes, (h.shape[-1], *[d.shape[-1] for d in nodes[:-1]]))):
         return None
     J, mask = h.jacobian.data, h.jacobian.x0_idx
     proj, aligned = None, False
@@ -1226,9 +1226,7 @@ def _reduce_tensor(t: torch.Tensor, lead: int, axes, alpha=1.0, window=None) -> 
 
 
 def _reduce_tensors(ts, leads, axes, alpha=1.0, window=None):
-    """``_reduce_tensor`` of several arrays with the same logical axes, on the GPU in one launch an axis."""
-    if not ts[0].is_cuda:
-        return [_reduce_tensor(t, lead, axes, alpha, window) for t, lead in zip(ts, leads)]
+    """``_reduce_tensor`` of several arrays with the same logical axes, in one launch an axis."""
     for ax in sorted(axes, reverse=True):
         ts = K.reduce_sum_arrays([t.contiguous() for t in ts], [ax + lead for lead in leads], alpha, window)
         alpha = 1.0

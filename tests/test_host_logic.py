@@ -1210,3 +1210,83 @@ def test_one_number_on_the_device_is_one_entry():
         assert math.copysign(1.0, so.scalar_const(0.0, cpu).item()) == 1.0
         assert math.copysign(1.0, so.scalar_const(-0.0, cpu).item()) == -1.0
     assert len(so.cached_tensors()) == 4
+
+
+_CW = [np.random.default_rng(30 + i).normal(size=s).astype(np.float32) / 2 for i, s in enumerate(((4, 12), (12, 12), (12, 7), (7, 12), (12, 1), (12, 1)))]
+_CB = np.linspace(-1, 1, 12).astype(np.float32)
+
+
+def _layers(xp, h, *Ws):
+    for W in Ws:
+        h = xp.silu(xp.dot(h, W))
+    return h
+
+
+def _chain_read_twice(xp, x):
+    h = _layers(xp, x, *_CW[:2])
+    return xp.add(xp.sum(_layers(xp, h, _CW[2])), xp.sum(h))
+
+
+def _chain_two_vectors(xp, x):        # what the first one reads is handed back for the second
+    h = _layers(xp, x, *_CW[:2])
+    return xp.add(xp.sum(xp.dot(h, _CW[4])), xp.sum(xp.tanh(xp.dot(h, _CW[5]))))
+
+
+def _chain_with_skip(xp, x):
+    h = _layers(xp, x, _CW[0])
+    return xp.sum(xp.add(_layers(xp, h, _CW[1]), h))
+
+
+def _chain_of_a_slice(xp, x):
+    return xp.sum(_layers(xp, xp.getitem(_layers(xp, x, _CW[0]), (slice(0, 2),)), _CW[1], _CW[2]))
+
+
+def _chain_through_a_reshape(xp, x):
+    return xp.sum(_layers(xp, xp.reshape(_layers(xp, x, _CW[0], _CW[1]), (1, -1, 12)), _CW[2], _CW[3]))
+
+
+def _chain_over_mixed_coordinates(xp, x):   # rows of several nodes at a position
+    return xp.sum(_layers(xp, xp.multiply(x, xp.flip(x, 0)), *_CW[:3]))
+
+
+# (function, layers in each launch with 4 to 6 Jacobian rows; None: it depends)
+CHAINS = {
+    'plain': (lambda xp, x: xp.sum(xp.add(xp.dot(_layers(xp, x, *_CW[:2]), _CW[4]), 0.3)), [3]),
+    'no_vector': (lambda xp, x: xp.sum(_layers(xp, x, *_CW[:4])), [4]),
+    'bias': (lambda xp, x: xp.sum(xp.tanh(xp.add(xp.dot(_layers(xp, x, _CW[0]), _CW[1]), _CB))), [2]),
+    'read_twice': (_chain_read_twice, [2]),
+    'two_vectors': (_chain_two_vectors, [3]),
+    'with_skip': (_chain_with_skip, []),
+    'of_a_slice': (_chain_of_a_slice, []),
+    'through_a_reshape': (_chain_through_a_reshape, [3]),
+    'over_mixed_coordinates': (_chain_over_mixed_coordinates, None),
+    'no_function': (lambda xp, x: xp.sum(xp.dot(xp.dot(x, _CW[0]), _CW[1])), []),
+    'too_wide': (lambda xp, x: xp.sum(_layers(xp, x, np.tile(_CW[0], (1, 11)), np.tile(_CW[1], (11, 1)))), []),
+}
+
+
+@pytest.mark.parametrize('nodes,thr', [(3, 6), (3, 4), (3, 0), (1, 0)])
+@pytest.mark.parametrize('name', CHAINS)
+def test_chains_of_narrow_layers(monkeypatch, name, nodes, thr):
+    """What becomes one launch, what is handed back to others, how sparse rows enter: the same results as layer by layer."""
+    import folx_amd.kernels as K
+
+    fn, taken = CHAINS[name]
+    nodes = max(nodes, 2) if name == 'of_a_slice' else nodes
+    x = np.random.default_rng(8).normal(size=(2, nodes, 4)).astype(np.float32)
+    want = run_product(fn, x, thr)
+    monkeypatch.undo()                              # the stand-ins of the other tests, which take chains apart
+    cpu_kernels.install(monkeypatch, chains=True)
+    launches, one = [], K.dense_chain
+    monkeypatch.setattr(K, 'dense_chain', lambda layers, *a: (launches.append(len(layers)), one(layers, *a))[1])
+    got = run_product(fn, x, thr)
+    if taken is not None and (thr >= 4 or nodes == 1):
+        assert launches == taken, launches
+    if thr == 0 and nodes == 3:
+        assert not launches                         # 12 Jacobian rows
+    assert got.jacobian.weak == want.jacobian.weak
+    if got.jacobian.weak:
+        assert np.array_equal(got.jacobian.x0_idx, want.jacobian.x0_idx)
+    for a, b in ((got.x, want.x), (got.jacobian.dense_array, want.jacobian.dense_array), (got.laplacian, want.laplacian)):
+        # every rule's result is rounded to 32 bits layer by layer, once in a chain
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5 * float(b.abs().max()))
