@@ -243,7 +243,6 @@ extern "C" int folx_hip_gather_rows(void* stream, const float* data, const int32
   if (k_out == 0 || B == 0 || S == 0) return FOLX_HIP_OK;
   if (!out || (n_slots > 0 && (!take || (k_in > 0 && !data)))) return FOLX_HIP_EINVAL;
   if (k_out > 65535) return FOLX_HIP_ENOTSUP;
-  if (B > 8 * 65535LL) return FOLX_HIP_ENOTSUP;
   const bool vec = (S_inner % 4 == 0) && folx_aligned16(data) && folx_aligned16(out);
   const int64_t blocks = (B * S + (vec ? 1023 : 255)) / (vec ? 1024 : 256);
   if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;

@@ -273,7 +273,7 @@ __global__ __launch_bounds__(NT, 4) void mhsa_sparse_kernel(SAArgs a) {
     // alpha[e][s][j] = a_es . k[j],  beta[e][s][i] = q[i] . b_es,  gp[e][s] = a_es . b_es
     sa_products_nt<NT>(aS, dp, ne * K, kS, dp, n, bS, dp, ne * K, qS, dp, n, d4, tid,
                    [&](bool beta, int es, int x, float v) { (beta ? beS : alS)[es * n + x] = v; });
-    if (tid >= NT - ne * K) {  // the last wavefront has no tile when n <= 48
+    if (tid >= NT - ne * K) {  // of 512 threads the last wavefront has no tile when n <= 48; of fewer it goes on behind its tiles
       const int es = NT - 1 - tid;
       gpS[es] = sa_dot(aS + es * dp, bS + es * dp, d4);
     }

@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize('k_in,k_out,n_slots,B,S_outer,S_inner', [
     (2, 1, 1, 1, 1, 1), (3, 3, 5, 7, 3, 4), (3, 4, 4, 5, 3, 4), (3, 5, 3, 5, 3, 3), (1, 7, 1, 257, 1, 1), (4, 9, 2, 33, 4, 8),
     (3, 8, 9, 20, 11, 1), (2, 3, 4, 3, 2, 6), (3, 66, 1, 64, 5, 64), (0, 5, 1, 3, 2, 4), (3, 6, 0, 3, 2, 4),
+    (2, 5, 2, 524281, 1, 3), (1, 1, 1, 600000, 1, 4),                       # more walkers than 8 x 65535
 ])
 def test_gather_rows_in_slot_order(k_in, k_out, n_slots, B, S_outer, S_inner):
     print(f'case gather k {k_in} -> {k_out} slots {n_slots} B={B} S={S_outer} x {S_inner}', flush=True)
