@@ -130,6 +130,12 @@ def clear_caches():
     index_algebra._BY_IDENTITY.clear()
 
 
+def aligned(t: torch.Tensor) -> torch.Tensor:
+    """``t``, or a copy of it where it starts off a 16-byte boundary (a caller's view into a larger array): what kernels with
+    128-bit loads only need."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def zeros(shape, device) -> torch.Tensor:
     """Zero tensor produced by a fill kernel (never by a memset node, so that the call can
     sit inside a captured HIP graph)."""

@@ -2005,9 +2005,8 @@ def mhsa_forward_laplacian(args, kwargs, sparsity_threshold):
         sparse = _position_sparse_index(q, k, v)
         if sparse is not None:
             index, P, all_named = sparse
-            o, oj, ol = K.mhsa_sparse(
-                q.x, q.jacobian.data, q.laplacian, k.x, k.jacobian.data, k.laplacian, v.x, v.jacobian.data,
-                v.laplacian, so.device_table(index, dev), P, all_named)
+            flat = [so.aligned(a) for t in (q, k, v) for a in (t.x, t.jacobian.data, t.laplacian)]
+            o, oj, ol = K.mhsa_sparse(*flat, so.device_table(index, dev), P, all_named)
             return FwdLaplArray(o, FwdJacobian(oj, None), ol)
     trip = (q, k, v) if bias is None else (q, k, v, bias)
     Js = [t.jacobian.dense_array for t in trip]
@@ -2026,7 +2025,8 @@ def mhsa_forward_laplacian(args, kwargs, sparsity_threshold):
         assert im.shape[0] == P, 'input_mask must have one entry per Jacobian row'
         it = _mask_tensor(im, (P, B), dev)
     edge = None if bias is None else (bias.x, Js[3], bias.laplacian)
-    o, oj, ol = K.mhsa(q.x, Js[0], q.laplacian, k.x, Js[1], k.laplacian, v.x, Js[2], v.laplacian, mt, it, edge)
+    flat = [so.aligned(a) for t, J in zip((q, k, v), Js) for a in (t.x, J, t.laplacian)]
+    o, oj, ol = K.mhsa(*flat, mt, it, edge)
     return FwdLaplArray(o, FwdJacobian(oj, None), ol)
 
 

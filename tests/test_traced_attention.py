@@ -180,3 +180,18 @@ def test_a_trace_that_fails_to_finish_is_not_kept(monkeypatch):
     want = fx.forward_laplacian_torch(matmul, 0).batched(x)
     got = traced.batched(x)
     assert torch.equal(got.x, want.x) and torch.equal(got.laplacian, want.laplacian)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n,thr', [(3, 0), (5, 0), (5, 4)])
+def test_attention_on_operands_off_a_16_byte_boundary(n, thr):
+    """Queries, keys and values read from a view into a larger array: the results of an array of their own."""
+    import folx_amd
+
+    print(f'case attention off the boundary n={n} thr={thr}', flush=True)
+    fl = folx_amd.vmap(folx_amd.forward_laplacian_torch(lambda x: softmax(x @ x.T / 2) @ x, thr))
+    buffer = torch.randn(3 * n * 4 + 1, device='cuda', generator=torch.Generator(device='cuda').manual_seed(0))
+    x = buffer[1:].reshape(3, n, 4)
+    got, want = fl(x), fl(x.clone())
+    assert torch.equal(got.x, want.x) and torch.equal(got.laplacian, want.laplacian)
+    assert torch.equal(got.jacobian.dense_array, want.jacobian.dense_array)
