@@ -664,6 +664,7 @@ def _dot_then_act(h, W, kwargs, thr: int):
         if k_pad:
             padk = lambda t: torch.nn.functional.pad(t, (0, k_pad))
             hx, J, hl = padk(hx), padk(J), padk(hl)
+        hx, J, hl = so.aligned(hx), so.aligned(J), so.aligned(hl)
         if (_is(residual) and K.dense_act_residual_supported(*np.shape(W))
                 and tuple(residual.shape) == (*h.shape[:-1], np.shape(W)[1])
                 and residual.jacobian.data.shape[0] == J.shape[0]):

@@ -133,6 +133,25 @@ def test_front_door_chains_what_nobody_else_reads():
         assert torch.equal(got.jacobian.dense_array, want.jacobian.dense_array)
 
 
+@pytest.mark.parametrize('B,widths', [(3, (4, 100)), (3, (4, 24, 24)), (8000, (4, 4, 128))])
+def test_layers_of_an_input_off_a_16_byte_boundary(B, widths):
+    """One layer, layers in one launch, layers whose chain would be slower: the results of an aligned array."""
+    print(f'case layers off the boundary B={B} widths={widths}', flush=True)
+    g = torch.Generator(device='cuda').manual_seed(5)
+    Ws = [torch.randn(a, b, device='cuda', generator=g) / a ** 0.5 for a, b in zip(widths, widths[1:])]
+
+    def fn(r):
+        for W in Ws:
+            r = fnp.tanh(fnp.dot(r, W))
+        return fnp.sum(r)
+
+    fl = folx_amd.vmap(folx_amd.forward_laplacian(fn, 4))
+    x = torch.randn(B * 50 * 4 + 1, device='cuda', generator=g)[1:].reshape(B, 50, 4)
+    got, want = fl(x), fl(x.clone())
+    assert torch.equal(got.x, want.x) and torch.equal(got.laplacian, want.laplacian)
+    assert torch.equal(got.jacobian.dense_array, want.jacobian.dense_array)
+
+
 def test_chain_with_a_large_tile_under_graph_replay():
     """More than 64 KB of LDS (P = 6, 128 features, 16 positions a workgroup): every replay returns the bits of the eager call."""
     print('case captured chain R=6200 P=6 128 x 128 x 128', flush=True)
