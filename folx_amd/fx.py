@@ -918,8 +918,8 @@ def _steps(gm: torch.fx.GraphModule):
 def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None, steps=None, on_device=None):
     """One pass over the equations of a traced graph (folx/interpreter.py:218-264): constant equations come from
     ``fold_constants``, the others go through ``RULES``.  Who evaluates a graph often and changes it no more keeps both,
-    ``consts`` and ``steps`` (``_steps``).  ``on_device``: device copies of some constants, for the equations in
-    ``_DEVICE_READERS`` that meet a triplet; all others take the constants as they are."""
+    ``consts`` and ``steps`` (``_steps``).  ``on_device``: for some equations, the positions of operands to look at and
+    ``(position, device copy)`` of constants, which are taken where one of those is a triplet."""
     env = dict(fold_constants(gm) if consts is None else consts)
     it = iter(inputs)
     look = lambda a: env[a] if isinstance(a, torch.fx.Node) else a
@@ -937,8 +937,11 @@ def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None, steps=None, on
             env[node] = next(it)
         elif step.op == 'call_function':
             args = [take(kind, a) for kind, a in step.args]
-            if on_device and step.target in _DEVICE_READERS and any(fnp._is_triplet(a) for a in args):
-                args = [on_device.get(a, v) if kind == 1 else v for (kind, a), v in zip(step.args, args)]
+            if on_device and node in on_device:
+                others, copies = on_device[node]
+                if any([fnp._is_triplet(args[i]) for i in others]):
+                    for i, copy in copies:
+                        args[i] = copy
             kwargs = {k: take(kind, a) for k, kind, a in step.kwargs}
             rule = RULES.get(step.target)
             functional = _functional_form(node.target) if rule is None else None
@@ -1055,17 +1058,26 @@ class TracedForwardLaplacian(ForwardLaplacianFn):
         return gm
 
     def _on_device(self, shapes, device):
-        """Device copies of the constants that sums, products and weights read, made once per device."""
+        """``evaluate_graph``'s device copies of the constants that sums, products and weights read, made once per device."""
         key = (shapes, str(device))
         hit = self.constants.get(key)
         if hit is None:
-            def wanted(n, v):
-                if not (isinstance(v, np.ndarray) and v.dtype == np.float32 and v.ndim >= 1):
-                    return False
-                return any(u.target in _OPERAND_READERS or (u.target in _WEIGHT_READERS and v.size >= _DEVICE_CONST_MIN) for u in n.users)
-
-            hit = self.constants[key] = {n: torch.as_tensor(np.ascontiguousarray(v)).to(device)
-                                         for n, v in self.constants[shapes].items() if wanted(n, v)}
+            consts, tensors, hit = self.constants[shapes], {}, {}
+            for node in self.graphs[shapes].graph.nodes:
+                if node in consts or node.target not in _DEVICE_READERS:
+                    continue
+                least = 1 if node.target in _OPERAND_READERS else _DEVICE_CONST_MIN
+                copies = []
+                for i, a in enumerate(node.args):
+                    v = consts.get(a) if isinstance(a, torch.fx.Node) else None
+                    if isinstance(v, np.ndarray) and v.dtype == np.float32 and v.ndim >= 1 and v.size >= least:
+                        if a not in tensors:
+                            tensors[a] = torch.as_tensor(np.ascontiguousarray(v)).to(device)
+                        copies.append((i, tensors[a]))
+                if copies:
+                    others = [i for i, a in enumerate(node.args) if isinstance(a, torch.fx.Node) and a not in consts]
+                    hit[node] = others, copies
+            self.constants[key] = hit
         return hit
 
     def _run(self, *lapl_args):
