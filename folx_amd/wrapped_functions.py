@@ -657,7 +657,7 @@ def _dot_then_act(h, W, kwargs, thr: int):
         W = W[:K_in]
     if fused:
         dev = h.x.device
-        Wt = so.device_const(W, dev)
+        Wt = so.aligned(so.device_const(W, dev))
         bt = None if bias is None else so.device_const(bias, dev)
         res = None
         hx, hl = h.x, h.laplacian
@@ -1100,8 +1100,8 @@ def _dot_parts(lc: LazyConcat, W, kwargs, thr: int):
     res = None  # a skip connection with the same dense rows goes into the kernel's epilogue
     if (_is(residual) and residual.jacobian.x0_idx is None and residual.jacobian.data.shape[0] == P
             and tuple(residual.shape) == (*lead, np.shape(W)[1])):
-        res = (residual.x.contiguous(), residual.jacobian.data.contiguous(), residual.laplacian.contiguous())
-    Wt = so.device_const(W, dev)
+        res = tuple(so.aligned(t.contiguous()) for t in (residual.x, residual.jacobian.data, residual.laplacian))
+    Wt = so.aligned(so.device_const(W, dev))
     w_const = not isinstance(W, torch.Tensor)  # a numpy constant: its device copy is never written again
     bt = None if bias is None else so.device_const(bias, dev)
     is_b = [isinstance(t, LazyBroadcast) for t in lc.parts]

@@ -8,7 +8,9 @@ import torch
 from oracle import rules
 from tolerances import assert_lap, assert_val
 
+import folx_amd
 from folx_amd import kernels as K
+from folx_amd import numpy as fnp
 
 pytestmark = pytest.mark.gpu
 dev = lambda v: torch.as_tensor(np.asarray(v, dtype=np.float32)).cuda()
@@ -62,3 +64,32 @@ def test_gelu_far_from_zero(name, P, k, n):
     for a, want in zip(got, (y, d, d)):
         a = a.cpu().numpy()
         np.testing.assert_array_equal(a, np.broadcast_to(want, a.shape))
+
+
+def off_the_boundary(t):
+    """``t`` as a view into a larger array, 4 bytes behind a 16-byte boundary."""
+    view = torch.empty(t.numel() + 1, device='cuda')[1:].reshape(t.shape)
+    return view.copy_(t)
+
+
+@pytest.mark.parametrize('k,n', [(4, 16), (32, 132), (20, 160), (256, 256)])
+def test_gelu_layer_of_arrays_off_a_16_byte_boundary(k, n):
+    """Weights, a skip connection and the input itself that a caller reads from a larger array: the results of aligned ones."""
+    print(f'case gelu layer off the boundary {k} x {n}', flush=True)
+    g = torch.Generator(device='cuda').manual_seed(k)
+    rn = lambda *s: torch.randn(*s, device='cuda', generator=g)
+    x, W, W2, b = rn(12, 4, k), rn(k, n) / k ** 0.5, rn(n + 32, k) / n ** 0.5, rn(n)
+
+    def model(x, W, W2, b):
+        h = fnp.gelu(fnp.add(fnp.dot(x, W), b), approximate=False)
+        # a layer that reads a concatenation in parts where it is wide, with the input as its skip connection
+        parts = fnp.concatenate([h, fnp.tanh(fnp.dot(x, W[:, :16].contiguous())), fnp.tanh(fnp.dot(x, W[:, -16:].contiguous()))], axis=-1)
+        return fnp.add(x, fnp.gelu(fnp.dot(parts, W2)))
+
+    run = lambda x, *weights: folx_amd.vmap(folx_amd.forward_laplacian(lambda t: model(t, *weights), 0))(x)
+    want = run(x, W, W2, b)
+    for at in range(4):
+        got = run(*[off_the_boundary(t) if i == at else t for i, t in enumerate((x, W, W2, b))])
+        for u, v in ((got.x, want.x), (got.jacobian.dense_array, want.jacobian.dense_array), (got.laplacian, want.laplacian)):
+            # the plain product of unaligned operands adds in another order
+            torch.testing.assert_close(u, v, rtol=1e-4, atol=1e-5 * float(v.abs().max()))
