@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/folx_hip.h"
 
 #define FOLX_WAVE 64
@@ -10,6 +12,21 @@
 static inline int folx_launch_status() {
   return hipGetLastError() == hipSuccess ? FOLX_HIP_OK : FOLX_HIP_ELAUNCH;
 }
+
+// The permission that a kernel needs for more than 64 KB of dynamic LDS: asked for once per device (the runtime keeps it for the
+// current one only), not on every launch and not inside every stream capture.
+struct FolxLdsGrant {
+  std::atomic<uint64_t> devices{0};
+  bool ask(const void* kernel, int bytes) {
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return false;
+    const uint64_t bit = dev < 64 ? 1ull << dev : 0;
+    if (devices.load() & bit) return true;
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return false;
+    devices.fetch_or(bit);
+    return true;
+  }
+};
 
 static inline bool folx_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

@@ -27,8 +27,6 @@
 // Weights through a descriptor and operands one chunk ahead: 8 to 14 % of the time.  80 registers for a third workgroup a
 // CU spilled 70 of them (429 -> 631 us).  us, layers one by one -> chain: ten layers of 100, P = 4: 2000 positions
 // 101 -> 43, 25 600 503 -> 390; four of 50, P = 3, 15 750: 106 -> 31; six of 128, P = 6, 100 000: 1408 -> 1156.
-#include <atomic>
-
 #include "activations.h"
 
 namespace {
@@ -359,14 +357,8 @@ double layers_time(int32_t L, const int32_t* widths, int64_t R, int32_t P) {
 template <int NR, int PB>
 int launch_chain(hipStream_t st, const ChainParams& prm, const ChainPlan& pl) {
   if (pl.lds > 65536) {
-    // once per process, not on every launch and not inside every stream capture
-    static std::atomic<bool> granted{false};
-    if (!granted.load()) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_chain_kernel<NR, PB>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
-        return FOLX_HIP_ELAUNCH;
-      granted.store(true);
-    }
+    static FolxLdsGrant grant;
+    if (!grant.ask(reinterpret_cast<const void*>(&dense_chain_kernel<NR, PB>), 160 * 1024)) return FOLX_HIP_ELAUNCH;
   }
   dense_chain_kernel<NR, PB><<<dim3((unsigned)pl.blocks), dim3(64 * pl.waves), pl.lds, st>>>(prm);
   return folx_launch_status();

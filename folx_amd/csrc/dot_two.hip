@@ -21,7 +21,6 @@
 // operand is one 128-bit LDS read per four MFMAs.
 //
 // Up to 32 x 32 x 32 nothing has to be shared: dot_two_small_kernel (its mapping stands there).
-#include <atomic>
 
 #include "common.h"
 
@@ -432,16 +431,10 @@ extern "C" int folx_hip_dot_two_fwdlap(void* stream, const float* a, const float
     else dot_two_kernel<8, false><<<grid, block, lds, st>>>(g);
   } else {
     if (lds > 64 * 1024) {
-      // raised once per process (not a stream operation, so never issued inside a stream capture twice)
-      static std::atomic<bool> granted{false};
-      if (!granted.load()) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(dot_two_kernel<16, false>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess ||
-            hipFuncSetAttribute(reinterpret_cast<const void*>(dot_two_kernel<16, true>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess)
-          return FOLX_HIP_ENOTSUP;
-        granted.store(true);
-      }
+      static FolxLdsGrant grant[2];
+      const void* kernel = constb ? reinterpret_cast<const void*>(dot_two_kernel<16, true>)
+                                  : reinterpret_cast<const void*>(dot_two_kernel<16, false>);
+      if (!grant[constb ? 1 : 0].ask(kernel, 96 * 1024)) return FOLX_HIP_ENOTSUP;
     }
     if (constb) dot_two_kernel<16, true><<<grid, block, lds, st>>>(g);
     else dot_two_kernel<16, false><<<grid, block, lds, st>>>(g);

@@ -23,7 +23,6 @@
 // different rows cover all banks); the n x n x d products (scores, alpha, beta, the Laplacian's
 // score term) run on the matrix cores from those rows, the sums over j on 128-bit LDS reads; the
 // vectors of the next group of positions are fetched while the current one is worked on.
-#include <atomic>
 
 #include "common.h"
 
@@ -450,15 +449,8 @@ __global__ __launch_bounds__(NT, 4) void mhsa_sparse_kernel(SAArgs a) {
 template <int NT, int RL, int NP>
 int launch_sa(hipStream_t st, const SAArgs& a, size_t lds) {
   if (lds > 64 * 1024) {
-    // raised once per process to the largest size asked for so far (not a stream operation,
-    // and then never issued again inside a stream capture)
-    static std::atomic<size_t> granted{0};
-    if (lds > granted.load()) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(mhsa_sparse_kernel<NT, RL, NP>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
-        return FOLX_HIP_ENOTSUP;
-      granted.store(160 * 1024);
-    }
+    static FolxLdsGrant grant;
+    if (!grant.ask(reinterpret_cast<const void*>(mhsa_sparse_kernel<NT, RL, NP>), 160 * 1024)) return FOLX_HIP_ENOTSUP;
   }
   mhsa_sparse_kernel<NT, RL, NP><<<dim3((unsigned)(a.B * a.H)), dim3(NT), lds, st>>>(a);
   return folx_launch_status();

@@ -258,3 +258,36 @@ def test_questions_about_a_shape(lib):
     assert tile(1550, 100, 256, 256) == 128 and tile(3000, 98, 512, 100) == 128
     assert tile(64, 3, 32, 64) == tile(64, 3, 40, 128) == tile(64, 3, 32, 130) == _lib.ENOTSUP
     assert form(-1, 4, 100, 100, 0) == faster(64, 33, 256, 256, 0) == _lib.EINVAL
+
+
+def test_lds_permission_is_asked_for_once_per_device(tmp_path):
+    """The helper on the host, with the two runtime calls it makes replaced: a second device of the process asks for itself."""
+    import subprocess
+
+    from folx_amd import build
+
+    (tmp_path / 'grant.hip').write_text(r'''
+#include "common.h"
+static int device = 0, asked = 0;
+static hipError_t answer = hipSuccess;
+extern "C" hipError_t hipGetDevice(int* d) { *d = device; return hipSuccess; }
+extern "C" hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { ++asked; return answer; }
+int main() {
+  FolxLdsGrant g;
+  answer = hipErrorInvalidValue;
+  if (g.ask(&g, 1) || asked != 1) return 1;                                  // refused: asked again
+  answer = hipSuccess;
+  if (!g.ask(&g, 1) || !g.ask(&g, 1) || asked != 2) return 2;
+  device = 3;
+  if (!g.ask(&g, 1) || !g.ask(&g, 1) || asked != 3) return 3;
+  device = 0;
+  if (!g.ask(&g, 1) || asked != 3) return 4;
+  device = 64;                                                               // beyond the mask: every time
+  if (!g.ask(&g, 1) || !g.ask(&g, 1) || asked != 5) return 5;
+  return 0;
+}
+''')
+    exe = str(tmp_path / 'grant')
+    subprocess.run([build._hipcc(), '--offload-arch=gfx950', '-I', build.CSRC, '-x', 'hip', str(tmp_path / 'grant.hip'), '-o', exe],
+                   check=True, capture_output=True)
+    assert subprocess.run([exe]).returncode == 0
