@@ -24,6 +24,7 @@ from . import numpy as fnp
 from .api import BatchedArray, FwdLaplArray
 from .fx_attention import attention, fuse_attention
 from .interpreter import ForwardLaplacianFn
+from .wrapped_functions import Deferred
 
 aten = torch.ops.aten
 
@@ -56,8 +57,6 @@ def multi_head_self_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor)
 
 
 def _is_t(v):
-    from .wrapped_functions import Deferred
-
     return isinstance(v, (FwdLaplArray, BatchedArray, Deferred))
 
 
@@ -921,6 +920,7 @@ def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None, steps=None, on
     ``consts`` and ``steps`` (``_steps``).  ``on_device``: for some equations, the positions of operands to look at and
     ``(position, device copy)`` of constants, which are taken where one of those is a triplet."""
     env = dict(fold_constants(gm) if consts is None else consts)
+    on_device = on_device or {}
     it = iter(inputs)
     look = lambda a: env[a] if isinstance(a, torch.fx.Node) else a
     take = lambda kind, a: a if kind == 0 else (env[a] if kind == 1 else torch.fx.node.map_arg(a, look))   # noqa: E731
@@ -937,11 +937,13 @@ def evaluate_graph(gm: torch.fx.GraphModule, inputs, consts=None, steps=None, on
             env[node] = next(it)
         elif step.op == 'call_function':
             args = [take(kind, a) for kind, a in step.args]
-            if on_device and node in on_device:
-                others, copies = on_device[node]
-                if any([fnp._is_triplet(args[i]) for i in others]):
-                    for i, copy in copies:
-                        args[i] = copy
+            at_hand = on_device.get(node)
+            if at_hand is not None:
+                for i in at_hand[0]:
+                    if isinstance(args[i], (FwdLaplArray, Deferred)):
+                        for j, copy in at_hand[1]:
+                            args[j] = copy
+                        break
             kwargs = {k: take(kind, a) for k, kind, a in step.kwargs}
             rule = RULES.get(step.target)
             functional = _functional_form(node.target) if rule is None else None
