@@ -50,8 +50,7 @@ def parse():
     ap.add_argument('--cpu-seconds', type=float, default=20.0, help='budget of the CPU baseline sample')
     ap.add_argument('--no-cpu', action='store_true')
     ap.add_argument('--gemm', choices=('f32', 'bf16x3'), default='f32',
-                    help='products of the wide dense rules: FP32 matrix instructions (default) or the exact '
-                         'three-piece bf16 split on the bf16 matrix pipe')
+                    help='product mode; the wide layers of the workloads take exact three-piece bf16 splits with fp32 sums in both')
     ap.add_argument('--no-split-leg', action='store_true',
                     help='skip the short second measurement with --gemm bf16x3 that a default run appends')
     ap.add_argument('--no-other', action='store_true',
@@ -167,12 +166,19 @@ def roofline_of(dname, dkey, dn, dms, gemm):
     hbm = lambda nbytes, kernel: {'bound': 'hbm', 'achieved': nbytes / avg_s / 1e9, 'peak': PEAK_HBM_GBS, 'unit': 'GB/s',
                                   'frac': nbytes / avg_s / 1e9 / PEAK_HBM_GBS, 'traffic': None, 'kernel': kernel,
                                   'launches': dn, 'avg_launch_ms': dms / dn}
+    def pieces(rec):  # wide layers: six bf16 piece products per fp32 product, so the matrix pipe's bf16 peak over six
+        rec['peak'] = PEAK_BF16_MFMA_TFLOPS / 6.0
+        rec['frac'] = rec['achieved'] / rec['peak']
+        rec['peak_note'] = 'bf16 dense peak 2500 TFLOP/s / 6 exact piece products per fp32 product'
+        return rec
+
     if dname == 'dense_fwdlap':
         R, P, Kd, N, has_res = dkey
         if N == 1:  # matrix-vector form
             return hbm(4.0 * (P + 2) * R * (Kd + 1), f'dense_n1 kernels R={R} P={P} K={Kd}')
-        kern = (('dense_split_kernel' if gemm == 'bf16x3' and N > 128 else 'dense_dma_kernel')
-                if Kd % 16 == 0 and N % 4 == 0 else 'dense_kernel')
+        if Kd % 16 == 0 and N % 4 == 0 and N > 128 and (Kd >= 128 or not has_res):
+            return pieces(mfma(2.0 * (P + 2) * R * Kd * N, f'dense_pieces_kernel R={R} P={P} K={Kd} N={N} residual={has_res}'))
+        kern = 'dense_dma_kernel' if Kd % 16 == 0 and N % 4 == 0 else 'dense_kernel'
         return mfma(2.0 * (P + 2) * R * Kd * N, kern + f' R={R} P={P} K={Kd} N={N} residual={has_res}')
     if dname == 'mhsa_fwdlap':
         Bc, n, H, d, P = dkey
@@ -182,12 +188,11 @@ def roofline_of(dname, dkey, dn, dms, gemm):
         # plus short launches for the x / lap rows; the events bracket the whole entry point
         act, R, P, Kd, N = dkey
         norm = dname == 'norm_dense_fwdlap'
-        return mfma(2.0 * (P + 2) * R * Kd * N,
-                    f'dense_wide_kernel<{"true" if norm else "false"}, {"false" if act is None else "true"}, '
-                    f'{"32, false" if norm else "16 | 32, parts"}, {"true" if gemm == "bf16x3" else "false"}> '
-                    f'+ the short launches of its entry point '
-                    f'({dname}: x / lap rows GEMM, finish; with LayerNorm also weight fold and per-position rows), '
-                    f'act={act} R={R} P={P} K={Kd} N={N}')
+        return pieces(mfma(2.0 * (P + 2) * R * Kd * N,
+                           f'wide_pieces_kernel<8 | 4, {"true" if norm else "false"}, {"false" if act is None else "true"}> '
+                           f'+ the short launches of its entry point '
+                           f'({dname}: x / lap rows GEMM, finish; with LayerNorm also weight fold and per-position rows), '
+                           f'act={act} R={R} P={P} K={Kd} N={N}'))
     if dname == 'dense_act_fwdlap':
         act, R, P, Kd, N = dkey
         if P <= 6:  # layers in a row are one launch, on record by their shares of it: the triplets between them never move
@@ -434,6 +439,7 @@ def main():
             'chunk': args.chunk,
             'jacobian_rows': int(out.jacobian.dense_array.shape[0]),
             'gemm': args.gemm,
+            'products': 'fp32 operands of wide layers split exactly into three bf16 pieces, six exact piece products summed in fp32',
             'front_door': args.front_door,
         },
         'roofline': roof,
@@ -444,14 +450,8 @@ def main():
         roof['traffic_source'] = ('profiles/psiformer32_forward_laplacian.txt, table "HBM counters": rocprofv3 --pmc FETCH_SIZE / '
                                   'WRITE_SIZE of this command in earlier runs, summed over the launches of the entry point '
                                   '(counters cannot be read inside the timed run)')
-    if args.gemm == 'bf16x3' and roof is not None and roof['bound'] == 'mfma' and 'mhsa' not in roof['kernel']:
-        # six bf16 piece products per fp32 product: the matrix pipe's bf16 peak over six
-        roof['peak'] = PEAK_BF16_MFMA_TFLOPS / 6.0
-        roof['frac'] = roof['achieved'] / roof['peak']
-        roof['peak_note'] = 'bf16 dense peak 2500 TFLOP/s / 6 piece products per fp32 product'
     if args.gemm == 'f32' and not args.no_split_leg and not args.graph:
-        # the same step with the products of the wide dense rules on the bf16 pipe (three exact bf16
-        # pieces per operand): reported beside the headline, never as `value`
+        # the same step in the other product mode (the rules of this step take the same kernels in both)
         K.set_gemm_mode('bf16x3')
         out2 = None
         try:

@@ -25,9 +25,13 @@ SIGNATURES = {
     'folx_hip_get_gemm_mode': (c_int, []),
     'folx_hip_dense_fwdlap': (c_int, [_P] * 12 + [c_int64, c_int32, c_int32, c_int32]),
     'folx_hip_dense_rows_fwdlap': (c_int, [_P] * 12 + [c_int64, c_int32, c_int32, c_int32, c_int64, c_int64]),
+    'folx_hip_dense_workspace_bytes': (c_int64, [c_int32, c_int32]),
+    'folx_hip_dense_ws_fwdlap': (c_int, [_P] * 12 + [c_int64, c_int32, c_int32, c_int32, c_int64, c_int64, _P, c_int64]),
     'folx_hip_dense_act_workspace_bytes': (c_int64, [c_int64, c_int32, c_int32, c_int32]),
     'folx_hip_dense_act_form': (c_int, [c_int64, c_int32, c_int32, c_int32, c_int32]),
     'folx_hip_dense_act_faster': (c_int, [c_int64, c_int32, c_int32, c_int32, c_int32]),
+    'folx_hip_dense_act_pieces_bytes': (c_int64, [c_int64, c_int32, c_int32, c_int32]),
+    'folx_hip_dense_act_pieces_faster': (c_int, [c_int64, c_int32, c_int32, c_int32, c_int32]),
     'folx_hip_dense_form': (c_int, [c_int64, c_int32, c_int32, c_int32]),
     'folx_hip_dense_act_fwdlap': (c_int, [_P, c_int32, c_float] + [_P] * 11 + [c_int64, c_int32, c_int32, c_int32, _P, c_int64]),
     'folx_hip_dense_act_parts_fwdlap': (c_int, [_P, c_int32, c_float, _P, _P, c_int32, _P, _P, _P, c_int32] + [_P] * 11

@@ -74,8 +74,11 @@ __device__ __forceinline__ void store_tile(const floatx16 (&acc)[TM][TN], const 
                                            float* __restrict__ C, const float* __restrict__ Rs, int64_t rows,
                                            int32_t N, int64_t row0, int32_t col0, int wr, int wc, int l32,
                                            int lh) {
-  const bool full_tile = (row0 + BM <= rows) && (col0 + BN <= N);
-  if (full_tile) {
+  const int cols = N - col0 - wc;  // of this wavefront's first block and to the right of it
+  int whole = 0;                   // blocks of 32 columns that are there whole, and with all rows
+  if (row0 + BM <= rows && cols >= 32) {
+    whole = cols >= 32 * TN ? TN : cols / 32;
+    const int steps = 4 * whole;  // their groups of 8 rows
     const uint32_t voff = (uint32_t)((4 * lh * N + l32) * 4);
     float* cs = C + (row0 + wr) * (int64_t)N + col0 + wc;
     const float* rsb = HAS_RES ? Rs + (row0 + wr) * (int64_t)N + col0 + wc : nullptr;
@@ -92,44 +95,64 @@ __device__ __forceinline__ void store_tile(const floatx16 (&acc)[TM][TN], const 
         dst[r] = __builtin_nontemporal_load((const float*)(p + voff));
       }
     };
-    if constexpr (HAS_RES) fetch(0, rs[0]);
+    auto blocks = [&](auto all, auto stream) __attribute__((always_inline)) {
+      constexpr bool ALL = decltype(all)::value;
+      if constexpr (HAS_RES) fetch(0, rs[0]);
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+      for (int i = 0; i < TM; ++i) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
+        for (int j = 0; j < TN; ++j) {
+          if (!ALL && 4 * j >= steps) continue;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int step = (i * TN + j) * 4 + g;
-          if constexpr (HAS_RES)
-            if (step + 1 < TM * TN * 4) fetch(step + 1, rs[(step + 1) & 1]);
+          for (int g = 0; g < 4; ++g) {
+            const int step = (i * TN + j) * 4 + g;
+            if constexpr (HAS_RES)
+              if (step + 1 < TM * TN * 4 && (ALL || (step + 1) % (4 * TN) < steps)) fetch(step + 1, rs[(step + 1) & 1]);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            char* p = (char*)(cs + (int64_t)(i * 32 + 8 * g + r) * N + j * 32);
-            float o = acc[i][j][4 * g + r] + bvals[j];
-            if constexpr (HAS_RES) o += rs[step & 1][r];
-            __builtin_nontemporal_store(o, (float*)(p + voff));  // written once, read by a later launch
+            for (int r = 0; r < 4; ++r) {
+              char* p = (char*)(cs + (int64_t)(i * 32 + 8 * g + r) * N + j * 32);
+              float o = acc[i][j][4 * g + r] + bvals[j];
+              if constexpr (HAS_RES) o += rs[step & 1][r];
+              if constexpr (decltype(stream)::value) __builtin_nontemporal_store(o, (float*)(p + voff));
+              else *(float*)(p + voff) = o;
+            }
           }
         }
       }
+    };
+    // Written once and read by a later launch; but rows that do not end on a line share it with their neighbours, and pieces of a
+    // line are put together in the caches only if the stores may stay there (2 million rows of 200, K = 32: 898 -> 729 us).
+    if (N % 32 == 0) {
+      if (whole == TN) blocks(std::true_type{}, std::true_type{});
+      else blocks(std::false_type{}, std::true_type{});
+    } else {
+      if (whole == TN) blocks(std::true_type{}, std::false_type{});
+      else blocks(std::false_type{}, std::false_type{});
     }
-    return;
+    if (whole == TN) return;
   }
+  // Edge tiles: the skip connection of a block is asked for in one go in front of its stores.
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int gc = col0 + wc + j * 32 + l32;
-      const bool cok = gc < N;
-      if (cok) {
+      if (j < whole || gc >= N) continue;
+      const int64_t first = row0 + wr + i * 32 + 4 * lh;
+      const int left = (int)(rows - first < 32 ? rows - first : 32);
+      const int64_t at = first * (int64_t)N + gc;
+      float rs[16];
+      if constexpr (HAS_RES) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int64_t gr = row0 + wr + i * 32 + 8 * (r / 4) + 4 * lh + (r % 4);
-          if (gr < rows) {
-            float o = acc[i][j][r] + bvals[j];
-            if constexpr (HAS_RES) o += Rs[gr * (int64_t)N + gc];
-            C[gr * (int64_t)N + gc] = o;
-          }
+          const int row = 8 * (r / 4) + r % 4;
+          rs[r] = row < left ? Rs[at + (int64_t)row * N] : 0.0f;
         }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = 8 * (r / 4) + r % 4;
+        if (row < left) C[at + (int64_t)row * N] = acc[i][j][r] + bvals[j] + (HAS_RES ? rs[r] : 0.0f);
       }
     }
   }
@@ -616,6 +639,75 @@ __global__ __launch_bounds__(512, 4) void dense_split_kernel(Segs sg, const floa
                                       wr, wc, l32, lh);
 }
 
+// The pieces of W for the kernel below: a thread an octet of k of one column, zeros in the columns that pad the last block.
+__global__ __launch_bounds__(256) void split_weights_kernel(const float* __restrict__ W, char* __restrict__ pieces, int32_t K,
+                                                            int32_t N, int32_t blocks) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int32_t n = (int32_t)(i % (32 * blocks));
+  const int64_t octet = i / (32 * blocks);
+  if (octet >= K / 8) return;
+  float w[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) w[e] = n < N ? W[(octet * 8 + e) * N + n] : 0.0f;
+  folx_split::store_octet(w, pieces, (int32_t)octet, n, blocks);
+}
+
+// The rule on SplitTile (split_bf16.h): tiles of 128 rows x 32 CB columns on 4 wavefronts, the products on the bf16 matrix pipe
+// from operands split into three bf16 pieces each, those of W prepared or (FLY) formed here; KEEP: the first row tile
+// then writes them to `pieces`.  Same epilogue as the fp32 kernels.  Requires K % 16 == 0 and 16-byte aligned rows.
+template <int CB, bool HAS_RES, bool APART, bool FLY, bool KEEP>
+__global__ __launch_bounds__(256, 2) void dense_pieces_kernel(Segs sg, const float* __restrict__ W, char* pieces,
+                                                              const float* __restrict__ bias, int32_t K, int32_t N,
+                                                              int64_t row_tiles, int32_t col_tiles) {
+  using Tile = folx_split::SplitTile<CB, false, APART, FLY, KEEP>;
+  __shared__ __attribute__((aligned(16))) char ws0[Tile::STAGE];
+  __shared__ __attribute__((aligned(16))) char ws1[Tile::STAGE];
+
+  const int64_t id = blockIdx.x;
+  const int64_t xcd = id % NXCD;
+  const int64_t slot = id / NXCD;
+  const int64_t rt = (slot / col_tiles) * NXCD + xcd;
+  const int32_t ct = (int32_t)(slot % col_tiles);
+  if (rt >= row_tiles) return;
+  int seg = 0;
+  int64_t t = rt;
+  if (t >= sg.tiles[0]) { t -= sg.tiles[0]; seg = 1; if (t >= sg.tiles[1]) { t -= sg.tiles[1]; seg = 2; } }
+  const float* __restrict__ A = sg.in[seg];
+  const int64_t rows = sg.rows[seg];
+  const int64_t row0 = t * Tile::BM;
+  const int32_t col0 = ct * Tile::BN;
+
+  const int lane = threadIdx.x % 64;
+  const int wr = 32 * folx_wave_id();
+  const int l32 = lane % 32;
+  const int lh = lane / 32;
+
+  int64_t gr = row0 + wr + l32;
+  if (gr >= rows) gr = rows - 1;  // rows past the end: copies of the last one, never stored
+  const float* a_src = A + phys_row(sg, gr) * (int64_t)K + 8 * lh;
+  const int32_t blocks = (N + 31) / 32;
+
+  floatx16 acc[1][CB];
+  Tile::products(
+      acc, ws0, ws1, FLY && (!KEEP || rt > 0) ? nullptr : pieces + (int64_t)(col0 / 32) * 1024, blocks,
+      blocks - col0 / 32, K / 16, [](int) __attribute__((always_inline)) { return folx_split::zeros(); },
+      [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < CB; ++j) acc[0][j] = folx_split::zeros();
+      },
+      [&](int kt) __attribute__((always_inline)) { return a_src + kt * 16; },
+      [](int, const float4&, const float4&) __attribute__((always_inline)) {}, []() __attribute__((always_inline)) {},
+      W + col0, N, N - col0);
+  float bvals[CB];
+#pragma unroll
+  for (int j = 0; j < CB; ++j) {
+    const int gc = col0 + j * 32 + l32;
+    bvals[j] = (seg == 0 && bias != nullptr && gc < N) ? bias[gc] : 0.0f;
+  }
+  store_tile<Tile::BM, Tile::BN, 1, CB, HAS_RES>(acc, bvals, sg.out[seg], HAS_RES ? sg.res[seg] : nullptr, rows, N, row0,
+                                                 col0, wr, 0, l32, lh);
+}
+
 // N = 1 (a layer with one output per position, e.g. the last layer of a node-wise network): the
 // rule is a matrix-vector product, bound by reading the rows once.  A group of 32 lanes owns a
 // row at a time: 128-bit loads of up to 128 features per pass, the weights in registers, the
@@ -786,6 +878,36 @@ int launch_cfg(hipStream_t st, Segs& sg, const float* W, const float* bias, int3
   return folx_launch_status();
 }
 
+template <int CB, bool HAS_RES, bool APART, bool FLY, bool KEEP>
+int launch_tiles(hipStream_t st, Segs& sg, const float* W, char* pieces, const float* bias, int32_t K, int32_t N) {
+  int64_t row_tiles = 0;
+  for (int s = 0; s < 3; ++s) { sg.tiles[s] = (sg.rows[s] + 127) / 128; row_tiles += sg.tiles[s]; }
+  const int32_t col_tiles = (N + 32 * CB - 1) / (32 * CB);
+  const int64_t blocks = (row_tiles + NXCD - 1) / NXCD * NXCD * col_tiles;
+  if (blocks > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
+  dense_pieces_kernel<CB, HAS_RES, APART, FLY, KEEP><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(sg, W, pieces, bias, K, N, row_tiles,
+                                                                                             col_tiles);
+  return folx_launch_status();
+}
+
+int split_weights(hipStream_t st, const float* W, char* pieces, int32_t K, int32_t N) {
+  const int32_t blocks = (N + 31) / 32;
+  const int64_t grid = ((int64_t)K / 8 * 32 * blocks + 255) / 256;
+  if (grid > 0x7fffffffLL) return FOLX_HIP_ENOTSUP;
+  split_weights_kernel<<<dim3((unsigned)grid), dim3(256), 0, st>>>(W, pieces, K, N, blocks);
+  return folx_launch_status();
+}
+
+// From W itself where the launch is small (KEEP: `pieces` then holds those of W afterwards all the same), else its pieces first.
+template <bool HAS_RES, bool APART, bool KEEP>
+int launch_pieces(hipStream_t st, Segs& sg, const float* W, char* pieces, const float* bias, int32_t K, int32_t N) {
+  const int cb = folx_pieces_columns(sg.rows, K, N);
+  if (cb == 2) return launch_tiles<2, HAS_RES, APART, true, KEEP>(st, sg, W, pieces, bias, K, N);
+  if (cb == 4) return launch_tiles<4, HAS_RES, APART, true, KEEP>(st, sg, W, pieces, bias, K, N);
+  const int rc = split_weights(st, W, pieces, K, N);
+  return rc != FOLX_HIP_OK ? rc : launch_tiles<8, HAS_RES, APART, false, false>(st, sg, W, pieces, bias, K, N);
+}
+
 }  // namespace
 
 extern "C" int folx_hip_dense_form(int64_t R, int32_t P, int32_t K, int32_t N) {
@@ -797,11 +919,13 @@ extern "C" int folx_hip_dense_form(int64_t R, int32_t P, int32_t K, int32_t N) {
   return small ? 64 : 128;
 }
 
-extern "C" int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const float* jac,
-                                          const float* lap, const float* W, const float* bias,
-                                          const float* res, const float* res_jac, const float* res_lap,
-                                          float* y, float* y_jac, float* y_lap, int64_t R, int32_t P,
-                                          int32_t K, int32_t N, int64_t group, int64_t group_stride) {
+namespace {
+
+// The arguments of the rule as segments; FOLX_HIP_OK, or what the call returns instead (`done` for R = 0).
+int make_segs(Segs& sg, const float* x, const float* jac, const float* lap, const float* W, const float* res,
+              const float* res_jac, const float* res_lap, float* y, float* y_jac, float* y_lap, int64_t R, int32_t P, int32_t K,
+              int32_t N, int64_t group, int64_t group_stride, bool& done) {
+  done = true;
   if (R < 0 || P < 0 || K <= 0 || N <= 0 || group < 0 || (group > 0 && group_stride < group))
     return FOLX_HIP_EINVAL;
   if (R == 0) return FOLX_HIP_OK;
@@ -809,13 +933,27 @@ extern "C" int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const fl
   if (!x || !lap || !W || !y || !y_lap || (P > 0 && (!jac || !y_jac))) return FOLX_HIP_EINVAL;
   if ((res != nullptr) != (res_lap != nullptr) || (P > 0 && (res != nullptr) != (res_jac != nullptr)))
     return FOLX_HIP_EINVAL;
-  Segs sg;
   sg.res[0] = res; sg.res[1] = res_jac; sg.res[2] = res_lap;
   sg.in[0] = x; sg.in[1] = jac; sg.in[2] = lap;
   sg.out[0] = y; sg.out[1] = y_jac; sg.out[2] = y_lap;
   sg.rows[0] = R; sg.rows[1] = (int64_t)P * R; sg.rows[2] = R;
   sg.group = group; sg.gstride = group_stride;
   if (P == 0) { sg.in[1] = x; sg.out[1] = y; sg.res[1] = res; }  // never dereferenced: 0 tiles
+  done = false;
+  return FOLX_HIP_OK;
+}
+
+}  // namespace
+
+extern "C" int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const float* jac,
+                                          const float* lap, const float* W, const float* bias,
+                                          const float* res, const float* res_jac, const float* res_lap,
+                                          float* y, float* y_jac, float* y_lap, int64_t R, int32_t P,
+                                          int32_t K, int32_t N, int64_t group, int64_t group_stride) {
+  Segs sg;
+  bool done;
+  const int rc = make_segs(sg, x, jac, lap, W, res, res_jac, res_lap, y, y_jac, y_lap, R, P, K, N, group, group_stride, done);
+  if (done) return rc;
   const bool vec = (K % 4 == 0) && (N % 4 == 0) && folx_aligned16(x) && folx_aligned16(jac) &&
                    folx_aligned16(lap) && folx_aligned16(W);
   const bool has_res = res != nullptr;
@@ -843,6 +981,53 @@ extern "C" int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const fl
   if (N > 64) return launch_cfg<128, 128, 2, 2, 3>(st, sg, W, bias, K, N, vec, has_res);
   if (N > 32) return launch_cfg<128, 64, 4, 1, 3>(st, sg, W, bias, K, N, vec, has_res);
   return launch_cfg<128, 32, 4, 1, 3>(st, sg, W, bias, K, N, vec, has_res);
+}
+
+extern "C" int64_t folx_hip_dense_workspace_bytes(int32_t K, int32_t N) {
+  if (K <= 0 || N <= 0) return FOLX_HIP_EINVAL;
+  return K % BK == 0 && N > 128 && N % 4 == 0 ? folx_split::pieces_bytes(K, N) : 0;
+}
+
+extern "C" int folx_hip_dense_ws_fwdlap(void* stream, const float* x, const float* jac, const float* lap, const float* W,
+                                        const float* bias, const float* res, const float* res_jac, const float* res_lap,
+                                        float* y, float* y_jac, float* y_lap, int64_t R, int32_t P, int32_t K, int32_t N,
+                                        int64_t group, int64_t group_stride, void* workspace, int64_t workspace_bytes) {
+  Segs sg;
+  bool done;
+  const int rc = make_segs(sg, x, jac, lap, W, res, res_jac, res_lap, y, y_jac, y_lap, R, P, K, N, group, group_stride, done);
+  if (done) return rc;
+  const int64_t need = folx_hip_dense_workspace_bytes(K, N);
+  // With a skip connection the traffic of a short sum takes longer than its products on either pipe, and the fp32 kernels keep more
+  // wavefronts in flight (us, pieces / fp32: 409 600 rows, N = 160, K = 16 124 / 95, K = 64 168 / 155; 51 200, N = 256, K = 64
+  // 37 / 35, K = 128 46 / 50).
+  if (need == 0 || (res != nullptr && K < 128) || !folx_aligned16(x) || !folx_aligned16(jac) || !folx_aligned16(lap))
+    return folx_hip_dense_rows_fwdlap(stream, x, jac, lap, W, bias, res, res_jac, res_lap, y, y_jac, y_lap, R, P, K, N, group,
+                                      group_stride);
+  if (!workspace || workspace_bytes < need || !folx_aligned16(workspace)) return FOLX_HIP_EINVAL;
+  hipStream_t st = (hipStream_t)stream;
+  if (res != nullptr)
+    return K > folx_split::APART_K ? launch_pieces<true, true, false>(st, sg, W, (char*)workspace, bias, K, N)
+                                   : launch_pieces<true, false, false>(st, sg, W, (char*)workspace, bias, K, N);
+  return K > folx_split::APART_K ? launch_pieces<false, true, false>(st, sg, W, (char*)workspace, bias, K, N)
+                                 : launch_pieces<false, false, false>(st, sg, W, (char*)workspace, bias, K, N);
+}
+
+int folx_dense_values(hipStream_t st, const float* x, const float* lap, const float* W, char* pieces, const float* bias, float* y,
+                      float* y_lap, int64_t R, int32_t K, int32_t N) {
+  Segs sg;
+  sg.in[0] = sg.in[1] = x; sg.in[2] = lap;
+  sg.res[0] = sg.res[1] = sg.res[2] = nullptr;
+  sg.out[0] = sg.out[1] = y; sg.out[2] = y_lap;
+  sg.rows[0] = sg.rows[2] = R; sg.rows[1] = 0;
+  sg.group = sg.gstride = 0;
+  if (W != nullptr)
+    return K > folx_split::APART_K ? launch_pieces<false, true, true>(st, sg, W, pieces, bias, K, N)
+                                   : launch_pieces<false, false, true>(st, sg, W, pieces, bias, K, N);
+  switch (folx_pieces_columns(sg.rows, K, N)) {
+    case 8: return launch_tiles<8, false, false, false, false>(st, sg, W, pieces, bias, K, N);
+    case 4: return launch_tiles<4, false, false, false, false>(st, sg, W, pieces, bias, K, N);
+    default: return launch_tiles<2, false, false, false, false>(st, sg, W, pieces, bias, K, N);
+  }
 }
 
 extern "C" int folx_hip_dense_fwdlap(void* stream, const float* x, const float* jac,

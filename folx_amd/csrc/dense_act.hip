@@ -541,6 +541,18 @@ extern "C" int folx_hip_dense_act_form(int64_t R, int32_t P, int32_t K, int32_t 
   return folx_dense_act_wide_group(R, P, K, N);
 }
 
+extern "C" int64_t folx_hip_dense_act_pieces_bytes(int64_t R, int32_t P, int32_t K, int32_t N) {
+  if (R < 0 || P < 0 || K <= 0 || N <= 0) return FOLX_HIP_EINVAL;
+  DAPlan pl;
+  return plan_dense_act(R, P, K, N, pl) ? FOLX_HIP_ENOTSUP : folx_wide_pieces_ws_bytes(R, P, K, N);
+}
+
+extern "C" int folx_hip_dense_act_pieces_faster(int64_t R, int32_t P, int32_t K, int32_t N, int32_t plain_K) {
+  if (R < 0 || P < 0 || K <= 0 || N <= 0 || plain_K <= 0) return FOLX_HIP_EINVAL;
+  DAPlan pl;
+  return plan_dense_act(R, P, K, N, pl) ? FOLX_HIP_ENOTSUP : folx_wide_pieces_faster(R, P, K, N, plain_K);
+}
+
 extern "C" int folx_hip_dense_act_faster(int64_t R, int32_t P, int32_t K, int32_t N, int32_t plain_K) {
   DAPlan pl;
   if (R <= 0 || P < 0 || plain_K <= 0) return FOLX_HIP_EINVAL;

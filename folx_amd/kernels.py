@@ -122,11 +122,11 @@ class _timed_chain:
 
 
 def set_gemm_mode(mode: str):
-    """How the wide dense rules form their fp32 products: ``'f32'`` (FP32 matrix instructions, the
-    default) or ``'bf16x3'`` (operands split exactly into three bf16 pieces, six exact piece
-    products per product accumulated in fp32: same accuracy, the faster matrix pipe).  Process
-    wide; the environment variable ``FOLX_AMD_GEMM`` sets it when the library is loaded.  A HIP
-    graph captured by ``folx_amd.jit`` keeps the kernels of the mode it was captured under."""
+    """The product mode of the C entry points that take no workspace (``folx_hip_dense_fwdlap``): ``'f32'`` (FP32 matrix
+    instructions, the default) or ``'bf16x3'``.  The rules of this module bring a workspace, and take the products of wide layers
+    from operands split exactly into three bf16 pieces in either mode (six exact piece products per product accumulated in fp32,
+    with less rounding than the FP32 instructions).  Process wide; the environment variable ``FOLX_AMD_GEMM`` sets it when
+    the library is loaded."""
     if mode not in _lib.GEMM_MODE:
         raise ValueError(f'gemm mode {mode!r}: expected one of {sorted(_lib.GEMM_MODE)}')
     _lib.check(_lib.load().folx_hip_set_gemm_mode(_lib.GEMM_MODE[mode]), 'set_gemm_mode')
@@ -183,11 +183,14 @@ def dense(x, jac, lap, W, bias=None, res=None, row_slice=None):
     y = torch.empty((*lead, N), device=x.device, dtype=torch.float32)
     yj = torch.empty((P, *lead, N), device=x.device, dtype=torch.float32)
     yl = torch.empty_like(y)
+    lib = _lib.load()
+    nbytes = int(lib.folx_hip_dense_workspace_bytes(K, N))
+    ws = torch.empty(nbytes // 4, device=x.device, dtype=torch.float32) if nbytes > 0 else None
     with _timed('dense_fwdlap', (R, P, K, N, res is not None)):
         check(
-            _lib.load().folx_hip_dense_rows_fwdlap(
+            lib.folx_hip_dense_ws_fwdlap(
                 _stream(), xp, jp, lp, _p(W), _p(bias), _p(rx), _p(rj), _p(rl),
-                _p(y), _p(yj), _p(yl), R, P, K, N, group, gstride
+                _p(y), _p(yj), _p(yl), R, P, K, N, group, gstride, _p(ws), nbytes
             ),
             'dense_fwdlap',
         )
@@ -203,18 +206,27 @@ def dense_act_supported(name, K, N, rows=None, P=None, spared=None):
     (K, N <= 128), and wide ones (N > 128, K a multiple of 16) over a multiple of 4 rows.
     With ``P`` (Jacobian rows) given, also whether the wide kernel is expected to be faster than the plain product over
     ``spared`` features (the whole concatenation, where the fused form reads it in parts; else ``K``) and the activation
-    after it: the library knows the tiles of both (folx_hip_dense_act_faster)."""
+    after it: the library knows the tiles of both (folx_hip_dense_act_pieces_faster)."""
     if name not in FUSED_ACTS:
         return False
     if 4 <= K <= 128 and K % 4 == 0 and 1 <= N <= 128:
         return True
     return (rows is not None and rows > 0 and rows % 4 == 0 and K % 16 == 0 and N > 128 and N % 4 == 0
-            and (P is None or _lib.load().folx_hip_dense_act_faster(rows, P, K, N, spared or K) == 1))
+            and (P is None or _lib.load().folx_hip_dense_act_pieces_faster(rows, P, K, N, spared or K) == 1))
 
 
 def dense_act_residual_supported(K, N):
     """Layers whose fused kernel adds a skip connection in its epilogue (the narrow ones)."""
     return 4 <= K <= 128 and K % 4 == 0 and N <= 128
+
+
+def _dense_act_workspace(lib, R, P, K, N):
+    nbytes = int(lib.folx_hip_dense_act_pieces_bytes(R, P, K, N))  # wide layers
+    if nbytes < 0:
+        nbytes = int(lib.folx_hip_dense_act_workspace_bytes(R, P, K, N))
+        if nbytes < 0:
+            check(nbytes, 'dense_act_workspace_bytes')
+    return nbytes
 
 
 def dense_act(name, x, jac, lap, W, bias=None, param=0.0, res=None):
@@ -228,9 +240,7 @@ def dense_act(name, x, jac, lap, W, bias=None, param=0.0, res=None):
     lead = tuple(x.shape[:-1])
     R = int(math.prod(lead))
     lib = _lib.load()
-    nbytes = int(lib.folx_hip_dense_act_workspace_bytes(R, P, K, N))
-    if nbytes < 0:
-        check(nbytes, 'dense_act_workspace_bytes')
+    nbytes = _dense_act_workspace(lib, R, P, K, N)
     ws = torch.empty(nbytes // 4, device=x.device, dtype=torch.float32) if nbytes > 0 else None
     y = torch.empty((*lead, N), device=x.device, dtype=torch.float32)
     yj = torch.empty((P, *lead, N), device=x.device, dtype=torch.float32)
@@ -319,9 +329,7 @@ def dense_act_parts(name, x, lap, jac_parts, widths, broadcast, group, W, bias=N
         assert J.is_contiguous() and J.shape[0] == P and J.numel() == P * (R // group if bc else R) * w
     x, lap = x.contiguous(), lap.contiguous()
     lib = _lib.load()
-    nbytes = int(lib.folx_hip_dense_act_workspace_bytes(R, P, K, N))
-    if nbytes < 0:
-        check(nbytes, 'dense_act_workspace_bytes')
+    nbytes = _dense_act_workspace(lib, R, P, K, N)
     ws = torch.empty(max(nbytes // 4, 1), device=x.device, dtype=torch.float32)
     y = torch.empty((*lead, N), device=x.device, dtype=torch.float32)
     yj = torch.empty((P, *lead, N), device=x.device, dtype=torch.float32)

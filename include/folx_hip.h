@@ -31,8 +31,8 @@ extern "C" {
 #define FOLX_HIP_ELAUNCH (-3)  /* hipGetLastError() != hipSuccess after the launch     */
 #define FOLX_HIP_ESCRATCH (-4) /* needs more than FOLX_HIP_STATIC_SCRATCH_BYTES of scratch */
 
-/* Size of the library's own scratch array (folx_hip_norm_dense_static_fwdlap): 64 MiB of
- * device memory on every GPU the library has been used on, held until the process ends. */
+/* What folx_hip_norm_dense_workspace_bytes may say at most for folx_hip_norm_dense_static_fwdlap, whose scratch array is
+ * the library's own: this much and 33 MiB more of device memory on every GPU the library has been used on, held until the process ends. */
 #define FOLX_HIP_STATIC_SCRATCH_BYTES (64ll << 20)
 
 /* Library version (major * 10000 + minor * 100 + patch). */
@@ -43,17 +43,18 @@ const char* folx_hip_strerror(int code);
 /* How the wide dense rules (K % 16 == 0, N > 128, 16-byte aligned operands) form their fp32
  * products.  No counterpart in the reference, which leaves the choice to XLA
  * (jax.default_matmul_precision).
+ * With memory to prepare W's pieces in (folx_hip_dense_ws_fwdlap, folx_hip_norm_dense_fwdlap, and dense_act /
+ * dense_act_parts with folx_hip_dense_act_pieces_bytes of it) it is done alike in both modes: every operand element is split exactly into three bf16 pieces and a product
+ * is the sum of the six piece products of weight >= 2^-16, each exact, accumulated in fp32 on
+ * v_mfma_f32_32x32x16_bf16.  The dropped terms weigh <= 2^-24 of a product, the rounding of one fp32 multiply-add,
+ * and there are fewer roundings than with the fp32 instructions: against float64 the rms error is 0.4 to 0.85 of
+ * theirs.  Inputs, outputs and accumulators stay fp32.  Where an operand element is infinite or NaN, or rounds to a
+ * bf16 infinity (within 2^-9 of FLT_MAX), the rows it reaches are multiplied again with the fp32 instructions.
+ * Elements below 2^-109 keep the bits above 2^-133.
+ * Without (folx_hip_dense_fwdlap, folx_hip_dense_rows_fwdlap, the wide forms of dense_act with less workspace):
  *   FOLX_HIP_GEMM_F32    v_mfma_f32_32x32x2_f32 on the fp32 operands (the default).
- *   FOLX_HIP_GEMM_BF16X3 every operand element is split exactly into three bf16 pieces and a
- *                        product is the sum of the six piece products of weight >= 2^-16, each
- *                        exact, accumulated in fp32 on v_mfma_f32_32x32x16_bf16.  The dropped
- *                        terms weigh <= 2^-24 of a product, the rounding of one fp32
- *                        multiply-add, so results agree with the fp32 form to fp32 rounding;
- *                        inputs, outputs and accumulators stay fp32.  Kernels without a split
- *                        form run as under FOLX_HIP_GEMM_F32.  Where the two forms differ: an
- *                        infinite operand element (or one within 2^-9 of FLT_MAX, which rounds
- *                        to a bf16 infinity) gives NaN instead of an infinity, because its
- *                        remainder x - bf16(x) is inf - inf.
+ *   FOLX_HIP_GEMM_BF16X3 the split above in every workgroup; an infinite operand element gives NaN there instead of
+ *                        an infinity, because its remainder x - bf16(x) is inf - inf.
  * The mode is process wide and read at every launch; set it before launching, not while other
  * threads launch.  folx_hip_set_gemm_mode returns FOLX_HIP_EINVAL for any other value. */
 #define FOLX_HIP_GEMM_F32 0
@@ -145,6 +146,15 @@ int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const float* jac, c
                                float* y_lap, int64_t R, int32_t P, int32_t K, int32_t N,
                                int64_t group, int64_t group_stride);
 
+/* The same rule with a workspace of folx_hip_dense_workspace_bytes(K, N) bytes (16-byte aligned, device memory, not read on
+ * entry; 0: none is used and workspace may be NULL): wide layers (K % 16 == 0, N > 128, N % 4 == 0, operands 16-byte aligned)
+ * take their products from bf16 pieces in either product mode, W's prepared in the workspace. */
+int64_t folx_hip_dense_workspace_bytes(int32_t K, int32_t N);
+int folx_hip_dense_ws_fwdlap(void* stream, const float* x, const float* jac, const float* lap, const float* W,
+                             const float* bias, const float* res, const float* res_jac, const float* res_lap, float* y,
+                             float* y_jac, float* y_lap, int64_t R, int32_t P, int32_t K, int32_t N, int64_t group,
+                             int64_t group_stride, void* workspace, int64_t workspace_bytes);
+
 /*
  * Elementwise activation rule  y = f(x), y_jac[p] = f'(x) * jac[p],
  * y_lap = f'(x) * lap + f''(x) * sum_p jac[p]^2   in one pass over the Jacobian.
@@ -208,6 +218,8 @@ int folx_hip_dense_act_fwdlap(void* stream, int32_t act, float param, const floa
  * folx_hip_dense_act_faster: 1 where the fused rule is expected to be faster than
  * folx_hip_dense_fwdlap over plain_K features (K, or the whole concatenation whose parts the fused rule
  * reads) followed by folx_hip_elementwise_fwdlap, 0 where it is not.
+ * folx_hip_dense_act_pieces_faster: the same question for a wide layer with a workspace of folx_hip_dense_act_pieces_bytes
+ * against folx_hip_dense_ws_fwdlap, in either mode.
  * folx_hip_dense_form: rows of the tiles (64 or 128) that folx_hip_dense_fwdlap cuts 16-byte aligned operands with N > 64,
  * N % 4 == 0 and K % 16 == 0 into.
  * FOLX_HIP_ENOTSUP for shapes that the rule does not take (folx_hip_dense_form: for any other).
@@ -216,6 +228,10 @@ int folx_hip_dense_act_fwdlap(void* stream, int32_t act, float param, const floa
 #define FOLX_HIP_FORM_FEW 2
 int folx_hip_dense_act_form(int64_t R, int32_t P, int32_t K, int32_t N, int32_t has_res);
 int folx_hip_dense_act_faster(int64_t R, int32_t P, int32_t K, int32_t N, int32_t plain_K);
+int folx_hip_dense_act_pieces_faster(int64_t R, int32_t P, int32_t K, int32_t N, int32_t plain_K);
+/* Bytes of workspace with which folx_hip_dense_act_fwdlap and folx_hip_dense_act_parts_fwdlap take a wide layer's products from
+ * bf16 pieces (see folx_hip_set_gemm_mode); FOLX_HIP_ENOTSUP for a narrow layer and for shapes the rule does not take. */
+int64_t folx_hip_dense_act_pieces_bytes(int64_t R, int32_t P, int32_t K, int32_t N);
 int folx_hip_dense_form(int64_t R, int32_t P, int32_t K, int32_t N);
 
 /*
