@@ -176,7 +176,7 @@ def roofline_of(dname, dkey, dn, dms, gemm):
         R, P, Kd, N, has_res = dkey
         if N == 1:  # matrix-vector form
             return hbm(4.0 * (P + 2) * R * (Kd + 1), f'dense_n1 kernels R={R} P={P} K={Kd}')
-        if Kd % 16 == 0 and N % 4 == 0 and N > 128 and (Kd >= 128 or not has_res):
+        if Kd % 16 == 0 and N % 4 == 0 and (N > 128 and (Kd >= 128 or not has_res) or N > 32 and Kd > 128):
             return pieces(mfma(2.0 * (P + 2) * R * Kd * N, f'dense_pieces_kernel R={R} P={P} K={Kd} N={N} residual={has_res}'))
         kern = 'dense_dma_kernel' if Kd % 16 == 0 and N % 4 == 0 else 'dense_kernel'
         return mfma(2.0 * (P + 2) * R * Kd * N, kern + f' R={R} P={P} K={Kd} N={N} residual={has_res}')

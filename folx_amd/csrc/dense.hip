@@ -983,9 +983,12 @@ extern "C" int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const fl
   return launch_cfg<128, 32, 4, 1, 3>(st, sg, W, bias, K, N, vec, has_res);
 }
 
+// Wide layers; and those of more than 32 columns with sums that are long enough to be bound by the matrix pipe, which no fused narrow
+// kernel takes (us, fp32 -> pieces: 1.6 million rows, K = 256, N = 128 958 -> 734, N = 80 914 -> 700, N = 48 551 -> 487; 152 000 rows, K = 256,
+// N = 112 109 -> 76, N = 64 56 -> 48; 19 000 rows: the same).
 extern "C" int64_t folx_hip_dense_workspace_bytes(int32_t K, int32_t N) {
   if (K <= 0 || N <= 0) return FOLX_HIP_EINVAL;
-  return K % BK == 0 && N > 128 && N % 4 == 0 ? folx_split::pieces_bytes(K, N) : 0;
+  return K % BK == 0 && (N > 128 || (N > 32 && K > 128)) && N % 4 == 0 ? folx_split::pieces_bytes(K, N) : 0;
 }
 
 extern "C" int folx_hip_dense_ws_fwdlap(void* stream, const float* x, const float* jac, const float* lap, const float* W,

@@ -147,7 +147,7 @@ int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const float* jac, c
                                int64_t group, int64_t group_stride);
 
 /* The same rule with a workspace of folx_hip_dense_workspace_bytes(K, N) bytes (16-byte aligned, device memory, not read on
- * entry; 0: none is used and workspace may be NULL): wide layers (K % 16 == 0, N > 128, N % 4 == 0, operands 16-byte aligned)
+ * entry; 0: none is used and workspace may be NULL): layers with K % 16 == 0, N % 4 == 0 and N > 128, or N > 32 and K > 128, operands 16-byte aligned,
  * take their products from bf16 pieces in either product mode, W's prepared in the workspace. */
 int64_t folx_hip_dense_workspace_bytes(int32_t K, int32_t N);
 int folx_hip_dense_ws_fwdlap(void* stream, const float* x, const float* jac, const float* lap, const float* W,
