@@ -25,7 +25,7 @@ SIGNATURES = {
     'folx_hip_get_gemm_mode': (c_int, []),
     'folx_hip_dense_fwdlap': (c_int, [_P] * 12 + [c_int64, c_int32, c_int32, c_int32]),
     'folx_hip_dense_rows_fwdlap': (c_int, [_P] * 12 + [c_int64, c_int32, c_int32, c_int32, c_int64, c_int64]),
-    'folx_hip_dense_workspace_bytes': (c_int64, [c_int32, c_int32]),
+    'folx_hip_dense_workspace_bytes': (c_int64, [c_int64, c_int32, c_int32, c_int32]),
     'folx_hip_dense_ws_fwdlap': (c_int, [_P] * 12 + [c_int64, c_int32, c_int32, c_int32, c_int64, c_int64, _P, c_int64]),
     'folx_hip_dense_act_workspace_bytes': (c_int64, [c_int64, c_int32, c_int32, c_int32]),
     'folx_hip_dense_act_form': (c_int, [c_int64, c_int32, c_int32, c_int32, c_int32]),

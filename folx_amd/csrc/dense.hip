@@ -986,9 +986,14 @@ extern "C" int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const fl
 // Wide layers; and those of more than 32 columns with sums that are long enough to be bound by the matrix pipe, which no fused narrow
 // kernel takes (us, fp32 -> pieces: 1.6 million rows, K = 256, N = 128 958 -> 734, N = 80 914 -> 700, N = 48 551 -> 487; 152 000 rows, K = 256,
 // N = 112 109 -> 76, N = 64 56 -> 48; 19 000 rows: the same).
-extern "C" int64_t folx_hip_dense_workspace_bytes(int32_t K, int32_t N) {
-  if (K <= 0 || N <= 0) return FOLX_HIP_EINVAL;
-  return K % BK == 0 && (N > 128 || (N > 32 && K > 128)) && N % 4 == 0 ? folx_split::pieces_bytes(K, N) : 0;
+static bool takes_pieces(int32_t K, int32_t N) {
+  return K % BK == 0 && (N > 128 || (N > 32 && K > 128)) && N % 4 == 0;
+}
+
+extern "C" int64_t folx_hip_dense_workspace_bytes(int64_t R, int32_t P, int32_t K, int32_t N) {
+  if (R < 0 || P < 0 || K <= 0 || N <= 0) return FOLX_HIP_EINVAL;
+  const int64_t rows[3] = {R, P * R, R};
+  return takes_pieces(K, N) && folx_pieces_columns(rows, K, N) == 8 ? folx_split::pieces_bytes(K, N) : 0;
 }
 
 extern "C" int folx_hip_dense_ws_fwdlap(void* stream, const float* x, const float* jac, const float* lap, const float* W,
@@ -999,14 +1004,14 @@ extern "C" int folx_hip_dense_ws_fwdlap(void* stream, const float* x, const floa
   bool done;
   const int rc = make_segs(sg, x, jac, lap, W, res, res_jac, res_lap, y, y_jac, y_lap, R, P, K, N, group, group_stride, done);
   if (done) return rc;
-  const int64_t need = folx_hip_dense_workspace_bytes(K, N);
   // With a skip connection the traffic of a short sum takes longer than its products on either pipe, and the fp32 kernels keep more
   // wavefronts in flight (us, pieces / fp32: 409 600 rows, N = 160, K = 16 124 / 95, K = 64 168 / 155; 51 200, N = 256, K = 64
   // 37 / 35, K = 128 46 / 50).
-  if (need == 0 || (res != nullptr && K < 128) || !folx_aligned16(x) || !folx_aligned16(jac) || !folx_aligned16(lap))
+  if (!takes_pieces(K, N) || (res != nullptr && K < 128) || !folx_aligned16(x) || !folx_aligned16(jac) || !folx_aligned16(lap))
     return folx_hip_dense_rows_fwdlap(stream, x, jac, lap, W, bias, res, res_jac, res_lap, y, y_jac, y_lap, R, P, K, N, group,
                                       group_stride);
-  if (!workspace || workspace_bytes < need || !folx_aligned16(workspace)) return FOLX_HIP_EINVAL;
+  const int64_t need = folx_hip_dense_workspace_bytes(R, P, K, N);
+  if (need > 0 && (!workspace || workspace_bytes < need || !folx_aligned16(workspace))) return FOLX_HIP_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   if (res != nullptr)
     return K > folx_split::APART_K ? launch_pieces<true, true, false>(st, sg, W, (char*)workspace, bias, K, N)

@@ -8,6 +8,7 @@ contiguous and on the GPU.  Layout: x (B, *s), jac (P, B, *s), lap (B, *s).
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import numpy as np
@@ -158,6 +159,27 @@ def _dims(*vals):
     return (ctypes.c_int64 * len(vals))(*[int(v) for v in vals])
 
 
+# What the library says about a shape, whatever the product mode: asked for once per shape, not once per call.
+@functools.lru_cache(maxsize=1024)
+def _dense_workspace(R, P, K, N):
+    return int(_lib.load().folx_hip_dense_workspace_bytes(R, P, K, N))
+
+
+@functools.lru_cache(maxsize=1024)
+def _dense_act_pieces(R, P, K, N):
+    return int(_lib.load().folx_hip_dense_act_pieces_bytes(R, P, K, N))
+
+
+@functools.lru_cache(maxsize=1024)
+def _dense_act_pieces_faster(R, P, K, N, plain):
+    return _lib.load().folx_hip_dense_act_pieces_faster(R, P, K, N, plain) == 1
+
+
+@functools.lru_cache(maxsize=1024)
+def _norm_dense_workspace(R, P, K, N, act):
+    return int(_lib.load().folx_hip_norm_dense_workspace_bytes(R, P, K, N, act))
+
+
 def dense(x, jac, lap, W, bias=None, res=None, row_slice=None):
     """x (.., K), jac (P, .., K), lap (.., K), W (K, N) -> triplet with last dim N.
     ``res`` = optional (x, jac, lap) residual triplet of the output shape, added in the
@@ -184,7 +206,7 @@ def dense(x, jac, lap, W, bias=None, res=None, row_slice=None):
     yj = torch.empty((P, *lead, N), device=x.device, dtype=torch.float32)
     yl = torch.empty_like(y)
     lib = _lib.load()
-    nbytes = int(lib.folx_hip_dense_workspace_bytes(K, N))
+    nbytes = _dense_workspace(R, P, K, N)
     ws = torch.empty(nbytes // 4, device=x.device, dtype=torch.float32) if nbytes > 0 else None
     with _timed('dense_fwdlap', (R, P, K, N, res is not None)):
         check(
@@ -212,7 +234,7 @@ def dense_act_supported(name, K, N, rows=None, P=None, spared=None):
     if 4 <= K <= 128 and K % 4 == 0 and 1 <= N <= 128:
         return True
     return (rows is not None and rows > 0 and rows % 4 == 0 and K % 16 == 0 and N > 128 and N % 4 == 0
-            and (P is None or _lib.load().folx_hip_dense_act_pieces_faster(rows, P, K, N, spared or K) == 1))
+            and (P is None or _dense_act_pieces_faster(rows, P, K, N, spared or K)))
 
 
 def dense_act_residual_supported(K, N):
@@ -221,7 +243,7 @@ def dense_act_residual_supported(K, N):
 
 
 def _dense_act_workspace(lib, R, P, K, N):
-    nbytes = int(lib.folx_hip_dense_act_pieces_bytes(R, P, K, N))  # wide layers
+    nbytes = _dense_act_pieces(R, P, K, N)  # wide layers
     if nbytes < 0:
         nbytes = int(lib.folx_hip_dense_act_workspace_bytes(R, P, K, N))
         if nbytes < 0:
@@ -374,7 +396,7 @@ def norm_dense(name, x, jac, lap, gamma, beta, eps, W, bias=None, param=0.0):
     R = int(math.prod(lead))
     act = -1 if name is None else ACT[name]
     lib = _lib.load()
-    nbytes = int(lib.folx_hip_norm_dense_workspace_bytes(R, P, K, N, act))
+    nbytes = _norm_dense_workspace(R, P, K, N, act)
     if nbytes < 0:
         check(nbytes, 'norm_dense_workspace_bytes')
     ws = torch.empty(nbytes // 4, device=x.device, dtype=torch.float32)

@@ -146,10 +146,10 @@ int folx_hip_dense_rows_fwdlap(void* stream, const float* x, const float* jac, c
                                float* y_lap, int64_t R, int32_t P, int32_t K, int32_t N,
                                int64_t group, int64_t group_stride);
 
-/* The same rule with a workspace of folx_hip_dense_workspace_bytes(K, N) bytes (16-byte aligned, device memory, not read on
+/* The same rule with a workspace of folx_hip_dense_workspace_bytes(R, P, K, N) bytes (16-byte aligned, device memory, not read on
  * entry; 0: none is used and workspace may be NULL): layers with K % 16 == 0, N % 4 == 0 and N > 128, or N > 32 and K > 128, operands 16-byte aligned,
- * take their products from bf16 pieces in either product mode, W's prepared in the workspace. */
-int64_t folx_hip_dense_workspace_bytes(int32_t K, int32_t N);
+ * take their products from bf16 pieces in either product mode, W's prepared in the workspace (small calls: none). */
+int64_t folx_hip_dense_workspace_bytes(int64_t R, int32_t P, int32_t K, int32_t N);
 int folx_hip_dense_ws_fwdlap(void* stream, const float* x, const float* jac, const float* lap, const float* W,
                              const float* bias, const float* res, const float* res_jac, const float* res_lap, float* y,
                              float* y_jac, float* y_lap, int64_t R, int32_t P, int32_t K, int32_t N, int64_t group,
