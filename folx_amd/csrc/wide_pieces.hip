@@ -23,10 +23,10 @@
 // a_p, b_p and mean(t_p^2) are summed from the A tile while it feeds the MFMAs.
 //
 // Launches on the caller's stream:
-//  1. (LayerNorm only) fold gamma / beta into the weights (Wg, w1, c0 = bias + beta @ W), and
-//     one wavefront per position for xh, rs, LN(x) and the linear part of LN's lap row;
-//  2. the plain dense kernel on the x and lap rows only (2 R of the (P + 2) R rows): z goes to
-//     y, the linear part of zl to y_lap;
+//  1. (LayerNorm only) fold gamma / beta into the weights (the pieces of Wg, w1, c0 = bias + beta @ W), and
+//     one wavefront per position for xh, rs and the linear part of LN's lap row before gamma;
+//  2. the plain dense kernel on the x and lap rows only (2 R of the (P + 2) R rows; xh @ Wg + c0 behind LayerNorm): z goes to
+//     y, the linear part of zl to y_lap; without LayerNorm it leaves the pieces of W as well;
 //  3. the Jacobian GEMM below, whose 128-row tiles are cut ACROSS Jacobian rows: a tile holds
 //     4 consecutive positions x 32 consecutive p, ordered position-major, so that each 32 x 32
 //     accumulator block belongs to ONE position.  f'(z), w1, w2 and rs of a block are then one
@@ -40,12 +40,14 @@
 // share) and adds a skip connection in its epilogue, so that a layer fed by
 // [own features, per-walker means, ...] forms neither the broadcasts nor the concatenation.
 //
-// The main loop is the one of the dense kernel: K in chunks of 16 through double-buffered LDS
-// tiles filled by global_load_lds_dwordx4, a 128 x 256 tile on 8 wavefronts of 64 x 64,
-// v_mfma_f32_32x32x2_f32 with the k order inside a group of 8 permuted to fit 128-bit reads
-// (lane l, register j of group t <-> k = 8 t + 4 (l / 32) + j), piece c of an A row stored at
-// slot c ^ ((row / 2) % 4).  Only the address a lane asks for differs: tile row m is
-// Jacobian row p0 + m % 32 of position r0 + m / 32.
+// The products are SplitTile's (split_bf16.h), a wavefront's 32 rows one position (32 Jacobian rows), two or four; what the epilogue
+// needs per position and column (z - c0, f'(z)) waits in LDS.
+//
+// What bounds it: the power cap, as for the plain product; beyond that, us for K = N = 256, P = 96, 32 768 positions: 2700 behind LayerNorm and
+// 2780 with tanh as well against 2330 plain (the row sums and the rank-2 correction are as many vector instructions as the split of A;
+// with the fp32 instructions 3670 and 3760).  Read in parts, K = 320, P = 48 in groups of 16, 16 384 positions: 1300 -> 990.
+// What the accumulators start from (the per-walker term) has to be put together block by block, and the loop to exist once: the registers
+// of two would be spilled (29 -> 25 ms for the whole of such a model).
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -513,8 +515,8 @@ __device__ __forceinline__ void norm_rows(const float* __restrict__ x, const flo
 
 // Both in one launch, the blocks of the weights first: neither reads what the other writes.  K = N = 256: 16.5 us for the weights
 // (64 columns a block, 16 requests in a row each) and 4.9 us for the rows of 640 positions, each its own launch, became 6 us.
-// The fused form is the one for any number of positions, also where LayerNorm and a product with 64 x 64 tiles would be faster (us, fused
-// / the two rules, K = N = 256: P = 30, R = 64 56 / 16, 640 62 / 41, 1920 102 / 98; P = 96, R = 64 56 / 28): the two round differently, and a
+// The fused form is the one for any number of positions, also where LayerNorm and the plain product would be faster (P R < 30 000: 1.4 times
+// in the mean over 77 sizes): the two round differently, and a
 // walker's Jacobian then depended on how many walkers a call has, by up to 1.5e-3 of it behind a determinant of 20 electrons.
 __global__ __launch_bounds__(256) void norm_prepare_kernel(const float* x, const float* lap, const float* W, const float* bias,
                                                            const float* gamma, const float* beta, float* xhat, float* rs,
