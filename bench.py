@@ -169,6 +169,7 @@ def roofline_of(dname, dkey, dn, dms, gemm):
     def pieces(rec):  # wide layers: six bf16 piece products per fp32 product, so the matrix pipe's bf16 peak over six
         rec['peak'] = PEAK_BF16_MFMA_TFLOPS / 6.0
         rec['frac'] = rec['achieved'] / rec['peak']
+        rec['traffic'] = None  # counted for the fp32 kernels only
         rec['peak_note'] = 'bf16 dense peak 2500 TFLOP/s / 6 exact piece products per fp32 product'
         return rec
 
